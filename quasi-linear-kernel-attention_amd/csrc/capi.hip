@@ -454,6 +454,83 @@ int run_pipeline(int P, const Plan& pl, void* ws, size_t copy, hipStream_t st, P
     return w == hipSuccess ? QLKA_OK : hip_status((int)w, "join");
 }
 
+// ---- the forward sums column by column (col.hip): sort k and q, merge them into the stream the columns walk, the column
+// sums, and the finish that turns columns into rows (with the v == 1 terms and, for a layer, its epilogue). Segments of
+// N + M <= COL_MAX elements take it whatever the dense cutoff leaves; longer ones walk ranges of keys into a slab of
+// contribution rows. Measured against that walk on MI355X: see col.hip.
+// The chunks run in order on the caller's stream: the sums keep every CU's LDS, so nothing would run beside them. Its
+// workspace is smaller than the walk's but for many more keys than queries, where the *_ws_bytes queries return the
+// larger of the two.
+struct ColWs { SortedWs s; ColStream str; float* u; float* cols; float* wt; char* extra; };
+
+size_t col_part(const ColPlan& pl, int P, int D, int N, int M, int C, int i) {
+    const size_t S = (size_t)P * D;
+    switch (i) {
+        case 0: case 1: return align256(S * N * 4);
+        case 2: case 3: return align256(S * M * 4);
+        case 4: return align256(sort_scratch_need(WsSpec{P, D, N, M, C, N, 0, false}));
+        case 5: return align256(col_stream_bytes(pl, (int)S));
+        case 6: return align256(S * M * 4);
+        case 7: return align256((size_t)P * pl.DS * C * M * 4);
+        case 8: return align256((size_t)P * C * N * 4);
+    }
+    return 0;
+}
+
+constexpr int COL_PARTS = 9;
+
+// Workspace of a chunk of P p, the columns sized for the most feature shares: their number depends on the whole call's P,
+// and neither the sizes nor (the plan being the whole call's) the results may depend on the chunking.
+size_t col_bytes(int kind, int P, int D, int N, int M, int C) {
+    if (!col_applies(D, N, M)) return 0;
+    ColPlan pl = col_plan(kind, 1, D, N, M, C);
+    pl.DS = std::min(D, COL_SHARES);
+    size_t b = 0;
+    for (int i = 0; i < COL_PARTS; ++i) b += col_part(pl, P, D, N, M, C, i);
+    return b;
+}
+
+ColWs col_carve(ColPlan pl, void* ws, int P, int D, int N, int M, int C) {
+    pl.DS = std::min(D, COL_SHARES);
+    char* part[COL_PARTS];
+    char* b = (char*)ws;
+    for (int i = 0; i < COL_PARTS; ++i) { part[i] = b; b += col_part(pl, P, D, N, M, C, i); }
+    ColWs r{};
+    r.s.ks = (float*)part[0]; r.s.kp = (uint32_t*)part[1]; r.s.qs = (float*)part[2]; r.s.qp = (uint32_t*)part[3];
+    r.s.sort_scratch = part[4];
+    r.str = col_stream(pl, part[5], P * D);
+    r.u = (float*)part[6];
+    r.cols = (float*)part[7];
+    r.wt = (float*)part[8];
+    r.extra = b;
+    return r;
+}
+
+// sort(p0, np, w, stream) leaves the sorted k and q in w.s; finish(p0, np, w, plan, stream) reads w.cols and w.u (null
+// without want_u). extra(np): bytes of the caller's own after the columns (w.extra).
+template <class Extra, class Sort, class Finish>
+int run_columns(int kind, const float* v, const uint8_t* keep, bool want_u, int P, int D, int N, int M, int C, void* ws,
+                size_t given, hipStream_t st, Extra extra, Sort sort, Finish finish) {
+    const ColPlan pl = col_plan(kind, P, D, N, M, C);
+    auto bytes = [&](int pc) { return col_bytes(kind, pc, D, N, M, C) + extra(pc); };
+    const int pc = fit_chunk(P, given, bytes);
+    if (int e = check_ws(ws, given, bytes(pc))) return e;
+    return for_chunks(P, pc, [&](int p0, int np) {
+        ColWs w = col_carve(pl, ws, np, D, N, M, C);
+        if (!want_u) w.u = nullptr;
+        const size_t p = (size_t)p0;
+        if (int e = sort(p0, np, w, st)) return e;
+        const uint8_t* kc = keep ? keep + p * N : nullptr;
+        if (int e = col_merge_launch(kind, pl, w.s.qs, w.s.qp, w.s.ks, w.s.kp, kc, w.str, w.u, np * D, D, N, M, st))
+            return hip_status(e, "merge of q and k");
+        if (int e = col_weights_launch(v + p * N * C, kc, w.wt, np, N, C, st)) return hip_status(e, "weight columns");
+        if (int e = col_sum_launch(kind, pl, w.str, w.wt, w.cols, np, D, N, M, C, st))
+            return hip_status(e, "column sums");
+        return finish(p0, np, w, pl, st); });
+}
+
+inline size_t no_extra(int) { return 0; }
+
 }  // namespace
 
 extern "C" {
@@ -473,10 +550,15 @@ size_t qlka_set_workspace_budget(size_t bytes) { return g_ws_budget.exchange(byt
 // ------------------------------------------------------------------------------------------------ laplace forward
 static WsSpec laplace_spec(int P, int D, int N, int M, int C) { return WsSpec{P, D, N, M, C, N, M, true}; }
 
+// one chunk of P p, by columns or by ranges
+static size_t laplace_ws(int P, int D, int N, int M, int C) {
+    return std::max(ws_bytes(laplace_spec(P, D, N, M, C)), col_bytes(1, P, D, N, M, C));
+}
+
 size_t qlka_laplace_fwd_ws_bytes(int P, int D, int N, int M, int C) {
     if (P <= 0 || D <= 0 || N <= 0 || M <= 0 || C <= 0) return 0;
     if (dense_laplace_fwd(N, M)) return 0;        // the dense route takes no workspace
-    auto b1 = [&](int pc) { return ws_bytes(laplace_spec(pc, D, N, M, C)); };
+    auto b1 = [&](int pc) { return laplace_ws(pc, D, N, M, C); };
     return plan_bytes(plan_chunks(P, g_ws_budget.load(std::memory_order_relaxed), pipelined(P, D, M), b1), b1);
 }
 
@@ -488,9 +570,18 @@ int qlka_laplace_fwd(const float* q, const float* k, const float* v, float* out_
     hipStream_t st = (hipStream_t)stream;
     if (dense_laplace_fwd(N, M))
         return hip_status(direct_fwd(1, q, k, v, out_w, out_u, P, D, N, M, C, st), "laplace direct sum");
-    auto b1 = [&](int pc) { return ws_bytes(laplace_spec(pc, D, N, M, C)); };
+    auto b1 = [&](int pc) { return laplace_ws(pc, D, N, M, C); };
     const Plan pl = plan_chunks(P, ws_bytes_given, pipelined(P, D, M), b1);
     if (int e = check_ws(ws, ws_bytes_given, plan_bytes(pl, b1))) return e;
+    if (col_applies(D, N, M))
+        return run_columns(1, v, nullptr, true, P, D, N, M, C, ws, ws_bytes_given, st, no_extra,
+            [&](int p0, int np, ColWs& w, hipStream_t s) {
+                const size_t p = (size_t)p0;
+                return sort_both(q + p * D * M, k + p * D * N, w.s, np * D, N, M, s); },
+            [&](int p0, int np, ColWs& w, const ColPlan& cp, hipStream_t s) {
+                const size_t p = (size_t)p0;
+                return hip_status(col_finish_launch(1, -1, false, cp, w.cols, w.u, out_w + p * M * C, out_u + p * M,
+                                                    ReduceEpilogue{}, np, D, M, C, s), "columns to rows"); });
     // per chunk: sort k and group q; range passes and walk; reduce
     auto prep = [&](int p0, int np, void* buf, hipStream_t s) {
         SortedWs w = carve(buf, laplace_spec(np, D, N, M, C));
@@ -530,10 +621,14 @@ static size_t abs_dense_ws(int P, int pc, int D, int N, int M, int C) {
     return dense_sign(P, N, M) ? 0 : align256(sort_scratch_need(abs_fwd_spec(pc, D, N, M, C, true)));
 }
 
+static size_t abs_fwd_ws(int P, int D, int N, int M, int C) {
+    return std::max(ws_bytes(abs_fwd_spec(P, D, N, M, C, true)), col_bytes(0, P, D, N, M, C));
+}
+
 size_t qlka_abs_fwd_ws_bytes(int P, int D, int N, int M, int C) {
     if (P <= 0 || D <= 0 || N <= 0 || M <= 0 || C <= 0) return 0;
     if (dense_abs_fwd(N, M)) return budget_bytes(P, [&](int pc) { return abs_dense_ws(P, pc, D, N, M, C); });
-    auto b1 = [&](int pc) { return ws_bytes(abs_fwd_spec(pc, D, N, M, C, true)); };
+    auto b1 = [&](int pc) { return abs_fwd_ws(pc, D, N, M, C); };
     return plan_bytes(plan_chunks(P, g_ws_budget.load(std::memory_order_relaxed), pipelined(P, D, M), b1), b1);
 }
 
@@ -604,9 +699,27 @@ int abs_fwd_impl(const float* q, const float* k, const float* v, float* out_w, f
         return hip_status(direct_fwd(0, q, k, v, out_w, out_u, P, D, N, M, C, st), "abs direct sum");
     }
     // the workspace is sized for the _full op (an upper bound of the plain one), so one size serves both
-    auto b1 = [&](int pc) { return ws_bytes(abs_fwd_spec(pc, D, N, M, C, true)); };
+    auto b1 = [&](int pc) { return abs_fwd_ws(pc, D, N, M, C); };
     const Plan pl = plan_chunks(P, ws_bytes_given, pipelined(P, D, M), b1);
     if (int e = check_ws(ws, ws_bytes_given, plan_bytes(pl, b1))) return e;
+    if (col_applies(D, N, M) && !keep_states) {
+        const int e = run_columns(0, v, nullptr, out_u != nullptr, P, D, N, M, C, ws, ws_bytes_given, st, no_extra,
+            [&](int p0, int np, ColWs& w, hipStream_t s) {
+                const size_t p = (size_t)p0;
+                if (keep_sorts) {
+                    const Presorted ks = offset(*keep, p, D, N, M);
+                    w.s.ks = ks.ks; w.s.kp = ks.kp; w.s.qs = ks.qs; w.s.qp = ks.qp;
+                }
+                return sort_both(q + p * D * M, k + p * D * N, w.s, np * D, N, M, s); },
+            [&](int p0, int np, ColWs& w, const ColPlan& cp, hipStream_t s) {
+                const size_t p = (size_t)p0;
+                return hip_status(col_finish_launch(0, -1, false, cp, w.cols, w.u, out_w + p * M * C,
+                                                    out_u ? out_u + p * M : nullptr, ReduceEpilogue{}, np, D, M, C, s),
+                                  "columns to rows"); });
+        if (e) return e;
+        if (keep_sorts) *kept = 1;
+        return QLKA_OK;
+    }
     const int mode = out_u ? (ABS_ROW | ABS_ONES) : ABS_ROW;
     // the chunk's workspace view, with the sorted arrays in the caller's buffers when the sorts are kept
     auto view = [&](int p0, int np, void* buf, SortedWs& w, AbsWalkArgs& a) {
@@ -1098,9 +1211,26 @@ static bool layer_pipelined(int kind, int P, int D, int M, int C) {
     return (kind != LAYER_ADD_BUMP || reduce_folds_epilogue(M, C)) && pipelined(P, D, M);
 }
 
+// add_laplace / add_riesz by columns: the op's columns with the layer's epilogue in their finish. Masked keys weigh 0;
+// their sort values are replaced as for the walks (mask_keys, fill_masked_keys), so that whatever they hold, the distances
+// run between kept keys.
+static size_t layer_col_extra(int kind, int P, int D, int N, int M, int C) {
+    return align256((size_t)P * M * 4) + (kind == LAYER_ADD_RIESZ ? align256(riesz_prefix_bytes(P, N, C))
+                                                                  : align256((size_t)P * D * N * 4));
+}
+
+static bool col_layer(int kind, int D, int N, int M) { return kind != LAYER_ADD_BUMP && col_applies(D, N, M); }
+
+// one chunk of P p, by columns or by ranges
+static size_t layer_ws(int kind, int P, int D, int N, int M, int C) {
+    const size_t ranges = layer_ws_bytes(kind, WsSpec{P, D, N, M, C, N, M, true});
+    if (!col_layer(kind, D, N, M)) return ranges;
+    return std::max(ranges, col_bytes(kind == LAYER_ADD_LAPLACE, P, D, N, M, C) + layer_col_extra(kind, P, D, N, M, C));
+}
+
 size_t qlka_layer_fwd_ws_bytes(int kind, int P, int D, int N, int M, int C) {
     if (P <= 0 || D <= 0 || N <= 0 || M <= 0 || C <= 0 || kind < 0 || kind > 2) return 0;
-    auto b1 = [&](int pc) { return layer_ws_bytes(kind, WsSpec{pc, D, N, M, C, N, M, true}); };
+    auto b1 = [&](int pc) { return layer_ws(kind, pc, D, N, M, C); };
     const size_t cap = g_ws_budget.load(std::memory_order_relaxed);
     return plan_bytes(plan_chunks(P, cap, layer_pipelined(kind, P, D, M, C), b1), b1);
 }
@@ -1163,13 +1293,45 @@ static int bump_chunk_unfolded(const float* q, const float* k, const float* v, c
     return hip_status(e, "layer epilogue");
 }
 
+static int layer_columns(int kind, const float* q, const float* k, const float* v, const float* n_pad,
+                         const uint8_t* keep, float* out, int P, int D, int N, int M, int C, void* ws, size_t given,
+                         hipStream_t st) {
+    const bool riesz = kind == LAYER_ADD_RIESZ;
+    return run_columns(riesz ? 0 : 1, v, keep, true, P, D, N, M, C, ws, given, st,
+        [&](int pc) { return layer_col_extra(kind, pc, D, N, M, C); },
+        [&](int p0, int np, ColWs& w, hipStream_t s) {
+            const size_t p = (size_t)p0;
+            const float* kc = k + p * D * N;
+            const uint8_t* keepc = keep ? keep + p * N : nullptr;
+            if (keepc && !riesz) {
+                float* km = (float*)(w.extra + align256((size_t)np * M * 4));
+                if (int e = hip_status(mask_keys(kc, keepc, km, np, D, N, s), "masked keys")) return e;
+                kc = km;
+            }
+            if (int e = sort_both(q + p * D * M, kc, w.s, np * D, N, M, s)) return e;
+            if (keepc && riesz) return hip_status(fill_masked_keys(w.s.ks, w.s.kp, keepc, np, D, N, s), "masked keys");
+            return (int)QLKA_OK; },
+        [&](int p0, int np, ColWs& w, const ColPlan& cp, hipStream_t s) {
+            const size_t p = (size_t)p0;
+            void* pre = w.extra + align256((size_t)np * M * 4);
+            if (riesz)
+                if (int e = riesz_prefix(k + p * D * N, v + p * N * C, keep ? keep + p * N : nullptr, pre, np, D, N, C, s))
+                    return hip_status(e, "riesz prefixes");
+            ReduceEpilogue ep{};
+            if (int e = layer_epilogue_params(kind, keep != nullptr, q + p * D * M, n_pad ? n_pad + p : nullptr, pre,
+                                              (float*)w.extra, out + p * M * C, np, D, M, C, &ep, s))
+                return hip_status(e, "layer query terms");
+            return hip_status(col_finish_launch(riesz ? 0 : 1, kind, keep != nullptr, cp, w.cols, w.u, nullptr, nullptr, ep, np, D, M, C,
+                                                s), "columns to rows"); });
+}
+
 static int layer_fwd(int kind, const float* q, const float* k, const float* v, const float* n_pad,
                      const uint8_t* keep, float* out, int P, int D, int N, int M, int C, void* ws,
                      size_t ws_bytes_given, void* stream) {
     if (kind < 0 || kind > 2) return fail(QLKA_EINVAL, "kind must be 0 (add_laplace), 1 (add_riesz) or 2 (add_bump)");
     if (int e = check_dims(P, D, N, M, C)) return e;
     if (!q || !k || !v || !out) return fail(QLKA_EINVAL, "q, k, v and out must be non-null");
-    auto b1 = [&](int pc) { return layer_ws_bytes(kind, WsSpec{pc, D, N, M, C, N, M, true}); };
+    auto b1 = [&](int pc) { return layer_ws(kind, pc, D, N, M, C); };
     const Plan pl = plan_chunks(P, ws_bytes_given, layer_pipelined(kind, P, D, M, C), b1);
     if (int e = check_ws(ws, ws_bytes_given, plan_bytes(pl, b1))) return e;
     hipStream_t st = (hipStream_t)stream;
@@ -1180,6 +1342,8 @@ static int layer_fwd(int kind, const float* q, const float* k, const float* v, c
         npc = n_pad ? n_pad + p : nullptr; keepc = keep ? keep + p * N : nullptr; outc = out + p * M * C;
     };
     const bool bump = kind == LAYER_ADD_BUMP;
+    if (col_layer(kind, D, N, M) && !(kind == LAYER_ADD_RIESZ && keep == nullptr && few_keys(N)))
+        return layer_columns(kind, q, k, v, n_pad, keep, out, P, D, N, M, C, ws, ws_bytes_given, st);
     if (kind == LAYER_ADD_RIESZ && keep == nullptr && few_keys(N))   // the abs sums dense (few_keys), then the epilogue
         return for_chunks(P, pl.pc, [&](int p0, int np) {
             const float *qc, *kc, *vc, *npc; const uint8_t* keepc; float* outc;
@@ -1366,6 +1530,6 @@ int validate_dims(int P, int D, int N, int M, int C) {
     g_err.clear();
     return check_dims(P, D, N, M, C);
 }
-size_t laplace_fwd_chunk_ws(int pc, int D, int N, int M, int C) { return ws_bytes(laplace_spec(pc, D, N, M, C)); }
+size_t laplace_fwd_chunk_ws(int pc, int D, int N, int M, int C) { return laplace_ws(pc, D, N, M, C); }
 int report_error(int code, const char* msg) { return fail(code, "%s", msg); }
 }  // namespace qlka

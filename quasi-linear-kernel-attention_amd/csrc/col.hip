@@ -1,0 +1,889 @@
+// The forward sums column by column (segments with N + M <= COL_MAX elements).
+//
+//   abs      out[p,m,c] = sum_{d,n} |k[p,d,n] - q[p,d,m]| v[p,n,c]
+//   Laplace  out[p,m,c] = sum_{d,n} e^{-|k[p,d,n] - q[p,d,m]|} v[p,n,c]
+//
+// One workgroup owns CH channels of one p: their columns of v (N words each) and their accumulators (M words each) stay
+// in LDS while it runs over the features d. Per feature it walks the merged sorted sequence of keys and queries: each
+// thread owns E consecutive elements, reads their words from LDS (a key's v, a query's accumulator; random access), the
+// prefix states are combined over threads by a scan, and each query adds its feature's value to its accumulator. The D
+// sum happens in LDS, so no per-feature contribution ever goes to memory, which is what a walk with one row per (p, d,
+// query) has to write and a reduce to read back (6.6 of 10.4 GB per call at P = 12, D = 64, N = M = 16384, C = 64).
+//
+// The merged sequence of a segment does not depend on the channel: col_merge writes it once (6 bytes per element) and the
+// C / CH workgroups of a p read it, neighbours on one XCD at about the same time, so from its L2.
+//   val[s][E/4][T][4]   abs: the value less the thread's anchor, the end of its elements that lies towards the segment's
+//                       median key; Laplace: e^-distance to the previous element
+//   tag[s][E/4][T][4]   16-bit word index: m for query m, M + n for key n, N + M for padding
+//   xe[s][T]            abs: each thread's anchor less the median key; Laplace: e^-(extent of its elements)
+// With 4 elements per 16-byte (8-byte) load, a wave's loads are contiguous.
+//
+// What bounds col_sum: per element and channel one LDS read and, for a query, one masked write at random addresses (about
+// 8 and 6 cycles a wave, bank conflicts of 64 random words), beside some 10 (abs) or 15 (Laplace) vector instructions; at
+// N = M = 16384, one channel per workgroup, that is 0.6 ms of LDS and 0.5 ms of VALU for the measured 0.81 ms (abs,
+// P = 12, D = C = 64; Laplace 0.91). LDS float atomics in place of the read and the write ran at 100 cycles a wave
+// (4.3 ms). Whole calls against the walk: abs 1.70 -> 1.40 ms, Laplace 1.69 -> 1.55 ms at that size, Laplace 0.81 ->
+// 0.58 ms at N = M = 8192, add_riesz 0.97 -> 0.68 ms at 24 x 3111.
+#include <algorithm>
+
+#include "qlka_common.h"
+#include "qlka_internal.h"
+
+namespace qlka {
+
+#define LDS_AS __attribute__((address_space(3)))
+
+typedef float f2_t __attribute__((ext_vector_type(2)));
+typedef unsigned int u2_t __attribute__((ext_vector_type(2)));
+
+enum ColKind : int { COL_ABS = 0, COL_LAPLACE = 1 };
+
+// ---------------------------------------------------------------------------------------------------------------
+// DPP helpers: the value of another lane, or `old` where the pattern has no source lane
+// ---------------------------------------------------------------------------------------------------------------
+template <int CTRL>
+__device__ __forceinline__ float dpp(float old, float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(x), CTRL, 0xf, 0xf, false));
+}
+constexpr int WAVE_SHR1 = 0x138, WAVE_SHL1 = 0x130;
+
+// Steps of the scans as one DPP instruction each (the compiler's form moves the other lane's value first): x += y of the
+// lane the pattern names, x = a y + x and a *= that lane's a; lanes without a source keep x. A DPP read needs two wait
+// states after the register's write (as a lane read does after the last step: settle), which the compiler does not
+// know of around an asm statement.
+#define QLKA_DPP_STEP(NAME, PATTERN)                                                                                  \
+    struct NAME {                                                                                                     \
+        __device__ static __forceinline__ void add(float& x) {                                                        \
+            asm("s_nop 1\n\tv_add_f32_dpp %0, %0, %0 " PATTERN : "+v"(x));                                            \
+        }                                                                                                             \
+        __device__ static __forceinline__ void fma(float& x, float a) {                                               \
+            asm("s_nop 1\n\tv_fmac_f32_dpp %0, %0, %1 " PATTERN : "+v"(x) : "v"(a));                                  \
+        }                                                                                                             \
+        __device__ static __forceinline__ void mul(float& x) {                                                        \
+            asm("s_nop 1\n\tv_mul_f32_dpp %0, %0, %0 " PATTERN : "+v"(x));                                            \
+        }                                                                                                             \
+    }
+QLKA_DPP_STEP(Up1, "row_shr:1 row_mask:0xf bank_mask:0xf");
+QLKA_DPP_STEP(Up2, "row_shr:2 row_mask:0xf bank_mask:0xf");
+QLKA_DPP_STEP(Up4, "row_shr:4 row_mask:0xf bank_mask:0xf");
+QLKA_DPP_STEP(Up8, "row_shr:8 row_mask:0xf bank_mask:0xf");
+QLKA_DPP_STEP(UpRow, "row_bcast:15 row_mask:0xa bank_mask:0xf");
+QLKA_DPP_STEP(UpHalf, "row_bcast:31 row_mask:0xc bank_mask:0xf");
+QLKA_DPP_STEP(Down1, "row_shl:1 row_mask:0xf bank_mask:0xf");
+QLKA_DPP_STEP(Down2, "row_shl:2 row_mask:0xf bank_mask:0xf");
+QLKA_DPP_STEP(Down4, "row_shl:4 row_mask:0xf bank_mask:0xf");
+QLKA_DPP_STEP(Down8, "row_shl:8 row_mask:0xf bank_mask:0xf");
+#undef QLKA_DPP_STEP
+
+__device__ __forceinline__ void settle(float& x) { asm("s_nop 1" : "+v"(x)); }
+
+// inclusive prefix sum over the wave's lanes
+__device__ __forceinline__ float wave_scan_sum(float x) {
+    Up1::add(x);
+    Up2::add(x);
+    Up4::add(x);
+    Up8::add(x);
+    UpRow::add(x);
+    UpHalf::add(x);
+    settle(x);
+    return x;
+}
+// the same within rows of 16 lanes, over W <= 16 entries
+template <int W>
+__device__ __forceinline__ float row_scan_sum(float x) {
+    if constexpr (W > 1) Up1::add(x);
+    if constexpr (W > 2) Up2::add(x);
+    if constexpr (W > 4) Up4::add(x);
+    if constexpr (W > 8) Up8::add(x);
+    settle(x);
+    return x;
+}
+// one step of the inclusive scan of y <- a y' + b, y' from the lane the step names
+template <int CH>
+__device__ __forceinline__ void settle(float& a, float (&b)[CH]) {
+    settle(a);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) settle(b[c]);
+}
+template <class Step, int CH>
+__device__ __forceinline__ void affine_step(float& a, float (&b)[CH]) {
+#pragma unroll
+    for (int c = 0; c < CH; ++c) Step::fma(b[c], a);
+    Step::mul(a);
+}
+template <int CH>
+__device__ __forceinline__ void wave_affine_up(float& a, float (&b)[CH]) {      // lane order
+    affine_step<Up1>(a, b);
+    affine_step<Up2>(a, b);
+    affine_step<Up4>(a, b);
+    affine_step<Up8>(a, b);
+    affine_step<UpRow>(a, b);
+    affine_step<UpHalf>(a, b);
+    settle(a, b);
+}
+template <int CH>
+__device__ __forceinline__ void wave_affine_down(float& a, float (&b)[CH]) {    // reverse lane order
+    affine_step<Down1>(a, b);
+    affine_step<Down2>(a, b);
+    affine_step<Down4>(a, b);
+    affine_step<Down8>(a, b);
+    settle(a, b);
+    // rows above, last first (no DPP pattern reads the next row): their totals are in their first lanes
+    const int row = lane_id() >> 4;
+    const float a1 = bcast(a, 16), a2 = bcast(a, 32), a3 = bcast(a, 48);
+    const float ain = row == 0 ? a1 * (a2 * a3) : row == 1 ? a2 * a3 : row == 2 ? a3 : 1.f;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        const float b3 = bcast(b[c], 48);
+        const float b2 = fmaf(a2, b3, bcast(b[c], 32));
+        const float b1 = fmaf(a1, b2, bcast(b[c], 16));
+        const float bin = row == 0 ? b1 : row == 1 ? b2 : row == 2 ? b3 : 0.f;
+        b[c] = fmaf(a, bin, b[c]);
+    }
+    a *= ain;
+}
+// the same over W <= 16 entries of a row
+template <int W, int CH>
+__device__ __forceinline__ void row_affine_up(float& a, float (&b)[CH]) {
+    if constexpr (W > 1) affine_step<Up1>(a, b);
+    if constexpr (W > 2) affine_step<Up2>(a, b);
+    if constexpr (W > 4) affine_step<Up4>(a, b);
+    if constexpr (W > 8) affine_step<Up8>(a, b);
+    settle(a, b);
+}
+template <int W, int CH>
+__device__ __forceinline__ void row_affine_down(float& a, float (&b)[CH]) {
+    if constexpr (W > 1) affine_step<Down1>(a, b);
+    if constexpr (W > 2) affine_step<Down2>(a, b);
+    if constexpr (W > 4) affine_step<Down4>(a, b);
+    if constexpr (W > 8) affine_step<Down8>(a, b);
+    settle(a, b);
+}
+
+// words of CH channels at an LDS byte address
+template <int CH>
+__device__ __forceinline__ void lds_read(float (&x)[CH], uint32_t byte) {
+    if constexpr (CH == 1) {
+        x[0] = *(LDS_AS const float*)byte;
+    } else {
+        const f2_t v = *(LDS_AS const f2_t*)byte;
+        x[0] = v.x;
+        x[1] = v.y;
+    }
+}
+// Store in the lanes of `mask` only, without a branch around it (the compiler's form of a masked store jumps over it when
+// no lane stores, which costs more than the store: half of a wave's elements are queries). Every lane of the wave is
+// active here. The compiler does not count this store: a wait for lgkmcnt(0) must come before the next barrier.
+template <int CH>
+__device__ __forceinline__ void lds_write_masked(const float (&x)[CH], uint32_t byte, uint64_t mask) {
+    if constexpr (CH == 1) {
+        asm volatile("s_mov_b64 exec, %2\n\tds_write_b32 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(byte), "v"(x[0]), "s"(mask)
+                     : "memory");
+    } else {
+        f2_t v;
+        v.x = x[0];
+        v.y = x[1];
+        asm volatile("s_mov_b64 exec, %2\n\tds_write_b64 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(byte), "v"(v), "s"(mask)
+                     : "memory");
+    }
+}
+// Byte address of the low / high 16-bit word index of a tag pair, words of B bytes (one instruction each; the compiler takes
+// two for the low half).
+template <int B>
+__device__ __forceinline__ uint32_t tag_addr(uint32_t pair, bool high) {
+    uint32_t r;
+    const uint32_t sh = B == 4 ? 2 : 3;
+    if (high)
+        asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_1"
+            : "=v"(r) : "v"(sh), "v"(pair));
+    else
+        asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_0"
+            : "=v"(r) : "v"(sh), "v"(pair));
+    return r;
+}
+// b where the lane's bit of mask is set, else a; the empty asm keeps it one select (the compiler otherwise branches around
+// the arithmetic that follows)
+__device__ __forceinline__ float pick(float a, float b, uint64_t mask) {
+    float r = __builtin_amdgcn_inverse_ballot_w64(mask) ? b : a;
+    asm("" : "+v"(r));
+    return r;
+}
+__device__ __forceinline__ float unless(float a, uint64_t mask) { return pick(a, 0.f, mask); }
+
+// ---------------------------------------------------------------------------------------------------------------
+// col_merge: one workgroup per segment
+// ---------------------------------------------------------------------------------------------------------------
+// e^-x, x >= 0, rounded to nearest for the small x that the sums multiply by the thousands: near 1 the library's expf is
+// off to one side by up to an ulp, which such products add up (Laplace at N = 16384: 1.2e-6 of the result against 64 bits)
+__device__ __forceinline__ float decay(float x) { return x < 0.5f ? 1.f + expm1f(-x) : expf(-x); }
+
+struct ColMergeArgs {
+    const float* qs; const uint32_t* qp; const float* ks; const uint32_t* kp;   // sorted queries and keys
+    const uint8_t* keep;             // (P, N) key mask or null: masked keys weigh 0 in the v == 1 terms
+    float* val; uint16_t* tag; float* xe;
+    float* u;                        // (S, M) v == 1 terms in query order, or null
+    int D, N, M;
+};
+
+// dynamic LDS: N + M words (values, then word indices, then the v == 1 terms), then the scan's aggregates
+template <int KIND, int T, int E>
+__global__ __launch_bounds__(T)
+void col_merge(const ColMergeArgs A)
+{
+    constexpr int W = T / WAVE;
+    extern __shared__ float sm[];
+    const int s = blockIdx.x, p = s / A.D, tid = threadIdx.x;
+    const int N = A.N, M = A.M, n = N + M;
+    const float* qs = A.qs + (size_t)s * M;
+    const float* ks = A.ks + (size_t)s * N;
+#pragma unroll 8
+    for (int i = tid; i < M; i += T) sm[i] = qs[i];
+#pragma unroll 8
+    for (int i = tid; i < N; i += T) sm[M + i] = ks[i];
+    __syncthreads();
+    const float* sq = sm;
+    const float* sk = sm + M;
+    const float x0 = sk[N / 2];
+    // merge path: queries before `diag` (queries come first among equal values)
+    const int diag = min(tid * E, n);
+    int lo = max(0, diag - N), hi = min(diag, M);
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (sq[mid] <= sk[diag - 1 - mid]) lo = mid + 1;
+        else hi = mid;
+    }
+    int i = lo, j = diag - lo;
+    float prev = 0.f;
+    if (diag == 0) prev = fminf(sq[0], sk[0]);
+    else if (i == 0) prev = sk[j - 1];
+    else if (j == 0) prev = sq[i - 1];
+    else prev = fmaxf(sq[i - 1], sk[j - 1]);
+    const float xs = prev;
+    float qa = sq[min(i, M - 1)], kb = sk[min(j, N - 1)];
+    float dist[E];                      // abs: the element's value; Laplace: its distance to the previous element
+    int src[E];                         // word of the element in sq / sk
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const bool live = diag + e < n;
+        const bool tq = j >= N || (i < M && qa <= kb);
+        const float r = tq ? qa : kb;
+        src[e] = live ? (tq ? i : M + j) : n;
+        if constexpr (KIND == COL_LAPLACE) dist[e] = (live && r != prev) ? r - prev : 0.f;   // equal infinities: 0 apart
+        else dist[e] = live ? r : prev;
+        if (live) {
+            prev = r;
+            if (tq) { ++i; qa = sq[min(i, M - 1)]; }
+            else { ++j; kb = sk[min(j, N - 1)]; }
+        }
+    }
+    const float xn = prev, xs0 = KIND == COL_ABS ? dist[0] : 0.f;      // last and first value
+    __syncthreads();
+    {   // word indices over the values
+        uint32_t* w = (uint32_t*)sm;
+        const uint32_t* qp = A.qp + (size_t)s * M;
+        const uint32_t* kp = A.kp + (size_t)s * N;
+#pragma unroll 8
+        for (int x = tid; x < M; x += T) w[x] = qp[x];
+#pragma unroll 8
+        for (int x = tid; x < N; x += T) w[M + x] = M + kp[x];
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < E; ++e) src[e] = src[e] < n ? (int)w[src[e]] : n;
+    }
+    // A thread's values are taken relative to its anchor, so that where a gap splits its elements, those on the median's
+    // side stay precise: every value an element's sums are formed from is then bounded by distances to keys
+    float anchor = 0.f;
+    if constexpr (KIND == COL_ABS) {
+        const float xa = xn <= x0 ? xn : xs0;
+        anchor = xa - x0;
+#pragma unroll
+        for (int e = 0; e < E; ++e) dist[e] -= xa;
+    }
+    // e^-distance once per element for all channels
+    float dec = 1.f;
+    if constexpr (KIND == COL_LAPLACE) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) dist[e] = decay(dist[e]);
+        dec = xn != xs ? decay(xn - xs) : 1.f;
+    }
+    float* vo = A.val + (size_t)s * T * E;
+    uint16_t* to = A.tag + (size_t)s * T * E;
+#pragma unroll
+    for (int g = 0; g < E / 4; ++g) {
+        f4_t x;
+        u2_t y;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = dist[4 * g + e];
+        y.x = (uint32_t)src[4 * g] | ((uint32_t)src[4 * g + 1] << 16);
+        y.y = (uint32_t)src[4 * g + 2] | ((uint32_t)src[4 * g + 3] << 16);
+        *(f4_t*)(vo + ((size_t)g * T + tid) * 4) = x;
+        *(u2_t*)(to + ((size_t)g * T + tid) * 4) = y;
+    }
+    A.xe[(size_t)s * T + tid] = KIND == COL_ABS ? anchor : dec;
+    if (A.u == nullptr) return;
+
+    // v == 1: the same walk as col_sum's with every kept key's weight 1
+    float wt[E];
+    const uint8_t* keep = A.keep ? A.keep + (size_t)p * N : nullptr;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const bool key = src[e] >= M && src[e] < n;
+        wt[e] = key ? (keep ? (keep[src[e] - M] ? 1.f : 0.f) : 1.f) : 0.f;
+    }
+    const int lane = lane_id(), wv = wave_in_block();
+    float* agg = sm + n;
+    float out[E];
+    if constexpr (KIND == COL_ABS) {
+        float sw = 0.f, sk_ = 0.f;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            out[e] = fmaf(dist[e], sw, -sk_);
+            sw += wt[e];
+            sk_ = fmaf(dist[e], wt[e], sk_);
+        }
+        float we = sw, ke = fmaf(anchor, sw, sk_);
+        const float wi = wave_scan_sum(we), ki = wave_scan_sum(ke);
+        we = wi - we;
+        ke = ki - ke;
+        if (lane == WAVE - 1) { agg[2 * wv] = wi; agg[2 * wv + 1] = ki; }
+        __syncthreads();
+        float wp = 0.f, kp = 0.f, wtot = 0.f, ktot = 0.f;
+        for (int x = 0; x < W; ++x) {
+            const float a = agg[2 * x], b = agg[2 * x + 1];
+            if (x < wv) { wp += a; kp += b; }
+            wtot += a;
+            ktot += b;
+        }
+        const float S = we + fmaf(-0.5f, wtot, wp);
+        const float F = fmaf(anchor, S, -(ke + fmaf(-0.5f, ktot, kp)));
+#pragma unroll
+        for (int e = 0; e < E; ++e) out[e] = 2.f * (out[e] + fmaf(dist[e], S, F));
+    } else {
+        float l = 0.f, r = 0.f, pr = 1.f;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            l = fmaf(dist[e], l, wt[e]);
+            pr *= dist[e];
+            r = fmaf(pr, wt[e], r);
+        }
+        float up[1] = {l}, dn[1] = {r}, au = dec, ad = dec;
+        wave_affine_up(au, up);
+        wave_affine_down(ad, dn);
+        if (lane == WAVE - 1) { agg[3 * wv] = up[0]; agg[3 * wv + 2] = au; }
+        if (lane == 0) agg[3 * wv + 1] = dn[0];
+        float L = dpp<WAVE_SHR1>(0.f, up[0]), R = dpp<WAVE_SHL1>(0.f, dn[0]);
+        const float aL = dpp<WAVE_SHR1>(1.f, au), aR = dpp<WAVE_SHL1>(1.f, ad);
+        __syncthreads();
+        float lin = 0.f, rin = 0.f;
+        for (int x = 0; x < wv; ++x) lin = fmaf(agg[3 * x + 2], lin, agg[3 * x]);
+        for (int x = W - 1; x > wv; --x) rin = fmaf(agg[3 * x + 2], rin, agg[3 * x + 1]);
+        L = fmaf(aL, lin, L);
+        R = fmaf(aR, rin, R);
+#pragma unroll
+        for (int e = E - 1; e >= 0; --e) {               // R at the element (later keys), then at the one before
+            R += wt[e];
+            out[e] = R;                                  // a query's weight is 0
+            R *= dist[e];
+        }
+#pragma unroll
+        for (int e = 0; e < E; ++e) { L = fmaf(dist[e], L, wt[e]); out[e] += L; }
+    }
+    // to query order through LDS (every thread has read its word indices before the scan's barrier)
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+        if (src[e] < M) sm[src[e]] = out[e];
+    __syncthreads();
+    float* uo = A.u + (size_t)s * M;
+    for (int x = tid; x < M; x += T) uo[x] = sm[x];
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// col_sum: one workgroup per (p, feature share, CH channels)
+// ---------------------------------------------------------------------------------------------------------------
+struct ColSumArgs {
+    const float* val; const uint16_t* tag; const float* xe;
+    const float* w;                  // (P, C, Nw) weight columns (col_weights): of v, or of g_w with SWAP
+    float* out;                      // [P][DS][C][Ma]
+    int P, D, N, M, C, DS;
+};
+
+// SWAP: the queries carry the weights and the keys the accumulators (the grad_v of the abs sums)
+template <int KIND, int T, int E, int CH, bool SWAP, int WPE>
+__global__ __launch_bounds__(T, WPE)
+void col_sum(const ColSumArgs A)
+{
+    constexpr int W = T / WAVE;
+    extern __shared__ float sm[];
+    const int tid = threadIdx.x, lane = lane_id(), wv = wave_in_block();
+    const int D = A.D, N = A.N, M = A.M, C = A.C, DS = A.DS;
+    const int Nw = SWAP ? M : N, Ma = SWAP ? N : M, w0 = SWAP ? 0 : M, a0 = SWAP ? M : 0;
+    const int CG = (C + CH - 1) / CH;
+    const int b = xcd_slice_block(blockIdx.x, gridDim.x);
+    const int p = b / (DS * CG), ds = (b / CG) % DS, c = (b % CG) * CH;
+    const int d0 = (int)((long)D * ds / DS), d1 = (int)((long)D * (ds + 1) / DS);
+    // LDS words: [N + M + 1][CH] (the last: padding's), then the aggregates of two features
+#pragma unroll
+    for (int h = 0; h < CH; ++h) {
+        const float* wp = A.w + ((size_t)p * C + min(c + h, C - 1)) * Nw;
+#pragma unroll 8
+        for (int i = tid; i < Nw; i += T) sm[(w0 + i) * CH + h] = wp[i];
+    }
+    for (int i = tid; i < Ma * CH; i += T) sm[a0 * CH + i] = 0.f;
+    if (tid < CH) sm[(N + M) * CH + tid] = 0.f;
+    const uint32_t aggb = ((uint32_t)(N + M + 1) * CH * 4 + 15) & ~15u;
+    constexpr uint32_t AGGS = (KIND == COL_ABS ? 2 : 3) * CH * W * 4;    // bytes of one feature's aggregates
+    __syncthreads();
+    if (d0 >= d1) {                                      // more shares than features
+        for (int h = 0; h < CH; ++h)
+            if (c + h < C)
+                for (int i = tid; i < Ma; i += T) A.out[((size_t)(p * DS + ds) * C + c + h) * Ma + i] = 0.f;
+        return;
+    }
+
+    const size_t s0 = (size_t)p * D;
+    const rsrc_t rv = make_rsrc(A.val + s0 * T * E, (uint32_t)(D * T * E * 4));
+    const rsrc_t rt = make_rsrc(A.tag + s0 * T * E, (uint32_t)(D * T * E * 2));
+    float dv[E];
+    uint32_t tg[E / 2];
+    auto load = [&](int d, int g) {                      // elements 4g .. 4g + 3
+        const f4_t x = buf_load4(rv, tid * 16, d * (T * E * 4) + g * (T * 16));
+        const u2_t y = __builtin_bit_cast(u2_t, __builtin_amdgcn_raw_buffer_load_b64(rt, tid * 8,
+                                                                 d * (T * E * 2) + g * (T * 8), 0));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dv[4 * g + e] = x[e];
+        tg[2 * g] = y.x;
+        tg[2 * g + 1] = y.y;
+    };
+#pragma unroll
+    for (int g = 0; g < E / 4; ++g) load(d0, g);
+    const float* xp = A.xe + (s0 + d0) * T + tid;
+    float xs = *xp;
+    const uint32_t split = (uint32_t)M * CH * 4;         // queries' words lie below, keys' above
+    auto addr = [&](int e) { return tag_addr<CH * 4>(tg[e / 2], e & 1); };
+    for (int d = d0; d < d1; ++d) {
+        float a[E][CH];
+        uint64_t acc[E];                                 // lanes whose element is an accumulator
+        // One workgroup per CU (CH = 1): reads run AHEAD elements before their use, in that order, so that a wave's arithmetic
+        // overlaps the other waves' reads (abs at N = M = 16384: 957 -> 856 us with the reads first and in order). With
+        // several workgroups per CU the compiler's order is better (text size, 16384 elements: 302 against 336 us).
+        auto read = [&](int e) {
+            const uint32_t x = addr(e);
+            lds_read<CH>(a[e], x);
+            acc[e] = SWAP ? __ballot(x >= split) : __ballot(x < split);
+        };
+        constexpr int AHEAD = CH == 1 ? 12 : E;
+#pragma unroll
+        for (int e = 0; e < AHEAD && e < E; ++e) read(e);
+        const int dn = min(d + 1, d1 - 1);
+        const uint32_t ab = aggb + (uint32_t)(d & 1) * AGGS;
+        const int el = min(lane & 15, W - 1);            // the wave whose aggregate this lane scans
+        if constexpr (KIND == COL_ABS) {
+            // Half of sum_n |k_n - x| w_n is sum_{k < x} (x - k) w less half of the sum over all keys of (x - k) w. With x
+            // and k relative to the thread's anchor, a thread's own keys below give x W - K from its running sums
+            // W = sum w, K = sum k w; the keys of the threads before, and the totals, then make one linear term S x + F
+            // per thread. Across threads K runs relative to the median
+            // key: |k - median| w sums to no more than the terms |k - q| w that the result is measured by.
+            float own[E][CH], sw[CH], sk[CH], we[CH], ke[CH];
+#pragma unroll
+            for (int h = 0; h < CH; ++h) sw[h] = sk[h] = 0.f;
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                if (CH == 1 && (e & 3) == 0) {
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int i = e + AHEAD; i < e + AHEAD + 4 && i < E; ++i) read(i);
+                }
+#pragma unroll
+                for (int h = 0; h < CH; ++h) {
+                    const float x = unless(a[e][h], acc[e]);
+                    if (e > 0) {
+                        own[e][h] = fmaf(dv[e], sw[h], -sk[h]);
+                        asm("" : "+v"(own[e][h]));    // now, or every element's sw and sk stay live
+                        sw[h] += x;
+                        sk[h] = fmaf(dv[e], x, sk[h]);
+                    } else {
+                        own[e][h] = 0.f;
+                        sw[h] = x;
+                        sk[h] = dv[e] * x;
+                    }
+                }
+            }
+            float wi[CH], ki[CH];
+#pragma unroll
+            for (int h = 0; h < CH; ++h) {
+                we[h] = sw[h];
+                ke[h] = fmaf(xs, sw[h], sk[h]);
+                wi[h] = wave_scan_sum(we[h]);
+                ki[h] = wave_scan_sum(ke[h]);
+                we[h] = wi[h] - we[h];
+                ke[h] = ki[h] - ke[h];
+            }
+            if (lane == WAVE - 1) {
+#pragma unroll
+                for (int h = 0; h < CH; ++h) {
+                    f2_t x;
+                    x.x = wi[h];
+                    x.y = ki[h];
+                    *(LDS_AS f2_t*)(ab + (wv * CH + h) * 8) = x;
+                }
+            }
+            __syncthreads();
+            float S[CH], F[CH];
+#pragma unroll
+            for (int h = 0; h < CH; ++h) {
+                const f2_t x = *(LDS_AS const f2_t*)(ab + (el * CH + h) * 8);
+                const float ww = row_scan_sum<W>(x.x), kk = row_scan_sum<W>(x.y);
+                const float wtot = bcast(ww, W - 1), ktot = bcast(kk, W - 1);
+                const float wb = wv ? bcast(ww, wv ? wv - 1 : 0) : 0.f, kb = wv ? bcast(kk, wv ? wv - 1 : 0) : 0.f;
+                S[h] = we[h] + fmaf(-0.5f, wtot, wb);
+                F[h] = fmaf(xs, S[h], -(ke[h] + fmaf(-0.5f, ktot, kb)));
+            }
+#pragma unroll
+            for (int g = 0; g < E / 2; ++g) asm volatile("" : "+v"(tg[g]));    // addresses again, not kept in registers
+            xp += T;
+            if (d + 1 < d1) xs = *xp;
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                float o[CH];
+#pragma unroll
+                for (int h = 0; h < CH; ++h) {
+                    o[h] = a[e][h] + fmaf(dv[e], S[h], F[h] + own[e][h]);
+                }
+                lds_write_masked<CH>(o, addr(e), acc[e]);
+                if ((e & 3) == 3) {                      // the next feature's elements over the ones just used
+                    load(dn, e / 4);
+                    __builtin_amdgcn_sched_barrier(0x1 | 0x2 | 0x4 | 0x80 | 0x100 | 0x200 | 0x400);
+                }
+            }
+        } else {
+            // L = sum over the keys below of e^-(x - k) w, R the same above. A thread's own sums, then the states
+            // entering it from both sides, then each query adds L + R.
+            float l[CH], r[CH], au = xs, ad = xs, pr = 1.f;
+#pragma unroll
+            for (int h = 0; h < CH; ++h) l[h] = r[h] = 0.f;
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                if (CH == 1 && (e & 3) == 0) {
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int i = e + AHEAD; i < e + AHEAD + 4 && i < E; ++i) read(i);
+                }
+                pr *= dv[e];
+#pragma unroll
+                for (int h = 0; h < CH; ++h) {
+                    const float x = unless(a[e][h], acc[e]);
+                    l[h] = fmaf(dv[e], l[h], x);
+                    r[h] = fmaf(pr, x, r[h]);
+                }
+            }
+            wave_affine_up(au, l);
+            wave_affine_down(ad, r);
+            if (lane == WAVE - 1) {
+#pragma unroll
+                for (int h = 0; h < CH; ++h) *(LDS_AS float*)(ab + (wv * CH + h) * 4) = l[h];
+                *(LDS_AS float*)(ab + (2 * W * CH + wv) * 4) = au;
+            }
+            if (lane == 0) {
+#pragma unroll
+                for (int h = 0; h < CH; ++h) *(LDS_AS float*)(ab + (W * CH + wv * CH + h) * 4) = r[h];
+            }
+            float L[CH], R[CH];
+#pragma unroll
+            for (int h = 0; h < CH; ++h) {
+                L[h] = dpp<WAVE_SHR1>(0.f, l[h]);
+                R[h] = dpp<WAVE_SHL1>(0.f, r[h]);
+            }
+            const float aL = dpp<WAVE_SHR1>(1.f, au), aR = dpp<WAVE_SHL1>(1.f, ad);
+            __syncthreads();
+            {
+                const float a0_ = *(LDS_AS const float*)(ab + (2 * W * CH + el) * 4);
+                float up[CH], dw[CH], a1 = a0_, a2 = a0_;
+                const bool in = (lane & 15) < W;         // entries past the last wave are the identity
+#pragma unroll
+                for (int h = 0; h < CH; ++h) {
+                    up[h] = *(LDS_AS const float*)(ab + (el * CH + h) * 4);
+                    dw[h] = in ? *(LDS_AS const float*)(ab + (W * CH + el * CH + h) * 4) : 0.f;
+                }
+                row_affine_up<W>(a1, up);
+                row_affine_down<W>(a2, dw);
+#pragma unroll
+                for (int h = 0; h < CH; ++h) {
+                    const float lin = wv > 0 ? bcast(up[h], wv > 0 ? wv - 1 : 0) : 0.f;
+                    const float rin = wv < W - 1 ? bcast(dw[h], wv < W - 1 ? wv + 1 : 0) : 0.f;
+                    L[h] = fmaf(aL, lin, L[h]);
+                    R[h] = fmaf(aR, rin, R[h]);
+                }
+            }
+#pragma unroll
+            for (int g = 0; g < E / 2; ++g) asm volatile("" : "+v"(tg[g]));
+            xp += T;
+            if (d + 1 < d1) xs = *xp;
+#pragma unroll
+            for (int e = E - 1; e >= 0; --e) {
+#pragma unroll
+                for (int h = 0; h < CH; ++h) {           // R: at the element, without its own weight
+                    const float t = a[e][h] + R[h];      // query: its word + R; key: R past it
+                    R[h] = dv[e] * pick(t, R[h], acc[e]);
+                    a[e][h] = pick(a[e][h], t, acc[e]);
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                float o[CH];
+#pragma unroll
+                for (int h = 0; h < CH; ++h) {
+                    const float x = dv[e] * L[h];
+                    o[h] = a[e][h] + x;                  // query: its word + R + L; key: L past it
+                    L[h] = pick(o[h], x, acc[e]);
+                }
+                lds_write_masked<CH>(o, addr(e), acc[e]);
+                if ((e & 3) == 3) {
+                    load(dn, e / 4);
+                    __builtin_amdgcn_sched_barrier(0x1 | 0x2 | 0x4 | 0x80 | 0x100 | 0x200 | 0x400);
+                }
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // the masked stores (lds_write_masked)
+        __syncthreads();
+    }
+    for (int h = 0; h < CH; ++h) {
+        if (c + h >= C) break;
+        float* o = A.out + ((size_t)(p * DS + ds) * C + c + h) * Ma;
+        for (int i = tid; i < Ma; i += T) o[i] = sm[(a0 + i) * CH + h];
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// col_weights: the weight rows (P, Nw, C) as columns (P, C, Nw), masked rows 0
+// ---------------------------------------------------------------------------------------------------------------
+constexpr int CF_T = 256, CF_M = 64;        // threads, rows per workgroup (also of col_finish)
+
+__global__ __launch_bounds__(CF_T)
+void col_weights(const float* __restrict__ w, const uint8_t* __restrict__ keep, float* __restrict__ out, const int Nw,
+                 const int C)
+{
+    __shared__ float tile[128][CF_M + 1];
+    const int nb = (Nw + CF_M - 1) / CF_M;
+    const int p = blockIdx.x / nb, n0 = (blockIdx.x - p * nb) * CF_M;
+    const int rows = min(CF_M, Nw - n0);
+    const float* src = w + ((size_t)p * Nw + n0) * C;
+    int r = threadIdx.x / C, c = threadIdx.x - r * C;
+    const int dr = CF_T / C, dc = CF_T - dr * C;
+    for (int i = threadIdx.x; i < rows * C; i += CF_T) {
+        const float x = src[i];
+        tile[c][r] = (!keep || keep[(size_t)p * Nw + n0 + r] != 0) ? x : 0.f;
+        r += dr;
+        c += dc;
+        if (c >= C) { c -= C; ++r; }
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & (CF_M - 1);
+    float* dst = out + (size_t)p * C * Nw + n0;
+    if (lane < rows)
+        for (int cc = threadIdx.x / CF_M; cc < C; cc += CF_T / CF_M) dst[(size_t)cc * Nw + lane] = tile[cc][lane];
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// col_finish: the feature shares' columns summed, turned into rows, with the v == 1 terms summed over the features
+// ---------------------------------------------------------------------------------------------------------------
+// scale: 2 for the abs sums, whose columns hold halves. kind < 0: out = w and out_u = u; else the layer's epilogue on
+// them, as layer_epilogue_kernel
+__global__ __launch_bounds__(CF_T)
+void col_finish(const float* __restrict__ cols, const float* __restrict__ u, float* __restrict__ out,
+                float* __restrict__ out_u, const float scale, const int kind, const int masked, const ReduceEpilogue ep,
+                const int D, const int M, const int C, const int DS)
+{
+    __shared__ float tile[128][CF_M + 1];
+    __shared__ float us[CF_T / CF_M][CF_M];
+    const int mb = (M + CF_M - 1) / CF_M;
+    const int p = blockIdx.x / mb, m0 = (blockIdx.x - p * mb) * CF_M;
+    const int lane = threadIdx.x & (CF_M - 1), wv = threadIdx.x / CF_M;
+    const int m = min(m0 + lane, M - 1);
+    const float* src = cols + (size_t)p * DS * C * M + m;
+#pragma unroll 4
+    for (int c = wv; c < C; c += CF_T / CF_M) {
+        float x = src[(size_t)c * M];
+        for (int s = 1; s < DS; ++s) x += src[(size_t)(s * C + c) * M];
+        tile[c][lane] = scale * x;
+    }
+    if (u) {
+        const float* up = u + (size_t)p * D * M + m;
+        float x = 0.f;
+#pragma unroll 8
+        for (int d = wv; d < D; d += CF_T / CF_M) x += up[(size_t)d * M];
+        us[wv][lane] = x;
+    }
+    __syncthreads();
+    const int rows = min(CF_M, M - m0);
+    if (u && kind < 0 && threadIdx.x < rows)
+        out_u[(size_t)p * M + m0 + lane] = (us[0][lane] + us[1][lane]) + (us[2][lane] + us[3][lane]);
+    float* dst = (kind < 0 ? out : ep.out) + ((size_t)p * M + m0) * C;
+    const float np = (kind >= 0 && ep.n_pad) ? ep.n_pad[p] : 0.f;
+    int r = threadIdx.x / C, c = threadIdx.x - r * C;
+    const int dr = CF_T / C, dc = CF_T - dr * C;
+    for (int i = threadIdx.x; i < rows * C; i += CF_T) {
+        float x = tile[c][r];
+        if (kind >= 0) {
+            const float uu = (us[0][r] + us[1][r]) + (us[2][r] + us[3][r]);
+            const float qv = ep.qt[(size_t)p * M + m0 + r];
+            float den;
+            if (kind == LAYER_ADD_RIESZ) {
+                const float aqe = qv + LAYER_EPS;
+                den = masked ? aqe * ((float)M - np) + ep.sak[p] - uu
+                             : aqe * (float)M + ep.sak[p] - uu - LAYER_EPS * np;
+                x = aqe * ep.vsum[(size_t)p * C + c] + ep.akv[(size_t)p * C + c] - x;
+            } else {
+                den = masked ? uu : uu - np * qv;
+            }
+            x /= fmaxf(den, LAYER_CLAMP);
+        }
+        dst[i] = x;
+        r += dr;
+        c += dc;
+        if (c >= C) { c -= C; ++r; }
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// host
+// ---------------------------------------------------------------------------------------------------------------
+namespace {
+
+constexpr size_t LDS_BYTES = 160 * 1024;
+
+size_t sum_lds(int kind, int T, int CH, int n) {
+    return (((size_t)(n + 1) * CH * 4 + 15) & ~size_t(15)) + 2 * (size_t)(kind == COL_ABS ? 2 : 3) * CH * (T / WAVE) * 4;
+}
+
+// Workgroups of one col_sum launch that a CU holds at once: by LDS, and by the wave slots of 4 waves per SIMD (128 VGPRs)
+int wgs_per_cu(int kind, int T, int CH, int n) {
+    return std::max(1, std::min((int)(LDS_BYTES / sum_lds(kind, T, CH, n)), 1024 / T));
+}
+
+}  // namespace
+
+bool col_applies(int D, int N, int M) {
+    if ((int64_t)N + M > COL_MAX) return false;
+    const ColPlan pl = col_plan(COL_ABS, 1, D, N, M, 2);
+    return (int64_t)D * pl.T * pl.E * 4 <= (int64_t)INT32_MAX;      // a p's stream within 32-bit buffer offsets
+}
+
+ColPlan col_plan(int kind, int P, int D, int N, int M, int C) {
+    const int n = N + M;
+    ColPlan pl{};
+    // Two channels per workgroup where their words fit LDS (an 8-byte LDS read costs what a 4-byte one does, and the
+    // stream is read once for both); the smallest workgroup whose threads hold at most 16 elements then, so that
+    // several run per CU and fill each other's waits.
+    if (C >= 2 && n <= COL_MAX2) {
+        pl.CH = 2;
+        pl.T = 64;
+        while (pl.T < 1024 && pl.T * (pl.T < 512 ? 16 : 20) < n) pl.T *= 2;
+        pl.E = n <= pl.T * 12 ? 12 : n <= pl.T * 16 ? 16 : 20;
+    } else {
+        pl.CH = 1;
+        pl.T = n <= 16384 ? 512 : 1024;
+        pl.E = n <= pl.T * 20 ? 20 : n <= pl.T * 24 ? 24 : n <= pl.T * 28 ? 28 : 32;
+    }
+    // Shares of the features: the fewest rounds of workgroups over the chip, in features walked one after another (plus
+    // about two features' time per round for loading and storing the columns).
+    const int64_t wgs = (int64_t)P * ((C + pl.CH - 1) / pl.CH), slots = 256 * (int64_t)wgs_per_cu(kind, pl.T, pl.CH, n);
+    int64_t best = -1;
+    for (int s = 1; s <= std::min(D, COL_SHARES); ++s) {
+        const int64_t cost = ((wgs * s + slots - 1) / slots) * ((D + s - 1) / s + 2);
+        if (best < 0 || cost < best) { best = cost; pl.DS = s; }
+    }
+    return pl;
+}
+
+size_t col_stream_bytes(const ColPlan& pl, int S) {
+    const size_t L = (size_t)pl.T * pl.E;
+    auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
+    return al((size_t)S * L * 4) + al((size_t)S * L * 2) + al((size_t)S * pl.T * 4);
+}
+
+ColStream col_stream(const ColPlan& pl, void* base, int S) {
+    const size_t L = (size_t)pl.T * pl.E;
+    auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
+    char* b = (char*)base;
+    ColStream r;
+    r.val = (float*)b;     b += al((size_t)S * L * 4);
+    r.tag = (uint16_t*)b;  b += al((size_t)S * L * 2);
+    r.xe = (float*)b;
+    return r;
+}
+
+namespace {
+
+// every workgroup shape col_plan returns
+template <class F>
+int dispatch_shape(const ColPlan& pl, F f) {
+#define QLKA_COL(TT, EE, CC) \
+    if (pl.T == TT && pl.E == EE && pl.CH == CC) \
+        return f(std::integral_constant<int, TT>{}, std::integral_constant<int, EE>{}, std::integral_constant<int, CC>{})
+    QLKA_COL(64, 12, 2); QLKA_COL(64, 16, 2); QLKA_COL(128, 12, 2); QLKA_COL(128, 16, 2); QLKA_COL(256, 12, 2);
+    QLKA_COL(256, 16, 2); QLKA_COL(512, 12, 2); QLKA_COL(512, 16, 2); QLKA_COL(1024, 12, 2); QLKA_COL(1024, 16, 2);
+    QLKA_COL(512, 20, 2); QLKA_COL(1024, 20, 2);
+    QLKA_COL(512, 20, 1); QLKA_COL(512, 24, 1); QLKA_COL(512, 28, 1); QLKA_COL(512, 32, 1);
+    QLKA_COL(1024, 20, 1); QLKA_COL(1024, 24, 1); QLKA_COL(1024, 28, 1); QLKA_COL(1024, 32, 1);
+#undef QLKA_COL
+    return (int)hipErrorInvalidValue;
+}
+
+template <class K>
+hipError_t allow_lds(K kernel) {
+    return hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_BYTES);
+}
+
+template <int KIND, int T, int E>
+int launch_merge(const ColMergeArgs& a, int S, hipStream_t st) {
+    static const hipError_t once = allow_lds(col_merge<KIND, T, E>);
+    if (once != hipSuccess) return (int)once;
+    const size_t lds = (size_t)(a.N + a.M + 3 * (T / WAVE)) * 4;
+    hipLaunchKernelGGL((col_merge<KIND, T, E>), dim3((unsigned)S), dim3(T), lds, st, a);
+    return (int)hipGetLastError();
+}
+
+template <int KIND, int T, int E, int CH, bool SWAP>
+int launch_sum(const ColSumArgs& a, hipStream_t st) {
+    static const hipError_t once = allow_lds(col_sum<KIND, T, E, CH, SWAP, 4>);
+    if (once != hipSuccess) return (int)once;
+    const unsigned blocks = (unsigned)(a.P * a.DS * ((a.C + CH - 1) / CH));
+    hipLaunchKernelGGL((col_sum<KIND, T, E, CH, SWAP, 4>), dim3(blocks), dim3(T), sum_lds(KIND, T, CH, a.N + a.M), st, a);
+    return (int)hipGetLastError();
+}
+
+}  // namespace
+
+int col_merge_launch(int kind, const ColPlan& pl, const float* qs, const uint32_t* qp, const float* ks,
+                     const uint32_t* kp, const uint8_t* keep, ColStream str, float* u, int S, int D, int N, int M,
+                     hipStream_t st) {
+    const ColMergeArgs a{qs, qp, ks, kp, keep, str.val, str.tag, str.xe, u, D, N, M};
+    StageTimer t("col_merge", st);
+    return dispatch_shape(pl, [&](auto T, auto E, auto) {
+        return kind == COL_ABS ? launch_merge<COL_ABS, T(), E()>(a, S, st) : launch_merge<COL_LAPLACE, T(), E()>(a, S, st); });
+}
+
+int col_weights_launch(const float* w, const uint8_t* keep, float* wt, int P, int Nw, int C, hipStream_t st) {
+    StageTimer t("col_weights", st);
+    hipLaunchKernelGGL(col_weights, dim3((unsigned)(P * ((Nw + CF_M - 1) / CF_M))), dim3(CF_T), 0, st, w, keep, wt, Nw, C);
+    return (int)hipGetLastError();
+}
+
+int col_sum_launch(int kind, const ColPlan& pl, ColStream str, const float* wt, float* cols, int P, int D, int N, int M,
+                   int C, hipStream_t st) {
+    const ColSumArgs a{str.val, str.tag, str.xe, wt, cols, P, D, N, M, C, pl.DS};
+    StageTimer t(kind == COL_ABS ? "col_sum_abs" : "col_sum_laplace", st);
+    return dispatch_shape(pl, [&](auto T, auto E, auto CH) {
+        return kind == COL_ABS ? launch_sum<COL_ABS, T(), E(), CH(), false>(a, st)
+                               : launch_sum<COL_LAPLACE, T(), E(), CH(), false>(a, st); });
+}
+
+int col_finish_launch(int kind, int layer, bool masked, const ColPlan& pl, const float* cols, const float* u, float* out,
+                      float* out_u, const ReduceEpilogue& ep, int P, int D, int M, int C, hipStream_t st) {
+    StageTimer t("col_finish", st);
+    hipLaunchKernelGGL(col_finish, dim3((unsigned)(P * ((M + CF_M - 1) / CF_M))), dim3(CF_T), 0, st, cols, u, out, out_u,
+                       kind == COL_ABS ? 2.f : 1.f, layer, masked ? 1 : 0, ep, D, M, C, pl.DS);
+    return (int)hipGetLastError();
+}
+
+}  // namespace qlka

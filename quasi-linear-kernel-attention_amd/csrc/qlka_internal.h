@@ -258,6 +258,29 @@ int reduce_slabs_layer(int kind, bool masked, const ReduceEpilogue& ep, const fl
 int reduce_slabs_bump(bool masked, const ReduceEpilogue& ep, const float* const slab[3], const float* const uq[3],
                       int P, int D, int M, int C, hipStream_t st);
 
+// ---- col.hip: the forward sums column by column, for segments of N + M <= COL_MAX elements
+constexpr int COL_MAX = 32768;           // 32 elements for each of 1024 threads
+constexpr int COL_MAX2 = 20352;          // two channels per workgroup: 2 words of LDS per element
+constexpr int COL_SHARES = 16;           // most shares of the features
+struct ColPlan { int T, E, CH, DS; };    // threads, elements per thread, channels per workgroup, shares of the features
+struct ColStream { float* val; uint16_t* tag; float* xe; };
+bool col_applies(int D, int N, int M);
+ColPlan col_plan(int kind, int P, int D, int N, int M, int C);      // kind 0 abs, 1 Laplace (as below)
+size_t col_stream_bytes(const ColPlan& pl, int S);
+ColStream col_stream(const ColPlan& pl, void* base, int S);
+// the merged stream of S sorted segments, and the v == 1 terms u (S, M) in query order (null: none; masked keys weigh 0)
+int col_merge_launch(int kind, const ColPlan& pl, const float* qs, const uint32_t* qp, const float* ks,
+                     const uint32_t* kp, const uint8_t* keep, ColStream str, float* u, int S, int D, int N, int M,
+                     hipStream_t st);
+// wt (P, C, Nw) from rows w (P, Nw, C), rows masked by keep (null: none) 0
+int col_weights_launch(const float* w, const uint8_t* keep, float* wt, int P, int Nw, int C, hipStream_t st);
+// cols[P][DS][C][M]: the sums of each feature share over the weights wt (P, C, N); half of them for kind 0
+int col_sum_launch(int kind, const ColPlan& pl, ColStream str, const float* wt, float* cols, int P, int D, int N, int M,
+                   int C, hipStream_t st);
+// layer < 0: out (P, M, C) and, with u, out_u (P, M); else the epilogue of layer kind `layer` written to ep.out
+int col_finish_launch(int kind, int layer, bool masked, const ColPlan& pl, const float* cols, const float* u, float* out,
+                      float* out_u, const ReduceEpilogue& ep, int P, int D, int M, int C, hipStream_t st);
+
 // ---- capi.hip helpers for noalloc.hip
 // check_dims of the C ABI (clears the thread's error first); the workspace of a Laplace forward over pc p at a time;
 // set the thread's error message and return code

@@ -1,0 +1,122 @@
+"""GPU checks of the column route of the forward sums (csrc/col.hip) at the edges of its workgroup shapes: the element
+counts N + M where the threads or elements per thread change, the switch from two channels per workgroup to one, odd
+channel counts, more feature shares than features, one-sided sizes and the last size before the ranges take over.
+
+Against the fp64 oracle on a subsample of the queries, at the bar of every forward sum: 1e-5 of sum |term|. The fp32 error
+of these sums is a few roundings of partial sums no larger than sum |term| (measured: below 1e-6), so 1e-5 has room.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import brute, inputs
+
+pytestmark = pytest.mark.gpu
+
+REL = 1e-5
+# N + M just at and past every capacity of col_plan (threads x elements per thread), CH = 2 up to 20352 elements
+EDGES = [768, 769, 1024, 1025, 1536, 1537, 2048, 2049, 4096, 4097, 6144, 6145, 8192, 8193, 10240, 10241, 12288, 12289,
+         16384, 16385, 20352, 20353, 20480, 20481, 24576, 24577, 28672, 28673, 32768, 32769]
+
+
+def _data(P, D, N, M, C, kind, seed):
+    rng = np.random.default_rng(seed)
+    if kind == "ties":
+        q = (rng.integers(-6, 7, size=(P, D, M)) / 4).astype(np.float32)
+        k = (rng.integers(-6, 7, size=(P, D, N)) / 4).astype(np.float32)
+    else:
+        q = rng.standard_normal((P, D, M), dtype=np.float32)
+        k = rng.standard_normal((P, D, N), dtype=np.float32)
+        if kind == "far":                          # offset by 300, with keys and queries far out on both sides
+            q += 300
+            k += 300
+            q[..., 0] = -4000
+            k[..., -1] = 9000
+    return q, k, rng.standard_normal((P, N, C), dtype=np.float32)
+
+
+def _check(dev, P, D, N, M, C, kind, seed):
+    from weighted_abs_sum import weighted_abs_sum_full
+    from weighted_laplace_sum import weighted_laplace_sum
+    print(f"columns P={P} D={D} N={N} M={M} C={C} {kind}", flush=True)
+    q, k, v = _data(P, D, N, M, C, kind, seed)
+    tq, tk, tv = (torch.from_numpy(a).to(dev) for a in (q, k, v))
+    idx = inputs.query_subsample(P, M, per_p=24, seed=seed)
+    for name, op, oracle in (("abs", lambda *a: weighted_abs_sum_full(*a, backend="cuda"), brute.abs_sum),
+                             ("laplace", weighted_laplace_sum, brute.laplace_sum)):
+        w, u = (t.cpu().numpy() for t in op(tq, tk, tv))
+        assert np.isfinite(w).all() and np.isfinite(u).all(), name
+        ow, ou, nw = oracle(q, k, v, qidx=idx)
+        w = np.stack([w[p][idx[p]] for p in range(P)])
+        u = np.stack([u[p][idx[p]] for p in range(P)])
+        assert float(brute.rel_err(w, ow, nw).max()) <= REL, f"{name} out_w"
+        assert float(brute.rel_err(u, ou, ou).max()) <= REL, f"{name} out_u"
+
+
+@pytest.fixture
+def no_dense():
+    from qlka import _lib
+    lib = _lib.load()
+    prev = lib.qlka_set_direct_max(0)
+    yield
+    lib.qlka_set_direct_max(prev)
+
+
+@pytest.mark.parametrize("kind", ["normal", "ties"])
+@pytest.mark.parametrize("n", EDGES)
+def test_column_capacity_edges(dev, no_dense, n, kind):
+    N = n // 2 + 3
+    _check(dev, 1, 3, N, n - N, 3, kind, seed=n)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 17, 1, 1), (2, 1, 18, 40, 2), (1, 2, 32000, 700, 5), (1, 2, 700, 32000, 2),
+                                   (3, 33, 900, 1100, 7), (40, 2, 1200, 900, 128), (2, 64, 5003, 3001, 33)])
+@pytest.mark.parametrize("kind", ["normal", "far"])
+def test_column_shapes(dev, no_dense, shape, kind):
+    _check(dev, *shape, kind, seed=sum(shape))
+
+
+def test_laplace_infinite_keys_and_queries(dev, no_dense):
+    # an infinite key adds 0 to every finite query, an infinite query sums to 0 over finite keys; neighbours stay exact
+    from weighted_laplace_sum import weighted_laplace_sum
+    P, D, N, M, C = 1, 2, 2000, 1500, 3
+    q, k, v = _data(P, D, N, M, C, "normal", 5)
+    k[0, 0, [3, 40]] = np.inf
+    k[0, 1, 7] = -np.inf
+    q[0, 0, 11] = np.inf
+    w, u = (t.cpu().numpy() for t in weighted_laplace_sum(*(torch.from_numpy(a).to(dev) for a in (q, k, v))))
+    with np.errstate(invalid="ignore"):            # inf - inf, set below
+        a = [np.exp(-np.abs(q[0, d, :, None].astype(np.float64) - k[0, d][None])) for d in range(D)]
+    a[0][11, [3, 40]] = 1.0                        # equal infinities are 0 apart
+    A = a[0] + a[1]
+    assert float(brute.rel_err(w[0], A @ v[0], A @ np.abs(v[0]).astype(np.float64)).max()) <= REL
+    assert float(brute.rel_err(u[0], A.sum(1), A.sum(1)).max()) <= REL
+
+
+@pytest.mark.parametrize("kernel", ["add_laplace", "add_riesz"])
+@pytest.mark.parametrize("N,M,C", [(1030, 1020, 6), (3111, 3111, 64), (12000, 9000, 31)])
+def test_masked_layer_columns(dev, kernel, N, M, C):
+    # masked rows weigh 0 whatever they hold (NaN in v, large k), against the float64 layer over the kept keys
+    from qlka import layers
+    P, D = 2, 4
+    q, k, v = _data(P, D, N, M, C, "normal", N)
+    keep = np.random.default_rng(N).random((P, N)) < 0.7
+    k[np.broadcast_to(~keep[:, None], k.shape)] = 50.0
+    v[~keep] = np.nan
+    got = layers.layer_forward(kernel, *(torch.from_numpy(a).to(dev) for a in (q, k, v)),
+                               keep=torch.from_numpy(keep).to(dev)).cpu().numpy()
+    rows = np.arange(0, M, max(1, M // 50))
+    for p in range(P):
+        kk, vv, qq = k[p][:, keep[p]].astype(np.float64), v[p][keep[p]].astype(np.float64), q[p][:, rows].astype(np.float64)
+        dist = np.abs(qq[:, :, None] - kk[:, None])
+        if kernel == "add_laplace":
+            A = np.exp(-dist).sum(0)
+        else:
+            A = np.abs(qq).sum(0)[:, None] + np.abs(kk).sum(0)[None] - dist.sum(0) + layers.EPS
+        den = A.sum(1)
+        if kernel == "add_riesz":
+            den = den + (np.abs(qq).sum(0) + layers.EPS) * (M - N)
+        num = A @ vv
+        scale = np.abs(A) @ np.abs(vv)
+        np.testing.assert_array_less(np.abs(got[p][rows] * den[:, None] - num), 2e-4 * (scale + np.abs(num)) + 1e-6)
