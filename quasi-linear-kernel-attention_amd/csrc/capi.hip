@@ -472,7 +472,7 @@ size_t col_part(const ColPlan& pl, int P, int D, int N, int M, int C, int i) {
         case 5: return align256(col_stream_bytes(pl, (int)S));
         case 6: return align256(S * M * 4);
         case 7: return align256((size_t)P * pl.DS * C * M * 4);
-        case 8: return align256((size_t)P * C * N * 4);
+        case 8: return align256((size_t)P * (C + 1) * N * 4);
     }
     return 0;
 }
@@ -521,15 +521,84 @@ int run_columns(int kind, const float* v, const uint8_t* keep, bool want_u, int 
         const size_t p = (size_t)p0;
         if (int e = sort(p0, np, w, st)) return e;
         const uint8_t* kc = keep ? keep + p * N : nullptr;
-        if (int e = col_merge_launch(kind, pl, w.s.qs, w.s.qp, w.s.ks, w.s.kp, kc, w.str, w.u, np * D, D, N, M, st))
+        if (int e = col_merge_launch(kind, pl, w.s.qs, w.s.qp, w.s.ks, w.s.kp, kc, w.str, w.u, np * D, D, N, M, false,
+                                     st))
             return hip_status(e, "merge of q and k");
-        if (int e = col_weights_launch(v + p * N * C, kc, w.wt, np, N, C, st)) return hip_status(e, "weight columns");
+        if (int e = col_weights_launch(pl, v + p * N * C, kc, false, nullptr, w.wt, np, N, C, st))
+            return hip_status(e, "weight columns");
         if (int e = col_sum_launch(kind, pl, w.str, w.wt, w.cols, np, D, N, M, C, st))
             return hip_status(e, "column sums");
         return finish(p0, np, w, pl, st); });
 }
 
 inline size_t no_extra(int) { return 0; }
+
+// The abs backward by columns (col.hip), and the sgn sum, its grad_q negated: the merge of the sorted k and q, the columns
+// of g_w and v (with g_u: one more channel, g_u against ones), grad_q and grad_k per segment, grad_v by the forward's
+// column sums with the roles of q and k exchanged. Workspace of a chunk of P p: as the forward's, the columns of N rows,
+// and those of g_w.
+ColPlan col_bwd_plan(int P, int D, int N, int M, int C) { return col_plan(0, P, D, N, M, std::max(C, 2)); }
+
+size_t col_bwd_part(const ColPlan& pl, int P, int D, int N, int M, int C, int i) {
+    const size_t S = (size_t)P * D, C1 = (size_t)(C + 1 + pl.CH) / pl.CH * pl.CH;      // C + 1 channels in whole groups
+    switch (i) {
+        case 0: case 1: return align256(S * N * 4);
+        case 2: case 3: return align256(S * M * 4);
+        case 4: return align256(sort_scratch_need(WsSpec{P, D, N, M, C, N, 0, false}));
+        case 5: return align256(col_stream_bytes(pl, (int)S));
+        case 6: return align256((size_t)P * C1 * N * 4);
+        case 7: return align256((size_t)P * C1 * M * 4);
+        case 8: return align256((size_t)P * std::min(D, COL_SHARES) * C * N * 4);
+    }
+    return 0;
+}
+
+size_t col_bwd_bytes(int P, int D, int N, int M, int C) {
+    if (!col_bwd_applies(D, N, M)) return 0;
+    const ColPlan pl = col_bwd_plan(1, D, N, M, C);
+    size_t b = 0;
+    for (int i = 0; i < COL_PARTS; ++i) b += col_bwd_part(pl, P, D, N, M, C, i);
+    return b;
+}
+
+// pre: sorted arrays of the whole call (as Presorted, offset by the caller) or null; sort(p0, np, w, st) otherwise.
+// grad_k and grad_v are null for the sgn sum.
+template <class Sorts>
+int run_bwd_columns(const float* v, const float* g_w, const float* g_u, float scale, float* grad_q, float* grad_k,
+                    float* grad_v, int P, int D, int N, int M, int C, void* ws, size_t given, hipStream_t st,
+                    Sorts sorts) {
+    const ColPlan pl = col_bwd_plan(P, D, N, M, C);
+    auto bytes = [&](int pc) { return col_bwd_bytes(pc, D, N, M, C); };
+    const int pc = fit_chunk(P, given, bytes);
+    if (int e = check_ws(ws, given, bytes(pc))) return e;
+    return for_chunks(P, pc, [&](int p0, int np) {
+        char* part[COL_PARTS];
+        char* b = (char*)ws;
+        for (int i = 0; i < COL_PARTS; ++i) { part[i] = b; b += col_bwd_part(pl, np, D, N, M, C, i); }
+        SortedWs w{};
+        w.ks = (float*)part[0]; w.kp = (uint32_t*)part[1]; w.qs = (float*)part[2]; w.qp = (uint32_t*)part[3];
+        w.sort_scratch = part[4];
+        const ColStream str = col_stream(pl, part[5], np * D);
+        float *vt = (float*)part[6], *gt = (float*)part[7], *cols = (float*)part[8];
+        const size_t p = (size_t)p0;
+        const int CW = (C + (g_u ? 1 : 0) + pl.CH - 1) / pl.CH;
+        if (int e = sorts(p0, np, w, st)) return e;
+        if (int e = col_merge_launch(0, pl, w.qs, w.qp, w.ks, w.kp, nullptr, str, nullptr, np * D, D, N, M, true, st))
+            return hip_status(e, "merge of q and k");
+        if (int e = col_weights_launch(pl, v + p * N * C, nullptr, g_u != nullptr, nullptr, vt, np, N, C, st))
+            return hip_status(e, "value columns");
+        if (int e = col_weights_launch(pl, g_w + p * M * C, nullptr, g_u != nullptr, g_u ? g_u + p * M : nullptr, gt, np, M,
+                                       C, st))
+            return hip_status(e, "gradient columns");
+        if (grad_v) {
+            if (int e = col_grad_v_launch(pl, str, gt, CW, cols, np, D, N, M, C, st)) return hip_status(e, "grad_v columns");
+            if (int e = col_finish_launch(0, -1, false, pl, cols, nullptr, grad_v + p * N * C, nullptr, ReduceEpilogue{}, np, D,
+                                          N, C, st))
+                return hip_status(e, "columns to rows");
+        }
+        return hip_status(col_dot_launch(pl, str, gt, vt, CW, scale, grad_q + p * D * M,
+                                         grad_k ? grad_k + p * D * N : nullptr, np * D, D, N, M, st), "column dots"); });
+}
 
 }  // namespace
 
@@ -702,7 +771,8 @@ int abs_fwd_impl(const float* q, const float* k, const float* v, float* out_w, f
     auto b1 = [&](int pc) { return abs_fwd_ws(pc, D, N, M, C); };
     const Plan pl = plan_chunks(P, ws_bytes_given, pipelined(P, D, M), b1);
     if (int e = check_ws(ws, ws_bytes_given, plan_bytes(pl, b1))) return e;
-    if (col_applies(D, N, M) && !keep_states) {
+    // (the backward by columns reads no range states, so none are written; *kept still says that a buffer was taken)
+    if (col_applies(D, N, M) && (!keep_states || col_bwd_applies(D, N, M))) {
         const int e = run_columns(0, v, nullptr, out_u != nullptr, P, D, N, M, C, ws, ws_bytes_given, st, no_extra,
             [&](int p0, int np, ColWs& w, hipStream_t s) {
                 const size_t p = (size_t)p0;
@@ -717,7 +787,7 @@ int abs_fwd_impl(const float* q, const float* k, const float* v, float* out_w, f
                                                     out_u ? out_u + p * M : nullptr, ReduceEpilogue{}, np, D, M, C, s),
                                   "columns to rows"); });
         if (e) return e;
-        if (keep_sorts) *kept = 1;
+        if (keep_sorts) *kept = keep_states ? 3 : 1;
         return QLKA_OK;
     }
     const int mode = out_u ? (ABS_ROW | ABS_ONES) : ABS_ROW;
@@ -914,10 +984,10 @@ size_t qlka_abs_bwd_ws_bytes(int P, int D, int N, int M, int C) {
     if (P <= 0 || D <= 0 || N <= 0 || M <= 0 || C <= 0) return 0;
     if (dense_sign(P, N, M)) return 0;            // the dense route takes no workspace
     if (mbw_applies(C)) {
-        auto bm = [&](int pc) { return mbw_ws_bytes(pc, D, N, M, C); };
+        auto bm = [&](int pc) { return std::max(mbw_ws_bytes(pc, D, N, M, C), col_bwd_bytes(pc, D, N, M, C)); };
         return plan_bytes(plan_chunks(P, g_ws_budget.load(std::memory_order_relaxed), pipelined(P, D, N), bm), bm);
     }
-    auto b1 = [&](int pc) { return ws_bytes(abs_bwd_spec(pc, D, N, M, C)); };
+    auto b1 = [&](int pc) { return std::max(ws_bytes(abs_bwd_spec(pc, D, N, M, C)), col_bwd_bytes(pc, D, N, M, C)); };
     return plan_bytes(plan_chunks(P, g_ws_budget.load(std::memory_order_relaxed), pipelined(P, D, N), b1), b1);
 }
 
@@ -989,6 +1059,16 @@ int abs_bwd_impl(const float* q, const float* k, const float* v, const float* g_
     hipStream_t st = (hipStream_t)stream;
     if (dense_sign(P, N, M))     // the walks' convention: a tie counts -1 in both gradients
         return dense_bwd(-1.f, q, k, v, g_w, g_u, grad_q, grad_k, grad_v, P, D, N, M, C, st);
+    if (col_bwd_applies(D, N, M)) {
+        if (int e = check_ws(ws, ws_bytes_given, col_bwd_bytes(1, D, N, M, C))) return e;
+        return run_bwd_columns(v, g_w, g_u, 2.f, grad_q, grad_k, grad_v, P, D, N, M, C, ws, ws_bytes_given, st,
+            [&](int p0, int np, SortedWs& w, hipStream_t s) {
+                const size_t p = (size_t)p0;
+                if (!pre) return sort_both(q + p * D * M, k + p * D * N, w, np * D, N, M, s);
+                const Presorted ps = offset(*pre, p, D, N, M);
+                w.ks = ps.ks; w.kp = ps.kp; w.qs = ps.qs; w.qp = ps.qp;
+                return (int)QLKA_OK; });
+    }
     if (mbw_applies(C))
         return abs_bwd_mbw(q, k, v, g_w, g_u, grad_q, grad_k, grad_v, P, D, N, M, C, pre, ws, ws_bytes_given, st);
     auto b1 = [&](int pc) { return ws_bytes(abs_bwd_spec(pc, D, N, M, C)); };
@@ -1080,7 +1160,8 @@ static WsSpec sgn_spec(int P, int D, int N, int M, int C) { return WsSpec{P, D, 
 size_t qlka_sgn_fwd_ws_bytes(int P, int D, int N, int M, int C) {
     if (P <= 0 || D <= 0 || N <= 0 || M <= 0 || C <= 0) return 0;
     if (dense_sign(P, N, M)) return 0;            // the dense route takes no workspace
-    return budget_bytes(P, [&](int pc) { return ws_bytes(sgn_spec(pc, D, N, M, C)); });
+    return budget_bytes(P, [&](int pc) {
+        return std::max(ws_bytes(sgn_spec(pc, D, N, M, C)), col_bwd_bytes(pc, D, N, M, C)); });
 }
 
 int qlka_sgn_fwd(const float* q, const float* k, const float* v, const float* g, float* out,
@@ -1091,6 +1172,11 @@ int qlka_sgn_fwd(const float* q, const float* k, const float* v, const float* g,
     hipStream_t st = (hipStream_t)stream;
     if (dense_sign(P, N, M))     // sgn(k - q) with a tie counted +1 == -(s(q - k) with a tie counted -1)
         return hip_status(direct_sign(true, q, k, g, v, nullptr, out, -1.f, -1.f, P, D, M, N, C, st), "dense sgn sum");
+    if (col_bwd_applies(D, N, M))   // sgn(k - q) with a tie counted +1, as above: -grad_q
+        return run_bwd_columns(v, g, nullptr, -2.f, out, nullptr, nullptr, P, D, N, M, C, ws, ws_bytes_given, st,
+            [&](int p0, int np, SortedWs& w, hipStream_t s) {
+                const size_t p = (size_t)p0;
+                return sort_both(q + p * D * M, k + p * D * N, w, np * D, N, M, s); });
     auto bytes = [&](int pc) { return ws_bytes(sgn_spec(pc, D, N, M, C)); };
     const int pc = fit_chunk(P, ws_bytes_given, bytes);
     if (int e = check_ws(ws, ws_bytes_given, bytes(pc))) return e;

@@ -14,8 +14,9 @@
 // C / CH workgroups of a p read it, neighbours on one XCD at about the same time, so from its L2.
 //   val[s][E/4][T][4]   abs: the value less the thread's anchor, the end of its elements that lies towards the segment's
 //                       median key; Laplace: e^-distance to the previous element
-//   tag[s][E/4][T][4]   16-bit word index: m for query m, M + n for key n, N + M for padding
+//   tag[s][E/4][T][4]   16-bit word index: m for query m, K0 + n for key n, K0 + N for padding (K0 = M, or M rounded up)
 //   xe[s][T]            abs: each thread's anchor less the median key; Laplace: e^-(extent of its elements)
+//   eq[s][T]            (abs backward) bit e: element e of the thread has the value of the element before it
 // With 4 elements per 16-byte (8-byte) load, a wave's loads are contiguous.
 //
 // What bounds col_sum: per element and channel one LDS read and, for a query, one masked write at random addresses (about
@@ -25,6 +26,7 @@
 // (4.3 ms). Whole calls against the walk: abs 1.70 -> 1.40 ms, Laplace 1.69 -> 1.55 ms at that size, Laplace 0.81 ->
 // 0.58 ms at N = M = 8192, add_riesz 0.97 -> 0.68 ms at 24 x 3111.
 #include <algorithm>
+#include <utility>
 
 #include "qlka_common.h"
 #include "qlka_internal.h"
@@ -209,6 +211,24 @@ __device__ __forceinline__ float pick(float a, float b, uint64_t mask) {
     return r;
 }
 __device__ __forceinline__ float unless(float a, uint64_t mask) { return pick(a, 0.f, mask); }
+// All ones where bit e of x is set, else 0; and b where m is all ones, a where it is 0. As asm, or the compiler turns the
+// bits of a loop into one lane mask each, more than there are scalar registers.
+template <int e>
+__device__ __forceinline__ uint32_t bit_mask(uint32_t x) {
+    uint32_t r;
+    asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(r) : "v"(x), "n"(e));
+    return r;
+}
+__device__ __forceinline__ float bit_pick(float a, float b, uint32_t m) {
+    float r;
+    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(r) : "v"(m), "v"(b), "v"(a));
+    return r;
+}
+// f(integral_constant<int, 0>) ... f(integral_constant<int, E - 1>)
+template <class F, int... I>
+__device__ __forceinline__ void each_of(F f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+template <int E, class F>
+__device__ __forceinline__ void each(F f) { each_of(f, std::make_integer_sequence<int, E>{}); }
 
 // ---------------------------------------------------------------------------------------------------------------
 // col_merge: one workgroup per segment
@@ -220,9 +240,9 @@ __device__ __forceinline__ float decay(float x) { return x < 0.5f ? 1.f + expm1f
 struct ColMergeArgs {
     const float* qs; const uint32_t* qp; const float* ks; const uint32_t* kp;   // sorted queries and keys
     const uint8_t* keep;             // (P, N) key mask or null: masked keys weigh 0 in the v == 1 terms
-    float* val; uint16_t* tag; float* xe;
+    float* val; uint16_t* tag; float* xe; uint32_t* eq;      // eq: null unless wanted
     float* u;                        // (S, M) v == 1 terms in query order, or null
-    int D, N, M;
+    int D, N, M, K0;
 };
 
 // dynamic LDS: N + M words (values, then word indices, then the v == 1 terms), then the scan's aggregates
@@ -260,6 +280,7 @@ void col_merge(const ColMergeArgs A)
     else prev = fmaxf(sq[i - 1], sk[j - 1]);
     const float xs = prev;
     float qa = sq[min(i, M - 1)], kb = sk[min(j, N - 1)];
+    uint32_t eq = 0;
     float dist[E];                      // abs: the element's value; Laplace: its distance to the previous element
     int src[E];                         // word of the element in sq / sk
 #pragma unroll
@@ -268,6 +289,7 @@ void col_merge(const ColMergeArgs A)
         const bool tq = j >= N || (i < M && qa <= kb);
         const float r = tq ? qa : kb;
         src[e] = live ? (tq ? i : M + j) : n;
+        if (live && diag + e > 0 && r == prev) eq |= 1u << e;
         if constexpr (KIND == COL_LAPLACE) dist[e] = (live && r != prev) ? r - prev : 0.f;   // equal infinities: 0 apart
         else dist[e] = live ? r : prev;
         if (live) {
@@ -285,11 +307,12 @@ void col_merge(const ColMergeArgs A)
 #pragma unroll 8
         for (int x = tid; x < M; x += T) w[x] = qp[x];
 #pragma unroll 8
-        for (int x = tid; x < N; x += T) w[M + x] = M + kp[x];
+        for (int x = tid; x < N; x += T) w[M + x] = A.K0 + kp[x];
         __syncthreads();
 #pragma unroll
-        for (int e = 0; e < E; ++e) src[e] = src[e] < n ? (int)w[src[e]] : n;
+        for (int e = 0; e < E; ++e) src[e] = src[e] < n ? (int)w[src[e]] : A.K0 + N;
     }
+    if (A.eq) A.eq[(size_t)s * T + tid] = eq;
     // A thread's values are taken relative to its anchor, so that where a gap splits its elements, those on the median's
     // side stay precise: every value an element's sums are formed from is then bounded by distances to keys
     float anchor = 0.f;
@@ -327,8 +350,8 @@ void col_merge(const ColMergeArgs A)
     const uint8_t* keep = A.keep ? A.keep + (size_t)p * N : nullptr;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-        const bool key = src[e] >= M && src[e] < n;
-        wt[e] = key ? (keep ? (keep[src[e] - M] ? 1.f : 0.f) : 1.f) : 0.f;
+        const int key = src[e] - A.K0;
+        wt[e] = key >= 0 && key < N ? (keep ? (keep[key] ? 1.f : 0.f) : 1.f) : 0.f;
     }
     const int lane = lane_id(), wv = wave_in_block();
     float* agg = sm + n;
@@ -402,9 +425,9 @@ void col_merge(const ColMergeArgs A)
 // ---------------------------------------------------------------------------------------------------------------
 struct ColSumArgs {
     const float* val; const uint16_t* tag; const float* xe;
-    const float* w;                  // (P, C, Nw) weight columns (col_weights): of v, or of g_w with SWAP
+    const float* w;                  // [P][CW][Nw][CH] weight columns (col_weights): of v, or of g_w with SWAP
     float* out;                      // [P][DS][C][Ma]
-    int P, D, N, M, C, DS;
+    int P, D, N, M, C, DS, K0, CW;
 };
 
 // SWAP: the queries carry the weights and the keys the accumulators (the grad_v of the abs sums)
@@ -416,21 +439,20 @@ void col_sum(const ColSumArgs A)
     extern __shared__ float sm[];
     const int tid = threadIdx.x, lane = lane_id(), wv = wave_in_block();
     const int D = A.D, N = A.N, M = A.M, C = A.C, DS = A.DS;
-    const int Nw = SWAP ? M : N, Ma = SWAP ? N : M, w0 = SWAP ? 0 : M, a0 = SWAP ? M : 0;
+    const int Nw = SWAP ? M : N, Ma = SWAP ? N : M, w0 = SWAP ? 0 : A.K0, a0 = SWAP ? A.K0 : 0;
     const int CG = (C + CH - 1) / CH;
     const int b = xcd_slice_block(blockIdx.x, gridDim.x);
     const int p = b / (DS * CG), ds = (b / CG) % DS, c = (b % CG) * CH;
     const int d0 = (int)((long)D * ds / DS), d1 = (int)((long)D * (ds + 1) / DS);
-    // LDS words: [N + M + 1][CH] (the last: padding's), then the aggregates of two features
-#pragma unroll
-    for (int h = 0; h < CH; ++h) {
-        const float* wp = A.w + ((size_t)p * C + min(c + h, C - 1)) * Nw;
+    // LDS words: [K0 + N + 1][CH] (the last: padding's), then the aggregates of two features
+    {
+        const float* wp = A.w + ((size_t)p * A.CW + c / CH) * Nw * CH;
 #pragma unroll 8
-        for (int i = tid; i < Nw; i += T) sm[(w0 + i) * CH + h] = wp[i];
+        for (int i = tid; i < Nw * CH; i += T) sm[w0 * CH + i] = wp[i];
     }
     for (int i = tid; i < Ma * CH; i += T) sm[a0 * CH + i] = 0.f;
-    if (tid < CH) sm[(N + M) * CH + tid] = 0.f;
-    const uint32_t aggb = ((uint32_t)(N + M + 1) * CH * 4 + 15) & ~15u;
+    if (tid < CH) sm[(A.K0 + N) * CH + tid] = 0.f;
+    const uint32_t aggb = ((uint32_t)(A.K0 + N + 1) * CH * 4 + 15) & ~15u;
     constexpr uint32_t AGGS = (KIND == COL_ABS ? 2 : 3) * CH * W * 4;    // bytes of one feature's aggregates
     __syncthreads();
     if (d0 >= d1) {                                      // more shares than features
@@ -458,7 +480,7 @@ void col_sum(const ColSumArgs A)
     for (int g = 0; g < E / 4; ++g) load(d0, g);
     const float* xp = A.xe + (s0 + d0) * T + tid;
     float xs = *xp;
-    const uint32_t split = (uint32_t)M * CH * 4;         // queries' words lie below, keys' above
+    const uint32_t split = (uint32_t)A.K0 * CH * 4;      // queries' words lie below, keys' above
     auto addr = [&](int e) { return tag_addr<CH * 4>(tg[e / 2], e & 1); };
     for (int d = d0; d < d1; ++d) {
         float a[E][CH];
@@ -654,18 +676,248 @@ void col_sum(const ColSumArgs A)
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// col_weights: the weight rows (P, Nw, C) as columns (P, C, Nw), masked rows 0
+// col_dot: one workgroup per segment (p, d), all channels: the gradients of the abs sums in q and k
+//
+//   grad_q[m] = sum_c g_mc (2 W_c - Wtot_c), W_c the sum of v_nc over the keys below q_m      (an equal key counts above)
+//   grad_k[n] = sum_c v_nc (2 G_c - Gtot_c), G_c the sum of g_mc over the queries below k_n   (an equal query counts above)
+//
+// The transposed loop of col_sum: a segment's merged order stays in registers (tags, and each element's running dot
+// product), and the columns of g_w and v of one channel group after another go through LDS (copied there without
+// registers while the previous group's arithmetic finishes). Per element and channel one random LDS read, two running
+// sums and two multiply-adds. With g_u there is one more channel, g_u against ones.
+// Queries come before equal keys in the merged order, so W is right as it runs; G is taken where the key's run of equal
+// values began: kept as the thread goes, and where a run crosses threads (else a workgroup skips it) through LDS from the
+// thread in which it began.
+// ---------------------------------------------------------------------------------------------------------------
+struct ColDotArgs {
+    const uint16_t* tag; const uint32_t* eq;
+    const float* gt; const float* vt;        // [P][CW][M][CH], [P][CW][N][CH]
+    float* gq; float* gk;                    // (P, D, M) and, or null, (P, D, N)
+    float* sums;                             // [S][E/4][T][4] scratch: the dot products, where they are not in registers
+    float scale;                             // 2, or -2 for the sgn sum
+    int D, N, M, K0, NP, CW;                 // NP: keys' words, N rounded up like K0
+};
+
+template <int T, int E, int CH>
+__global__ __launch_bounds__(T, 4)
+void col_dot(const ColDotArgs A)
+{
+    constexpr int W = T / WAVE;
+    extern __shared__ float sm[];
+    const int tid = threadIdx.x, lane = lane_id(), wv = wave_in_block();
+    const int s = xcd_slice_block(blockIdx.x, gridDim.x), p = s / A.D;
+    const int N = A.N, M = A.M, K0 = A.K0;
+    // LDS words: queries [K0][CH], keys [NP + 1][CH], then aggregates [W][2 CH], then run starts [T][CH]
+    const uint32_t aggb = ((uint32_t)(K0 + A.NP + 1) * CH * 4 + 15) & ~15u;
+    const uint32_t runb = aggb + W * 2 * CH * 4;
+    if (tid < CH) sm[(K0 + A.NP) * CH + tid] = 0.f;          // padding's word where N fills its region
+
+    uint32_t tg[E / 2];
+    {
+        const u2_t* tp = (const u2_t*)(A.tag + (size_t)s * T * E) + tid;
+#pragma unroll
+        for (int g = 0; g < E / 4; ++g) {
+            const u2_t y = tp[(size_t)g * T];
+            tg[2 * g] = y.x;
+            tg[2 * g + 1] = y.y;
+        }
+    }
+    const uint32_t split = (uint32_t)K0 * CH * 4;
+    auto addr = [&](int e) { return tag_addr<CH * 4>(tg[e / 2], e & 1); };
+    uint64_t isq[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) isq[e] = __ballot(addr(e) < split);
+
+    // runs of equal values within the thread (eq), and the elements that continue the run before it (cont)
+    constexpr uint32_t FULL = E == 32 ? 0xffffffffu : (1u << E) - 1;
+    const uint32_t eq = A.eq[(size_t)s * T + tid];
+    const uint32_t cont = eq & ~(eq + 1);                    // trailing ones: elements of the run from before
+    // the last thread before this one in which a run starts
+    int from = 0;
+    bool crossing = false;                                   // some run crosses threads
+    {
+        int* any = (int*)((char*)sm + aggb);
+        const uint64_t b = __ballot(eq & 1);
+        if (lane == 0) any[wv] = b != 0;
+        __syncthreads();
+        for (int i = 0; i < W; ++i) crossing |= any[i] != 0;
+        crossing = uniform_u32(crossing) != 0;
+        __syncthreads();
+    }
+    if (crossing) {
+        int x = eq != FULL ? tid : -1;
+#pragma unroll
+        for (int off = 1; off < WAVE; off <<= 1) {
+            const int y = __shfl_up(x, off, WAVE);
+            if (lane >= off) x = max(x, y);
+        }
+        int* last = (int*)((char*)sm + aggb);
+        if (lane == WAVE - 1) last[wv] = x;
+        int ex = __shfl_up(x, 1, WAVE);
+        if (lane == 0) ex = -1;
+        __syncthreads();
+        for (int i = 0; i < wv; ++i) ex = max(ex, last[i]);
+        from = max(ex, 0);
+    }
+
+    // one channel group's columns into LDS: chunks of 64 x 16 bytes, shared out over the waves; lanes past a column read 0
+    auto fetch = [&](int cg) {
+        const rsrc_t rg = make_rsrc(A.gt + ((size_t)p * A.CW + cg) * M * CH, (uint32_t)(M * CH * 4));
+        const rsrc_t rv = make_rsrc(A.vt + ((size_t)p * A.CW + cg) * N * CH, (uint32_t)(N * CH * 4));
+        const int qc = K0 * CH / 256, kc = A.NP * CH / 256;
+        for (int i = wv; i < qc; i += W)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rg, (LDS_AS void*)(uint32_t)(i * 1024), 16, lane * 16, i * 1024, 0, 0);
+        for (int i = wv; i < kc; i += W)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (LDS_AS void*)(uint32_t)((qc + i) * 1024), 16, lane * 16, i * 1024,
+                                                     0, 0);
+    };
+    // The dot products over 8 groups at a time, then over those: sequential sums over all channels lost half a digit. The
+    // latter in memory where registers do not hold both (spilled, their reloads would wait for the columns in flight).
+    constexpr bool IN_MEMORY = CH == 1 && E > 24;
+    float sum[IN_MEMORY ? 1 : E], part[E];
+    f4_t* sums = (f4_t*)(A.sums + (size_t)s * T * E) + tid;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        part[e] = 0.f;
+        if constexpr (!IN_MEMORY) sum[e] = 0.f;
+    }
+    __syncthreads();
+    fetch(0);
+    for (int cg = 0; cg < A.CW; ++cg) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        float a[E][CH];
+        constexpr int AHEAD = CH == 1 ? 12 : E;              // as in col_sum
+#pragma unroll
+        for (int e = 0; e < AHEAD && e < E; ++e) lds_read<CH>(a[e], addr(e));
+        uint32_t eqc = eq, contc = cont;
+        asm volatile("" : "+v"(eqc), "+v"(contc));           // their bits' masks are formed here, not kept from channel to channel
+        float w[CH], g[CH], gr[CH];                          // running W and G, G where the element's run of equals began
+#pragma unroll
+        for (int h = 0; h < CH; ++h) w[h] = g[h] = gr[h] = 0.f;
+        each<E>([&](auto ec) {
+            constexpr int e = ec();
+            if constexpr (CH == 1 && (e & 3) == 0) {
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = e + AHEAD; i < e + AHEAD + 4 && i < E; ++i) lds_read<CH>(a[i], addr(i));
+            }
+            const uint32_t same = bit_mask<e>(eqc);
+#pragma unroll
+            for (int h = 0; h < CH; ++h) {
+                gr[h] = e > 0 ? bit_pick(g[h], gr[h], same) : 0.f;
+                part[e] = fmaf(a[e][h], pick(gr[h], w[h], isq[e]), part[e]);
+                w[h] += unless(a[e][h], isq[e]);
+                g[h] += pick(0.f, a[e][h], isq[e]);
+            }
+            asm("" : "+v"(part[e]));
+        });
+        float w0[CH], g0[CH], wt[CH], gt[CH];
+#pragma unroll
+        for (int h = 0; h < CH; ++h) {
+            w0[h] = wave_scan_sum(w[h]);
+            g0[h] = wave_scan_sum(g[h]);
+        }
+        if (lane == WAVE - 1) {
+#pragma unroll
+            for (int h = 0; h < CH; ++h) {
+                f2_t x;
+                x.x = w0[h];
+                x.y = g0[h];
+                *(LDS_AS f2_t*)(aggb + (wv * CH + h) * 8) = x;
+            }
+        }
+        __syncthreads();                                     // every wave has its words: the next group may land
+        if (cg + 1 < A.CW) fetch(cg + 1);
+        const int el = min(lane & 15, W - 1);
+#pragma unroll
+        for (int h = 0; h < CH; ++h) {
+            const f2_t x = *(LDS_AS const f2_t*)(aggb + (el * CH + h) * 8);
+            const float ww = row_scan_sum<W>(x.x), gg = row_scan_sum<W>(x.y);
+            wt[h] = bcast(ww, W - 1);
+            gt[h] = bcast(gg, W - 1);
+            w0[h] += (wv ? bcast(ww, wv ? wv - 1 : 0) : 0.f) - w[h];
+            g0[h] += (wv ? bcast(gg, wv ? wv - 1 : 0) : 0.f) - g[h];
+        }
+#pragma unroll
+        for (int h = 0; h < CH; ++h) {
+            w0[h] = fmaf(-0.5f, wt[h], w0[h]);
+            gt[h] *= -0.5f;
+        }
+        if (!crossing) {
+#pragma unroll
+            for (int h = 0; h < CH; ++h) g0[h] += gt[h];
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+#pragma unroll
+                for (int h = 0; h < CH; ++h) part[e] = fmaf(a[e][h], pick(g0[h], w0[h], isq[e]), part[e]);
+        } else {
+            float gc[CH];                                    // G where the run from before began
+#pragma unroll
+            for (int h = 0; h < CH; ++h) *(LDS_AS float*)(runb + (tid * CH + h) * 4) = g0[h] + gr[h];
+            __syncthreads();
+#pragma unroll
+            for (int h = 0; h < CH; ++h) {
+                gc[h] = *(LDS_AS const float*)(runb + (from * CH + h) * 4) + gt[h];
+                g0[h] += gt[h];
+            }
+#pragma unroll
+            for (int h = 0; h < CH; ++h)
+                each<E>([&](auto ec) {
+                    constexpr int e = ec();
+                    const float z = bit_pick(g0[h], gc[h], bit_mask<e>(contc));
+                    part[e] = fmaf(a[e][h], pick(z, w0[h], isq[e]), part[e]);
+                });
+        }
+        if ((cg & 7) == 7 && cg + 1 < A.CW) {
+            if constexpr (IN_MEMORY) {
+#pragma unroll
+                for (int g4 = 0; g4 < E / 4; ++g4) {
+                    f4_t x = {part[4 * g4], part[4 * g4 + 1], part[4 * g4 + 2], part[4 * g4 + 3]};
+                    if (cg > 7) x += sums[(size_t)g4 * T];
+                    sums[(size_t)g4 * T] = x;
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                if constexpr (!IN_MEMORY) sum[e] += part[e];
+                part[e] = 0.f;
+            }
+        }
+    }
+    __syncthreads();                                         // every wave has read its last words
+#pragma unroll
+    for (int e = 0; e < E; ++e) {                            // to query and key order through LDS (one word per element)
+        const uint32_t t = tg[e / 2];
+        float x = part[e];
+        if constexpr (!IN_MEMORY) x += sum[e];
+        else if (A.CW > 8) x += sums[(size_t)(e / 4) * T][e % 4];
+        sm[(e & 1) ? t >> 16 : t & 0xffffu] = A.scale * x;
+    }
+    __syncthreads();
+    float* gq = A.gq + (size_t)s * M;
+    for (int i = tid; i < M; i += T) gq[i] = sm[i];
+    if (A.gk) {
+        float* gk = A.gk + (size_t)s * N;
+        for (int i = tid; i < N; i += T) gk[i] = sm[K0 + i];
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// col_weights: the weight rows (P, Nw, C) as columns [P][CW][Nw][CH], masked rows 0. With C1 = C + 1 there is one more
+// channel, `extra` (P, Nw) or all ones.
 // ---------------------------------------------------------------------------------------------------------------
 constexpr int CF_T = 256, CF_M = 64;        // threads, rows per workgroup (also of col_finish)
 
+template <int CH>
 __global__ __launch_bounds__(CF_T)
-void col_weights(const float* __restrict__ w, const uint8_t* __restrict__ keep, float* __restrict__ out, const int Nw,
-                 const int C)
+void col_weights(const float* __restrict__ w, const float* __restrict__ extra, const uint8_t* __restrict__ keep,
+                 float* __restrict__ out, const int Nw, const int C, const int C1)
 {
-    __shared__ float tile[128][CF_M + 1];
+    __shared__ float tile[130][CF_M + 1];
     const int nb = (Nw + CF_M - 1) / CF_M;
     const int p = blockIdx.x / nb, n0 = (blockIdx.x - p * nb) * CF_M;
-    const int rows = min(CF_M, Nw - n0);
+    const int rows = min(CF_M, Nw - n0), CW = (C1 + CH - 1) / CH;
     const float* src = w + ((size_t)p * Nw + n0) * C;
     int r = threadIdx.x / C, c = threadIdx.x - r * C;
     const int dr = CF_T / C, dc = CF_T - dr * C;
@@ -676,11 +928,22 @@ void col_weights(const float* __restrict__ w, const uint8_t* __restrict__ keep, 
         c += dc;
         if (c >= C) { c -= C; ++r; }
     }
-    __syncthreads();
     const int lane = threadIdx.x & (CF_M - 1);
-    float* dst = out + (size_t)p * C * Nw + n0;
-    if (lane < rows)
-        for (int cc = threadIdx.x / CF_M; cc < C; cc += CF_T / CF_M) dst[(size_t)cc * Nw + lane] = tile[cc][lane];
+    for (int cc = C + threadIdx.x / CF_M; cc < CW * CH; cc += CF_T / CF_M)
+        if (lane < rows) tile[cc][lane] = cc < C1 ? (extra ? extra[(size_t)p * Nw + n0 + lane] : 1.f) : 0.f;
+    __syncthreads();
+    if (lane >= rows) return;
+    float* dst = out + ((size_t)p * CW * Nw + n0 + lane) * CH;
+    for (int g = threadIdx.x / CF_M; g < CW; g += CF_T / CF_M) {
+        if constexpr (CH == 1) {
+            dst[(size_t)g * Nw] = tile[g][lane];
+        } else {
+            f2_t x;
+            x.x = tile[2 * g][lane];
+            x.y = tile[2 * g + 1][lane];
+            *(f2_t*)(dst + (size_t)g * Nw * 2) = x;
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -755,6 +1018,14 @@ size_t sum_lds(int kind, int T, int CH, int n) {
     return (((size_t)(n + 1) * CH * 4 + 15) & ~size_t(15)) + 2 * (size_t)(kind == COL_ABS ? 2 : 3) * CH * (T / WAVE) * 4;
 }
 
+// words of a region rounded up to the 1 KB chunks col_dot copies
+int pad_words(int n, int CH) { return (n + 256 / CH - 1) / (256 / CH) * (256 / CH); }
+
+size_t dot_lds(int T, int CH, int N, int M) {
+    const size_t words = ((size_t)(pad_words(M, CH) + pad_words(N, CH) + 1) * CH * 4 + 15) & ~size_t(15);
+    return words + (size_t)(T / WAVE) * 2 * CH * 4 + (size_t)T * CH * 4;
+}
+
 // Workgroups of one col_sum launch that a CU holds at once: by LDS, and by the wave slots of 4 waves per SIMD (128 VGPRs)
 int wgs_per_cu(int kind, int T, int CH, int n) {
     return std::max(1, std::min((int)(LDS_BYTES / sum_lds(kind, T, CH, n)), 1024 / T));
@@ -795,10 +1066,19 @@ ColPlan col_plan(int kind, int P, int D, int N, int M, int C) {
     return pl;
 }
 
+// The plan of the abs backward's stream: col_dot's LDS also holds the regions' padding and the run starts.
+bool col_bwd_applies(int D, int N, int M) {
+    if (!col_applies(D, N, M)) return false;
+    const ColPlan pl = col_plan(COL_ABS, 1, D, N, M, 2);
+    return dot_lds(pl.T, pl.CH, N, M) <= LDS_BYTES && sum_lds(COL_ABS, pl.T, pl.CH, pad_words(M, pl.CH) + N) <= LDS_BYTES;
+}
+
+int col_key0(const ColPlan& pl, int M) { return pad_words(M, pl.CH); }
+
 size_t col_stream_bytes(const ColPlan& pl, int S) {
     const size_t L = (size_t)pl.T * pl.E;
     auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
-    return al((size_t)S * L * 4) + al((size_t)S * L * 2) + al((size_t)S * pl.T * 4);
+    return al((size_t)S * L * 4) + al((size_t)S * L * 2) + 2 * al((size_t)S * pl.T * 4);
 }
 
 ColStream col_stream(const ColPlan& pl, void* base, int S) {
@@ -808,7 +1088,8 @@ ColStream col_stream(const ColPlan& pl, void* base, int S) {
     ColStream r;
     r.val = (float*)b;     b += al((size_t)S * L * 4);
     r.tag = (uint16_t*)b;  b += al((size_t)S * L * 2);
-    r.xe = (float*)b;
+    r.xe = (float*)b;      b += al((size_t)S * pl.T * 4);
+    r.eq = (uint32_t*)b;
     return r;
 }
 
@@ -848,7 +1129,7 @@ int launch_sum(const ColSumArgs& a, hipStream_t st) {
     static const hipError_t once = allow_lds(col_sum<KIND, T, E, CH, SWAP, 4>);
     if (once != hipSuccess) return (int)once;
     const unsigned blocks = (unsigned)(a.P * a.DS * ((a.C + CH - 1) / CH));
-    hipLaunchKernelGGL((col_sum<KIND, T, E, CH, SWAP, 4>), dim3(blocks), dim3(T), sum_lds(KIND, T, CH, a.N + a.M), st, a);
+    hipLaunchKernelGGL((col_sum<KIND, T, E, CH, SWAP, 4>), dim3(blocks), dim3(T), sum_lds(KIND, T, CH, a.K0 + a.N), st, a);
     return (int)hipGetLastError();
 }
 
@@ -856,26 +1137,50 @@ int launch_sum(const ColSumArgs& a, hipStream_t st) {
 
 int col_merge_launch(int kind, const ColPlan& pl, const float* qs, const uint32_t* qp, const float* ks,
                      const uint32_t* kp, const uint8_t* keep, ColStream str, float* u, int S, int D, int N, int M,
-                     hipStream_t st) {
-    const ColMergeArgs a{qs, qp, ks, kp, keep, str.val, str.tag, str.xe, u, D, N, M};
+                     bool bwd, hipStream_t st) {
+    const ColMergeArgs a{qs, qp, ks, kp, keep, str.val, str.tag, str.xe, bwd ? str.eq : nullptr, u, D, N, M,
+                         bwd ? col_key0(pl, M) : M};
     StageTimer t("col_merge", st);
     return dispatch_shape(pl, [&](auto T, auto E, auto) {
         return kind == COL_ABS ? launch_merge<COL_ABS, T(), E()>(a, S, st) : launch_merge<COL_LAPLACE, T(), E()>(a, S, st); });
 }
 
-int col_weights_launch(const float* w, const uint8_t* keep, float* wt, int P, int Nw, int C, hipStream_t st) {
+int col_weights_launch(const ColPlan& pl, const float* w, const uint8_t* keep, bool more, const float* extra, float* wt,
+                       int P, int Nw, int C, hipStream_t st) {
     StageTimer t("col_weights", st);
-    hipLaunchKernelGGL(col_weights, dim3((unsigned)(P * ((Nw + CF_M - 1) / CF_M))), dim3(CF_T), 0, st, w, keep, wt, Nw, C);
+    const dim3 grid((unsigned)(P * ((Nw + CF_M - 1) / CF_M)));
+    if (pl.CH == 2)
+        hipLaunchKernelGGL(col_weights<2>, grid, dim3(CF_T), 0, st, w, extra, keep, wt, Nw, C, C + (more ? 1 : 0));
+    else
+        hipLaunchKernelGGL(col_weights<1>, grid, dim3(CF_T), 0, st, w, extra, keep, wt, Nw, C, C + (more ? 1 : 0));
     return (int)hipGetLastError();
 }
 
 int col_sum_launch(int kind, const ColPlan& pl, ColStream str, const float* wt, float* cols, int P, int D, int N, int M,
                    int C, hipStream_t st) {
-    const ColSumArgs a{str.val, str.tag, str.xe, wt, cols, P, D, N, M, C, pl.DS};
+    const ColSumArgs a{str.val, str.tag, str.xe, wt, cols, P, D, N, M, C, pl.DS, M, (C + pl.CH - 1) / pl.CH};
     StageTimer t(kind == COL_ABS ? "col_sum_abs" : "col_sum_laplace", st);
     return dispatch_shape(pl, [&](auto T, auto E, auto CH) {
         return kind == COL_ABS ? launch_sum<COL_ABS, T(), E(), CH(), false>(a, st)
                                : launch_sum<COL_LAPLACE, T(), E(), CH(), false>(a, st); });
+}
+
+int col_grad_v_launch(const ColPlan& pl, ColStream str, const float* gt, int CW, float* cols, int P, int D, int N, int M,
+                      int C, hipStream_t st) {
+    const ColSumArgs a{str.val, str.tag, str.xe, gt, cols, P, D, N, M, C, pl.DS, col_key0(pl, M), CW};
+    StageTimer t("col_grad_v", st);
+    return dispatch_shape(pl, [&](auto T, auto E, auto CH) { return launch_sum<COL_ABS, T(), E(), CH(), true>(a, st); });
+}
+
+int col_dot_launch(const ColPlan& pl, ColStream str, const float* gt, const float* vt, int CW, float scale, float* gq,
+                   float* gk, int S, int D, int N, int M, hipStream_t st) {
+    const ColDotArgs a{str.tag, str.eq, gt, vt, gq, gk, str.val, scale, D, N, M, col_key0(pl, M), pad_words(N, pl.CH), CW};
+    StageTimer t("col_dot", st);
+    return dispatch_shape(pl, [&](auto T, auto E, auto CH) {
+        static const hipError_t once = allow_lds(col_dot<T(), E(), CH()>);
+        if (once != hipSuccess) return (int)once;
+        hipLaunchKernelGGL((col_dot<T(), E(), CH()>), dim3((unsigned)S), dim3(T()), dot_lds(T(), CH(), N, M), st, a);
+        return (int)hipGetLastError(); });
 }
 
 int col_finish_launch(int kind, int layer, bool masked, const ColPlan& pl, const float* cols, const float* u, float* out,

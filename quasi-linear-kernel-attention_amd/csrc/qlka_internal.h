@@ -263,17 +263,28 @@ constexpr int COL_MAX = 32768;           // 32 elements for each of 1024 threads
 constexpr int COL_MAX2 = 20352;          // two channels per workgroup: 2 words of LDS per element
 constexpr int COL_SHARES = 16;           // most shares of the features
 struct ColPlan { int T, E, CH, DS; };    // threads, elements per thread, channels per workgroup, shares of the features
-struct ColStream { float* val; uint16_t* tag; float* xe; };
+struct ColStream { float* val; uint16_t* tag; float* xe; uint32_t* eq; };
 bool col_applies(int D, int N, int M);
 ColPlan col_plan(int kind, int P, int D, int N, int M, int C);      // kind 0 abs, 1 Laplace (as below)
 size_t col_stream_bytes(const ColPlan& pl, int S);
 ColStream col_stream(const ColPlan& pl, void* base, int S);
-// the merged stream of S sorted segments, and the v == 1 terms u (S, M) in query order (null: none; masked keys weigh 0)
+// the merged stream of S sorted segments, and the v == 1 terms u (S, M) in query order (null: none; masked keys weigh 0).
+// bwd: the stream of the abs backward (keys' words from col_key0, runs of equal values).
 int col_merge_launch(int kind, const ColPlan& pl, const float* qs, const uint32_t* qp, const float* ks,
                      const uint32_t* kp, const uint8_t* keep, ColStream str, float* u, int S, int D, int N, int M,
-                     hipStream_t st);
-// wt (P, C, Nw) from rows w (P, Nw, C), rows masked by keep (null: none) 0
-int col_weights_launch(const float* w, const uint8_t* keep, float* wt, int P, int Nw, int C, hipStream_t st);
+                     bool bwd, hipStream_t st);
+// wt: the columns of rows w (P, Nw, C) in groups of pl.CH, rows masked by keep (null: none) 0; `more`: one more channel,
+// extra (P, Nw) or ones
+int col_weights_launch(const ColPlan& pl, const float* w, const uint8_t* keep, bool more, const float* extra, float* wt,
+                       int P, int Nw, int C, hipStream_t st);
+// The abs backward over a bwd stream and the columns gt, vt (CW groups each) of g_w and v: cols[P][DS][C][N] = half of
+// grad_v; and gq = scale / 2 times grad_q, gk (or null) the same of grad_k (last: it overwrites str.val)
+bool col_bwd_applies(int D, int N, int M);
+int col_key0(const ColPlan& pl, int M);
+int col_grad_v_launch(const ColPlan& pl, ColStream str, const float* gt, int CW, float* cols, int P, int D, int N, int M,
+                      int C, hipStream_t st);
+int col_dot_launch(const ColPlan& pl, ColStream str, const float* gt, const float* vt, int CW, float scale, float* gq,
+                   float* gk, int S, int D, int N, int M, hipStream_t st);
 // cols[P][DS][C][M]: the sums of each feature share over the weights wt (P, C, N); half of them for kind 0
 int col_sum_launch(int kind, const ColPlan& pl, ColStream str, const float* wt, float* cols, int P, int D, int N, int M,
                    int C, hipStream_t st);
