@@ -463,14 +463,14 @@ int run_pipeline(int P, const Plan& pl, void* ws, size_t copy, hipStream_t st, P
 // larger of the two.
 struct ColWs { SortedWs s; ColStream str; float* u; float* cols; float* wt; char* extra; };
 
-size_t col_part(const ColPlan& pl, int P, int D, int N, int M, int C, int i) {
+size_t col_part(const ColPlan& pl, int P, int D, int N, int M, int C, int sets, int i) {
     const size_t S = (size_t)P * D;
     switch (i) {
         case 0: case 1: return align256(S * N * 4);
         case 2: case 3: return align256(S * M * 4);
         case 4: return align256(sort_scratch_need(WsSpec{P, D, N, M, C, N, 0, false}));
-        case 5: return align256(col_stream_bytes(pl, (int)S));
-        case 6: return align256(S * M * 4);
+        case 5: return align256(col_stream_bytes(pl, (int)S * sets));
+        case 6: return align256(S * sets * M * 4);
         case 7: return align256((size_t)P * pl.DS * C * M * 4);
         case 8: return align256((size_t)P * (C + 1) * N * 4);
     }
@@ -481,24 +481,24 @@ constexpr int COL_PARTS = 9;
 
 // Workspace of a chunk of P p, the columns sized for the most feature shares: their number depends on the whole call's P,
 // and neither the sizes nor (the plan being the whole call's) the results may depend on the chunking.
-size_t col_bytes(int kind, int P, int D, int N, int M, int C) {
-    if (!col_applies(D, N, M)) return 0;
+size_t col_bytes(int kind, int P, int D, int N, int M, int C, int sets = 1) {
+    if (!col_applies(D * sets, N, M)) return 0;
     ColPlan pl = col_plan(kind, 1, D, N, M, C);
     pl.DS = std::min(D, COL_SHARES);
     size_t b = 0;
-    for (int i = 0; i < COL_PARTS; ++i) b += col_part(pl, P, D, N, M, C, i);
+    for (int i = 0; i < COL_PARTS; ++i) b += col_part(pl, P, D, N, M, C, sets, i);
     return b;
 }
 
-ColWs col_carve(ColPlan pl, void* ws, int P, int D, int N, int M, int C) {
+ColWs col_carve(ColPlan pl, void* ws, int P, int D, int N, int M, int C, int sets) {
     pl.DS = std::min(D, COL_SHARES);
     char* part[COL_PARTS];
     char* b = (char*)ws;
-    for (int i = 0; i < COL_PARTS; ++i) { part[i] = b; b += col_part(pl, P, D, N, M, C, i); }
+    for (int i = 0; i < COL_PARTS; ++i) { part[i] = b; b += col_part(pl, P, D, N, M, C, sets, i); }
     ColWs r{};
     r.s.ks = (float*)part[0]; r.s.kp = (uint32_t*)part[1]; r.s.qs = (float*)part[2]; r.s.qp = (uint32_t*)part[3];
     r.s.sort_scratch = part[4];
-    r.str = col_stream(pl, part[5], P * D);
+    r.str = col_stream(pl, part[5], P * D * sets);
     r.u = (float*)part[6];
     r.cols = (float*)part[7];
     r.wt = (float*)part[8];
@@ -509,24 +509,25 @@ ColWs col_carve(ColPlan pl, void* ws, int P, int D, int N, int M, int C) {
 // sort(p0, np, w, stream) leaves the sorted k and q in w.s; finish(p0, np, w, plan, stream) reads w.cols and w.u (null
 // without want_u). extra(np): bytes of the caller's own after the columns (w.extra).
 template <class Extra, class Sort, class Finish>
-int run_columns(int kind, const float* v, const uint8_t* keep, bool want_u, int P, int D, int N, int M, int C, void* ws,
+int run_columns(int kind, int sets, const float* v, const uint8_t* keep, bool want_u, int P, int D, int N, int M, int C, void* ws,
                 size_t given, hipStream_t st, Extra extra, Sort sort, Finish finish) {
-    const ColPlan pl = col_plan(kind, P, D, N, M, C);
-    auto bytes = [&](int pc) { return col_bytes(kind, pc, D, N, M, C) + extra(pc); };
+    ColPlan pl = col_plan(kind, P, D * sets, N, M, C);
+    pl.DS = std::min(pl.DS, std::min(D, COL_SHARES));        // as many as the workspace is sized for
+    auto bytes = [&](int pc) { return col_bytes(kind, pc, D, N, M, C, sets) + extra(pc); };
     const int pc = fit_chunk(P, given, bytes);
     if (int e = check_ws(ws, given, bytes(pc))) return e;
     return for_chunks(P, pc, [&](int p0, int np) {
-        ColWs w = col_carve(pl, ws, np, D, N, M, C);
+        ColWs w = col_carve(pl, ws, np, D, N, M, C, sets);
         if (!want_u) w.u = nullptr;
         const size_t p = (size_t)p0;
         if (int e = sort(p0, np, w, st)) return e;
         const uint8_t* kc = keep ? keep + p * N : nullptr;
         if (int e = col_merge_launch(kind, pl, w.s.qs, w.s.qp, w.s.ks, w.s.kp, kc, w.str, w.u, np * D, D, N, M, false,
-                                     st))
+                                     sets, st))
             return hip_status(e, "merge of q and k");
         if (int e = col_weights_launch(pl, v + p * N * C, kc, false, nullptr, w.wt, np, N, C, st))
             return hip_status(e, "weight columns");
-        if (int e = col_sum_launch(kind, pl, w.str, w.wt, w.cols, np, D, N, M, C, st))
+        if (int e = col_sum_launch(kind, pl, w.str, w.wt, w.cols, np, D, N, M, C, sets, st))
             return hip_status(e, "column sums");
         return finish(p0, np, w, pl, st); });
 }
@@ -583,7 +584,8 @@ int run_bwd_columns(const float* v, const float* g_w, const float* g_u, float sc
         const size_t p = (size_t)p0;
         const int CW = (C + (g_u ? 1 : 0) + pl.CH - 1) / pl.CH;
         if (int e = sorts(p0, np, w, st)) return e;
-        if (int e = col_merge_launch(0, pl, w.qs, w.qp, w.ks, w.kp, nullptr, str, nullptr, np * D, D, N, M, true, st))
+        if (int e = col_merge_launch(0, pl, w.qs, w.qp, w.ks, w.kp, nullptr, str, nullptr, np * D, D, N, M, true, 1,
+                                     st))
             return hip_status(e, "merge of q and k");
         if (int e = col_weights_launch(pl, v + p * N * C, nullptr, g_u != nullptr, nullptr, vt, np, N, C, st))
             return hip_status(e, "value columns");
@@ -643,7 +645,7 @@ int qlka_laplace_fwd(const float* q, const float* k, const float* v, float* out_
     const Plan pl = plan_chunks(P, ws_bytes_given, pipelined(P, D, M), b1);
     if (int e = check_ws(ws, ws_bytes_given, plan_bytes(pl, b1))) return e;
     if (col_applies(D, N, M))
-        return run_columns(1, v, nullptr, true, P, D, N, M, C, ws, ws_bytes_given, st, no_extra,
+        return run_columns(1, 1, v, nullptr, true, P, D, N, M, C, ws, ws_bytes_given, st, no_extra,
             [&](int p0, int np, ColWs& w, hipStream_t s) {
                 const size_t p = (size_t)p0;
                 return sort_both(q + p * D * M, k + p * D * N, w.s, np * D, N, M, s); },
@@ -773,7 +775,7 @@ int abs_fwd_impl(const float* q, const float* k, const float* v, float* out_w, f
     if (int e = check_ws(ws, ws_bytes_given, plan_bytes(pl, b1))) return e;
     // (the backward by columns reads no range states, so none are written; *kept still says that a buffer was taken)
     if (col_applies(D, N, M) && (!keep_states || col_bwd_applies(D, N, M))) {
-        const int e = run_columns(0, v, nullptr, out_u != nullptr, P, D, N, M, C, ws, ws_bytes_given, st, no_extra,
+        const int e = run_columns(0, 1, v, nullptr, out_u != nullptr, P, D, N, M, C, ws, ws_bytes_given, st, no_extra,
             [&](int p0, int np, ColWs& w, hipStream_t s) {
                 const size_t p = (size_t)p0;
                 if (keep_sorts) {
@@ -1297,21 +1299,23 @@ static bool layer_pipelined(int kind, int P, int D, int M, int C) {
     return (kind != LAYER_ADD_BUMP || reduce_folds_epilogue(M, C)) && pipelined(P, D, M);
 }
 
-// add_laplace / add_riesz by columns: the op's columns with the layer's epilogue in their finish. Masked keys weigh 0;
+// The layers by columns: the op's columns with the layer's epilogue in their finish; add_bump's three abs sums as three
+// weighted streams per feature into one accumulator. Masked keys weigh 0;
 // their sort values are replaced as for the walks (mask_keys, fill_masked_keys), so that whatever they hold, the distances
 // run between kept keys.
 static size_t layer_col_extra(int kind, int P, int D, int N, int M, int C) {
-    return align256((size_t)P * M * 4) + (kind == LAYER_ADD_RIESZ ? align256(riesz_prefix_bytes(P, N, C))
-                                                                  : align256((size_t)P * D * N * 4));
+    return align256((size_t)P * M * 4) + (kind == LAYER_ADD_RIESZ     ? align256(riesz_prefix_bytes(P, N, C))
+                                          : kind == LAYER_ADD_LAPLACE ? align256((size_t)P * D * N * 4) : 0);
 }
 
-static bool col_layer(int kind, int D, int N, int M) { return kind != LAYER_ADD_BUMP && col_applies(D, N, M); }
+static bool col_layer(int kind, int D, int N, int M) { return col_applies(kind == LAYER_ADD_BUMP ? 3 * D : D, N, M); }
 
 // one chunk of P p, by columns or by ranges
 static size_t layer_ws(int kind, int P, int D, int N, int M, int C) {
     const size_t ranges = layer_ws_bytes(kind, WsSpec{P, D, N, M, C, N, M, true});
     if (!col_layer(kind, D, N, M)) return ranges;
-    return std::max(ranges, col_bytes(kind == LAYER_ADD_LAPLACE, P, D, N, M, C) + layer_col_extra(kind, P, D, N, M, C));
+    return std::max(ranges, col_bytes(kind == LAYER_ADD_LAPLACE, P, D, N, M, C, kind == LAYER_ADD_BUMP ? 3 : 1) +
+                            layer_col_extra(kind, P, D, N, M, C));
 }
 
 size_t qlka_layer_fwd_ws_bytes(int kind, int P, int D, int N, int M, int C) {
@@ -1382,20 +1386,21 @@ static int bump_chunk_unfolded(const float* q, const float* k, const float* v, c
 static int layer_columns(int kind, const float* q, const float* k, const float* v, const float* n_pad,
                          const uint8_t* keep, float* out, int P, int D, int N, int M, int C, void* ws, size_t given,
                          hipStream_t st) {
-    const bool riesz = kind == LAYER_ADD_RIESZ;
-    return run_columns(riesz ? 0 : 1, v, keep, true, P, D, N, M, C, ws, given, st,
+    const bool riesz = kind == LAYER_ADD_RIESZ, laplace = kind == LAYER_ADD_LAPLACE;
+    const int sets = kind == LAYER_ADD_BUMP ? 3 : 1;
+    return run_columns(laplace ? 1 : 0, sets, v, keep, true, P, D, N, M, C, ws, given, st,
         [&](int pc) { return layer_col_extra(kind, pc, D, N, M, C); },
         [&](int p0, int np, ColWs& w, hipStream_t s) {
             const size_t p = (size_t)p0;
             const float* kc = k + p * D * N;
             const uint8_t* keepc = keep ? keep + p * N : nullptr;
-            if (keepc && !riesz) {
+            if (keepc && laplace) {
                 float* km = (float*)(w.extra + align256((size_t)np * M * 4));
                 if (int e = hip_status(mask_keys(kc, keepc, km, np, D, N, s), "masked keys")) return e;
                 kc = km;
             }
             if (int e = sort_both(q + p * D * M, kc, w.s, np * D, N, M, s)) return e;
-            if (keepc && riesz) return hip_status(fill_masked_keys(w.s.ks, w.s.kp, keepc, np, D, N, s), "masked keys");
+            if (keepc && !laplace) return hip_status(fill_masked_keys(w.s.ks, w.s.kp, keepc, np, D, N, s), "masked keys");
             return (int)QLKA_OK; },
         [&](int p0, int np, ColWs& w, const ColPlan& cp, hipStream_t s) {
             const size_t p = (size_t)p0;
@@ -1407,7 +1412,8 @@ static int layer_columns(int kind, const float* q, const float* k, const float* 
             if (int e = layer_epilogue_params(kind, keep != nullptr, q + p * D * M, n_pad ? n_pad + p : nullptr, pre,
                                               (float*)w.extra, out + p * M * C, np, D, M, C, &ep, s))
                 return hip_status(e, "layer query terms");
-            return hip_status(col_finish_launch(riesz ? 0 : 1, kind, keep != nullptr, cp, w.cols, w.u, nullptr, nullptr, ep, np, D, M, C,
+            return hip_status(col_finish_launch(laplace ? 1 : 0, kind, keep != nullptr, cp, w.cols, w.u, nullptr, nullptr, ep, np,
+                                                D * sets, M, C,
                                                 s), "columns to rows"); });
 }
 

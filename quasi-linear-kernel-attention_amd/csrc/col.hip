@@ -243,7 +243,13 @@ struct ColMergeArgs {
     float* val; uint16_t* tag; float* xe; uint32_t* eq;      // eq: null unless wanted
     float* u;                        // (S, M) v == 1 terms in query order, or null
     int D, N, M, K0;
+    int sets;                        // 1, or 3: streams of q, q + 1 and q - 1 per segment (add_bump), their v == 1 terms weighted
 };
+
+// add_bump: max(0, 1 - |x|) = (|x + 1| + |x - 1|) / 2 - |x|, one feature's three abs sums after one another. The same sorted
+// order serves all three: adding a constant in fp32 is monotone.
+__device__ __forceinline__ float set_shift(int set) { return set == 0 ? 0.f : set == 1 ? 1.f : -1.f; }
+__device__ __forceinline__ float set_weight(int sets, int set) { return sets == 1 ? 1.f : set == 0 ? -1.f : 0.5f; }
 
 // dynamic LDS: N + M words (values, then word indices, then the v == 1 terms), then the scan's aggregates
 template <int KIND, int T, int E>
@@ -252,12 +258,13 @@ void col_merge(const ColMergeArgs A)
 {
     constexpr int W = T / WAVE;
     extern __shared__ float sm[];
-    const int s = blockIdx.x, p = s / A.D, tid = threadIdx.x;
+    const int s = blockIdx.x, seg = s / A.sets, p = seg / A.D, tid = threadIdx.x;     // stream, segment
     const int N = A.N, M = A.M, n = N + M;
-    const float* qs = A.qs + (size_t)s * M;
-    const float* ks = A.ks + (size_t)s * N;
+    const float* qs = A.qs + (size_t)seg * M;
+    const float* ks = A.ks + (size_t)seg * N;
+    const float shift = set_shift(s - seg * A.sets);
 #pragma unroll 8
-    for (int i = tid; i < M; i += T) sm[i] = qs[i];
+    for (int i = tid; i < M; i += T) sm[i] = qs[i] + shift;
 #pragma unroll 8
     for (int i = tid; i < N; i += T) sm[M + i] = ks[i];
     __syncthreads();
@@ -302,8 +309,8 @@ void col_merge(const ColMergeArgs A)
     __syncthreads();
     {   // word indices over the values
         uint32_t* w = (uint32_t*)sm;
-        const uint32_t* qp = A.qp + (size_t)s * M;
-        const uint32_t* kp = A.kp + (size_t)s * N;
+        const uint32_t* qp = A.qp + (size_t)seg * M;
+        const uint32_t* kp = A.kp + (size_t)seg * N;
 #pragma unroll 8
         for (int x = tid; x < M; x += T) w[x] = qp[x];
 #pragma unroll 8
@@ -380,7 +387,7 @@ void col_merge(const ColMergeArgs A)
         const float S = we + fmaf(-0.5f, wtot, wp);
         const float F = fmaf(anchor, S, -(ke + fmaf(-0.5f, ktot, kp)));
 #pragma unroll
-        for (int e = 0; e < E; ++e) out[e] = 2.f * (out[e] + fmaf(dist[e], S, F));
+        for (int e = 0; e < E; ++e) out[e] = 2.f * set_weight(A.sets, s - seg * A.sets) * (out[e] + fmaf(dist[e], S, F));
     } else {
         float l = 0.f, r = 0.f, pr = 1.f;
 #pragma unroll
@@ -428,6 +435,7 @@ struct ColSumArgs {
     const float* w;                  // [P][CW][Nw][CH] weight columns (col_weights): of v, or of g_w with SWAP
     float* out;                      // [P][DS][C][Ma]
     int P, D, N, M, C, DS, K0, CW;
+    int sets;                        // D counts streams: features x sets, a feature's sets next to each other
 };
 
 // SWAP: the queries carry the weights and the keys the accumulators (the grad_v of the abs sums)
@@ -564,13 +572,12 @@ void col_sum(const ColSumArgs A)
             for (int g = 0; g < E / 2; ++g) asm volatile("" : "+v"(tg[g]));    // addresses again, not kept in registers
             xp += T;
             if (d + 1 < d1) xs = *xp;
+            const float weight = set_weight(A.sets, A.sets == 1 ? 0 : d % 3);
 #pragma unroll
             for (int e = 0; e < E; ++e) {
                 float o[CH];
 #pragma unroll
-                for (int h = 0; h < CH; ++h) {
-                    o[h] = a[e][h] + fmaf(dv[e], S[h], F[h] + own[e][h]);
-                }
+                for (int h = 0; h < CH; ++h) o[h] = fmaf(weight, fmaf(dv[e], S[h], F[h] + own[e][h]), a[e][h]);
                 lds_write_masked<CH>(o, addr(e), acc[e]);
                 if ((e & 3) == 3) {                      // the next feature's elements over the ones just used
                     load(dn, e / 4);
@@ -1137,9 +1144,10 @@ int launch_sum(const ColSumArgs& a, hipStream_t st) {
 
 int col_merge_launch(int kind, const ColPlan& pl, const float* qs, const uint32_t* qp, const float* ks,
                      const uint32_t* kp, const uint8_t* keep, ColStream str, float* u, int S, int D, int N, int M,
-                     bool bwd, hipStream_t st) {
+                     bool bwd, int sets, hipStream_t st) {
     const ColMergeArgs a{qs, qp, ks, kp, keep, str.val, str.tag, str.xe, bwd ? str.eq : nullptr, u, D, N, M,
-                         bwd ? col_key0(pl, M) : M};
+                         bwd ? col_key0(pl, M) : M, sets};
+    S *= sets;
     StageTimer t("col_merge", st);
     return dispatch_shape(pl, [&](auto T, auto E, auto) {
         return kind == COL_ABS ? launch_merge<COL_ABS, T(), E()>(a, S, st) : launch_merge<COL_LAPLACE, T(), E()>(a, S, st); });
@@ -1157,8 +1165,8 @@ int col_weights_launch(const ColPlan& pl, const float* w, const uint8_t* keep, b
 }
 
 int col_sum_launch(int kind, const ColPlan& pl, ColStream str, const float* wt, float* cols, int P, int D, int N, int M,
-                   int C, hipStream_t st) {
-    const ColSumArgs a{str.val, str.tag, str.xe, wt, cols, P, D, N, M, C, pl.DS, M, (C + pl.CH - 1) / pl.CH};
+                   int C, int sets, hipStream_t st) {
+    const ColSumArgs a{str.val, str.tag, str.xe, wt, cols, P, D * sets, N, M, C, pl.DS, M, (C + pl.CH - 1) / pl.CH, sets};
     StageTimer t(kind == COL_ABS ? "col_sum_abs" : "col_sum_laplace", st);
     return dispatch_shape(pl, [&](auto T, auto E, auto CH) {
         return kind == COL_ABS ? launch_sum<COL_ABS, T(), E(), CH(), false>(a, st)
@@ -1167,7 +1175,7 @@ int col_sum_launch(int kind, const ColPlan& pl, ColStream str, const float* wt, 
 
 int col_grad_v_launch(const ColPlan& pl, ColStream str, const float* gt, int CW, float* cols, int P, int D, int N, int M,
                       int C, hipStream_t st) {
-    const ColSumArgs a{str.val, str.tag, str.xe, gt, cols, P, D, N, M, C, pl.DS, col_key0(pl, M), CW};
+    const ColSumArgs a{str.val, str.tag, str.xe, gt, cols, P, D, N, M, C, pl.DS, col_key0(pl, M), CW, 1};
     StageTimer t("col_grad_v", st);
     return dispatch_shape(pl, [&](auto T, auto E, auto CH) { return launch_sum<COL_ABS, T(), E(), CH(), true>(a, st); });
 }

@@ -94,7 +94,7 @@ def test_laplace_infinite_keys_and_queries(dev, no_dense):
     assert float(brute.rel_err(u[0], A.sum(1), A.sum(1)).max()) <= REL
 
 
-@pytest.mark.parametrize("kernel", ["add_laplace", "add_riesz"])
+@pytest.mark.parametrize("kernel", ["add_laplace", "add_riesz", "add_bump"])
 @pytest.mark.parametrize("N,M,C", [(1030, 1020, 6), (3111, 3111, 64), (12000, 9000, 31)])
 def test_masked_layer_columns(dev, kernel, N, M, C):
     # masked rows weigh 0 whatever they hold (NaN in v, large k), against the float64 layer over the kept keys
@@ -112,6 +112,8 @@ def test_masked_layer_columns(dev, kernel, N, M, C):
         dist = np.abs(qq[:, :, None] - kk[:, None])
         if kernel == "add_laplace":
             A = np.exp(-dist).sum(0)
+        elif kernel == "add_bump":
+            A = np.maximum(0, 1 - dist).sum(0)
         else:
             A = np.abs(qq).sum(0)[:, None] + np.abs(kk).sum(0)[None] - dist.sum(0) + layers.EPS
         den = A.sum(1)
