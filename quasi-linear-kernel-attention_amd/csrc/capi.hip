@@ -506,10 +506,11 @@ ColWs col_carve(ColPlan pl, void* ws, int P, int D, int N, int M, int C, int set
     return r;
 }
 
-// sort(p0, np, w, stream) leaves the sorted k and q in w.s; finish(p0, np, w, plan, stream) reads w.cols and w.u (null
+// q and k (null: always by sort) go to the stream in one kernel where col_sort_applies; else
+// sort(p0, np, w, stream) leaves the sorted k and q in w.s, which are merged. finish(p0, np, w, plan, stream) reads w.cols and w.u (null
 // without want_u). extra(np): bytes of the caller's own after the columns (w.extra).
 template <class Extra, class Sort, class Finish>
-int run_columns(int kind, int sets, const float* v, const uint8_t* keep, bool want_u, int P, int D, int N, int M, int C, void* ws,
+int run_columns(int kind, int sets, const float* q, const float* k, const float* v, const uint8_t* keep, bool want_u, int P, int D, int N, int M, int C, void* ws,
                 size_t given, hipStream_t st, Extra extra, Sort sort, Finish finish) {
     ColPlan pl = col_plan(kind, P, D * sets, N, M, C);
     pl.DS = std::min(pl.DS, std::min(D, COL_SHARES));        // as many as the workspace is sized for
@@ -520,11 +521,16 @@ int run_columns(int kind, int sets, const float* v, const uint8_t* keep, bool wa
         ColWs w = col_carve(pl, ws, np, D, N, M, C, sets);
         if (!want_u) w.u = nullptr;
         const size_t p = (size_t)p0;
-        if (int e = sort(p0, np, w, st)) return e;
         const uint8_t* kc = keep ? keep + p * N : nullptr;
-        if (int e = col_merge_launch(kind, pl, w.s.qs, w.s.qp, w.s.ks, w.s.kp, kc, w.str, w.u, np * D, D, N, M, false,
-                                     sets, st))
-            return hip_status(e, "merge of q and k");
+        if (q && sets == 1 && col_sort_applies(pl)) {
+            if (int e = col_sort_launch(kind, pl, q + p * D * M, k + p * D * N, kc, w.str, w.u, np * D, D, N, M, st))
+                return hip_status(e, "sort of q and k");
+        } else {
+            if (int e = sort(p0, np, w, st)) return e;
+            if (int e = col_merge_launch(kind, pl, w.s.qs, w.s.qp, w.s.ks, w.s.kp, kc, w.str, w.u, np * D, D, N, M,
+                                         false, sets, st))
+                return hip_status(e, "merge of q and k");
+        }
         if (int e = col_weights_launch(pl, v + p * N * C, kc, false, nullptr, w.wt, np, N, C, st))
             return hip_status(e, "weight columns");
         if (int e = col_sum_launch(kind, pl, w.str, w.wt, w.cols, np, D, N, M, C, sets, st))
@@ -645,7 +651,7 @@ int qlka_laplace_fwd(const float* q, const float* k, const float* v, float* out_
     const Plan pl = plan_chunks(P, ws_bytes_given, pipelined(P, D, M), b1);
     if (int e = check_ws(ws, ws_bytes_given, plan_bytes(pl, b1))) return e;
     if (col_applies(D, N, M))
-        return run_columns(1, 1, v, nullptr, true, P, D, N, M, C, ws, ws_bytes_given, st, no_extra,
+        return run_columns(1, 1, q, k, v, nullptr, true, P, D, N, M, C, ws, ws_bytes_given, st, no_extra,
             [&](int p0, int np, ColWs& w, hipStream_t s) {
                 const size_t p = (size_t)p0;
                 return sort_both(q + p * D * M, k + p * D * N, w.s, np * D, N, M, s); },
@@ -775,7 +781,7 @@ int abs_fwd_impl(const float* q, const float* k, const float* v, float* out_w, f
     if (int e = check_ws(ws, ws_bytes_given, plan_bytes(pl, b1))) return e;
     // (the backward by columns reads no range states, so none are written; *kept still says that a buffer was taken)
     if (col_applies(D, N, M) && (!keep_states || col_bwd_applies(D, N, M))) {
-        const int e = run_columns(0, 1, v, nullptr, out_u != nullptr, P, D, N, M, C, ws, ws_bytes_given, st, no_extra,
+        const int e = run_columns(0, 1, keep_sorts ? nullptr : q, k, v, nullptr, out_u != nullptr, P, D, N, M, C, ws, ws_bytes_given, st, no_extra,
             [&](int p0, int np, ColWs& w, hipStream_t s) {
                 const size_t p = (size_t)p0;
                 if (keep_sorts) {
@@ -1388,7 +1394,7 @@ static int layer_columns(int kind, const float* q, const float* k, const float* 
                          hipStream_t st) {
     const bool riesz = kind == LAYER_ADD_RIESZ, laplace = kind == LAYER_ADD_LAPLACE;
     const int sets = kind == LAYER_ADD_BUMP ? 3 : 1;
-    return run_columns(laplace ? 1 : 0, sets, v, keep, true, P, D, N, M, C, ws, given, st,
+    return run_columns(laplace ? 1 : 0, sets, q, k, v, keep, true, P, D, N, M, C, ws, given, st,
         [&](int pc) { return layer_col_extra(kind, pc, D, N, M, C); },
         [&](int p0, int np, ColWs& w, hipStream_t s) {
             const size_t p = (size_t)p0;

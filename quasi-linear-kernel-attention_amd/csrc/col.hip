@@ -251,75 +251,15 @@ struct ColMergeArgs {
 __device__ __forceinline__ float set_shift(int set) { return set == 0 ? 0.f : set == 1 ? 1.f : -1.f; }
 __device__ __forceinline__ float set_weight(int sets, int set) { return sets == 1 ? 1.f : set == 0 ? -1.f : 0.5f; }
 
-// dynamic LDS: N + M words (values, then word indices, then the v == 1 terms), then the scan's aggregates
+// The stream and the v == 1 terms of one segment, from its merged order: thread t's elements as word indices src (padding:
+// K0 + N) and as values (abs) or distances to the element before (Laplace) in dist; x0 the median key, xs the value before
+// the thread's first element, xs0 and xn its first and last. sm: N + M words and the scan's aggregates, free to use.
 template <int KIND, int T, int E>
-__global__ __launch_bounds__(T)
-void col_merge(const ColMergeArgs A)
+__device__ __forceinline__ void emit_stream(const ColMergeArgs& A, float* sm, int s, float x0, float xs, float xs0, float xn,
+                                            float (&dist)[E], int (&src)[E])
 {
     constexpr int W = T / WAVE;
-    extern __shared__ float sm[];
-    const int s = blockIdx.x, seg = s / A.sets, p = seg / A.D, tid = threadIdx.x;     // stream, segment
-    const int N = A.N, M = A.M, n = N + M;
-    const float* qs = A.qs + (size_t)seg * M;
-    const float* ks = A.ks + (size_t)seg * N;
-    const float shift = set_shift(s - seg * A.sets);
-#pragma unroll 8
-    for (int i = tid; i < M; i += T) sm[i] = qs[i] + shift;
-#pragma unroll 8
-    for (int i = tid; i < N; i += T) sm[M + i] = ks[i];
-    __syncthreads();
-    const float* sq = sm;
-    const float* sk = sm + M;
-    const float x0 = sk[N / 2];
-    // merge path: queries before `diag` (queries come first among equal values)
-    const int diag = min(tid * E, n);
-    int lo = max(0, diag - N), hi = min(diag, M);
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (sq[mid] <= sk[diag - 1 - mid]) lo = mid + 1;
-        else hi = mid;
-    }
-    int i = lo, j = diag - lo;
-    float prev = 0.f;
-    if (diag == 0) prev = fminf(sq[0], sk[0]);
-    else if (i == 0) prev = sk[j - 1];
-    else if (j == 0) prev = sq[i - 1];
-    else prev = fmaxf(sq[i - 1], sk[j - 1]);
-    const float xs = prev;
-    float qa = sq[min(i, M - 1)], kb = sk[min(j, N - 1)];
-    uint32_t eq = 0;
-    float dist[E];                      // abs: the element's value; Laplace: its distance to the previous element
-    int src[E];                         // word of the element in sq / sk
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const bool live = diag + e < n;
-        const bool tq = j >= N || (i < M && qa <= kb);
-        const float r = tq ? qa : kb;
-        src[e] = live ? (tq ? i : M + j) : n;
-        if (live && diag + e > 0 && r == prev) eq |= 1u << e;
-        if constexpr (KIND == COL_LAPLACE) dist[e] = (live && r != prev) ? r - prev : 0.f;   // equal infinities: 0 apart
-        else dist[e] = live ? r : prev;
-        if (live) {
-            prev = r;
-            if (tq) { ++i; qa = sq[min(i, M - 1)]; }
-            else { ++j; kb = sk[min(j, N - 1)]; }
-        }
-    }
-    const float xn = prev, xs0 = KIND == COL_ABS ? dist[0] : 0.f;      // last and first value
-    __syncthreads();
-    {   // word indices over the values
-        uint32_t* w = (uint32_t*)sm;
-        const uint32_t* qp = A.qp + (size_t)seg * M;
-        const uint32_t* kp = A.kp + (size_t)seg * N;
-#pragma unroll 8
-        for (int x = tid; x < M; x += T) w[x] = qp[x];
-#pragma unroll 8
-        for (int x = tid; x < N; x += T) w[M + x] = A.K0 + kp[x];
-        __syncthreads();
-#pragma unroll
-        for (int e = 0; e < E; ++e) src[e] = src[e] < n ? (int)w[src[e]] : A.K0 + N;
-    }
-    if (A.eq) A.eq[(size_t)s * T + tid] = eq;
+    const int N = A.N, M = A.M, n = N + M, tid = threadIdx.x, seg = s / A.sets, p = seg / A.D;
     // A thread's values are taken relative to its anchor, so that where a gap splits its elements, those on the median's
     // side stay precise: every value an element's sums are formed from is then bounded by distances to keys
     float anchor = 0.f;
@@ -425,6 +365,267 @@ void col_merge(const ColMergeArgs A)
     __syncthreads();
     float* uo = A.u + (size_t)s * M;
     for (int x = tid; x < M; x += T) uo[x] = sm[x];
+}
+
+// dynamic LDS: N + M words (values, then word indices, then the v == 1 terms), then the scan's aggregates
+template <int KIND, int T, int E>
+__global__ __launch_bounds__(T)
+void col_merge(const ColMergeArgs A)
+{
+    extern __shared__ float sm[];
+    const int s = blockIdx.x, seg = s / A.sets, tid = threadIdx.x;     // stream, segment
+    const int N = A.N, M = A.M, n = N + M;
+    const float* qs = A.qs + (size_t)seg * M;
+    const float* ks = A.ks + (size_t)seg * N;
+    const float shift = set_shift(s - seg * A.sets);
+#pragma unroll 8
+    for (int i = tid; i < M; i += T) sm[i] = qs[i] + shift;
+#pragma unroll 8
+    for (int i = tid; i < N; i += T) sm[M + i] = ks[i];
+    __syncthreads();
+    const float* sq = sm;
+    const float* sk = sm + M;
+    const float x0 = sk[N / 2];
+    // merge path: queries before `diag` (queries come first among equal values)
+    const int diag = min(tid * E, n);
+    int lo = max(0, diag - N), hi = min(diag, M);
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (sq[mid] <= sk[diag - 1 - mid]) lo = mid + 1;
+        else hi = mid;
+    }
+    int i = lo, j = diag - lo;
+    float prev = 0.f;
+    if (diag == 0) prev = fminf(sq[0], sk[0]);
+    else if (i == 0) prev = sk[j - 1];
+    else if (j == 0) prev = sq[i - 1];
+    else prev = fmaxf(sq[i - 1], sk[j - 1]);
+    const float xs = prev;
+    float qa = sq[min(i, M - 1)], kb = sk[min(j, N - 1)];
+    uint32_t eq = 0;
+    float dist[E];                      // abs: the element's value; Laplace: its distance to the previous element
+    int src[E];                         // word of the element in sq / sk
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const bool live = diag + e < n;
+        const bool tq = j >= N || (i < M && qa <= kb);
+        const float r = tq ? qa : kb;
+        src[e] = live ? (tq ? i : M + j) : n;
+        if (live && diag + e > 0 && r == prev) eq |= 1u << e;
+        if constexpr (KIND == COL_LAPLACE) dist[e] = (live && r != prev) ? r - prev : 0.f;   // equal infinities: 0 apart
+        else dist[e] = live ? r : prev;
+        if (live) {
+            prev = r;
+            if (tq) { ++i; qa = sq[min(i, M - 1)]; }
+            else { ++j; kb = sk[min(j, N - 1)]; }
+        }
+    }
+    const float xn = prev, xs0 = KIND == COL_ABS ? dist[0] : 0.f;      // last and first value
+    __syncthreads();
+    {   // word indices over the values
+        uint32_t* w = (uint32_t*)sm;
+        const uint32_t* qp = A.qp + (size_t)seg * M;
+        const uint32_t* kp = A.kp + (size_t)seg * N;
+#pragma unroll 8
+        for (int x = tid; x < M; x += T) w[x] = qp[x];
+#pragma unroll 8
+        for (int x = tid; x < N; x += T) w[M + x] = A.K0 + kp[x];
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < E; ++e) src[e] = src[e] < n ? (int)w[src[e]] : A.K0 + N;
+    }
+    if (A.eq) A.eq[(size_t)s * T + tid] = eq;
+    emit_stream<KIND, T, E>(A, sm, s, x0, xs, xs0, xn, dist, src);
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// col_sort: one workgroup per segment, from the unsorted queries and keys (A.qs, A.ks) to the stream
+//
+// A stable radix sort of queries (first) and keys together, 4 passes of 8 bits. A wave owns 64 E consecutive positions and
+// takes them 64 at a time: the lanes with an equal digit find each other by 8 ballots, so that a position's rank in its
+// wave is a running count per digit (a wave's own 256 counters in LDS) plus the equal lanes below it; one scan over
+// (digit, wave) makes the counts first positions, and values and word indices go to their places through LDS. Nothing
+// is read from or written to memory between the inputs and the stream. Masked keys sort last, as padding.
+// What bounds it: about 50 vector instructions per element and pass (the ballots), 16 waves a CU.
+// ---------------------------------------------------------------------------------------------------------------
+__host__ __device__ constexpr int sort_words(int T, int E) { return T * E + T * E / 32 + 1 + 256 * (T / WAVE) + 32; }
+
+// lanes of the wave whose 8-bit digit equals this lane's
+__device__ __forceinline__ uint64_t equal_lanes(uint32_t digit) {
+    uint32_t lo = 0u, hi = 0u;                               // lanes that differ in some bit
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+        uint32_t t = (uint32_t)__builtin_amdgcn_sbfe((int)digit, b, 1);
+        asm("" : "+v"(t));                                   // one comparison below, not the bit taken again
+        const uint64_t v = __ballot(t != 0);
+        lo = __builtin_amdgcn_bitop3_b32(lo, (uint32_t)v, t, 0xf6);              // lo | (v ^ t)
+        hi = __builtin_amdgcn_bitop3_b32(hi, (uint32_t)(v >> 32), t, 0xf6);
+    }
+    return ~((uint64_t)lo | ((uint64_t)hi << 32));
+}
+
+// 16-bit halves of an array of pairs
+template <int E>
+struct Halves {
+    uint32_t w[E / 2];
+    __device__ __forceinline__ uint32_t get(int i) const { return (i & 1) ? w[i / 2] >> 16 : w[i / 2] & 0xffffu; }
+    __device__ __forceinline__ void set(int i, uint32_t x) {         // in order: the low half first
+        if (i & 1) w[i / 2] |= x << 16;
+        else w[i / 2] = x;
+    }
+};
+
+template <int KIND, int T, int E>
+__global__ __launch_bounds__(T)
+void col_sort(const ColMergeArgs A)
+{
+    constexpr int W = T / WAVE, L = T * E, LP = L + L / 32 + 1;
+    extern __shared__ float sm[];
+    uint32_t* buf = (uint32_t*)sm;
+    uint32_t* all = (uint32_t*)sm + LP;                      // [W][256] counters
+    uint32_t* misc = all + 256 * W;                          // [0] live elements, [4..7] [8..23] scans, [24] the median
+    const int s = blockIdx.x, p = s / A.D, tid = threadIdx.x, lane = lane_id(), wv = wave_in_block();
+    const int N = A.N, M = A.M, n = N + M;
+    uint32_t* cnt = all + 256 * wv;
+    const int first = wv * (WAVE * E) + lane;                // position of element j: first + 64 j
+    auto padded = [](int i) { return i + (i >> 5); };
+    uint32_t key[E], before_key = 0, last_key = 0;
+    Halves<E> idx;
+    int live = 0;
+    {
+        const float* q = A.qs + (size_t)s * M;
+        const float* k = A.ks + (size_t)s * N;
+        const uint8_t* keep = A.keep ? A.keep + (size_t)p * N : nullptr;
+#pragma unroll
+        for (int j = 0; j < E; ++j) {
+            const int i = first + WAVE * j;
+            const float x = i < M ? q[i] : k[min(i - M, N - 1)];
+            const bool on = i < n && (i < M || !keep || keep[i - M] != 0);
+            key[j] = on ? float_to_ordered(x + 0.f) : 0xffffffffu;
+            idx.set(j, on ? (uint32_t)i : (uint32_t)n);
+            live += (int)__popcll(__ballot(on));
+        }
+    }
+    if (tid == 0) misc[0] = 0;
+    __syncthreads();
+    if (lane == 0) atomicAdd(&misc[0], (uint32_t)live);      // an integer: the order does not matter
+    for (int shift = 0; shift < 32; shift += 8) {
+#pragma unroll
+        for (int i = 0; i < 256 / WAVE; ++i) cnt[lane + WAVE * i] = 0;
+        Halves<E> pos;
+#pragma unroll
+        for (int j = 0; j < E; ++j) {
+            const uint32_t digit = (key[j] >> shift) & 255u;
+            const uint64_t same = equal_lanes(digit);
+            const uint32_t before = cnt[digit], below = (uint32_t)lanes_below(same), total = (uint32_t)__popcll(same);
+            pos.set(j, before + below);
+            if (below + 1 == total) cnt[digit] = before + total;
+            if (j & 1) __builtin_amdgcn_sched_barrier(0);    // two positions' masks at a time, or all E are live
+        }
+        __syncthreads();
+        {   // counts to first positions: digits in order, the waves of a digit in order
+            constexpr int TD = T < 256 ? T : 256, DPT = 256 / TD;     // threads at work, digits each
+            uint32_t tot[DPT], sum = 0;
+            if (tid < TD) {
+#pragma unroll
+                for (int x = 0; x < DPT; ++x) {
+                    uint32_t c = 0;
+                    for (int w = 0; w < W; ++w) {
+                        uint32_t* a = all + 256 * w + tid * DPT + x;
+                        const uint32_t y = *a;
+                        *a = c;
+                        c += y;
+                    }
+                    tot[x] = c;
+                    sum += c;
+                }
+            }
+            uint32_t inc = sum;
+#pragma unroll
+            for (int off = 1; off < WAVE; off <<= 1) {
+                const uint32_t y = __shfl_up(inc, off, WAVE);
+                if (lane >= off) inc += y;
+            }
+            if (tid < TD && lane == WAVE - 1) misc[4 + wv] = inc;
+            __syncthreads();
+            if (tid < TD) {
+                uint32_t base = inc - sum;
+                for (int w = 0; w < wv; ++w) base += misc[4 + w];
+#pragma unroll
+                for (int x = 0; x < DPT; ++x) {
+                    for (int w = 0; w < W; ++w) all[256 * w + tid * DPT + x] += base;
+                    base += tot[x];
+                }
+            }
+            __syncthreads();
+        }
+        // the last pass pads every 32 words: threads then read E words in a row
+        const bool last = shift == 24;
+#pragma unroll
+        for (int j = 0; j < E; ++j) {
+            const uint32_t x = pos.get(j) + cnt[(key[j] >> shift) & 255u], y = last ? x + (x >> 5) : x;
+            if (j & 1) pos.w[j / 2] = (pos.w[j / 2] & 0xffffu) | (y << 16);
+            else pos.w[j / 2] = (pos.w[j / 2] & 0xffff0000u) | y;
+        }
+#pragma unroll
+        for (int j = 0; j < E; ++j) buf[pos.get(j)] = key[j];
+        __syncthreads();
+        if (last) {
+#pragma unroll
+            for (int j = 0; j < E; ++j) key[j] = buf[padded(tid * E + j)];
+            before_key = buf[padded(max(tid * E, 1) - 1)];
+            last_key = buf[padded((int)misc[0] - 1)];
+        } else {
+#pragma unroll
+            for (int j = 0; j < E; ++j) key[j] = buf[first + WAVE * j];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < E; ++j) buf[pos.get(j)] = idx.get(j);
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < E; ++j) idx.set(j, buf[last ? padded(tid * E + j) : first + WAVE * j]);
+    }
+    const int nl = (int)misc[0];                             // queries and kept keys
+    float x0 = 0.f;
+    if constexpr (KIND == COL_ABS) {                         // the median of the kept keys
+        int keys = 0;
+#pragma unroll
+        for (int e = 0; e < E; ++e) keys += (int)idx.get(e) >= M && (int)idx.get(e) < n;
+        int inc = keys;
+#pragma unroll
+        for (int off = 1; off < WAVE; off <<= 1) {
+            const int y = __shfl_up(inc, off, WAVE);
+            if (lane >= off) inc += y;
+        }
+        if (lane == WAVE - 1) misc[8 + wv] = (uint32_t)inc;
+        __syncthreads();
+        int at = (nl - M) / 2 - (inc - keys);                // the median's number among this thread's keys
+        for (int w = 0; w < wv; ++w) at -= (int)misc[8 + w];
+        if (at >= 0 && at < keys) {
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                if ((int)idx.get(e) >= M && (int)idx.get(e) < n && at-- == 0) misc[24] = key[e];
+        }
+        __syncthreads();
+        if (nl > M) x0 = ordered_to_float(misc[24]);
+    }
+    const float lastv = ordered_to_float(last_key);
+    float prev = tid == 0 ? ordered_to_float(key[0]) : tid * E - 1 < nl ? ordered_to_float(before_key) : lastv;
+    const float xs = prev;
+    float dist[E];
+    int src[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const float r = tid * E + e < nl ? ordered_to_float(key[e]) : prev;
+        if constexpr (KIND == COL_LAPLACE) dist[e] = r != prev ? r - prev : 0.f;      // equal infinities: 0 apart
+        else dist[e] = r;
+        prev = r;
+        src[e] = (int)idx.get(e);
+    }
+    const float xs0 = KIND == COL_ABS ? dist[0] : 0.f;
+    __syncthreads();                                         // buf is read; the emission uses it
+    emit_stream<KIND, T, E>(A, sm, s, x0, xs, xs0, prev, dist, src);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -1141,6 +1342,33 @@ int launch_sum(const ColSumArgs& a, hipStream_t st) {
 }
 
 }  // namespace
+
+// Against the two sorts and the merge, whole prep of a call: 1536 elements 66 -> 47 us (2048 segments), 8192 210 -> 126 us
+// (1536; with a key mask also the 60 us of its fill), 16384 178 -> 156 us (768). Threads of more than 16 elements spill
+// here (32768: 629 against 412 us).
+bool col_sort_applies(const ColPlan& pl) { return pl.E <= 16; }
+
+int col_sort_launch(int kind, const ColPlan& pl, const float* q, const float* k, const uint8_t* keep, ColStream str,
+                    float* u, int S, int D, int N, int M, hipStream_t st) {
+    const ColMergeArgs a{q, nullptr, k, nullptr, keep, str.val, str.tag, str.xe, nullptr, u, D, N, M, M, 1};
+    StageTimer t("col_sort", st);
+    return dispatch_shape(pl, [&](auto T, auto E, auto) {
+        if constexpr (E() > 16) {
+            return (int)hipErrorInvalidValue;
+        } else {
+            const size_t lds = (size_t)sort_words(T(), E()) * 4;
+            if (kind == COL_ABS) {
+                static const hipError_t once = allow_lds(col_sort<COL_ABS, T(), E()>);
+                if (once != hipSuccess) return (int)once;
+                hipLaunchKernelGGL((col_sort<COL_ABS, T(), E()>), dim3((unsigned)S), dim3(T()), lds, st, a);
+            } else {
+                static const hipError_t once = allow_lds(col_sort<COL_LAPLACE, T(), E()>);
+                if (once != hipSuccess) return (int)once;
+                hipLaunchKernelGGL((col_sort<COL_LAPLACE, T(), E()>), dim3((unsigned)S), dim3(T()), lds, st, a);
+            }
+            return (int)hipGetLastError();
+        } });
+}
 
 int col_merge_launch(int kind, const ColPlan& pl, const float* qs, const uint32_t* qp, const float* ks,
                      const uint32_t* kp, const uint8_t* keep, ColStream str, float* u, int S, int D, int N, int M,

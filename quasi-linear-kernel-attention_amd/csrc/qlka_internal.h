@@ -274,6 +274,10 @@ ColStream col_stream(const ColPlan& pl, void* base, int S);
 int col_merge_launch(int kind, const ColPlan& pl, const float* qs, const uint32_t* qp, const float* ks,
                      const uint32_t* kp, const uint8_t* keep, ColStream str, float* u, int S, int D, int N, int M,
                      bool bwd, int sets, hipStream_t st);
+// the same stream from unsorted q and k in one kernel, masked keys as padding
+bool col_sort_applies(const ColPlan& pl);
+int col_sort_launch(int kind, const ColPlan& pl, const float* q, const float* k, const uint8_t* keep, ColStream str,
+                    float* u, int S, int D, int N, int M, hipStream_t st);
 // wt: the columns of rows w (P, Nw, C) in groups of pl.CH, rows masked by keep (null: none) 0; `more`: one more channel,
 // extra (P, Nw) or ones
 int col_weights_launch(const ColPlan& pl, const float* w, const uint8_t* keep, bool more, const float* extra, float* wt,
