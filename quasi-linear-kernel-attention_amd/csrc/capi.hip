@@ -461,6 +461,26 @@ int run_pipeline(int P, const Plan& pl, void* ws, size_t copy, hipStream_t st, P
 // The chunks run in order on the caller's stream: the sums keep every CU's LDS, so nothing would run beside them. Its
 // workspace is smaller than the walk's but for many more keys than queries, where the *_ws_bytes queries return the
 // larger of the two.
+// Its longer chain of launches, each too small to fill the chip, costs more than the walk's below about half a million
+// elements (a million with fewer than 128 segments, one workgroup each in its sort) forward, and backward, whose dot
+// products also take one workgroup per segment, below a million, 128 segments, or 192 where a workgroup fills a CU.
+// (P, D, M = N, C = 64:) Laplace 114 against 87 us at 1 x 64 x 2000, 99 against 139 at 12 x 64 x 520, abs 132 against 114 at
+// 1 x 64 x 4200; forward + backward 258 against 160 us at 1 x 64 x 1500, even at 12 x 64 x 640, 322 against 368 at
+// 12 x 64 x 1100, 796 against 774 at 2 x 64 x 16000. With the dense cutoff at 0, which turns the routing by small size
+// off, every size takes it. The sgn sum takes it with two channels per workgroup only (12 x 64 x 3000: 253 against 277 us;
+// 16384: 1525 against 1439).
+inline bool col_enough(int P, int D, int N, int M, int64_t elements, int64_t segments) {
+    return ((int64_t)P * D * ((int64_t)N + M) >= elements && (int64_t)P * D >= segments) || direct_base() == 0;
+}
+inline bool col_fwd(int P, int D, int sets, int N, int M) {
+    return col_applies(D * sets, N, M) &&
+           (col_enough(P, D, N, M, 1 << 19, 128) || col_enough(P, D, N, M, 1 << 20, 1));
+}
+inline bool col_bwd(int P, int D, int N, int M) {
+    return col_bwd_applies(D, N, M) && col_enough(P, D, N, M, 1 << 20, N + M <= COL_MAX2 ? 128 : 192);
+}
+inline bool col_sgn(int P, int D, int N, int M) { return col_bwd(P, D, N, M) && N + M <= COL_MAX2; }
+
 struct ColWs { SortedWs s; ColStream str; float* u; float* cols; float* wt; char* extra; };
 
 size_t col_part(const ColPlan& pl, int P, int D, int N, int M, int C, int sets, int i) {
@@ -650,7 +670,7 @@ int qlka_laplace_fwd(const float* q, const float* k, const float* v, float* out_
     auto b1 = [&](int pc) { return laplace_ws(pc, D, N, M, C); };
     const Plan pl = plan_chunks(P, ws_bytes_given, pipelined(P, D, M), b1);
     if (int e = check_ws(ws, ws_bytes_given, plan_bytes(pl, b1))) return e;
-    if (col_applies(D, N, M))
+    if (col_fwd(P, D, 1, N, M))
         return run_columns(1, 1, q, k, v, nullptr, true, P, D, N, M, C, ws, ws_bytes_given, st, no_extra,
             [&](int p0, int np, ColWs& w, hipStream_t s) {
                 const size_t p = (size_t)p0;
@@ -780,7 +800,7 @@ int abs_fwd_impl(const float* q, const float* k, const float* v, float* out_w, f
     const Plan pl = plan_chunks(P, ws_bytes_given, pipelined(P, D, M), b1);
     if (int e = check_ws(ws, ws_bytes_given, plan_bytes(pl, b1))) return e;
     // (the backward by columns reads no range states, so none are written; *kept still says that a buffer was taken)
-    if (col_applies(D, N, M) && (!keep_states || col_bwd_applies(D, N, M))) {
+    if (col_fwd(P, D, 1, N, M) && (!keep_states || col_bwd(P, D, N, M))) {
         const int e = run_columns(0, 1, keep_sorts ? nullptr : q, k, v, nullptr, out_u != nullptr, P, D, N, M, C, ws, ws_bytes_given, st, no_extra,
             [&](int p0, int np, ColWs& w, hipStream_t s) {
                 const size_t p = (size_t)p0;
@@ -1067,7 +1087,7 @@ int abs_bwd_impl(const float* q, const float* k, const float* v, const float* g_
     hipStream_t st = (hipStream_t)stream;
     if (dense_sign(P, N, M))     // the walks' convention: a tie counts -1 in both gradients
         return dense_bwd(-1.f, q, k, v, g_w, g_u, grad_q, grad_k, grad_v, P, D, N, M, C, st);
-    if (col_bwd_applies(D, N, M)) {
+    if (col_bwd(P, D, N, M)) {
         if (int e = check_ws(ws, ws_bytes_given, col_bwd_bytes(1, D, N, M, C))) return e;
         return run_bwd_columns(v, g_w, g_u, 2.f, grad_q, grad_k, grad_v, P, D, N, M, C, ws, ws_bytes_given, st,
             [&](int p0, int np, SortedWs& w, hipStream_t s) {
@@ -1180,7 +1200,7 @@ int qlka_sgn_fwd(const float* q, const float* k, const float* v, const float* g,
     hipStream_t st = (hipStream_t)stream;
     if (dense_sign(P, N, M))     // sgn(k - q) with a tie counted +1 == -(s(q - k) with a tie counted -1)
         return hip_status(direct_sign(true, q, k, g, v, nullptr, out, -1.f, -1.f, P, D, M, N, C, st), "dense sgn sum");
-    if (col_bwd_applies(D, N, M))   // sgn(k - q) with a tie counted +1, as above: -grad_q
+    if (col_sgn(P, D, N, M))   // sgn(k - q) with a tie counted +1, as above: -grad_q
         return run_bwd_columns(v, g, nullptr, -2.f, out, nullptr, nullptr, P, D, N, M, C, ws, ws_bytes_given, st,
             [&](int p0, int np, SortedWs& w, hipStream_t s) {
                 const size_t p = (size_t)p0;
@@ -1440,7 +1460,7 @@ static int layer_fwd(int kind, const float* q, const float* k, const float* v, c
         npc = n_pad ? n_pad + p : nullptr; keepc = keep ? keep + p * N : nullptr; outc = out + p * M * C;
     };
     const bool bump = kind == LAYER_ADD_BUMP;
-    if (col_layer(kind, D, N, M) && !(kind == LAYER_ADD_RIESZ && keep == nullptr && few_keys(N)))
+    if (col_fwd(P, D, bump ? 3 : 1, N, M) && !(kind == LAYER_ADD_RIESZ && keep == nullptr && few_keys(N)))
         return layer_columns(kind, q, k, v, n_pad, keep, out, P, D, N, M, C, ws, ws_bytes_given, st);
     if (kind == LAYER_ADD_RIESZ && keep == nullptr && few_keys(N))   // the abs sums dense (few_keys), then the epilogue
         return for_chunks(P, pl.pc, [&](int p0, int np) {

@@ -96,7 +96,7 @@ def test_laplace_infinite_keys_and_queries(dev, no_dense):
 
 @pytest.mark.parametrize("kernel", ["add_laplace", "add_riesz", "add_bump"])
 @pytest.mark.parametrize("N,M,C", [(1030, 1020, 6), (3111, 3111, 64), (12000, 9000, 31)])
-def test_masked_layer_columns(dev, kernel, N, M, C):
+def test_masked_layer_columns(dev, no_dense, kernel, N, M, C):
     # masked rows weigh 0 whatever they hold (NaN in v, large k), against the float64 layer over the kept keys
     from qlka import layers
     P, D = 2, 4
@@ -122,3 +122,35 @@ def test_masked_layer_columns(dev, kernel, N, M, C):
         num = A @ vv
         scale = np.abs(A) @ np.abs(vv)
         np.testing.assert_array_less(np.abs(got[p][rows] * den[:, None] - num), 2e-4 * (scale + np.abs(num)) + 1e-6)
+
+
+@pytest.mark.parametrize("kind", ["normal", "ties", "runs"])
+@pytest.mark.parametrize("shape", [(1, 3, 18, 19, 1), (2, 2, 400, 369, 3), (1, 3, 700, 800, 65), (1, 2, 2100, 1990, 5),
+                                   (1, 2, 5000, 5239, 2), (1, 2, 9000, 7385, 9), (1, 2, 9900, 10453, 3),
+                                   (1, 2, 16384, 16384, 18), (1, 2, 31000, 900, 2), (2, 1, 900, 30000, 1)])
+def test_column_backward(dev, no_dense, shape, kind):
+    # grad_q, grad_k, grad_v with and without g_u, and the sgn sum, at the workgroup shapes' edges; "ties": runs of equal
+    # queries and keys that cross threads and waves, "runs": one value for long stretches. Ties count -1 (sgn: +1).
+    from weighted_abs_sum import _ext, weighted_sgn_sum
+    P, D, N, M, C = shape
+    print(f"column backward {shape} {kind}", flush=True)
+    q, k, v = _data(P, D, N, M, C, "normal" if kind == "normal" else "ties", seed=sum(shape))
+    if kind == "runs":
+        q[..., : M // 2] = 0.25
+        k[..., : N // 2] = 0.25
+    rng = np.random.default_rng(1)
+    g = rng.standard_normal((P, M, C), dtype=np.float32)
+    gu = rng.standard_normal((P, M), dtype=np.float32)
+    iq, ik = inputs.query_subsample(P, M, per_p=12, seed=2), inputs.query_subsample(P, N, per_p=12, seed=3)
+    t = [torch.from_numpy(a).to(dev) for a in (q, k, v, g, gu)]
+    pick = lambda a, i, ax: np.stack([np.take(a[p], i[p], axis=ax) for p in range(P)])  # noqa: E731
+    for u in (gu, None):
+        got = (_ext.weighted_abs_sum_full_backward(*t) if u is not None else _ext.weighted_abs_sum_backward(*t[:4]))
+        got = [x.cpu().numpy() for x in got]
+        (wq, wk, wv), (nq, nk, nv) = brute.abs_backward_sub(q, k, v, g, u, iq, ik)
+        for name, a, w, nn in (("grad_q", pick(got[0], iq, 1), wq, nq), ("grad_k", pick(got[1], ik, 1), wk, nk),
+                               ("grad_v", pick(got[2], ik, 0), wv, nv)):
+            assert float(brute.rel_err(a, w, nn).max()) <= REL, name
+    sgn = weighted_sgn_sum(*t[:4], backend="cuda").cpu().numpy()
+    (wq, _, _), (nq, _, _) = brute.abs_backward_sub(q, k, v, g, None, iq, ik)
+    assert float(brute.rel_err(pick(sgn, iq, 1), -wq, nq).max()) <= REL
