@@ -476,6 +476,19 @@ inline bool col_fwd(int P, int D, int sets, int N, int M) {
     return col_applies(D * sets, N, M) &&
            (col_enough(P, D, N, M, 1 << 19, 128) || col_enough(P, D, N, M, 1 << 20, 1));
 }
+// The Laplace sums with one channel per workgroup (N + M > COL_MAX2) run about as long as the walk, so there the rounds that
+// the chip needs decide, by estimates of both in us: 4.75 per feature and round of 32-element threads, the sorts and the
+// merge, against the walk at this width (P, D, M = N, C: 10 x 64 x 15000 x 64 1336 against 1306 us, 9 x 64 x 15000 x 64 1308
+// against 1197, but 8 x 64 x 16300 x 64 1035 against 1188 and 12 x 64 x 16384 x 64 1540 against 1690).
+inline bool col_laplace(int P, int D, int N, int M, int C) {
+    if (!col_fwd(P, D, 1, N, M)) return false;
+    if (N + M <= COL_MAX2 || direct_base() == 0) return true;
+    const ColPlan pl = col_plan(1, P, D, N, M, C);
+    const double el = (double)P * D * (N + M);
+    const double col = 60 + pl.cost * 4.75 * pl.E / 32 + el * 1.87e-5;
+    const double walk = el * 0.67e-4 * (C <= 32 ? 0.67 : C <= 64 ? 1 : 2.4) * (std::max(N, M) > LDS_SORT_MAX ? 1.35 : 1);
+    return col < walk;
+}
 inline bool col_bwd(int P, int D, int N, int M) {
     return col_bwd_applies(D, N, M) && col_enough(P, D, N, M, 1 << 20, N + M <= COL_MAX2 ? 128 : 192);
 }
@@ -670,7 +683,7 @@ int qlka_laplace_fwd(const float* q, const float* k, const float* v, float* out_
     auto b1 = [&](int pc) { return laplace_ws(pc, D, N, M, C); };
     const Plan pl = plan_chunks(P, ws_bytes_given, pipelined(P, D, M), b1);
     if (int e = check_ws(ws, ws_bytes_given, plan_bytes(pl, b1))) return e;
-    if (col_fwd(P, D, 1, N, M))
+    if (col_laplace(P, D, N, M, C))
         return run_columns(1, 1, q, k, v, nullptr, true, P, D, N, M, C, ws, ws_bytes_given, st, no_extra,
             [&](int p0, int np, ColWs& w, hipStream_t s) {
                 const size_t p = (size_t)p0;
@@ -1460,7 +1473,8 @@ static int layer_fwd(int kind, const float* q, const float* k, const float* v, c
         npc = n_pad ? n_pad + p : nullptr; keepc = keep ? keep + p * N : nullptr; outc = out + p * M * C;
     };
     const bool bump = kind == LAYER_ADD_BUMP;
-    if (col_fwd(P, D, bump ? 3 : 1, N, M) && !(kind == LAYER_ADD_RIESZ && keep == nullptr && few_keys(N)))
+    const bool columns = kind == LAYER_ADD_LAPLACE ? col_laplace(P, D, N, M, C) : col_fwd(P, D, bump ? 3 : 1, N, M);
+    if (columns && !(kind == LAYER_ADD_RIESZ && keep == nullptr && few_keys(N)))
         return layer_columns(kind, q, k, v, n_pad, keep, out, P, D, N, M, C, ws, ws_bytes_given, st);
     if (kind == LAYER_ADD_RIESZ && keep == nullptr && few_keys(N))   // the abs sums dense (few_keys), then the epilogue
         return for_chunks(P, pl.pc, [&](int p0, int np) {

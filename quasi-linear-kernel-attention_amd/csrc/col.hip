@@ -233,9 +233,21 @@ __device__ __forceinline__ void each(F f) { each_of(f, std::make_integer_sequenc
 // ---------------------------------------------------------------------------------------------------------------
 // col_merge: one workgroup per segment
 // ---------------------------------------------------------------------------------------------------------------
-// e^-x, x >= 0, rounded to nearest for the small x that the sums multiply by the thousands: near 1 the library's expf is
-// off to one side by up to an ulp, which such products add up (Laplace at N = 16384: 1.2e-6 of the result against 64 bits)
-__device__ __forceinline__ float decay(float x) { return x < 0.5f ? 1.f + expm1f(-x) : expf(-x); }
+// e^-x, x >= 0. Below 1/2 as 1 - h with h = 1 - e^-x by its Taylor series (9 terms: to 2^-26 of h), so that it rounds to
+// nearest for the small x that the sums multiply by the thousands: near 1 the library's expf is off to one side by up to an
+// ulp, which such products add up (Laplace at N = 16384: 1.2e-6 of the result against 64 bits, 1.8e-7 so).
+__device__ __forceinline__ float decay(float x) {
+    if (x >= 0.5f) return expf(-x);
+    float h = fmaf(x, -1.f / 362880.f, 1.f / 40320.f);
+    h = fmaf(x, -h, 1.f / 5040.f);
+    h = fmaf(x, -h, 1.f / 720.f);
+    h = fmaf(x, -h, 1.f / 120.f);
+    h = fmaf(x, -h, 1.f / 24.f);
+    h = fmaf(x, -h, 1.f / 6.f);
+    h = fmaf(x, -h, 0.5f);
+    h = fmaf(x, -h, 1.f);
+    return fmaf(-x, h, 1.f);
+}
 
 struct ColMergeArgs {
     const float* qs; const uint32_t* qp; const float* ks; const uint32_t* kp;   // sorted queries and keys
@@ -1278,14 +1290,16 @@ ColPlan col_plan(int kind, int P, int D, int N, int M, int C) {
         pl.T = n <= 16384 ? 512 : 1024;
         pl.E = n <= pl.T * 20 ? 20 : n <= pl.T * 24 ? 24 : n <= pl.T * 28 ? 28 : 32;
     }
-    // Shares of the features: the fewest rounds of workgroups over the chip, in features walked one after another (plus
-    // about two features' time per round for loading and storing the columns).
+    // Shares of the features: the fewest rounds of workgroups over the chip, in features walked one after another, plus the
+    // loading and storing of the columns per round: about six features' time where a workgroup has a CU to itself, two
+    // where others run beside it.
     const int64_t wgs = (int64_t)P * ((C + pl.CH - 1) / pl.CH), slots = 256 * (int64_t)wgs_per_cu(kind, pl.T, pl.CH, n);
     int64_t best = -1;
     for (int s = 1; s <= std::min(D, COL_SHARES); ++s) {
-        const int64_t cost = ((wgs * s + slots - 1) / slots) * ((D + s - 1) / s + 2);
+        const int64_t cost = ((wgs * s + slots - 1) / slots) * ((D + s - 1) / s + (pl.CH == 1 ? 6 : 2));
         if (best < 0 || cost < best) { best = cost; pl.DS = s; }
     }
+    pl.cost = best;
     return pl;
 }
 
