@@ -280,7 +280,7 @@ def _cpu_model():
 
 STAGES = ("lds_radix_sort", "lds_count_sort", "merge_runs", "group_queries", "query_bounds", "fill_zero", "lap_range_sums",
           "lap_range_scan", "lap_range_walk", "abs_range_sums", "abs_range_scan", "abs_range_walk", "u_to_query",
-          "u_sum", "slab_reduce")
+          "u_sum", "slab_reduce", "col_sort", "col_merge", "col_weights", "col_sum_laplace", "col_sum_abs", "col_finish")
 DENSE_STAGES = ("direct_fwd", "direct_sign")
 
 
@@ -289,13 +289,19 @@ def kernel_algorithmic_bytes(name):
     walks read the sorted keys and their perm, the grouped queries and their indices, gather v once per key and
     feature, and write one contribution row per (p, d, query) plus one v == 1 term; the reduce reads the D rows of
     each query and writes one output row + out_u; the sort reads keys and writes sorted keys + perm; the range
-    sums gather v once per key and feature; the query grouping reads q and writes values + indices."""
+    sums gather v once per key and feature; the query grouping reads q and writes values + indices. The column route:
+    one sort launch of q and k; the merge reads both with their perms and writes 6 bytes per element and the v == 1 terms;
+    the column sums read that stream once per p and v's columns, and write the output's; the finish makes them rows."""
     S = P * D
     walk = 4.0 * S * (2 * N + 2 * M + N * C + M * C + M)
     table = {
         "lap_range_walk": walk, "abs_range_walk": walk,
         "slab_reduce": 4.0 * P * M * (D * C + D + C + 1),
-        "lds_radix_sort": 12.0 * S * N, "lds_count_sort": 12.0 * S * N,
+        "lds_radix_sort": 12.0 * S * (N + M), "lds_count_sort": 12.0 * S * (N + M),
+        "col_merge": S * (14.0 * (N + M) + 4 * M),
+        "col_sum_laplace": 6.0 * S * (N + M) + 4.0 * P * C * (N + M),
+        "col_sum_abs": 6.0 * S * (N + M) + 4.0 * P * C * (N + M),
+        "col_weights": 8.0 * P * N * C, "col_finish": 8.0 * P * M * C + 4.0 * M * (S + P),
         "lap_range_sums": 4.0 * S * (2 * N + N * C), "abs_range_sums": 4.0 * S * (2 * N + N * C),
         "group_queries": 12.0 * S * M,
     }

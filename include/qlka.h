@@ -39,6 +39,8 @@ int qlka_version(void);
  * accuracy with a handful of keys). Default 512; 0 sorts and walks everything else. Process-wide; returns the previous
  * value (or -QLKA_EINVAL for n < 0). The C-level counterpart of the reference's set_keops_cutoff
  * (Weighted_Abs_Sum/weighted_abs_sum/ops.py:21-25), which picks the KeOps backend in Python.
+ * B = 0 turns every routing by small size off: the column route (segments of N + M <= 32768 elements), which small calls
+ * otherwise leave to the walks, then takes every size it can.
  */
 int qlka_set_direct_max(int n);
 /*

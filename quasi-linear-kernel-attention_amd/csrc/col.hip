@@ -23,8 +23,9 @@
 // 8 and 6 cycles a wave, bank conflicts of 64 random words), beside some 10 (abs) or 15 (Laplace) vector instructions; at
 // N = M = 16384, one channel per workgroup, that is 0.6 ms of LDS and 0.5 ms of VALU for the measured 0.81 ms (abs,
 // P = 12, D = C = 64; Laplace 0.91). LDS float atomics in place of the read and the write ran at 100 cycles a wave
-// (4.3 ms). Whole calls against the walk: abs 1.70 -> 1.40 ms, Laplace 1.69 -> 1.55 ms at that size, Laplace 0.81 ->
-// 0.58 ms at N = M = 8192, add_riesz 0.97 -> 0.68 ms at 24 x 3111.
+// (4.3 ms). Whole calls against the walk: abs 1.70 -> 1.36 ms, Laplace 1.69 -> 1.54 ms at that size, Laplace 0.81 ->
+// 0.52 ms at N = M = 8192, add_riesz 0.97 -> 0.55 ms at 24 x 3111, add_bump 8.9 -> 5.5 ms at 48 x 8192, abs forward +
+// backward 4.76 -> 3.65 ms at 12 x 16384.
 #include <algorithm>
 #include <utility>
 
@@ -458,7 +459,8 @@ void col_merge(const ColMergeArgs A)
 // wave is a running count per digit (a wave's own 256 counters in LDS) plus the equal lanes below it; one scan over
 // (digit, wave) makes the counts first positions, and values and word indices go to their places through LDS. Nothing
 // is read from or written to memory between the inputs and the stream. Masked keys sort last, as padding.
-// What bounds it: about 50 vector instructions per element and pass (the ballots), 16 waves a CU.
+// What bounds it: about 60 vector instructions per element and pass (the ballots), then some 38 cycles of LDS, one after the
+// other: 155 us for 768 segments of 16384 elements (the two sorts and the merge: 178).
 // ---------------------------------------------------------------------------------------------------------------
 __host__ __device__ constexpr int sort_words(int T, int E) { return T * E + T * E / 32 + 1 + 256 * (T / WAVE) + 32; }
 
