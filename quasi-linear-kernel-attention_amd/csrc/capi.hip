@@ -494,7 +494,7 @@ inline bool col_bwd(int P, int D, int N, int M) {
 }
 inline bool col_sgn(int P, int D, int N, int M) { return col_bwd(P, D, N, M) && N + M <= COL_MAX2; }
 
-struct ColWs { SortedWs s; ColStream str; float* u; float* cols; float* wt; char* extra; };
+struct ColWs { SortedWs s; ColStream str; float* u; float* cols; float* wt; float* bad; char* extra; };
 
 size_t col_part(const ColPlan& pl, int P, int D, int N, int M, int C, int sets, int i) {
     const size_t S = (size_t)P * D;
@@ -506,11 +506,12 @@ size_t col_part(const ColPlan& pl, int P, int D, int N, int M, int C, int sets, 
         case 6: return align256(S * sets * M * 4);
         case 7: return align256((size_t)P * pl.DS * C * M * 4);
         case 8: return align256((size_t)P * (C + 1) * N * 4);
+        case 9: return align256((size_t)P * M * 4);
     }
     return 0;
 }
 
-constexpr int COL_PARTS = 9;
+constexpr int COL_PARTS = 10;
 
 // Workspace of a chunk of P p, the columns sized for the most feature shares: their number depends on the whole call's P,
 // and neither the sizes nor (the plan being the whole call's) the results may depend on the chunking.
@@ -535,6 +536,7 @@ ColWs col_carve(ColPlan pl, void* ws, int P, int D, int N, int M, int C, int set
     r.u = (float*)part[6];
     r.cols = (float*)part[7];
     r.wt = (float*)part[8];
+    r.bad = (float*)part[9];
     r.extra = b;
     return r;
 }
@@ -555,17 +557,17 @@ int run_columns(int kind, int sets, const float* q, const float* k, const float*
         if (!want_u) w.u = nullptr;
         const size_t p = (size_t)p0;
         const uint8_t* kc = keep ? keep + p * N : nullptr;
+        if (int e = col_weights_launch(pl, v + p * N * C, kc, false, nullptr, w.wt, w.bad, np * M, np, N, C, st))
+            return hip_status(e, "weight columns");
         if (q && sets == 1 && col_sort_applies(pl)) {
-            if (int e = col_sort_launch(kind, pl, q + p * D * M, k + p * D * N, kc, w.str, w.u, np * D, D, N, M, st))
+            if (int e = col_sort_launch(kind, pl, q + p * D * M, k + p * D * N, kc, w.str, w.u, w.bad, np * D, D, N, M, st))
                 return hip_status(e, "sort of q and k");
         } else {
             if (int e = sort(p0, np, w, st)) return e;
-            if (int e = col_merge_launch(kind, pl, w.s.qs, w.s.qp, w.s.ks, w.s.kp, kc, w.str, w.u, np * D, D, N, M,
+            if (int e = col_merge_launch(kind, pl, w.s.qs, w.s.qp, w.s.ks, w.s.kp, kc, w.str, w.u, w.bad, np * D, D, N, M,
                                          false, sets, st))
                 return hip_status(e, "merge of q and k");
         }
-        if (int e = col_weights_launch(pl, v + p * N * C, kc, false, nullptr, w.wt, np, N, C, st))
-            return hip_status(e, "weight columns");
         if (int e = col_sum_launch(kind, pl, w.str, w.wt, w.cols, np, D, N, M, C, sets, st))
             return hip_status(e, "column sums");
         return finish(p0, np, w, pl, st); });
@@ -589,6 +591,7 @@ size_t col_bwd_part(const ColPlan& pl, int P, int D, int N, int M, int C, int i)
         case 6: return align256((size_t)P * C1 * N * 4);
         case 7: return align256((size_t)P * C1 * M * 4);
         case 8: return align256((size_t)P * std::min(D, COL_SHARES) * C * N * 4);
+        case 9: return align256((size_t)P * N * 4);
     }
     return 0;
 }
@@ -620,20 +623,22 @@ int run_bwd_columns(const float* v, const float* g_w, const float* g_u, float sc
         w.sort_scratch = part[4];
         const ColStream str = col_stream(pl, part[5], np * D);
         float *vt = (float*)part[6], *gt = (float*)part[7], *cols = (float*)part[8];
+        float* bad = grad_v ? (float*)part[9] : nullptr;
         const size_t p = (size_t)p0;
         const int CW = (C + (g_u ? 1 : 0) + pl.CH - 1) / pl.CH;
+        if (int e = col_weights_launch(pl, v + p * N * C, nullptr, g_u != nullptr, nullptr, vt, bad, bad ? np * N : 0, np,
+                                       N, C, st))
+            return hip_status(e, "value columns");
+        if (int e = col_weights_launch(pl, g_w + p * M * C, nullptr, g_u != nullptr, g_u ? g_u + p * M : nullptr, gt,
+                                       nullptr, 0, np, M, C, st))
+            return hip_status(e, "gradient columns");
         if (int e = sorts(p0, np, w, st)) return e;
-        if (int e = col_merge_launch(0, pl, w.qs, w.qp, w.ks, w.kp, nullptr, str, nullptr, np * D, D, N, M, true, 1,
+        if (int e = col_merge_launch(0, pl, w.qs, w.qp, w.ks, w.kp, nullptr, str, nullptr, bad, np * D, D, N, M, true, 1,
                                      st))
             return hip_status(e, "merge of q and k");
-        if (int e = col_weights_launch(pl, v + p * N * C, nullptr, g_u != nullptr, nullptr, vt, np, N, C, st))
-            return hip_status(e, "value columns");
-        if (int e = col_weights_launch(pl, g_w + p * M * C, nullptr, g_u != nullptr, g_u ? g_u + p * M : nullptr, gt, np, M,
-                                       C, st))
-            return hip_status(e, "gradient columns");
         if (grad_v) {
             if (int e = col_grad_v_launch(pl, str, gt, CW, cols, np, D, N, M, C, st)) return hip_status(e, "grad_v columns");
-            if (int e = col_finish_launch(0, -1, false, pl, cols, nullptr, grad_v + p * N * C, nullptr, ReduceEpilogue{}, np, D,
+            if (int e = col_finish_launch(0, -1, false, pl, cols, nullptr, bad, grad_v + p * N * C, nullptr, ReduceEpilogue{}, np, D,
                                           N, C, st))
                 return hip_status(e, "columns to rows");
         }
@@ -690,7 +695,7 @@ int qlka_laplace_fwd(const float* q, const float* k, const float* v, float* out_
                 return sort_both(q + p * D * M, k + p * D * N, w.s, np * D, N, M, s); },
             [&](int p0, int np, ColWs& w, const ColPlan& cp, hipStream_t s) {
                 const size_t p = (size_t)p0;
-                return hip_status(col_finish_launch(1, -1, false, cp, w.cols, w.u, out_w + p * M * C, out_u + p * M,
+                return hip_status(col_finish_launch(1, -1, false, cp, w.cols, w.u, w.bad, out_w + p * M * C, out_u + p * M,
                                                     ReduceEpilogue{}, np, D, M, C, s), "columns to rows"); });
     // per chunk: sort k and group q; range passes and walk; reduce
     auto prep = [&](int p0, int np, void* buf, hipStream_t s) {
@@ -824,7 +829,7 @@ int abs_fwd_impl(const float* q, const float* k, const float* v, float* out_w, f
                 return sort_both(q + p * D * M, k + p * D * N, w.s, np * D, N, M, s); },
             [&](int p0, int np, ColWs& w, const ColPlan& cp, hipStream_t s) {
                 const size_t p = (size_t)p0;
-                return hip_status(col_finish_launch(0, -1, false, cp, w.cols, w.u, out_w + p * M * C,
+                return hip_status(col_finish_launch(0, -1, false, cp, w.cols, w.u, w.bad, out_w + p * M * C,
                                                     out_u ? out_u + p * M : nullptr, ReduceEpilogue{}, np, D, M, C, s),
                                   "columns to rows"); });
         if (e) return e;
@@ -1451,7 +1456,8 @@ static int layer_columns(int kind, const float* q, const float* k, const float* 
             if (int e = layer_epilogue_params(kind, keep != nullptr, q + p * D * M, n_pad ? n_pad + p : nullptr, pre,
                                               (float*)w.extra, out + p * M * C, np, D, M, C, &ep, s))
                 return hip_status(e, "layer query terms");
-            return hip_status(col_finish_launch(laplace ? 1 : 0, kind, keep != nullptr, cp, w.cols, w.u, nullptr, nullptr, ep, np,
+            return hip_status(col_finish_launch(laplace ? 1 : 0, kind, keep != nullptr, cp, w.cols, w.u, w.bad, nullptr, nullptr, ep,
+                                                np,
                                                 D * sets, M, C,
                                                 s), "columns to rows"); });
 }

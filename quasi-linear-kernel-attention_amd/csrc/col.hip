@@ -27,6 +27,7 @@
 // 0.52 ms at N = M = 8192, add_riesz 0.97 -> 0.55 ms at 24 x 3111, add_bump 8.9 -> 5.5 ms at 48 x 8192, abs forward +
 // backward 4.76 -> 3.65 ms at 12 x 16384.
 #include <algorithm>
+#include <cfloat>
 #include <utility>
 
 #include "qlka_common.h"
@@ -255,6 +256,7 @@ struct ColMergeArgs {
     const uint8_t* keep;             // (P, N) key mask or null: masked keys weigh 0 in the v == 1 terms
     float* val; uint16_t* tag; float* xe; uint32_t* eq;      // eq: null unless wanted
     float* u;                        // (S, M) v == 1 terms in query order, or null
+    float* bad;                      // (P, M), bwd: (P, N): NaN at the rows whose own value makes them NaN, 0 else; or null
     int D, N, M, K0;
     int sets;                        // 1, or 3: streams of q, q + 1 and q - 1 per segment (add_bump), their v == 1 terms weighted
 };
@@ -264,30 +266,74 @@ struct ColMergeArgs {
 __device__ __forceinline__ float set_shift(int set) { return set == 0 ? 0.f : set == 1 ? 1.f : -1.f; }
 __device__ __forceinline__ float set_weight(int sets, int set) { return sets == 1 ? 1.f : set == 0 ? -1.f : 0.5f; }
 
+// A finite stand-in for an element that carries no weight: x, or the largest float on x's side. Its value enters the shared
+// sums as value x 0, which an infinity or a NaN would turn into NaN for every row of the p.
+__device__ __forceinline__ float bounded(float x) { return fabsf(x) <= FLT_MAX ? x : copysignf(FLT_MAX, x); }
+// a NaN as the infinity on its side
+__device__ __forceinline__ float no_nan(float x) { return x == x ? x : copysignf(__int_as_float(0x7f800000), x); }
+// Values with which all below is finite without looking at each (abs: their differences are; Laplace: not a NaN); a segment
+// with another one is `rare`
+template <int KIND>
+__device__ __forceinline__ bool ordinary(float x) { return KIND == COL_ABS ? fabsf(x) <= 1e37f : x == x; }
+// true in the whole workgroup if x is in any of its threads; flags: W words of LDS, read before they may be written again
+template <int W>
+__device__ __forceinline__ bool any_of(bool x, uint32_t* flags) {
+    const uint64_t b = __ballot(x);
+    if (lane_id() == 0) flags[wave_in_block()] = b != 0;
+    __syncthreads();
+    return __ballot(flags[lane_id() % W] != 0) != 0;
+}
+
 // The stream and the v == 1 terms of one segment, from its merged order: thread t's elements as word indices src (padding:
-// K0 + N) and as values (abs) or distances to the element before (Laplace) in dist; x0 the median key, xs the value before
-// the thread's first element, xs0 and xn its first and last. sm: N + M words and the scan's aggregates, free to use.
+// K0 + N) and as values val (padding: the value before); x0 the median key, xs the value before the thread's first element.
+// sm: N + M words and the scan's aggregates, free to use.
+//
+// A query (bwd: a key) only receives sums, so whatever it holds stays in its own row. In a rare segment abs sums take its
+// value bounded, Laplace sums a NaN as the infinity on its side, and the row is marked in A.bad, which the finish makes NaN:
+// for abs where the value is infinite or NaN (as the walks' rows are), for Laplace where it is NaN (an infinite one is far
+// from every finite key). poison: a NaN among the weights' values that val no longer shows; every row is NaN.
 template <int KIND, int T, int E>
-__device__ __forceinline__ void emit_stream(const ColMergeArgs& A, float* sm, int s, float x0, float xs, float xs0, float xn,
-                                            float (&dist)[E], int (&src)[E])
+__device__ __forceinline__ void emit_stream(const ColMergeArgs& A, float* sm, int s, float x0, float xs, float (&val)[E],
+                                            int (&src)[E], bool rare, bool poison)
 {
     constexpr int W = T / WAVE;
     const int N = A.N, M = A.M, n = N + M, tid = threadIdx.x, seg = s / A.sets, p = seg / A.D;
+    const int acc0 = A.eq ? A.K0 : 0, accs = A.eq ? N : M;       // the words that receive sums
+    auto receives = [&](int e) { return (uint32_t)(src[e] - acc0) < (uint32_t)accs; };
+    auto weightless = [&](int e) { return receives(e) || src[e] == A.K0 + N; };
+    if (rare) {
+        if constexpr (KIND == COL_LAPLACE) xs = no_nan(xs);
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const bool row = receives(e) && (KIND == COL_ABS ? !(fabsf(val[e]) <= FLT_MAX) : val[e] != val[e]);
+            if (row && A.bad) A.bad[(size_t)p * accs + (src[e] - acc0)] = __int_as_float(0x7fc00000);
+            if (weightless(e)) val[e] = KIND == COL_ABS ? bounded(val[e]) : no_nan(val[e]);
+        }
+    }
+    float dist[E];
     // A thread's values are taken relative to its anchor, so that where a gap splits its elements, those on the median's
     // side stay precise: every value an element's sums are formed from is then bounded by distances to keys
-    float anchor = 0.f;
+    float anchor = 0.f, dec = 1.f;
     if constexpr (KIND == COL_ABS) {
-        const float xa = xn <= x0 ? xn : xs0;
+        const float xa = val[E - 1] <= x0 ? val[E - 1] : val[0];
         anchor = xa - x0;
 #pragma unroll
-        for (int e = 0; e < E; ++e) dist[e] -= xa;
-    }
-    // e^-distance once per element for all channels
-    float dec = 1.f;
-    if constexpr (KIND == COL_LAPLACE) {
+        for (int e = 0; e < E; ++e) dist[e] = val[e] - xa;
+        if (rare) {
+            anchor = poison ? __int_as_float(0x7fc00000) : bounded(anchor);
 #pragma unroll
-        for (int e = 0; e < E; ++e) dist[e] = decay(dist[e]);
-        dec = xn != xs ? decay(xn - xs) : 1.f;
+            for (int e = 0; e < E; ++e)
+                if (weightless(e)) dist[e] = bounded(dist[e]);
+        }
+    } else {                                             // e^-distance once per element for all channels
+        float prev = xs;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            dist[e] = decay(val[e] != prev ? val[e] - prev : 0.f);       // equal infinities: 0 apart
+            prev = val[e];
+        }
+        dec = prev != xs ? decay(prev - xs) : 1.f;
+        if (rare && poison) dec = __int_as_float(0x7fc00000);
     }
     float* vo = A.val + (size_t)s * T * E;
     uint16_t* to = A.tag + (size_t)s * T * E;
@@ -391,11 +437,37 @@ void col_merge(const ColMergeArgs A)
     const float* qs = A.qs + (size_t)seg * M;
     const float* ks = A.ks + (size_t)seg * N;
     const float shift = set_shift(s - seg * A.sets);
+    bool odd = false;
 #pragma unroll 8
-    for (int i = tid; i < M; i += T) sm[i] = qs[i] + shift;
+    for (int i = tid; i < M; i += T) {
+        const float x = qs[i] + shift;
+        odd |= !ordinary<KIND>(x);
+        sm[i] = x;
+    }
 #pragma unroll 8
-    for (int i = tid; i < N; i += T) sm[M + i] = ks[i];
-    __syncthreads();
+    for (int i = tid; i < N; i += T) {
+        const float x = ks[i];
+        odd |= !ordinary<KIND>(x);
+        sm[M + i] = x;
+    }
+    const bool rare = any_of<T / WAVE>(odd, (uint32_t*)sm + n);
+    bool poison = false;
+    if (rare) {          // the merge compares floats: NaNs become infinities, on the side that the sort put them
+        bool nan = false;
+        for (int i = tid; i < n; i += T) {
+            const float x = sm[i];
+            if (x == x) continue;
+            sm[i] = no_nan(x);
+            const bool weight = (i >= M) == (A.eq == nullptr);
+            if (weight) nan = true;
+            else if (A.bad) {
+                const int row = i < M ? (int)A.qp[(size_t)seg * M + i] : (int)A.kp[(size_t)seg * N + i - M];
+                A.bad[(size_t)(seg / A.D) * (A.eq ? N : M) + row] = x;
+            }
+        }
+        __syncthreads();
+        poison = any_of<T / WAVE>(nan, (uint32_t*)sm + n);
+    }
     const float* sq = sm;
     const float* sk = sm + M;
     const float x0 = sk[N / 2];
@@ -416,7 +488,7 @@ void col_merge(const ColMergeArgs A)
     const float xs = prev;
     float qa = sq[min(i, M - 1)], kb = sk[min(j, N - 1)];
     uint32_t eq = 0;
-    float dist[E];                      // abs: the element's value; Laplace: its distance to the previous element
+    float val[E];
     int src[E];                         // word of the element in sq / sk
 #pragma unroll
     for (int e = 0; e < E; ++e) {
@@ -425,15 +497,13 @@ void col_merge(const ColMergeArgs A)
         const float r = tq ? qa : kb;
         src[e] = live ? (tq ? i : M + j) : n;
         if (live && diag + e > 0 && r == prev) eq |= 1u << e;
-        if constexpr (KIND == COL_LAPLACE) dist[e] = (live && r != prev) ? r - prev : 0.f;   // equal infinities: 0 apart
-        else dist[e] = live ? r : prev;
+        val[e] = live ? r : prev;
         if (live) {
             prev = r;
             if (tq) { ++i; qa = sq[min(i, M - 1)]; }
             else { ++j; kb = sk[min(j, N - 1)]; }
         }
     }
-    const float xn = prev, xs0 = KIND == COL_ABS ? dist[0] : 0.f;      // last and first value
     __syncthreads();
     {   // word indices over the values
         uint32_t* w = (uint32_t*)sm;
@@ -448,7 +518,7 @@ void col_merge(const ColMergeArgs A)
         for (int e = 0; e < E; ++e) src[e] = src[e] < n ? (int)w[src[e]] : A.K0 + N;
     }
     if (A.eq) A.eq[(size_t)s * T + tid] = eq;
-    emit_stream<KIND, T, E>(A, sm, s, x0, xs, xs0, xn, dist, src);
+    emit_stream<KIND, T, E>(A, sm, s, x0, xs, val, src, rare, poison);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -490,7 +560,7 @@ struct Halves {
 };
 
 template <int KIND, int T, int E>
-__global__ __launch_bounds__(T)
+__global__ __launch_bounds__(T, 4)
 void col_sort(const ColMergeArgs A)
 {
     constexpr int W = T / WAVE, L = T * E, LP = L + L / 32 + 1;
@@ -506,6 +576,7 @@ void col_sort(const ColMergeArgs A)
     uint32_t key[E], before_key = 0, last_key = 0;
     Halves<E> idx;
     int live = 0;
+    bool odd = false;
     {
         const float* q = A.qs + (size_t)s * M;
         const float* k = A.ks + (size_t)s * N;
@@ -515,13 +586,14 @@ void col_sort(const ColMergeArgs A)
             const int i = first + WAVE * j;
             const float x = i < M ? q[i] : k[min(i - M, N - 1)];
             const bool on = i < n && (i < M || !keep || keep[i - M] != 0);
-            key[j] = on ? float_to_ordered(x + 0.f) : 0xffffffffu;
+            odd |= on && !ordinary<KIND>(x);
+            key[j] = on ? min(float_to_ordered(x), 0xfffffffeu) : 0xffffffffu;
             idx.set(j, on ? (uint32_t)i : (uint32_t)n);
             live += (int)__popcll(__ballot(on));
         }
     }
     if (tid == 0) misc[0] = 0;
-    __syncthreads();
+    const bool rare = any_of<W>(odd, misc + 8);
     if (lane == 0) atomicAdd(&misc[0], (uint32_t)live);      // an integer: the order does not matter
     for (int shift = 0; shift < 32; shift += 8) {
 #pragma unroll
@@ -627,19 +699,16 @@ void col_sort(const ColMergeArgs A)
     const float lastv = ordered_to_float(last_key);
     float prev = tid == 0 ? ordered_to_float(key[0]) : tid * E - 1 < nl ? ordered_to_float(before_key) : lastv;
     const float xs = prev;
-    float dist[E];
+    float val[E];
     int src[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-        const float r = tid * E + e < nl ? ordered_to_float(key[e]) : prev;
-        if constexpr (KIND == COL_LAPLACE) dist[e] = r != prev ? r - prev : 0.f;      // equal infinities: 0 apart
-        else dist[e] = r;
-        prev = r;
+        if (tid * E + e < nl) prev = ordered_to_float(key[e]);
+        val[e] = prev;
         src[e] = (int)idx.get(e);
     }
-    const float xs0 = KIND == COL_ABS ? dist[0] : 0.f;
     __syncthreads();                                         // buf is read; the emission uses it
-    emit_stream<KIND, T, E>(A, sm, s, x0, xs, xs0, prev, dist, src);
+    emit_stream<KIND, T, E>(A, sm, s, x0, xs, val, src, rare, false);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -1142,16 +1211,17 @@ void col_dot(const ColDotArgs A)
 
 // ---------------------------------------------------------------------------------------------------------------
 // col_weights: the weight rows (P, Nw, C) as columns [P][CW][Nw][CH], masked rows 0. With C1 = C + 1 there is one more
-// channel, `extra` (P, Nw) or all ones.
+// channel, `extra` (P, Nw) or all ones. Also clears `bad` (bads words; null: 0) for the merge that comes after it.
 // ---------------------------------------------------------------------------------------------------------------
 constexpr int CF_T = 256, CF_M = 64;        // threads, rows per workgroup (also of col_finish)
 
 template <int CH>
 __global__ __launch_bounds__(CF_T)
 void col_weights(const float* __restrict__ w, const float* __restrict__ extra, const uint8_t* __restrict__ keep,
-                 float* __restrict__ out, const int Nw, const int C, const int C1)
+                 float* __restrict__ out, float* __restrict__ bad, const int bads, const int Nw, const int C, const int C1)
 {
     __shared__ float tile[130][CF_M + 1];
+    for (int i = blockIdx.x * CF_T + threadIdx.x; i < bads; i += gridDim.x * CF_T) bad[i] = 0.f;
     const int nb = (Nw + CF_M - 1) / CF_M;
     const int p = blockIdx.x / nb, n0 = (blockIdx.x - p * nb) * CF_M;
     const int rows = min(CF_M, Nw - n0), CW = (C1 + CH - 1) / CH;
@@ -1186,11 +1256,12 @@ void col_weights(const float* __restrict__ w, const float* __restrict__ extra, c
 // ---------------------------------------------------------------------------------------------------------------
 // col_finish: the feature shares' columns summed, turned into rows, with the v == 1 terms summed over the features
 // ---------------------------------------------------------------------------------------------------------------
-// scale: 2 for the abs sums, whose columns hold halves. kind < 0: out = w and out_u = u; else the layer's epilogue on
+// scale: 2 for the abs sums, whose columns hold halves. bad (P, M): NaN at the rows that are NaN whatever the columns hold
+// (emit_stream), 0 else. kind < 0: out = w and out_u = u; else the layer's epilogue on
 // them, as layer_epilogue_kernel
 __global__ __launch_bounds__(CF_T)
-void col_finish(const float* __restrict__ cols, const float* __restrict__ u, float* __restrict__ out,
-                float* __restrict__ out_u, const float scale, const int kind, const int masked, const ReduceEpilogue ep,
+void col_finish(const float* __restrict__ cols, const float* __restrict__ u, const float* __restrict__ bad,
+                float* __restrict__ out, float* __restrict__ out_u, const float scale, const int kind, const int masked, const ReduceEpilogue ep,
                 const int D, const int M, const int C, const int DS)
 {
     __shared__ float tile[128][CF_M + 1];
@@ -1200,11 +1271,12 @@ void col_finish(const float* __restrict__ cols, const float* __restrict__ u, flo
     const int lane = threadIdx.x & (CF_M - 1), wv = threadIdx.x / CF_M;
     const int m = min(m0 + lane, M - 1);
     const float* src = cols + (size_t)p * DS * C * M + m;
+    const float spoilt = bad[(size_t)p * M + m];         // 0 or NaN
 #pragma unroll 4
     for (int c = wv; c < C; c += CF_T / CF_M) {
         float x = src[(size_t)c * M];
         for (int s = 1; s < DS; ++s) x += src[(size_t)(s * C + c) * M];
-        tile[c][lane] = scale * x;
+        tile[c][lane] = spoilt == spoilt ? scale * x : spoilt;
     }
     if (u) {
         const float* up = u + (size_t)p * D * M + m;
@@ -1216,7 +1288,8 @@ void col_finish(const float* __restrict__ cols, const float* __restrict__ u, flo
     __syncthreads();
     const int rows = min(CF_M, M - m0);
     if (u && kind < 0 && threadIdx.x < rows)
-        out_u[(size_t)p * M + m0 + lane] = (us[0][lane] + us[1][lane]) + (us[2][lane] + us[3][lane]);
+        out_u[(size_t)p * M + m0 + lane] =
+            spoilt == spoilt ? (us[0][lane] + us[1][lane]) + (us[2][lane] + us[3][lane]) : spoilt;
     float* dst = (kind < 0 ? out : ep.out) + ((size_t)p * M + m0) * C;
     const float np = (kind >= 0 && ep.n_pad) ? ep.n_pad[p] : 0.f;
     int r = threadIdx.x / C, c = threadIdx.x - r * C;
@@ -1380,8 +1453,8 @@ int launch_sum(const ColSumArgs& a, hipStream_t st) {
 bool col_sort_applies(const ColPlan& pl) { return pl.E <= 16; }
 
 int col_sort_launch(int kind, const ColPlan& pl, const float* q, const float* k, const uint8_t* keep, ColStream str,
-                    float* u, int S, int D, int N, int M, hipStream_t st) {
-    const ColMergeArgs a{q, nullptr, k, nullptr, keep, str.val, str.tag, str.xe, nullptr, u, D, N, M, M, 1};
+                    float* u, float* bad, int S, int D, int N, int M, hipStream_t st) {
+    const ColMergeArgs a{q, nullptr, k, nullptr, keep, str.val, str.tag, str.xe, nullptr, u, bad, D, N, M, M, 1};
     StageTimer t("col_sort", st);
     return dispatch_shape(pl, [&](auto T, auto E, auto) {
         if constexpr (E() > 16) {
@@ -1402,9 +1475,9 @@ int col_sort_launch(int kind, const ColPlan& pl, const float* q, const float* k,
 }
 
 int col_merge_launch(int kind, const ColPlan& pl, const float* qs, const uint32_t* qp, const float* ks,
-                     const uint32_t* kp, const uint8_t* keep, ColStream str, float* u, int S, int D, int N, int M,
-                     bool bwd, int sets, hipStream_t st) {
-    const ColMergeArgs a{qs, qp, ks, kp, keep, str.val, str.tag, str.xe, bwd ? str.eq : nullptr, u, D, N, M,
+                     const uint32_t* kp, const uint8_t* keep, ColStream str, float* u, float* bad, int S, int D, int N,
+                     int M, bool bwd, int sets, hipStream_t st) {
+    const ColMergeArgs a{qs, qp, ks, kp, keep, str.val, str.tag, str.xe, bwd ? str.eq : nullptr, u, bad, D, N, M,
                          bwd ? col_key0(pl, M) : M, sets};
     S *= sets;
     StageTimer t("col_merge", st);
@@ -1413,13 +1486,15 @@ int col_merge_launch(int kind, const ColPlan& pl, const float* qs, const uint32_
 }
 
 int col_weights_launch(const ColPlan& pl, const float* w, const uint8_t* keep, bool more, const float* extra, float* wt,
-                       int P, int Nw, int C, hipStream_t st) {
+                       float* bad, int bads, int P, int Nw, int C, hipStream_t st) {
     StageTimer t("col_weights", st);
     const dim3 grid((unsigned)(P * ((Nw + CF_M - 1) / CF_M)));
     if (pl.CH == 2)
-        hipLaunchKernelGGL(col_weights<2>, grid, dim3(CF_T), 0, st, w, extra, keep, wt, Nw, C, C + (more ? 1 : 0));
+        hipLaunchKernelGGL(col_weights<2>, grid, dim3(CF_T), 0, st, w, extra, keep, wt, bad, bads, Nw, C,
+                           C + (more ? 1 : 0));
     else
-        hipLaunchKernelGGL(col_weights<1>, grid, dim3(CF_T), 0, st, w, extra, keep, wt, Nw, C, C + (more ? 1 : 0));
+        hipLaunchKernelGGL(col_weights<1>, grid, dim3(CF_T), 0, st, w, extra, keep, wt, bad, bads, Nw, C,
+                           C + (more ? 1 : 0));
     return (int)hipGetLastError();
 }
 
@@ -1450,10 +1525,10 @@ int col_dot_launch(const ColPlan& pl, ColStream str, const float* gt, const floa
         return (int)hipGetLastError(); });
 }
 
-int col_finish_launch(int kind, int layer, bool masked, const ColPlan& pl, const float* cols, const float* u, float* out,
-                      float* out_u, const ReduceEpilogue& ep, int P, int D, int M, int C, hipStream_t st) {
+int col_finish_launch(int kind, int layer, bool masked, const ColPlan& pl, const float* cols, const float* u,
+                      const float* bad, float* out, float* out_u, const ReduceEpilogue& ep, int P, int D, int M, int C, hipStream_t st) {
     StageTimer t("col_finish", st);
-    hipLaunchKernelGGL(col_finish, dim3((unsigned)(P * ((M + CF_M - 1) / CF_M))), dim3(CF_T), 0, st, cols, u, out, out_u,
+    hipLaunchKernelGGL(col_finish, dim3((unsigned)(P * ((M + CF_M - 1) / CF_M))), dim3(CF_T), 0, st, cols, u, bad, out, out_u,
                        kind == COL_ABS ? 2.f : 1.f, layer, masked ? 1 : 0, ep, D, M, C, pl.DS);
     return (int)hipGetLastError();
 }

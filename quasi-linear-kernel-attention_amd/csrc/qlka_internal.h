@@ -271,18 +271,19 @@ size_t col_stream_bytes(const ColPlan& pl, int S);
 ColStream col_stream(const ColPlan& pl, void* base, int S);
 // the merged stream of S sorted segments, and the v == 1 terms u (S, M) in query order (null: none; masked keys weigh 0).
 // bwd: the stream of the abs backward (keys' words from col_key0, runs of equal values). sets = 3 (kind 0): three streams
-// and rows of u per segment, of q, q + 1 and q - 1, which the sums weight -1, 1/2, 1/2 (add_bump); else 1.
+// and rows of u per segment, of q, q + 1 and q - 1, which the sums weight -1, 1/2, 1/2 (add_bump); else 1. bad (P, M), with
+// bwd (P, N), cleared before (col_weights_launch): NaN where a row's own value makes it NaN (null: not wanted).
 int col_merge_launch(int kind, const ColPlan& pl, const float* qs, const uint32_t* qp, const float* ks,
-                     const uint32_t* kp, const uint8_t* keep, ColStream str, float* u, int S, int D, int N, int M,
-                     bool bwd, int sets, hipStream_t st);
+                     const uint32_t* kp, const uint8_t* keep, ColStream str, float* u, float* bad, int S, int D, int N,
+                     int M, bool bwd, int sets, hipStream_t st);
 // the same stream from unsorted q and k in one kernel, masked keys as padding
 bool col_sort_applies(const ColPlan& pl);
 int col_sort_launch(int kind, const ColPlan& pl, const float* q, const float* k, const uint8_t* keep, ColStream str,
-                    float* u, int S, int D, int N, int M, hipStream_t st);
+                    float* u, float* bad, int S, int D, int N, int M, hipStream_t st);
 // wt: the columns of rows w (P, Nw, C) in groups of pl.CH, rows masked by keep (null: none) 0; `more`: one more channel,
-// extra (P, Nw) or ones
+// extra (P, Nw) or ones. Clears the `bads` words of bad.
 int col_weights_launch(const ColPlan& pl, const float* w, const uint8_t* keep, bool more, const float* extra, float* wt,
-                       int P, int Nw, int C, hipStream_t st);
+                       float* bad, int bads, int P, int Nw, int C, hipStream_t st);
 // The abs backward over a bwd stream and the columns gt, vt (CW groups each) of g_w and v: cols[P][DS][C][N] = half of
 // grad_v; and gq = scale / 2 times grad_q, gk (or null) the same of grad_k (last: it overwrites str.val)
 bool col_bwd_applies(int D, int N, int M);
@@ -294,9 +295,10 @@ int col_dot_launch(const ColPlan& pl, ColStream str, const float* gt, const floa
 // cols[P][DS][C][M]: the sums of each feature share over the weights wt (P, C, N); half of them for kind 0
 int col_sum_launch(int kind, const ColPlan& pl, ColStream str, const float* wt, float* cols, int P, int D, int N, int M,
                    int C, int sets, hipStream_t st);
-// layer < 0: out (P, M, C) and, with u, out_u (P, M); else the epilogue of layer kind `layer` written to ep.out
-int col_finish_launch(int kind, int layer, bool masked, const ColPlan& pl, const float* cols, const float* u, float* out,
-                      float* out_u, const ReduceEpilogue& ep, int P, int D, int M, int C, hipStream_t st);
+// layer < 0: out (P, M, C) and, with u, out_u (P, M); else the epilogue of layer kind `layer` written to ep.out. Rows marked
+// in bad are NaN.
+int col_finish_launch(int kind, int layer, bool masked, const ColPlan& pl, const float* cols, const float* u,
+                      const float* bad, float* out, float* out_u, const ReduceEpilogue& ep, int P, int D, int M, int C, hipStream_t st);
 
 // ---- capi.hip helpers for noalloc.hip
 // check_dims of the C ABI (clears the thread's error first); the workspace of a Laplace forward over pc p at a time;

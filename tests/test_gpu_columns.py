@@ -154,3 +154,97 @@ def test_column_backward(dev, no_dense, shape, kind):
     sgn = weighted_sgn_sum(*t[:4], backend="cuda").cpu().numpy()
     (wq, _, _), (nq, _, _) = brute.abs_backward_sub(q, k, v, g, None, iq, ik)
     assert float(brute.rel_err(pick(sgn, iq, 1), -wq, nq).max()) <= REL
+
+
+# ---- queries and keys that are not finite, or huge: their own row only
+
+BAD = {"inf": np.inf, "-inf": -np.inf, "nan": np.nan, "-nan": -np.nan, "huge": 3e38}
+
+
+def _layer64(kernel, q, k, v, keep, M):
+    """float64 num (rows, C) and den (rows) of one p's layer at queries q (D, rows) over its kept keys k (D, N) with rows v,
+    and the sums of |term| that the abs or Laplace sums and the epilogue form them from: each is within REL of those."""
+    from qlka import layers
+    n_pad = int((~keep).sum())
+    q, k, v = q.astype(np.float64), k[:, keep].astype(np.float64), v[keep].astype(np.float64)
+    x = q[:, :, None] - k[:, None]
+    if kernel == "add_laplace":
+        A = S = np.exp(-np.abs(x)).sum(0)
+    elif kernel == "add_bump":
+        A = np.maximum(0, 1 - np.abs(x)).sum(0)
+        S = ((np.abs(x + 1) + np.abs(x - 1)) / 2 + np.abs(x)).sum(0)
+    else:
+        near, far = np.abs(x).sum(0), np.abs(q).sum(0)[:, None] + np.abs(k).sum(0)[None] + layers.EPS
+        A, S = far - near, far + near
+    den, sden = A.sum(1), S.sum(1)
+    if kernel == "add_riesz":                      # it counts M keys (attention.py:78), less the masked ones
+        den = den + (np.abs(q).sum(0) + layers.EPS) * (M - n_pad - k.shape[1])
+    return A @ v, np.maximum(den, layers.CLAMP), S @ np.abs(v), sden
+
+
+def _assert_layer(kernel, got, q, k, v, keep, M):
+    num, den, snum, sden = _layer64(kernel, q, k, v, keep, M)
+    assert np.isfinite(got).all(), kernel
+    err = np.abs(got * den[:, None] - num)
+    np.testing.assert_array_less(err, REL * (snum + np.abs(got) * sden[:, None]) + 1e-30, err_msg=kernel)
+
+
+@pytest.mark.parametrize("bad", sorted(BAD))
+@pytest.mark.parametrize("shape", [(2, 3, 700, 650, 5), (1, 2, 12000, 11000, 3), (1, 2, 16000, 16000, 2)])
+def test_a_bad_query_spoils_only_its_row(dev, no_dense, shape, bad):
+    # as by the walks: abs and layer rows of an infinite or NaN query are NaN, Laplace's are 0 for an infinite one; every
+    # other row is what the oracle says. A huge finite query (differences past the largest float) spoils no other row.
+    from qlka import layers
+    from weighted_abs_sum import weighted_abs_sum, weighted_abs_sum_full
+    from weighted_laplace_sum import weighted_laplace_sum
+    P, D, N, M, C = shape
+    print(f"bad query {shape} {bad}", flush=True)
+    q, k, v = _data(P, D, N, M, C, "normal", 3)
+    at = 7
+    q[0, 1, at] = BAD[bad]
+    if bad == "huge":
+        q[0, 0, at] = -3e38
+    tq, tk, tv = (torch.from_numpy(a).to(dev) for a in (q, k, v))
+    assert bool(torch.signbit(tq[0, 1, at])) == bad.startswith("-")
+    idx = inputs.query_subsample(P, M, per_p=16, seed=5)
+    idx = [i[i != at] for i in idx]
+    rows = lambda a, p: a[p][idx[p]]  # noqa: E731
+    for name, op, oracle in (("abs", lambda: weighted_abs_sum_full(tq, tk, tv, backend="cuda"), brute.abs_sum),
+                             ("plain", lambda: (weighted_abs_sum(tq, tk, tv, backend="cuda"), None), brute.abs_sum),
+                             ("laplace", lambda: weighted_laplace_sum(tq, tk, tv), brute.laplace_sum)):
+        w, u = (t if t is None else t.cpu().numpy() for t in op())
+        for p in range(P):
+            ow, ou, nw = oracle(q[p:p + 1], k[p:p + 1], v[p:p + 1], qidx=idx[p:p + 1])
+            assert float(brute.rel_err(rows(w, p)[None], ow, nw).max()) <= REL, name
+            if u is not None:
+                assert float(brute.rel_err(rows(u, p)[None], ou, ou).max()) <= REL, name
+        if bad != "huge" and (name != "laplace" or "nan" in bad):
+            assert np.isnan(w[0, at]).all() and (u is None or np.isnan(u[0, at])), name
+        elif bad != "huge":                        # the features of a finite value alone
+            ow, ou, nw = oracle(np.delete(q, 1, 1), np.delete(k, 1, 1), v, qidx=[np.array([at])] * P)
+            assert float(brute.rel_err(w[:1, at:at + 1], ow[:1], nw[:1]).max()) <= REL
+    keep = np.random.default_rng(N).random((P, N)) < 0.7
+    for kernel in layers.KINDS:
+        for mask in (np.ones_like(keep), keep):
+            arg = None if mask.all() else torch.from_numpy(mask).to(dev)
+            got = layers.layer_forward(kernel, tq, tk, tv, keep=arg).cpu().numpy()
+            for p in range(P):
+                _assert_layer(kernel, rows(got, p), q[p][:, idx[p]], k[p], v[p], mask[p], M)
+            if bad != "huge" and (kernel != "add_laplace" or "nan" in bad):
+                assert np.isnan(got[0, at]).all(), kernel
+
+
+@pytest.mark.parametrize("bad", ["inf", "nan", "-nan"])
+@pytest.mark.parametrize("shape", [(2, 3, 700, 650, 5), (1, 2, 12000, 11000, 3)])
+def test_a_bad_key_spoils_only_its_row_of_grad_v(dev, no_dense, shape, bad):
+    from weighted_abs_sum import _ext
+    P, D, N, M, C = shape
+    q, k, v = _data(P, D, N, M, C, "normal", 4)
+    g = np.random.default_rng(6).standard_normal((P, M, C), dtype=np.float32)
+    k[0, 1, 9] = BAD[bad]
+    gv = _ext.weighted_abs_sum_backward(*(torch.from_numpy(a).to(dev) for a in (q, k, v, g)))[2].cpu().numpy()
+    assert np.isnan(gv[0, 9]).all()
+    idx = [i[i != 9] for i in inputs.query_subsample(P, N, per_p=16, seed=7)]
+    for p in range(P):                             # grad_v: the abs sum with q and k exchanged
+        w, _, nw = brute.abs_sum(k[p:p + 1], q[p:p + 1], g[p:p + 1], qidx=idx[p:p + 1])
+        assert float(brute.rel_err(gv[p][idx[p]][None], w, nw).max()) <= REL
