@@ -311,11 +311,12 @@ __device__ __forceinline__ void emit_stream(const ColMergeArgs& A, float* sm, in
         }
     }
     float dist[E];
-    // A thread's values are taken relative to its anchor, so that where a gap splits its elements, those on the median's
-    // side stay precise: every value an element's sums are formed from is then bounded by distances to keys
+    // A thread's values are taken relative to its anchor, its value nearest the median, so that every value an element's sums
+    // are formed from is bounded by distances to keys: on either side of the median the end towards it, and the median
+    // itself in a thread on both sides
     float anchor = 0.f, dec = 1.f;
     if constexpr (KIND == COL_ABS) {
-        const float xa = val[E - 1] <= x0 ? val[E - 1] : val[0];
+        const float xa = x0 <= val[0] ? val[0] : x0 >= val[E - 1] ? val[E - 1] : x0;
         anchor = xa - x0;
 #pragma unroll
         for (int e = 0; e < E; ++e) dist[e] = val[e] - xa;

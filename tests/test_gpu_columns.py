@@ -248,3 +248,20 @@ def test_a_bad_key_spoils_only_its_row_of_grad_v(dev, no_dense, shape, bad):
     for p in range(P):                             # grad_v: the abs sum with q and k exchanged
         w, _, nw = brute.abs_sum(k[p:p + 1], q[p:p + 1], g[p:p + 1], qidx=idx[p:p + 1])
         assert float(brute.rel_err(gv[p][idx[p]][None], w, nw).max()) <= REL
+
+
+def test_a_thread_on_both_sides_of_the_median(dev, no_dense):
+    # a far query, then the keys, all in the first thread's elements: the others' sums stay as precise as their distances to
+    # the keys are (1.5e-3 of sum |term| where such a thread's values were relative to the far query)
+    from weighted_abs_sum import weighted_abs_sum_full
+    P, D, N, M, C = 2, 2, 17, 700, 3
+    rng = np.random.default_rng(8)
+    q = (300.2 + 0.5 * rng.random((P, D, M))).astype(np.float32)
+    q[..., 0] = -4000
+    k = np.tile((300 + 0.01 * np.arange(N)).astype(np.float32), (P, D, 1))
+    v = rng.standard_normal((P, N, C), dtype=np.float32)
+    w, u = (t.cpu().numpy() for t in weighted_abs_sum_full(*(torch.from_numpy(a).to(dev) for a in (q, k, v)),
+                                                           backend="cuda"))
+    ow, ou, nw = brute.abs_sum(q, k, v)
+    assert float(brute.rel_err(w, ow, nw).max()) <= REL
+    assert float(brute.rel_err(u, ou, ou).max()) <= REL
