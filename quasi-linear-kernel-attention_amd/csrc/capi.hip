@@ -564,8 +564,10 @@ int run_columns(int kind, int sets, const float* q, const float* k, const float*
                 return hip_status(e, "sort of q and k");
         } else {
             if (int e = sort(p0, np, w, st)) return e;
-            if (int e = col_merge_launch(kind, pl, w.s.qs, w.s.qp, w.s.ks, w.s.kp, kc, w.str, w.u, w.bad, np * D, D, N, M,
-                                         false, sets, st))
+            // the Laplace layer's masked keys are already too far to count (mask_keys)
+            const uint8_t* km = kind == 0 ? kc : nullptr;
+            if (int e = col_merge_launch(kind, pl, w.s.qs, w.s.qp, w.s.ks, w.s.kp, km, w.str, w.u, w.bad, np * D, D, N,
+                                         M, false, sets, st))
                 return hip_status(e, "merge of q and k");
         }
         if (int e = col_sum_launch(kind, pl, w.str, w.wt, w.cols, np, D, N, M, C, sets, st))
@@ -1344,9 +1346,8 @@ static bool layer_pipelined(int kind, int P, int D, int M, int C) {
 }
 
 // The layers by columns: the op's columns with the layer's epilogue in their finish; add_bump's three abs sums as three
-// weighted streams per feature into one accumulator. Masked keys weigh 0;
-// their sort values are replaced as for the walks (mask_keys, fill_masked_keys), so that whatever they hold, the distances
-// run between kept keys.
+// weighted streams per feature into one accumulator. Masked keys are left out of the streams as padding, or, where the
+// Laplace sums sort k and q apart, lie too far away to count (mask_keys).
 static size_t layer_col_extra(int kind, int P, int D, int N, int M, int C) {
     return align256((size_t)P * M * 4) + (kind == LAYER_ADD_RIESZ     ? align256(riesz_prefix_bytes(P, N, C))
                                           : kind == LAYER_ADD_LAPLACE ? align256((size_t)P * D * N * 4) : 0);
@@ -1443,9 +1444,7 @@ static int layer_columns(int kind, const float* q, const float* k, const float* 
                 if (int e = hip_status(mask_keys(kc, keepc, km, np, D, N, s), "masked keys")) return e;
                 kc = km;
             }
-            if (int e = sort_both(q + p * D * M, kc, w.s, np * D, N, M, s)) return e;
-            if (keepc && !laplace) return hip_status(fill_masked_keys(w.s.ks, w.s.kp, keepc, np, D, N, s), "masked keys");
-            return (int)QLKA_OK; },
+            return sort_both(q + p * D * M, kc, w.s, np * D, N, M, s); },
         [&](int p0, int np, ColWs& w, const ColPlan& cp, hipStream_t s) {
             const size_t p = (size_t)p0;
             void* pre = w.extra + align256((size_t)np * M * 4);

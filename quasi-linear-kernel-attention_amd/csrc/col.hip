@@ -253,7 +253,7 @@ __device__ __forceinline__ float decay(float x) {
 
 struct ColMergeArgs {
     const float* qs; const uint32_t* qp; const float* ks; const uint32_t* kp;   // sorted queries and keys
-    const uint8_t* keep;             // (P, N) key mask or null: masked keys weigh 0 in the v == 1 terms
+    const uint8_t* keep;             // (P, N) key mask or null: masked keys become padding
     float* val; uint16_t* tag; float* xe; uint32_t* eq;      // eq: null unless wanted
     float* u;                        // (S, M) v == 1 terms in query order, or null
     float* bad;                      // (P, M), bwd: (P, N): NaN at the rows whose own value makes them NaN, 0 else; or null
@@ -284,8 +284,44 @@ __device__ __forceinline__ bool any_of(bool x, uint32_t* flags) {
     return __ballot(flags[lane_id() % W] != 0) != 0;
 }
 
-// The stream and the v == 1 terms of one segment, from its merged order: thread t's elements as word indices src (padding:
-// K0 + N) and as values val (padding: the value before); x0 the median key, xs the value before the thread's first element.
+__device__ __forceinline__ bool is_key(int word, const ColMergeArgs& A) { return (uint32_t)(word - A.K0) < (uint32_t)A.N; }
+
+// The median of a segment's keys that are not padding, from its merged order (as emit_stream's), 0 without any; scratch:
+// 1 + W words of LDS.
+template <int T, int E>
+__device__ __forceinline__ float median_key(const ColMergeArgs& A, const float (&val)[E], const int (&src)[E], uint32_t* scratch)
+{
+    constexpr int W = T / WAVE;
+    const int lane = lane_id(), wv = wave_in_block();
+    int keys = 0;
+#pragma unroll
+    for (int e = 0; e < E; ++e) keys += is_key(src[e], A);
+    int inc = keys;
+#pragma unroll
+    for (int off = 1; off < WAVE; off <<= 1) {
+        const int y = __shfl_up(inc, off, WAVE);
+        if (lane >= off) inc += y;
+    }
+    if (lane == WAVE - 1) scratch[1 + wv] = (uint32_t)inc;
+    if (threadIdx.x == 0) scratch[0] = 0;
+    __syncthreads();
+    int at = keys - inc, total = 0;                          // the median's number among this thread's keys
+    for (int w = 0; w < W; ++w) {
+        if (w < wv) at -= (int)scratch[1 + w];
+        total += (int)scratch[1 + w];
+    }
+    at += total / 2;
+    if (at >= 0 && at < keys) {
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            if (is_key(src[e], A) && at-- == 0) scratch[0] = __float_as_uint(val[e]);
+    }
+    __syncthreads();
+    return __uint_as_float(scratch[0]);
+}
+
+// The stream and the v == 1 terms of one segment, from its merged order: thread t's elements as word indices src (padding,
+// masked keys among it: K0 + N) and as values val (padding: the value before); x0 the median key, xs the value before the thread's first element.
 // sm: N + M words and the scan's aggregates, free to use.
 //
 // A query (bwd: a key) only receives sums, so whatever it holds stays in its own row. In a rare segment abs sums take its
@@ -352,14 +388,10 @@ __device__ __forceinline__ void emit_stream(const ColMergeArgs& A, float* sm, in
     A.xe[(size_t)s * T + tid] = KIND == COL_ABS ? anchor : dec;
     if (A.u == nullptr) return;
 
-    // v == 1: the same walk as col_sum's with every kept key's weight 1
+    // v == 1: the same walk as col_sum's with every key's weight 1
     float wt[E];
-    const uint8_t* keep = A.keep ? A.keep + (size_t)p * N : nullptr;
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const int key = src[e] - A.K0;
-        wt[e] = key >= 0 && key < N ? (keep ? (keep[key] ? 1.f : 0.f) : 1.f) : 0.f;
-    }
+    for (int e = 0; e < E; ++e) wt[e] = is_key(src[e], A) ? 1.f : 0.f;
     const int lane = lane_id(), wv = wave_in_block();
     float* agg = sm + n;
     float out[E];
@@ -438,6 +470,7 @@ void col_merge(const ColMergeArgs A)
     const float* qs = A.qs + (size_t)seg * M;
     const float* ks = A.ks + (size_t)seg * N;
     const float shift = set_shift(s - seg * A.sets);
+    const uint8_t* keep = A.keep ? A.keep + (size_t)(seg / A.D) * N : nullptr;       // without A.eq only
     bool odd = false;
 #pragma unroll 8
     for (int i = tid; i < M; i += T) {
@@ -460,18 +493,16 @@ void col_merge(const ColMergeArgs A)
             if (x == x) continue;
             sm[i] = no_nan(x);
             const bool weight = (i >= M) == (A.eq == nullptr);
-            if (weight) nan = true;
-            else if (A.bad) {
-                const int row = i < M ? (int)A.qp[(size_t)seg * M + i] : (int)A.kp[(size_t)seg * N + i - M];
-                A.bad[(size_t)(seg / A.D) * (A.eq ? N : M) + row] = x;
-            }
+            const int row = i < M ? (int)A.qp[(size_t)seg * M + i] : (int)A.kp[(size_t)seg * N + i - M];
+            if (weight) nan |= !keep || keep[row] != 0;
+            else if (A.bad) A.bad[(size_t)(seg / A.D) * (A.eq ? N : M) + row] = x;
         }
         __syncthreads();
         poison = any_of<T / WAVE>(nan, (uint32_t*)sm + n);
     }
     const float* sq = sm;
     const float* sk = sm + M;
-    const float x0 = sk[N / 2];
+    float x0 = sk[N / 2];
     // merge path: queries before `diag` (queries come first among equal values)
     const int diag = min(tid * E, n);
     int lo = max(0, diag - N), hi = min(diag, M);
@@ -513,12 +544,16 @@ void col_merge(const ColMergeArgs A)
 #pragma unroll 8
         for (int x = tid; x < M; x += T) w[x] = qp[x];
 #pragma unroll 8
-        for (int x = tid; x < N; x += T) w[M + x] = A.K0 + kp[x];
+        for (int x = tid; x < N; x += T) w[M + x] = A.K0 + (!keep || keep[kp[x]] != 0 ? kp[x] : (uint32_t)N);
         __syncthreads();
 #pragma unroll
         for (int e = 0; e < E; ++e) src[e] = src[e] < n ? (int)w[src[e]] : A.K0 + N;
     }
     if (A.eq) A.eq[(size_t)s * T + tid] = eq;
+    if (KIND == COL_ABS && keep) {
+        x0 = median_key<T, E>(A, val, src, (uint32_t*)sm + n);
+        __syncthreads();                                     // read; the emission writes there
+    }
     emit_stream<KIND, T, E>(A, sm, s, x0, xs, val, src, rare, poison);
 }
 
@@ -568,7 +603,7 @@ void col_sort(const ColMergeArgs A)
     extern __shared__ float sm[];
     uint32_t* buf = (uint32_t*)sm;
     uint32_t* all = (uint32_t*)sm + LP;                      // [W][256] counters
-    uint32_t* misc = all + 256 * W;                          // [0] live elements, [4..7] [8..23] scans, [24] the median
+    uint32_t* misc = all + 256 * W;                          // [0] live elements, [4 ...] scans, [7 ...] the median
     const int s = blockIdx.x, p = s / A.D, tid = threadIdx.x, lane = lane_id(), wv = wave_in_block();
     const int N = A.N, M = A.M, n = N + M;
     uint32_t* cnt = all + 256 * wv;
@@ -674,29 +709,6 @@ void col_sort(const ColMergeArgs A)
         for (int j = 0; j < E; ++j) idx.set(j, buf[last ? padded(tid * E + j) : first + WAVE * j]);
     }
     const int nl = (int)misc[0];                             // queries and kept keys
-    float x0 = 0.f;
-    if constexpr (KIND == COL_ABS) {                         // the median of the kept keys
-        int keys = 0;
-#pragma unroll
-        for (int e = 0; e < E; ++e) keys += (int)idx.get(e) >= M && (int)idx.get(e) < n;
-        int inc = keys;
-#pragma unroll
-        for (int off = 1; off < WAVE; off <<= 1) {
-            const int y = __shfl_up(inc, off, WAVE);
-            if (lane >= off) inc += y;
-        }
-        if (lane == WAVE - 1) misc[8 + wv] = (uint32_t)inc;
-        __syncthreads();
-        int at = (nl - M) / 2 - (inc - keys);                // the median's number among this thread's keys
-        for (int w = 0; w < wv; ++w) at -= (int)misc[8 + w];
-        if (at >= 0 && at < keys) {
-#pragma unroll
-            for (int e = 0; e < E; ++e)
-                if ((int)idx.get(e) >= M && (int)idx.get(e) < n && at-- == 0) misc[24] = key[e];
-        }
-        __syncthreads();
-        if (nl > M) x0 = ordered_to_float(misc[24]);
-    }
     const float lastv = ordered_to_float(last_key);
     float prev = tid == 0 ? ordered_to_float(key[0]) : tid * E - 1 < nl ? ordered_to_float(before_key) : lastv;
     const float xs = prev;
@@ -708,6 +720,7 @@ void col_sort(const ColMergeArgs A)
         val[e] = prev;
         src[e] = (int)idx.get(e);
     }
+    const float x0 = KIND == COL_ABS ? median_key<T, E>(A, val, src, misc + 7) : 0.f;
     __syncthreads();                                         // buf is read; the emission uses it
     emit_stream<KIND, T, E>(A, sm, s, x0, xs, val, src, rare, false);
 }

@@ -265,3 +265,30 @@ def test_a_thread_on_both_sides_of_the_median(dev, no_dense):
     ow, ou, nw = brute.abs_sum(q, k, v)
     assert float(brute.rel_err(w, ow, nw).max()) <= REL
     assert float(brute.rel_err(u, ou, ou).max()) <= REL
+
+
+@pytest.mark.parametrize("kernel", ["add_laplace", "add_riesz", "add_bump"])
+@pytest.mark.parametrize("far", ["low", "both", "nan"])
+@pytest.mark.parametrize("N,M,kept", [(3000, 2000, 0.4), (3000, 2000, 0.01), (12000, 11000, 0.4), (12000, 11000, 0.001)])
+def test_mostly_masked_keys_far_out(dev, no_dense, kernel, far, N, M, kept):
+    # masked keys weigh nothing wherever they lie: most of a segment's keys masked and far below the kept ones, on both sides
+    # of them, or NaN of either sign, with kept keys and queries of scale 1
+    from qlka import layers
+    P, D, C = 2, 3, 4
+    print(f"mostly masked {kernel} N={N} kept={kept} {far}", flush=True)
+    q, k, v = _data(P, D, N, M, C, "normal", N)
+    rng = np.random.default_rng(N + 1)
+    keep = rng.random((P, N)) < kept
+    keep[1] = rng.random(N) < 0.7
+    out = -1e4 * (1 + rng.random((P, D, N)))
+    if far == "both":
+        out *= np.where(rng.random((P, 1, N)) < 0.5, -1e3, 1.0)
+    out = out.astype(np.float32)
+    if far == "nan":
+        out = np.where(rng.random((P, 1, N)) < 0.5, np.float32(np.nan), -np.float32(np.nan))
+    k = np.where(keep[:, None], k, out).astype(np.float32)
+    got = layers.layer_forward(kernel, *(torch.from_numpy(a).to(dev) for a in (q, k, v)),
+                               keep=torch.from_numpy(keep).to(dev)).cpu().numpy()
+    idx = inputs.query_subsample(P, M, per_p=24, seed=9)
+    for p in range(P):
+        _assert_layer(kernel, got[p][idx[p]], q[p][:, idx[p]], k[p], v[p], keep[p], M)
