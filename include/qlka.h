@@ -36,13 +36,21 @@ int qlka_version(void);
  * abs forward goes dense for L <= 2B, the Laplace forward for L <= B, the backward and the sgn sum for L <= B or for
  * L <= 5B/4 when P * ceil(L / 32) >= 512. Whatever B (0 included) and the pinned path, the abs forward also goes
  * dense for N <= 16 keys, and the backward and the sgn sum for min(N, M) <= 16 (the walk's segment totals lose
- * accuracy with a handful of keys). Default 512; 0 sorts and walks everything else. Process-wide; returns the previous
+ * accuracy with a handful of keys). Default 512; 0 sorts everything else. Process-wide; returns the previous
  * value (or -QLKA_EINVAL for n < 0). The C-level counterpart of the reference's set_keops_cutoff
  * (Weighted_Abs_Sum/weighted_abs_sum/ops.py:21-25), which picks the KeOps backend in Python.
- * B = 0 turns every routing by small size off: the column route (segments of N + M <= 32768 elements), which small calls
- * otherwise leave to the walks, then takes every size it can.
  */
 int qlka_set_direct_max(int n);
+/*
+ * Which sorted route a call takes, for tests and measurements: segments of N + M <= 32768 elements can run column by
+ * column, all others walk. AUTO (the default) takes the columns where they were measured faster, NEVER walks everything,
+ * ALWAYS takes the columns wherever they apply. Results agree to fp32 rounding. What the dense evaluation takes stays
+ * there (qlka_set_direct_max). Process-wide; returns the previous mode (or -QLKA_EINVAL for another one).
+ */
+#define QLKA_COLUMNS_AUTO   0
+#define QLKA_COLUMNS_NEVER  1
+#define QLKA_COLUMNS_ALWAYS 2
+int qlka_set_columns(int mode);
 /*
  * Workspace budget in bytes (default 5 GiB). Every operator below runs its whole pipeline on chunks of consecutive
  * p = (batch, head) indices (every stage works on each p alone), taking the largest chunk the workspace it is given

@@ -53,6 +53,8 @@ inline size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 constexpr int FEW_KEYS = 16;
 std::atomic<int> g_direct_max{512};
 inline int64_t direct_base() { return g_direct_max.load(std::memory_order_relaxed); }
+std::atomic<int> g_columns{QLKA_COLUMNS_AUTO};
+inline int columns_mode() { return g_columns.load(std::memory_order_relaxed); }
 inline bool few_keys(int keys) { return keys <= FEW_KEYS; }
 inline bool dense_abs_fwd(int N, int M) { return std::max(N, M) <= 2 * direct_base() || few_keys(N); }
 inline bool dense_laplace_fwd(int N, int M) { return std::max(N, M) <= direct_base(); }
@@ -466,11 +468,12 @@ int run_pipeline(int P, const Plan& pl, void* ws, size_t copy, hipStream_t st, P
 // products also take one workgroup per segment, below a million, 128 segments, or 192 where a workgroup fills a CU.
 // (P, D, M = N, C = 64:) Laplace 114 against 87 us at 1 x 64 x 2000, 99 against 139 at 12 x 64 x 520, abs 132 against 114 at
 // 1 x 64 x 4200; forward + backward 258 against 160 us at 1 x 64 x 1500, even at 12 x 64 x 640, 322 against 368 at
-// 12 x 64 x 1100, 796 against 774 at 2 x 64 x 16000. With the dense cutoff at 0, which turns the routing by small size
-// off, every size takes it. The sgn sum takes it with two channels per workgroup only (12 x 64 x 3000: 253 against 277 us;
-// 16384: 1525 against 1439).
+// 12 x 64 x 1100, 796 against 774 at 2 x 64 x 16000. The sgn sum takes it with two channels per workgroup only
+// (12 x 64 x 3000: 253 against 277 us; 16384: 1525 against 1439). qlka_set_columns overrides all of this for tests.
 inline bool col_enough(int P, int D, int N, int M, int64_t elements, int64_t segments) {
-    return ((int64_t)P * D * ((int64_t)N + M) >= elements && (int64_t)P * D >= segments) || direct_base() == 0;
+    const int mode = columns_mode();
+    if (mode != QLKA_COLUMNS_AUTO) return mode == QLKA_COLUMNS_ALWAYS;
+    return (int64_t)P * D * ((int64_t)N + M) >= elements && (int64_t)P * D >= segments;
 }
 inline bool col_fwd(int P, int D, int sets, int N, int M) {
     return col_applies(D * sets, N, M) &&
@@ -482,7 +485,7 @@ inline bool col_fwd(int P, int D, int sets, int N, int M) {
 // against 1197, but 8 x 64 x 16300 x 64 1035 against 1188 and 12 x 64 x 16384 x 64 1540 against 1690).
 inline bool col_laplace(int P, int D, int N, int M, int C) {
     if (!col_fwd(P, D, 1, N, M)) return false;
-    if (N + M <= COL_MAX2 || direct_base() == 0) return true;
+    if (N + M <= COL_MAX2 || columns_mode() == QLKA_COLUMNS_ALWAYS) return true;
     const ColPlan pl = col_plan(1, P, D, N, M, C);
     const double el = (double)P * D * (N + M);
     const double col = 60 + pl.cost * 4.75 * pl.E / 32 + el * 1.87e-5;
@@ -660,6 +663,15 @@ int qlka_set_direct_max(int n) {
     g_err.clear();
     if (n < 0) return -fail(QLKA_EINVAL, "the dense cutoff must be >= 0");   // negative: not a cutoff
     return g_direct_max.exchange(n);
+}
+
+int qlka_set_columns(int mode) {
+    g_err.clear();
+    if (mode < QLKA_COLUMNS_AUTO || mode > QLKA_COLUMNS_ALWAYS) {
+        fail(QLKA_EINVAL, "mode must be 0 (auto), 1 (never) or 2 (always)");
+        return -QLKA_EINVAL;
+    }
+    return g_columns.exchange(mode);
 }
 
 size_t qlka_set_workspace_budget(size_t bytes) { return g_ws_budget.exchange(bytes); }

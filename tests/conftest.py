@@ -35,3 +35,28 @@ def pytest_collection_modifyitems(config, items):
 def dev():
     import torch
     return torch.device("cuda", 0)
+
+
+# The library's own routing by size ("auto"), or every short segment too through sort + walk or, where N + M allows it, sort +
+# column sums: dense cutoff (None: as it is), column mode.
+ROUTES = {"auto": (None, 0), "walk": (0, 1), "columns": (0, 2)}
+COLUMN_MAX = 32768                 # longest segment (N + M) that goes by columns
+
+
+@pytest.fixture
+def pin_route():
+    """pin_route(name) routes the library's calls as ROUTES says until the test ends."""
+    from qlka import _lib
+    lib = _lib.load()
+    cutoff, mode = lib.qlka_set_direct_max(512), lib.qlka_set_columns(0)
+    lib.qlka_set_direct_max(cutoff)
+
+    def pin(name):
+        direct_max, columns = ROUTES[name]
+        lib.qlka_set_direct_max(cutoff if direct_max is None else direct_max)
+        lib.qlka_set_columns(columns)
+        return name
+
+    yield pin
+    lib.qlka_set_direct_max(cutoff)
+    lib.qlka_set_columns(mode)

@@ -179,6 +179,18 @@ def test_direct_cutoff_setter(lib):
         lib.qlka_set_direct_max(prev)
 
 
+def test_column_mode_setter(lib):
+    prev = lib.qlka_set_columns(1)
+    try:
+        assert prev == 0                         # auto
+        assert lib.qlka_set_columns(2) == 1
+        for mode in (-1, 3):
+            assert lib.qlka_set_columns(mode) < 0 and b"mode must be" in lib.qlka_last_error()
+        assert lib.qlka_set_columns(prev) == 2   # a rejected value leaves the mode alone
+    finally:
+        lib.qlka_set_columns(prev)
+
+
 def test_keep_sorts_entries_validate(lib):
     import ctypes
     kept = ctypes.c_int(7)

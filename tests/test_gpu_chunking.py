@@ -36,7 +36,7 @@ def _inputs(P, D, N, M, C, seed, dev):
 
 
 def _all_ops(q, k, v, g, gu):
-    """Every operator that walks, on q, k, v: the forward ops, the backward (re-sorting and with kept sorts), the sgn
+    """Every operator that sorts, on q, k, v: the forward ops, the backward (re-sorting and with kept sorts), the sgn
     sum and the three fused layers with and without a key mask."""
     from qlka import layers
     from weighted_abs_sum import _ext, weighted_abs_sum_full, weighted_sgn_sum
@@ -61,11 +61,13 @@ def _all_ops(q, k, v, g, gu):
     return out
 
 
+@pytest.mark.parametrize("route", ["walk", "columns"])
 @pytest.mark.parametrize("shape", [(5, 4, 1500, 1300, 64), (3, 3, 20000, 700, 33)])
-def test_one_p_chunks_equal_unchunked(dev, budget, shape):
+def test_one_p_chunks_equal_unchunked(dev, budget, shape, route, pin_route):
     from qlka import _lib
     lib = _lib.load()
     P, D, N, M, C = shape
+    pin_route(route)
     q, k, v, g, gu = _inputs(P, D, N, M, C, seed=sum(shape), dev=dev)
     budget(8 << 30)
     whole = _all_ops(q, k, v, g, gu)
@@ -86,12 +88,14 @@ def test_one_p_chunks_equal_unchunked(dev, budget, shape):
     assert float(brute.rel_err(chunked["abs"][1].cpu().numpy(), ou, ou).max()) <= REL
 
 
-def test_workspace_between_chunk_sizes(dev, budget):
+@pytest.mark.parametrize("route", ["walk", "columns"])
+def test_workspace_between_chunk_sizes(dev, budget, route, pin_route):
     """A workspace that holds two p but not three runs in chunks of two (P = 5: 2 + 2 + 1), and a workspace below one
     p's is refused with the usual message."""
     from qlka import _lib
     from weighted_laplace_sum import weighted_laplace_sum
     lib = _lib.load()
+    pin_route(route)
     P, D, N, M, C = 5, 3, 2000, 1800, 16
     q, k, v, _, _ = _inputs(P, D, N, M, C, seed=3, dev=dev)
     want_w, want_u = weighted_laplace_sum(q, k, v)

@@ -55,12 +55,8 @@ def _check(dev, P, D, N, M, C, kind, seed):
 
 
 @pytest.fixture
-def no_dense():
-    from qlka import _lib
-    lib = _lib.load()
-    prev = lib.qlka_set_direct_max(0)
-    yield
-    lib.qlka_set_direct_max(prev)
+def no_dense(pin_route):
+    pin_route("columns")
 
 
 @pytest.mark.parametrize("kind", ["normal", "ties"])

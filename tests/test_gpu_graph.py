@@ -69,7 +69,11 @@ def _flat(out):
 @pytest.mark.parametrize("case", ["laplace_walk", "abs_full_walk", "abs_full_backward_walk", "add_bump_layer",
                                   "add_laplace_masked_layer", "laplace_noalloc", "abs_full_dense",
                                   "abs_backward_dense"])
-def test_graph_replays_equal_eager(dev, case):
+@pytest.mark.parametrize("route", ["auto", "columns"])
+def test_graph_replays_equal_eager(dev, case, route, pin_route):
+    if route == "columns" and "dense" in case:
+        pytest.skip("a dense case")
+    pin_route(route)
     shape, fn = _cases()[case]
     args = _inputs(dev, *shape, seed=sum(shape))
     with torch.no_grad():
@@ -96,10 +100,12 @@ def test_graph_replays_equal_eager(dev, case):
             torch.cuda.synchronize(dev)
 
 
-def test_first_call_of_a_thread_captured(dev):
+@pytest.mark.parametrize("route", ["auto", "columns"])
+def test_first_call_of_a_thread_captured(dev, route, pin_route):
     # A thread whose very first library call is captured has no side stream yet; creating one inside the capture would
     # invalidate it, so that call runs in order on the captured stream. Checked on a fresh thread, against eager.
     import threading
+    pin_route(route)
     shape, fn = _cases()["abs_full_walk"]
     args = _inputs(dev, *shape, seed=7)
     with torch.no_grad():

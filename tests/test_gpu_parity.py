@@ -68,25 +68,16 @@ SHAPES = [
 ]
 
 
-@pytest.fixture(params=["auto", "walk"])
-def route(request):
-    """auto: the library's size routing (dense kernels for short segments); walk: sort + walk at every size
-    (qlka_set_direct_max(0)), so the walks stay covered on the short segments the routing sends elsewhere."""
-    from qlka import _lib
-    lib = _lib.load()
-    if request.param == "auto":
-        yield "auto"
-        return
-    prev = lib.qlka_set_direct_max(0)
-    try:
-        yield "walk"
-    finally:
-        lib.qlka_set_direct_max(prev)
+@pytest.fixture(params=["auto", "walk", "columns"])
+def route(request, pin_route):
+    """auto: the library's size routing (dense kernels for short segments, columns for large calls); walk, columns: sort +
+    walk or sort + column sums at every size, so both stay covered on the short segments the routing sends elsewhere."""
+    return pin_route(request.param)
 
 
 def _same_route(route, N, M):
-    if route == "walk" and max(N, M) > 1024:
-        pytest.skip("above the dense cutoffs both routes walk")
+    if route == "columns" and N + M > 32768:
+        pytest.skip("too long for the columns: walks on every route")
 
 
 # ------------------------------------------------------------------------------------------------ sort / rank
@@ -165,7 +156,7 @@ def test_abs_forward_full(dev, shape, kind, route):
 
 
 @pytest.mark.parametrize("layout", ["all_equal", "all_above", "all_below", "on_range_ends"])
-def test_forward_query_grouping_edges(dev, layout):
+def test_forward_query_grouping_edges(dev, layout, route):
     # The forward ops group the queries by key chunk instead of sorting them: one bucket holding every query (its
     # LDS slot counter taken by every lane at once), every query above or below every key (the last and the first
     # range own them all), and queries equal to the last key of a range (their bucket is that range, rank at its end).
@@ -196,7 +187,7 @@ def test_forward_query_grouping_edges(dev, layout):
 
 
 @pytest.mark.parametrize("layout", ["all_equal", "long_runs", "on_key_ranks"])
-def test_backward_tie_runs_across_tiles_and_scan_blocks(dev, layout):
+def test_backward_tie_runs_across_tiles_and_scan_blocks(dev, layout, route):
     # The backward's merged walk takes a key's query sums where its run of equal values began, carried across ranges,
     # merge tiles (2048 merged elements) and scan workgroups (256 ranges) by the tie carry. N + M = 18000: 282 ranges,
     # 9 tiles, two scan workgroups per segment. Layouts: every query and key one value (one run over the whole
@@ -230,7 +221,7 @@ def test_backward_tie_runs_across_tiles_and_scan_blocks(dev, layout):
     _assert_rel(sub(_np(tv.grad), bk, 0), wv, nv, f"grad_v ({layout})")
 
 
-def test_abs_translation_far_from_zero(dev):
+def test_abs_translation_far_from_zero(dev, route):
     # keys and queries centred at 1000: the distance-relative walk must not cancel catastrophically
     from weighted_abs_sum import weighted_abs_sum_full
     q, k, v = _data(2, 3, 800, 600, 8, seed=7)
@@ -280,11 +271,11 @@ def test_abs_backward(dev, shape, full, kind, route):
 
 @pytest.mark.parametrize("shape", [(2, 3, 2000, 1500, 64), (1, 2, 600, 900, 128), (2, 2, 3000, 3000, 32)])
 @pytest.mark.parametrize("with_u", [False, True])
-def test_backward_error_against_reference_fp32_composition(dev, shape, with_u):
+def test_backward_error_against_reference_fp32_composition(dev, shape, with_u, route):
     """grad_q under the per-key normaliser sum_n |<g_m, v_n> (+ g_u)| (tighter than the elementary-product one of the
     other tests when a C-channel dot product cancels): the library's error must stay within twice the error of the
     reference's own fp32 composition (prefix sums in sorted order, <g, 2 PW - W_tot>, oracle grad_q_fp32_prefix)
-    and below 1e-4. Both walk and dense routes at these sizes are the library's own choice."""
+    and below 1e-4, on every route."""
     from weighted_abs_sum import _ext
     P, D, N, M, C = shape
     q, k, v = _data(P, D, N, M, C, seed=sum(shape))
@@ -401,7 +392,7 @@ def test_autograd_keeps_dense_matrix(dev, shape, full):
 @pytest.mark.parametrize("shape", [(2, 3, 1500, 1300, 18),      # one chunk
                                    (6, 64, 16384, 16384, 30),   # pipelined chunks of 2 p
                                    (2, 8, 40000, 30000, 65)])   # two-launch scans, two channel slots per lane
-def test_kept_range_states_match_recomputed(dev, shape):
+def test_kept_range_states_match_recomputed(dev, shape, pin_route):
     # A walking forward that keeps its sorts also leaves its range states and query bounds (a fifth tensor) at the
     # widths whose backward walks twice (C > 64 or C % 4 != 0): the backward over them (its grad_q walk skips its range
     # passes) must equal the backward over the sorts alone, which recomputes them, bit for bit, with and without g_u;
@@ -410,6 +401,7 @@ def test_kept_range_states_match_recomputed(dev, shape):
     from weighted_abs_sum import _ext
     P, D, N, M, C = shape
     print(f"kept range states {shape}", flush=True)
+    pin_route("walk")
     q, k, v = _data(P, D, N, M, C, seed=sum(shape) % 997, kind="ties")
     rng = np.random.default_rng(19)
     g_w = _t(rng.standard_normal((P, M, C)).astype(np.float32), dev)
@@ -434,7 +426,7 @@ def test_kept_range_states_match_recomputed(dev, shape):
 
 @pytest.mark.parametrize("shape", [(2, 3, 1500, 1300, 16),      # one chunk
                                    (6, 64, 16384, 16384, 32)])  # pipelined chunks of 2 p
-def test_merged_backward_over_kept_sorts(dev, shape):
+def test_merged_backward_over_kept_sorts(dev, shape, route):
     # At C <= 64 with C % 4 == 0 the backward walks once over the merged sorted keys and queries and reads no range
     # states: the forward keeps the four sorts only, and the backward over them equals, bit for bit, the backward that
     # sorts again, with and without g_u.
@@ -497,12 +489,13 @@ def test_backward_with_workspace_above_a_2gib_address_boundary(dev):
             assert torch.equal(a, b), f"{name} (C={C}): the workspace's address changed the result"
 
 
-def test_fwd_keep_leaves_unsized_states_untouched(dev):
+def test_fwd_keep_leaves_unsized_states_untouched(dev, pin_route):
     # Through the C ABI: where qlka_abs_keep_state_bytes is 0 (the merged backward, C <= 64, C % 4 == 0) the forward
     # keeps the sorts only (*kept = 1) even when handed a states pointer, and writes nothing through it; at a width whose
     # backward walks twice it fills a buffer of the stated size (*kept = 3).
     from qlka import _lib
     lib = _lib.load()
+    pin_route("walk")
     for C, want in ((64, 1), (62, 3)):
         P, D, N, M = 2, 3, 3000, 2500
         print(f"fwd_keep states C={C}", flush=True)
@@ -595,7 +588,7 @@ def test_pinned_paths_against_oracle(dev, backend, shape):
     _assert_rel(_np(w2), ow, nw, f"{backend} plain out_w")
 
 
-def test_non_default_stream_and_repeat(dev):
+def test_non_default_stream_and_repeat(dev, route):
     # every launch is on the current stream; repeated calls give identical results up to atomic ordering
     from weighted_laplace_sum import weighted_laplace_sum
     q, k, v = _data(2, 4, 700, 600, 64, seed=30)
@@ -613,7 +606,7 @@ def test_non_default_stream_and_repeat(dev):
 
 @pytest.mark.parametrize("fill", [0x00, 0xFF, 0x7F])
 @pytest.mark.parametrize("shape", [(3, 4, 129, 200, 64), (2, 2, 5000, 4097, 32), (2, 3, 1000, 700, 65)])
-def test_workspace_contents_do_not_matter(dev, shape, fill):
+def test_workspace_contents_do_not_matter(dev, shape, fill, route):
     # every op through the C ABI with the workspace pre-filled (NaN, zero, large): no stage may read workspace
     # memory before writing it, and no kernel may read memory it also writes
     from qlka import _lib

@@ -5,8 +5,8 @@ P in [1, 4], D in [1, 9], N and M log-uniform in [1, 6000] (M == N in about half
 dense cutoffs and the 64-key range and 16-key chunk boundaries at unplanned places), C from a list of awkward widths
 (1, odd, one below / above 32, 64 and 128's lane slots), and values N(0, s^2) with s in {0.1, 1, 8} (s = 8 underflows
 most Laplace terms) or the tie-heavy levels of the parity tests. Each case runs the Laplace and abs forwards, the abs
-backward through autograd (the kept sorts), the C-ABI backward and weighted_sgn_sum, on the library's own routing
-and with every segment walked (qlka_set_direct_max(0)). Bar: REL = 1e-5 of sum |term| per element.
+backward through autograd (the kept sorts), the C-ABI backward and weighted_sgn_sum, on the library's own routing,
+with every segment walked and with every one by columns. Bar: REL = 1e-5 of sum |term| per element.
 """
 
 import numpy as np
@@ -90,10 +90,9 @@ def _oracle(cache, i):
     return cache[i]
 
 
-@pytest.mark.parametrize("route", ["auto", "walk"])
+@pytest.mark.parametrize("route", ["auto", "walk", "columns"])
 @pytest.mark.parametrize("i", range(N_CASES), ids=[f"P{c[0]}D{c[1]}N{c[2]}M{c[3]}C{c[4]}-{c[5]}" for c in CASES])
-def test_random_shape(dev, oracle_cache, i, route):
-    from qlka import _lib
+def test_random_shape(dev, oracle_cache, i, route, pin_route):
     from weighted_abs_sum import _ext, weighted_abs_sum_full, weighted_sgn_sum
     from weighted_laplace_sum import weighted_laplace_sum
     P, D, N, M, C, kind, seed = CASES[i]
@@ -101,38 +100,33 @@ def test_random_shape(dev, oracle_cache, i, route):
     q, k, v, g_w, g_u = _data(P, D, N, M, C, kind, seed)
     want = _oracle(oracle_cache, i)
     tq, tk, tv, tgw, tgu = (_t(a, dev) for a in (q, k, v, g_w, g_u))
-    lib = _lib.load()
-    prev = lib.qlka_set_direct_max(0) if route == "walk" else None
-    try:
-        w, u = weighted_laplace_sum(tq, tk, tv)
-        ow, ou, nw = want["lap"]
-        _check(_np(w), ow, nw, "laplace out_w")
-        _check(_np(u), ou, ou, "laplace out_u")
+    pin_route(route)
+    w, u = weighted_laplace_sum(tq, tk, tv)
+    ow, ou, nw = want["lap"]
+    _check(_np(w), ow, nw, "laplace out_w")
+    _check(_np(u), ou, ou, "laplace out_u")
 
-        w, u = weighted_abs_sum_full(tq, tk, tv, backend="cuda")
-        ow, ou, nw = want["abs"]
-        _check(_np(w), ow, nw, "abs out_w")
-        _check(_np(u), ou, ou, "abs out_u")
+    w, u = weighted_abs_sum_full(tq, tk, tv, backend="cuda")
+    ow, ou, nw = want["abs"]
+    _check(_np(w), ow, nw, "abs out_w")
+    _check(_np(u), ou, ou, "abs out_u")
 
-        (wq, wk, wv), (nq, nk, nv) = want["bwd"]
-        aq, ak, av = (t.clone().requires_grad_(True) for t in (tq, tk, tv))
-        w, u = weighted_abs_sum_full(aq, ak, av, backend="cuda")
-        torch.autograd.backward([w, u], [tgw, tgu])
-        _check(_np(aq.grad), wq, nq, "autograd grad_q")
-        _check(_np(ak.grad), wk, nk, "autograd grad_k")
-        _check(_np(av.grad), wv, nv, "autograd grad_v")
+    (wq, wk, wv), (nq, nk, nv) = want["bwd"]
+    aq, ak, av = (t.clone().requires_grad_(True) for t in (tq, tk, tv))
+    w, u = weighted_abs_sum_full(aq, ak, av, backend="cuda")
+    torch.autograd.backward([w, u], [tgw, tgu])
+    _check(_np(aq.grad), wq, nq, "autograd grad_q")
+    _check(_np(ak.grad), wk, nk, "autograd grad_k")
+    _check(_np(av.grad), wv, nv, "autograd grad_v")
 
-        gq, gk, gv = _ext.weighted_abs_sum_full_backward(tq, tk, tv, tgw, tgu)
-        _check(_np(gq), wq, nq, "grad_q")
-        _check(_np(gk), wk, nk, "grad_k")
-        _check(_np(gv), wv, nv, "grad_v")
+    gq, gk, gv = _ext.weighted_abs_sum_full_backward(tq, tk, tv, tgw, tgu)
+    _check(_np(gq), wq, nq, "grad_q")
+    _check(_np(gk), wk, nk, "grad_k")
+    _check(_np(gv), wv, nv, "grad_v")
 
-        out = weighted_sgn_sum(tq, tk, tv, tgw, backend="cuda")
-        os_, ns = want["sgn"]
-        _check(_np(out), os_, ns, "sgn")
-    finally:
-        if prev is not None:
-            lib.qlka_set_direct_max(prev)
+    out = weighted_sgn_sum(tq, tk, tv, tgw, backend="cuda")
+    os_, ns = want["sgn"]
+    _check(_np(out), os_, ns, "sgn")
 
 
 # Shapes with a handful of keys on one side, where the abs walk's segment totals lose accuracy (one of them failed the

@@ -16,8 +16,8 @@ pytestmark = pytest.mark.gpu
 
 ITERS = 4
 THREADS = 2
-# P * D * M >= 2^22, so every op runs the two-copy chunk pipeline: at N = 16384 with the query grouping, at N = 22000
-# with the q sort and the merge passes; N = 600 takes the dense kernels (the backward forks grad_k)
+# P * D * M >= 2^22, so every op that walks runs the two-copy chunk pipeline: at N = 16384 with the query grouping, at
+# N = 22000 with the q sort and the merge passes; N = 600 takes the dense kernels (the backward forks grad_k)
 SHAPES = {
     "grouped": (4, 64, 16384, 16384, 64),
     "sorted_q": (3, 64, 22000, 22000, 32),
@@ -44,9 +44,10 @@ def _ops(q, k, v, g_w, g_u):
     return [w, u, aw, au, gq, gk, gv]
 
 
-@pytest.mark.parametrize("shape", list(SHAPES))
-def test_threads_on_own_streams_match_one_thread(dev, shape):
+@pytest.mark.parametrize("shape,route", [("grouped", "walk"), ("grouped", "columns"), ("sorted_q", "walk"), ("dense", "auto")])
+def test_threads_on_own_streams_match_one_thread(dev, shape, route, pin_route):
     P, D, N, M, C = SHAPES[shape]
+    pin_route(route)
     print(f"threads x{THREADS}: {shape} P={P} D={D} N={N} M={M} C={C}", flush=True)
     inputs = [_inputs(dev, P, D, N, M, C, seed=100 + i) for i in range(THREADS)]
     with torch.no_grad():
