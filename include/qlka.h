@@ -129,10 +129,8 @@ int qlka_abs_bwd(const float* q, const float* k, const float* v, const float* g_
  * dense kernels, or, at C <= 64 with C % 4 == 0, walks once over the merged sorted keys and queries): the forward
  * also leaves there the range states and query bounds of its walk over the sorted keys, which the backward's grad_q
  * walk would compute again (the same range sums, scan and bounds); it sets *kept = 3 when it wrote them (its own walk
- * ran; a forward on the dense kernels keeps only the sorts). Passing them to qlka_abs_bwd_sorted after *kept = 3
+ * ran; a forward on the dense kernels or by columns keeps only the sorts). Passing them to qlka_abs_bwd_sorted after *kept = 3
  * skips one range-sum pass, one scan and one bound search per chunk of the backward, with bit-identical gradients.
- * Segments of N + M <= 32768 elements whose forward and backward run column by column keep none (the buffer's contents
- * stay as they were, *kept as above): that backward reads none.
  */
 int qlka_abs_bwd_walks(int P, int N, int M);
 size_t qlka_abs_keep_state_bytes(int P, int D, int N, int M, int C);

@@ -831,7 +831,8 @@ int abs_fwd_impl(const float* q, const float* k, const float* v, float* out_w, f
     auto b1 = [&](int pc) { return abs_fwd_ws(pc, D, N, M, C); };
     const Plan pl = plan_chunks(P, ws_bytes_given, pipelined(P, D, M), b1);
     if (int e = check_ws(ws, ws_bytes_given, plan_bytes(pl, b1))) return e;
-    // (the backward by columns reads no range states, so none are written; *kept still says that a buffer was taken)
+    // By columns no range states are formed, so only the sorts are kept, where the backward is expected to need no states;
+    // should it walk all the same (the routes can be pinned in between), it forms its own.
     if (col_fwd(P, D, 1, N, M) && (!keep_states || col_bwd(P, D, N, M))) {
         const int e = run_columns(0, 1, keep_sorts ? nullptr : q, k, v, nullptr, out_u != nullptr, P, D, N, M, C, ws, ws_bytes_given, st, no_extra,
             [&](int p0, int np, ColWs& w, hipStream_t s) {
@@ -847,7 +848,7 @@ int abs_fwd_impl(const float* q, const float* k, const float* v, float* out_w, f
                                                     out_u ? out_u + p * M : nullptr, ReduceEpilogue{}, np, D, M, C, s),
                                   "columns to rows"); });
         if (e) return e;
-        if (keep_sorts) *kept = keep_states ? 3 : 1;
+        if (keep_sorts) *kept = 1;
         return QLKA_OK;
     }
     const int mode = out_u ? (ABS_ROW | ABS_ONES) : ABS_ROW;

@@ -917,3 +917,25 @@ def test_largest_inputs_dense(dev):
     _assert_rel(_np(gq[ps][:, :, bq[0]]), wq, nq, "largest dense grad_q")
     _assert_rel(_np(gk[ps][:, :, bk[0]]), wk, nk, "largest dense grad_k")
     _assert_rel(_np(gv[ps][:, bk[0]]), wv, nv, "largest dense grad_v")
+
+
+@pytest.mark.parametrize("forward,backward", [("columns", "walk"), ("walk", "columns"), ("columns", "columns")])
+def test_kept_sorts_across_routes(dev, pin_route, forward, backward):
+    # The two directions choose their routes apart, and the pins are process-wide: whatever the forward kept, the backward's
+    # gradients are right. By columns no range states are formed, so none are handed on (at C = 18, whose walking backward
+    # reads them).
+    from weighted_abs_sum import _ext
+    P, D, N, M, C = 2, 3, 1500, 1300, 18
+    print(f"kept sorts, forward {forward}, backward {backward}", flush=True)
+    q, k, v = _data(P, D, N, M, C, seed=71, kind="ties")
+    rng = np.random.default_rng(72)
+    g_w, g_u = rng.standard_normal((P, M, C)).astype(np.float32), rng.standard_normal((P, M)).astype(np.float32)
+    t = [_t(a, dev) for a in (q, k, v, g_w, g_u)]
+    pin_route(forward)
+    _, _, srt = _ext.weighted_abs_sum_forward_keep(*t[:3], -1, True)
+    assert len(srt) == (5 if forward == "walk" else 4)
+    pin_route(backward)
+    got = _ext.weighted_abs_sum_backward_sorted(*t, srt)
+    want, norm = brute.abs_backward(q, k, v, g_w, g_u)
+    for name, a, w, n in zip(("grad_q", "grad_k", "grad_v"), got, want, norm):
+        _assert_rel(_np(a), w, n, name)
