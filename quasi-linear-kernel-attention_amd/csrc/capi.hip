@@ -584,8 +584,6 @@ inline size_t no_extra(int) { return 0; }
 // of g_w and v (with g_u: one more channel, g_u against ones), grad_q and grad_k per segment, grad_v by the forward's
 // column sums with the roles of q and k exchanged. Workspace of a chunk of P p: as the forward's, the columns of N rows,
 // and those of g_w.
-ColPlan col_bwd_plan(int P, int D, int N, int M, int C) { return col_plan(0, P, D, N, M, std::max(C, 2)); }
-
 size_t col_bwd_part(const ColPlan& pl, int P, int D, int N, int M, int C, int i) {
     const size_t S = (size_t)P * D, C1 = (size_t)(C + 1 + pl.CH) / pl.CH * pl.CH;      // C + 1 channels in whole groups
     switch (i) {
@@ -603,7 +601,7 @@ size_t col_bwd_part(const ColPlan& pl, int P, int D, int N, int M, int C, int i)
 
 size_t col_bwd_bytes(int P, int D, int N, int M, int C) {
     if (!col_bwd_applies(D, N, M)) return 0;
-    const ColPlan pl = col_bwd_plan(1, D, N, M, C);
+    const ColPlan pl = col_plan(0, 1, D, N, M, C);
     size_t b = 0;
     for (int i = 0; i < COL_PARTS; ++i) b += col_bwd_part(pl, P, D, N, M, C, i);
     return b;
@@ -615,7 +613,7 @@ template <class Sorts>
 int run_bwd_columns(const float* v, const float* g_w, const float* g_u, float scale, float* grad_q, float* grad_k,
                     float* grad_v, int P, int D, int N, int M, int C, void* ws, size_t given, hipStream_t st,
                     Sorts sorts) {
-    const ColPlan pl = col_bwd_plan(P, D, N, M, C);
+    const ColPlan pl = col_plan(0, P, D, N, M, C);
     auto bytes = [&](int pc) { return col_bwd_bytes(pc, D, N, M, C); };
     const int pc = fit_chunk(P, given, bytes);
     if (int e = check_ws(ws, given, bytes(pc))) return e;

@@ -761,13 +761,6 @@ void col_sum(const ColSumArgs A)
     const uint32_t aggb = ((uint32_t)(A.K0 + N + 1) * CH * 4 + 15) & ~15u;
     constexpr uint32_t AGGS = (KIND == COL_ABS ? 2 : 3) * CH * W * 4;    // bytes of one feature's aggregates
     __syncthreads();
-    if (d0 >= d1) {                                      // more shares than features
-        for (int h = 0; h < CH; ++h)
-            if (c + h < C)
-                for (int i = tid; i < Ma; i += T) A.out[((size_t)(p * DS + ds) * C + c + h) * Ma + i] = 0.f;
-        return;
-    }
-
     const size_t s0 = (size_t)p * D;
     const rsrc_t rv = make_rsrc(A.val + s0 * T * E, (uint32_t)(D * T * E * 4));
     const rsrc_t rt = make_rsrc(A.tag + s0 * T * E, (uint32_t)(D * T * E * 2));
@@ -1359,7 +1352,7 @@ int wgs_per_cu(int kind, int T, int CH, int n) {
 
 bool col_applies(int D, int N, int M) {
     if ((int64_t)N + M > COL_MAX) return false;
-    const ColPlan pl = col_plan(COL_ABS, 1, D, N, M, 2);
+    const ColPlan pl = col_plan(COL_ABS, 1, D, N, M, 1);
     return (int64_t)D * pl.T * pl.E * 4 <= (int64_t)INT32_MAX;      // a p's stream within 32-bit buffer offsets
 }
 
@@ -1367,16 +1360,17 @@ ColPlan col_plan(int kind, int P, int D, int N, int M, int C) {
     const int n = N + M;
     ColPlan pl{};
     // Two channels per workgroup where their words fit LDS (an 8-byte LDS read costs what a 4-byte one does, and the
-    // stream is read once for both); the smallest workgroup whose threads hold at most 16 elements then, so that
-    // several run per CU and fill each other's waits.
-    if (C >= 2 && n <= COL_MAX2) {
+    // stream is read once for both; the second of one channel is 0); the smallest workgroup whose threads hold at most 16
+    // elements then, so that several run per CU and fill each other's waits. The shape depends on n alone: what a
+    // stream takes (col_applies) is the same for every C.
+    if (n <= COL_MAX2) {
         pl.CH = 2;
         pl.T = 64;
         while (pl.T < 1024 && pl.T * (pl.T < 512 ? 16 : 20) < n) pl.T *= 2;
         pl.E = n <= pl.T * 12 ? 12 : n <= pl.T * 16 ? 16 : 20;
     } else {
         pl.CH = 1;
-        pl.T = n <= 16384 ? 512 : 1024;
+        pl.T = 1024;
         pl.E = n <= pl.T * 20 ? 20 : n <= pl.T * 24 ? 24 : n <= pl.T * 28 ? 28 : 32;
     }
     // Shares of the features: the fewest rounds of workgroups over the chip, in features walked one after another, plus the
@@ -1395,7 +1389,7 @@ ColPlan col_plan(int kind, int P, int D, int N, int M, int C) {
 // The plan of the abs backward's stream: col_dot's LDS also holds the regions' padding and the run starts.
 bool col_bwd_applies(int D, int N, int M) {
     if (!col_applies(D, N, M)) return false;
-    const ColPlan pl = col_plan(COL_ABS, 1, D, N, M, 2);
+    const ColPlan pl = col_plan(COL_ABS, 1, D, N, M, 1);
     return dot_lds(pl.T, pl.CH, N, M) <= LDS_BYTES && sum_lds(COL_ABS, pl.T, pl.CH, pad_words(M, pl.CH) + N) <= LDS_BYTES;
 }
 
@@ -1430,7 +1424,6 @@ int dispatch_shape(const ColPlan& pl, F f) {
     QLKA_COL(64, 12, 2); QLKA_COL(64, 16, 2); QLKA_COL(128, 12, 2); QLKA_COL(128, 16, 2); QLKA_COL(256, 12, 2);
     QLKA_COL(256, 16, 2); QLKA_COL(512, 12, 2); QLKA_COL(512, 16, 2); QLKA_COL(1024, 12, 2); QLKA_COL(1024, 16, 2);
     QLKA_COL(512, 20, 2); QLKA_COL(1024, 20, 2);
-    QLKA_COL(512, 20, 1); QLKA_COL(512, 24, 1); QLKA_COL(512, 28, 1); QLKA_COL(512, 32, 1);
     QLKA_COL(1024, 20, 1); QLKA_COL(1024, 24, 1); QLKA_COL(1024, 28, 1); QLKA_COL(1024, 32, 1);
 #undef QLKA_COL
     return (int)hipErrorInvalidValue;

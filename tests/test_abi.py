@@ -179,6 +179,13 @@ def test_direct_cutoff_setter(lib):
         lib.qlka_set_direct_max(prev)
 
 
+def test_workspace_of_one_channel_is_not_larger_than_of_two(lib):
+    # the columns' shape depends on N + M alone (one channel once took 10240 elements for any short segment)
+    for N, M in ((600, 20), (20, 600), (700, 700), (9000, 9000)):
+        for fn in (lib.qlka_laplace_fwd_ws_bytes, lib.qlka_abs_fwd_ws_bytes, lib.qlka_abs_bwd_ws_bytes):
+            assert fn(4, 64, N, M, 1) <= fn(4, 64, N, M, 2)
+
+
 def test_column_mode_setter(lib):
     prev = lib.qlka_set_columns(1)
     try:

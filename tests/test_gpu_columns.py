@@ -1,6 +1,6 @@
 """GPU checks of the column route of the forward sums (csrc/col.hip) at the edges of its workgroup shapes: the element
 counts N + M where the threads or elements per thread change, the switch from two channels per workgroup to one, odd
-channel counts, more feature shares than features, one-sided sizes and the last size before the ranges take over.
+channel counts, one-sided sizes and the last size before the ranges take over.
 
 Against the fp64 oracle on a subsample of the queries, at the bar of every forward sum: 1e-5 of sum |term|. The fp32 error
 of these sums is a few roundings of partial sums no larger than sum |term| (measured: below 1e-6), so 1e-5 has room.
@@ -67,10 +67,15 @@ def test_column_capacity_edges(dev, no_dense, n, kind):
 
 
 @pytest.mark.parametrize("shape", [(1, 1, 17, 1, 1), (2, 1, 18, 40, 2), (1, 2, 32000, 700, 5), (1, 2, 700, 32000, 2),
-                                   (3, 33, 900, 1100, 7), (40, 2, 1200, 900, 128), (2, 64, 5003, 3001, 33)])
+                                   (2, 5, 600, 610, 1), (1, 2, 9000, 8000, 1), (3, 33, 900, 1100, 7), (40, 2, 1200, 900, 128), (2, 64, 5003, 3001, 33)])
 @pytest.mark.parametrize("kind", ["normal", "far"])
 def test_column_shapes(dev, no_dense, shape, kind):
     _check(dev, *shape, kind, seed=sum(shape))
+
+
+def test_one_channel_and_many_features(dev, no_dense):
+    # 60000 features: with 10240 elements a segment, as one channel once took, a p's stream passes 32-bit offsets
+    _check(dev, 1, 60000, 20, 600, 1, "normal", seed=2)
 
 
 def test_laplace_infinite_keys_and_queries(dev, no_dense):
