@@ -284,18 +284,29 @@ __device__ __forceinline__ bool any_of(bool x, uint32_t* flags) {
     return __ballot(flags[lane_id() % W] != 0) != 0;
 }
 
+// 16-bit word indices, two in a register
+template <int E>
+struct Halves {
+    uint32_t w[E / 2];
+    __device__ __forceinline__ uint32_t get(int i) const { return (i & 1) ? w[i / 2] >> 16 : w[i / 2] & 0xffffu; }
+    __device__ __forceinline__ void set(int i, uint32_t x) {         // in order: the low half first
+        if (i & 1) w[i / 2] |= x << 16;
+        else w[i / 2] = x;
+    }
+};
+
 __device__ __forceinline__ bool is_key(int word, const ColMergeArgs& A) { return (uint32_t)(word - A.K0) < (uint32_t)A.N; }
 
 // The median of a segment's keys that are not padding, from its merged order (as emit_stream's), 0 without any; scratch:
 // 1 + W words of LDS.
 template <int T, int E>
-__device__ __forceinline__ float median_key(const ColMergeArgs& A, const float (&val)[E], const int (&src)[E], uint32_t* scratch)
+__device__ __forceinline__ float median_key(const ColMergeArgs& A, const float (&val)[E], const Halves<E>& src, uint32_t* scratch)
 {
     constexpr int W = T / WAVE;
     const int lane = lane_id(), wv = wave_in_block();
     int keys = 0;
 #pragma unroll
-    for (int e = 0; e < E; ++e) keys += is_key(src[e], A);
+    for (int e = 0; e < E; ++e) keys += is_key((int)src.get(e), A);
     int inc = keys;
 #pragma unroll
     for (int off = 1; off < WAVE; off <<= 1) {
@@ -314,7 +325,7 @@ __device__ __forceinline__ float median_key(const ColMergeArgs& A, const float (
     if (at >= 0 && at < keys) {
 #pragma unroll
         for (int e = 0; e < E; ++e)
-            if (is_key(src[e], A) && at-- == 0) scratch[0] = __float_as_uint(val[e]);
+            if (is_key((int)src.get(e), A) && at-- == 0) scratch[0] = __float_as_uint(val[e]);
     }
     __syncthreads();
     return __uint_as_float(scratch[0]);
@@ -330,19 +341,19 @@ __device__ __forceinline__ float median_key(const ColMergeArgs& A, const float (
 // from every finite key). poison: a NaN among the weights' values that val no longer shows; every row is NaN.
 template <int KIND, int T, int E>
 __device__ __forceinline__ void emit_stream(const ColMergeArgs& A, float* sm, int s, float x0, float xs, float (&val)[E],
-                                            int (&src)[E], bool rare, bool poison)
+                                            const Halves<E>& src, bool rare, bool poison)
 {
     constexpr int W = T / WAVE;
     const int N = A.N, M = A.M, n = N + M, tid = threadIdx.x, seg = s / A.sets, p = seg / A.D;
     const int acc0 = A.eq ? A.K0 : 0, accs = A.eq ? N : M;       // the words that receive sums
-    auto receives = [&](int e) { return (uint32_t)(src[e] - acc0) < (uint32_t)accs; };
-    auto weightless = [&](int e) { return receives(e) || src[e] == A.K0 + N; };
+    auto receives = [&](int e) { return src.get(e) - (uint32_t)acc0 < (uint32_t)accs; };
+    auto weightless = [&](int e) { return receives(e) || (int)src.get(e) == A.K0 + N; };
     if (rare) {
         if constexpr (KIND == COL_LAPLACE) xs = no_nan(xs);
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             const bool row = receives(e) && (KIND == COL_ABS ? !(fabsf(val[e]) <= FLT_MAX) : val[e] != val[e]);
-            if (row && A.bad) A.bad[(size_t)p * accs + (src[e] - acc0)] = __int_as_float(0x7fc00000);
+            if (row && A.bad) A.bad[(size_t)p * accs + ((int)src.get(e) - acc0)] = __int_as_float(0x7fc00000);
             if (weightless(e)) val[e] = KIND == COL_ABS ? bounded(val[e]) : no_nan(val[e]);
         }
     }
@@ -380,8 +391,8 @@ __device__ __forceinline__ void emit_stream(const ColMergeArgs& A, float* sm, in
         u2_t y;
 #pragma unroll
         for (int e = 0; e < 4; ++e) x[e] = dist[4 * g + e];
-        y.x = (uint32_t)src[4 * g] | ((uint32_t)src[4 * g + 1] << 16);
-        y.y = (uint32_t)src[4 * g + 2] | ((uint32_t)src[4 * g + 3] << 16);
+        y.x = src.w[2 * g];
+        y.y = src.w[2 * g + 1];
         *(f4_t*)(vo + ((size_t)g * T + tid) * 4) = x;
         *(u2_t*)(to + ((size_t)g * T + tid) * 4) = y;
     }
@@ -391,7 +402,7 @@ __device__ __forceinline__ void emit_stream(const ColMergeArgs& A, float* sm, in
     // v == 1: the same walk as col_sum's with every key's weight 1
     float wt[E];
 #pragma unroll
-    for (int e = 0; e < E; ++e) wt[e] = is_key(src[e], A) ? 1.f : 0.f;
+    for (int e = 0; e < E; ++e) wt[e] = is_key((int)src.get(e), A) ? 1.f : 0.f;
     const int lane = lane_id(), wv = wave_in_block();
     float* agg = sm + n;
     float out[E];
@@ -453,7 +464,7 @@ __device__ __forceinline__ void emit_stream(const ColMergeArgs& A, float* sm, in
     // to query order through LDS (every thread has read its word indices before the scan's barrier)
 #pragma unroll
     for (int e = 0; e < E; ++e)
-        if (src[e] < M) sm[src[e]] = out[e];
+        if ((int)src.get(e) < M) sm[src.get(e)] = out[e];
     __syncthreads();
     float* uo = A.u + (size_t)s * M;
     for (int x = tid; x < M; x += T) uo[x] = sm[x];
@@ -521,13 +532,13 @@ void col_merge(const ColMergeArgs A)
     float qa = sq[min(i, M - 1)], kb = sk[min(j, N - 1)];
     uint32_t eq = 0;
     float val[E];
-    int src[E];                         // word of the element in sq / sk
+    Halves<E> src;                      // word of the element in sq / sk
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const bool live = diag + e < n;
         const bool tq = j >= N || (i < M && qa <= kb);
         const float r = tq ? qa : kb;
-        src[e] = live ? (tq ? i : M + j) : n;
+        src.set(e, (uint32_t)(live ? (tq ? i : M + j) : n));
         if (live && diag + e > 0 && r == prev) eq |= 1u << e;
         val[e] = live ? r : prev;
         if (live) {
@@ -547,7 +558,10 @@ void col_merge(const ColMergeArgs A)
         for (int x = tid; x < N; x += T) w[M + x] = A.K0 + (!keep || keep[kp[x]] != 0 ? kp[x] : (uint32_t)N);
         __syncthreads();
 #pragma unroll
-        for (int e = 0; e < E; ++e) src[e] = src[e] < n ? (int)w[src[e]] : A.K0 + N;
+        for (int e = 0; e < E; e += 2) {
+            const uint32_t x = src.get(e), y = src.get(e + 1), pad = (uint32_t)(A.K0 + N);
+            src.w[e / 2] = ((int)x < n ? w[x] : pad) | ((int)y < n ? w[y] : pad) << 16;
+        }
     }
     if (A.eq) A.eq[(size_t)s * T + tid] = eq;
     if (KIND == COL_ABS && keep) {
@@ -583,17 +597,6 @@ __device__ __forceinline__ uint64_t equal_lanes(uint32_t digit) {
     }
     return ~((uint64_t)lo | ((uint64_t)hi << 32));
 }
-
-// 16-bit halves of an array of pairs
-template <int E>
-struct Halves {
-    uint32_t w[E / 2];
-    __device__ __forceinline__ uint32_t get(int i) const { return (i & 1) ? w[i / 2] >> 16 : w[i / 2] & 0xffffu; }
-    __device__ __forceinline__ void set(int i, uint32_t x) {         // in order: the low half first
-        if (i & 1) w[i / 2] |= x << 16;
-        else w[i / 2] = x;
-    }
-};
 
 template <int KIND, int T, int E>
 __global__ __launch_bounds__(T, 4)
@@ -713,16 +716,14 @@ void col_sort(const ColMergeArgs A)
     float prev = tid == 0 ? ordered_to_float(key[0]) : tid * E - 1 < nl ? ordered_to_float(before_key) : lastv;
     const float xs = prev;
     float val[E];
-    int src[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         if (tid * E + e < nl) prev = ordered_to_float(key[e]);
         val[e] = prev;
-        src[e] = (int)idx.get(e);
     }
-    const float x0 = KIND == COL_ABS ? median_key<T, E>(A, val, src, misc + 7) : 0.f;
+    const float x0 = KIND == COL_ABS ? median_key<T, E>(A, val, idx, misc + 7) : 0.f;
     __syncthreads();                                         // buf is read; the emission uses it
-    emit_stream<KIND, T, E>(A, sm, s, x0, xs, val, src, rare, false);
+    emit_stream<KIND, T, E>(A, sm, s, x0, xs, val, idx, rare, false);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
