@@ -30,6 +30,7 @@
 #include <cfloat>
 #include <utility>
 
+#include "per_device.h"
 #include "qlka_common.h"
 #include "qlka_internal.h"
 
@@ -1430,15 +1431,27 @@ int dispatch_shape(const ColPlan& pl, F f) {
     return (int)hipErrorInvalidValue;
 }
 
+// Lets the kernel use all of a CU's LDS on the stream's device. The attribute belongs to one device's copy of the kernel (and
+// is set for the current device's), so `once`, one per kernel, keeps account by device.
 template <class K>
-hipError_t allow_lds(K kernel) {
-    return hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_BYTES);
+int allow_lds(K kernel, PerDevice& once, hipStream_t st) {
+    int cur = 0;
+    if (hipError_t e = hipGetDevice(&cur)) return (int)e;
+    hipDevice_t dev = cur;
+    if (st != nullptr)
+        if (hipError_t e = hipStreamGetDevice(st, &dev)) return (int)e;
+    return once(dev, [&] {
+        hipError_t e = dev == cur ? hipSuccess : hipSetDevice(dev);
+        if (e != hipSuccess) return (int)e;
+        e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_BYTES);
+        const hipError_t back = dev == cur ? hipSuccess : hipSetDevice(cur);
+        return (int)(e != hipSuccess ? e : back); });
 }
 
 template <int KIND, int T, int E>
 int launch_merge(const ColMergeArgs& a, int S, hipStream_t st) {
-    static const hipError_t once = allow_lds(col_merge<KIND, T, E>);
-    if (once != hipSuccess) return (int)once;
+    static PerDevice once;
+    if (int e = allow_lds(col_merge<KIND, T, E>, once, st)) return e;
     const size_t lds = (size_t)(a.N + a.M + 3 * (T / WAVE)) * 4;
     hipLaunchKernelGGL((col_merge<KIND, T, E>), dim3((unsigned)S), dim3(T), lds, st, a);
     return (int)hipGetLastError();
@@ -1446,8 +1459,8 @@ int launch_merge(const ColMergeArgs& a, int S, hipStream_t st) {
 
 template <int KIND, int T, int E, int CH, bool SWAP>
 int launch_sum(const ColSumArgs& a, hipStream_t st) {
-    static const hipError_t once = allow_lds(col_sum<KIND, T, E, CH, SWAP, 4>);
-    if (once != hipSuccess) return (int)once;
+    static PerDevice once;
+    if (int e = allow_lds(col_sum<KIND, T, E, CH, SWAP, 4>, once, st)) return e;
     const unsigned blocks = (unsigned)(a.P * a.DS * ((a.C + CH - 1) / CH));
     hipLaunchKernelGGL((col_sum<KIND, T, E, CH, SWAP, 4>), dim3(blocks), dim3(T), sum_lds(KIND, T, CH, a.K0 + a.N), st, a);
     return (int)hipGetLastError();
@@ -1470,12 +1483,12 @@ int col_sort_launch(int kind, const ColPlan& pl, const float* q, const float* k,
         } else {
             const size_t lds = (size_t)sort_words(T(), E()) * 4;
             if (kind == COL_ABS) {
-                static const hipError_t once = allow_lds(col_sort<COL_ABS, T(), E()>);
-                if (once != hipSuccess) return (int)once;
+                static PerDevice once;
+                if (int e = allow_lds(col_sort<COL_ABS, T(), E()>, once, st)) return e;
                 hipLaunchKernelGGL((col_sort<COL_ABS, T(), E()>), dim3((unsigned)S), dim3(T()), lds, st, a);
             } else {
-                static const hipError_t once = allow_lds(col_sort<COL_LAPLACE, T(), E()>);
-                if (once != hipSuccess) return (int)once;
+                static PerDevice once;
+                if (int e = allow_lds(col_sort<COL_LAPLACE, T(), E()>, once, st)) return e;
                 hipLaunchKernelGGL((col_sort<COL_LAPLACE, T(), E()>), dim3((unsigned)S), dim3(T()), lds, st, a);
             }
             return (int)hipGetLastError();
@@ -1527,8 +1540,8 @@ int col_dot_launch(const ColPlan& pl, ColStream str, const float* gt, const floa
     const ColDotArgs a{str.tag, str.eq, gt, vt, gq, gk, str.val, scale, D, N, M, col_key0(pl, M), pad_words(N, pl.CH), CW};
     StageTimer t("col_dot", st);
     return dispatch_shape(pl, [&](auto T, auto E, auto CH) {
-        static const hipError_t once = allow_lds(col_dot<T(), E(), CH()>);
-        if (once != hipSuccess) return (int)once;
+        static PerDevice once;
+        if (int e = allow_lds(col_dot<T(), E(), CH()>, once, st)) return e;
         hipLaunchKernelGGL((col_dot<T(), E(), CH()>), dim3((unsigned)S), dim3(T()), dot_lds(T(), CH(), N, M), st, a);
         return (int)hipGetLastError(); });
 }
