@@ -499,13 +499,13 @@ inline bool col_sgn(int P, int D, int N, int M) { return col_bwd(P, D, N, M) && 
 
 struct ColWs { SortedWs s; ColStream str; float* u; float* cols; float* wt; float* bad; char* extra; };
 
-size_t col_part(const ColPlan& pl, int P, int D, int N, int M, int C, int sets, int i) {
+size_t col_part(int kind, const ColPlan& pl, int P, int D, int N, int M, int C, int sets, int i) {
     const size_t S = (size_t)P * D;
     switch (i) {
         case 0: case 1: return align256(S * N * 4);
         case 2: case 3: return align256(S * M * 4);
         case 4: return align256(sort_scratch_need(WsSpec{P, D, N, M, C, N, 0, false}));
-        case 5: return align256(col_stream_bytes(pl, (int)S * sets));
+        case 5: return align256(col_stream_bytes(kind, pl, (int)S * sets));
         case 6: return align256(S * sets * M * 4);
         case 7: return align256((size_t)P * pl.DS * C * M * 4);
         case 8: return align256((size_t)P * (C + 1) * N * 4);
@@ -523,19 +523,19 @@ size_t col_bytes(int kind, int P, int D, int N, int M, int C, int sets = 1) {
     ColPlan pl = col_plan(kind, 1, D, N, M, C);
     pl.DS = std::min(D, COL_SHARES);
     size_t b = 0;
-    for (int i = 0; i < COL_PARTS; ++i) b += col_part(pl, P, D, N, M, C, sets, i);
+    for (int i = 0; i < COL_PARTS; ++i) b += col_part(kind, pl, P, D, N, M, C, sets, i);
     return b;
 }
 
-ColWs col_carve(ColPlan pl, void* ws, int P, int D, int N, int M, int C, int sets) {
+ColWs col_carve(int kind, ColPlan pl, void* ws, int P, int D, int N, int M, int C, int sets) {
     pl.DS = std::min(D, COL_SHARES);
     char* part[COL_PARTS];
     char* b = (char*)ws;
-    for (int i = 0; i < COL_PARTS; ++i) { part[i] = b; b += col_part(pl, P, D, N, M, C, sets, i); }
+    for (int i = 0; i < COL_PARTS; ++i) { part[i] = b; b += col_part(kind, pl, P, D, N, M, C, sets, i); }
     ColWs r{};
     r.s.ks = (float*)part[0]; r.s.kp = (uint32_t*)part[1]; r.s.qs = (float*)part[2]; r.s.qp = (uint32_t*)part[3];
     r.s.sort_scratch = part[4];
-    r.str = col_stream(pl, part[5], P * D * sets);
+    r.str = col_stream(kind, pl, part[5], P * D * sets);
     r.u = (float*)part[6];
     r.cols = (float*)part[7];
     r.wt = (float*)part[8];
@@ -556,7 +556,7 @@ int run_columns(int kind, int sets, const float* q, const float* k, const float*
     const int pc = fit_chunk(P, given, bytes);
     if (int e = check_ws(ws, given, bytes(pc))) return e;
     return for_chunks(P, pc, [&](int p0, int np) {
-        ColWs w = col_carve(pl, ws, np, D, N, M, C, sets);
+        ColWs w = col_carve(kind, pl, ws, np, D, N, M, C, sets);
         if (!want_u) w.u = nullptr;
         const size_t p = (size_t)p0;
         const uint8_t* kc = keep ? keep + p * N : nullptr;
@@ -590,7 +590,7 @@ size_t col_bwd_part(const ColPlan& pl, int P, int D, int N, int M, int C, int i)
         case 0: case 1: return align256(S * N * 4);
         case 2: case 3: return align256(S * M * 4);
         case 4: return align256(sort_scratch_need(WsSpec{P, D, N, M, C, N, 0, false}));
-        case 5: return align256(col_stream_bytes(pl, (int)S));
+        case 5: return align256(col_stream_bytes(0, pl, (int)S));
         case 6: return align256((size_t)P * C1 * N * 4);
         case 7: return align256((size_t)P * C1 * M * 4);
         case 8: return align256((size_t)P * std::min(D, COL_SHARES) * C * N * 4);
@@ -624,7 +624,7 @@ int run_bwd_columns(const float* v, const float* g_w, const float* g_u, float sc
         SortedWs w{};
         w.ks = (float*)part[0]; w.kp = (uint32_t*)part[1]; w.qs = (float*)part[2]; w.qp = (uint32_t*)part[3];
         w.sort_scratch = part[4];
-        const ColStream str = col_stream(pl, part[5], np * D);
+        const ColStream str = col_stream(0, pl, part[5], np * D);
         float *vt = (float*)part[6], *gt = (float*)part[7], *cols = (float*)part[8];
         float* bad = grad_v ? (float*)part[9] : nullptr;
         const size_t p = (size_t)p0;

@@ -15,7 +15,7 @@
 //   val[s][E/4][T][4]   abs: the value less the thread's anchor, the end of its elements that lies towards the segment's
 //                       median key; Laplace: e^-distance to the previous element
 //   tag[s][E/4][T][4]   16-bit word index: m for query m, K0 + n for key n, K0 + N for padding (K0 = M, or M rounded up)
-//   xe[s][T]            abs: each thread's anchor less the median key; Laplace: e^-(extent of its elements)
+//   xe[s][T]            abs: each thread's anchor less the median key; Laplace: its Decays
 //   eq[s][T]            (abs backward) bit e: element e of the thread has the value of the element before it
 // With 4 elements per 16-byte (8-byte) load, a wave's loads are contiguous.
 //
@@ -116,38 +116,62 @@ __device__ __forceinline__ void affine_step(float& a, float (&b)[CH]) {
     for (int c = 0; c < CH; ++c) Step::fma(b[c], a);
     Step::mul(a);
 }
+// lane_id() counted again, for a loop whose registers cannot hold it (spilled, its reload waits for every load in flight)
+__device__ __forceinline__ int lane_now() {
+    int r;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(r));
+    return r;
+}
+
+// The Laplace decays of a thread and around it in its wave, each formed from its own distance: a scan that multiplies the
+// threads' decays up doubles their errors at every step, to thousands of times a rounding that repeats (a grid of keys).
+struct Decays {
+    float own;                       // over the thread
+    float row, half;                 // from the start of its row of 16 lanes, and of lane 32, to the thread's end
+    float before, after;             // from the wave's start to the thread, and from it to the wave's end
+    float rest;                      // from the thread's start to its row's end
+};
+// inclusive scans of y <- a y' + b over the wave's threads
 template <int CH>
-__device__ __forceinline__ void wave_affine_up(float& a, float (&b)[CH]) {      // lane order
+__device__ __forceinline__ void wave_affine_up(const Decays& y, float (&b)[CH]) {       // lane order
+    float a = y.own;
     affine_step<Up1>(a, b);
     affine_step<Up2>(a, b);
     affine_step<Up4>(a, b);
-    affine_step<Up8>(a, b);
-    affine_step<UpRow>(a, b);
-    affine_step<UpHalf>(a, b);
-    settle(a, b);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) Up8::fma(b[c], a);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) UpRow::fma(b[c], y.row);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        UpHalf::fma(b[c], y.half);
+        settle(b[c]);
+    }
 }
 template <int CH>
-__device__ __forceinline__ void wave_affine_down(float& a, float (&b)[CH]) {    // reverse lane order
+__device__ __forceinline__ void wave_affine_down(const Decays& y, float (&b)[CH]) {     // reverse lane order
+    float a = y.own;
     affine_step<Down1>(a, b);
     affine_step<Down2>(a, b);
     affine_step<Down4>(a, b);
-    affine_step<Down8>(a, b);
-    settle(a, b);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        Down8::fma(b[c], a);
+        settle(b[c]);
+    }
     // rows above, last first (no DPP pattern reads the next row): their totals are in their first lanes
-    const int row = lane_id() >> 4;
-    const float a1 = bcast(a, 16), a2 = bcast(a, 32), a3 = bcast(a, 48);
-    const float ain = row == 0 ? a1 * (a2 * a3) : row == 1 ? a2 * a3 : row == 2 ? a3 : 1.f;
+    const int row = lane_now() >> 4;
+    const float a1 = bcast(y.row, 31), a2 = bcast(y.row, 47);
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
         const float b3 = bcast(b[c], 48);
         const float b2 = fmaf(a2, b3, bcast(b[c], 32));
         const float b1 = fmaf(a1, b2, bcast(b[c], 16));
         const float bin = row == 0 ? b1 : row == 1 ? b2 : row == 2 ? b3 : 0.f;
-        b[c] = fmaf(a, bin, b[c]);
+        b[c] = fmaf(y.rest, bin, b[c]);
     }
-    a *= ain;
 }
-// the same over W <= 16 entries of a row
+// the same over W <= 16 entries of a row, the decays multiplied up
 template <int W, int CH>
 __device__ __forceinline__ void row_affine_up(float& a, float (&b)[CH]) {
     if constexpr (W > 1) affine_step<Up1>(a, b);
@@ -236,10 +260,13 @@ __device__ __forceinline__ void each(F f) { each_of(f, std::make_integer_sequenc
 // ---------------------------------------------------------------------------------------------------------------
 // col_merge: one workgroup per segment
 // ---------------------------------------------------------------------------------------------------------------
-// e^-x, x >= 0. Below 1/2 as 1 - h with h = 1 - e^-x by its Taylor series (9 terms: to 2^-26 of h), so that it rounds to
-// nearest for the small x that the sums multiply by the thousands: near 1 the library's expf is off to one side by up to an
-// ulp, which such products add up (Laplace at N = 16384: 1.2e-6 of the result against 64 bits, 1.8e-7 so).
-__device__ __forceinline__ float decay(float x) {
+// e^-x, x >= 0, for a chain of products. Below 1/2 as 1 - h with h = 1 - e^-x by its Taylor series (9 terms: to 2^-26 of h),
+// so that it rounds to nearest: near 1 the library's expf is off to one side by up to an ulp, which thousands of factors add
+// up. And `rest`, what rounding the factors before has left to be taken off, is taken off here and left anew: where the
+// distances repeat (a grid) or are all below half an ulp, factors rounded one by one err to one side as well.
+// With this and Decays, Laplace at N = M = 8192, relative 2-norm against 64 bits, a grid over +-3 and uniform keys in +-2e-5:
+// 5.1e-6 and 3.5e-6 -> 3.9e-7 and 1.5e-7 (walks: 5.7e-7 and 2.1e-7); N(0, 1) 1.4e-7 -> 7.6e-8 (2.9e-7).
+__device__ __forceinline__ float decay(float x, float& rest) {
     if (x >= 0.5f) return expf(-x);
     float h = fmaf(x, -1.f / 362880.f, 1.f / 40320.f);
     h = fmaf(x, -h, 1.f / 5040.f);
@@ -249,13 +276,16 @@ __device__ __forceinline__ float decay(float x) {
     h = fmaf(x, -h, 1.f / 6.f);
     h = fmaf(x, -h, 0.5f);
     h = fmaf(x, -h, 1.f);
-    return fmaf(-x, h, 1.f);
+    h = fmaf(x, h, rest);
+    const float r = 1.f - h;
+    rest = h - (1.f - r);                                    // exact
+    return r;
 }
 
 struct ColMergeArgs {
     const float* qs; const uint32_t* qp; const float* ks; const uint32_t* kp;   // sorted queries and keys
     const uint8_t* keep;             // (P, N) key mask or null: masked keys become padding
-    float* val; uint16_t* tag; float* xe; uint32_t* eq;      // eq: null unless wanted
+    float* val; uint16_t* tag; float* xe; float* xe2; uint32_t* eq;  // eq: null unless wanted; xe2: Laplace only
     float* u;                        // (S, M) v == 1 terms in query order, or null
     float* bad;                      // (P, M), bwd: (P, N): NaN at the rows whose own value makes them NaN, 0 else; or null
     int D, N, M, K0;
@@ -334,7 +364,7 @@ __device__ __forceinline__ float median_key(const ColMergeArgs& A, const float (
 
 // The stream and the v == 1 terms of one segment, from its merged order: thread t's elements as word indices src (padding,
 // masked keys among it: K0 + N) and as values val (padding: the value before); x0 the median key, xs the value before the thread's first element.
-// sm: N + M words and the scan's aggregates, free to use.
+// sm: N + M words and 3 words a wave, free to use.
 //
 // A query (bwd: a key) only receives sums, so whatever it holds stays in its own row. In a rare segment abs sums take its
 // value bounded, Laplace sums a NaN as the infinity on its side, and the row is marked in A.bad, which the finish makes NaN:
@@ -362,7 +392,8 @@ __device__ __forceinline__ void emit_stream(const ColMergeArgs& A, float* sm, in
     // A thread's values are taken relative to its anchor, its value nearest the median, so that every value an element's sums
     // are formed from is bounded by distances to keys: on either side of the median the end towards it, and the median
     // itself in a thread on both sides
-    float anchor = 0.f, dec = 1.f;
+    float anchor = 0.f;
+    Decays dec;
     if constexpr (KIND == COL_ABS) {
         const float xa = x0 <= val[0] ? val[0] : x0 >= val[E - 1] ? val[E - 1] : x0;
         anchor = xa - x0;
@@ -375,14 +406,24 @@ __device__ __forceinline__ void emit_stream(const ColMergeArgs& A, float* sm, in
                 if (weightless(e)) dist[e] = bounded(dist[e]);
         }
     } else {                                             // e^-distance once per element for all channels
-        float prev = xs;
+        float prev = xs, rest = 0.f;
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            dist[e] = decay(val[e] != prev ? val[e] - prev : 0.f);       // equal infinities: 0 apart
+            dist[e] = decay(val[e] != prev ? val[e] - prev : 0.f, rest);         // equal infinities: 0 apart
             prev = val[e];
         }
-        dec = prev != xs ? decay(prev - xs) : 1.f;
-        if (rare && poison) dec = __int_as_float(0x7fc00000);
+        const int lane = lane_id();
+        auto over = [](float from, float to) {           // one distance's decay
+            float none = 0.f;
+            return decay(to != from ? to - from : 0.f, none);
+        };
+        dec.own = over(xs, prev);
+        dec.row = over(__shfl(xs, lane & 48, WAVE), prev);
+        dec.half = lane < 32 ? 1.f : over(__shfl(xs, 32, WAVE), prev);
+        dec.before = over(__shfl(xs, 0, WAVE), xs);
+        dec.after = over(prev, __shfl(prev, WAVE - 1, WAVE));
+        dec.rest = over(xs, __shfl(prev, lane | 15, WAVE));
+        if (rare && poison) dec.own = dec.row = dec.half = dec.before = dec.after = dec.rest = __int_as_float(0x7fc00000);
     }
     float* vo = A.val + (size_t)s * T * E;
     uint16_t* to = A.tag + (size_t)s * T * E;
@@ -397,7 +438,14 @@ __device__ __forceinline__ void emit_stream(const ColMergeArgs& A, float* sm, in
         *(f4_t*)(vo + ((size_t)g * T + tid) * 4) = x;
         *(u2_t*)(to + ((size_t)g * T + tid) * 4) = y;
     }
-    A.xe[(size_t)s * T + tid] = KIND == COL_ABS ? anchor : dec;
+    if constexpr (KIND == COL_ABS) {
+        A.xe[(size_t)s * T + tid] = anchor;
+    } else {
+        const f4_t x = {dec.own, dec.row, dec.half, dec.before};
+        const f2_t y = {dec.after, dec.rest};
+        ((f4_t*)A.xe)[(size_t)s * T + tid] = x;
+        ((f2_t*)A.xe2)[(size_t)s * T + tid] = y;
+    }
     if (A.u == nullptr) return;
 
     // v == 1: the same walk as col_sum's with every key's weight 1
@@ -440,19 +488,18 @@ __device__ __forceinline__ void emit_stream(const ColMergeArgs& A, float* sm, in
             pr *= dist[e];
             r = fmaf(pr, wt[e], r);
         }
-        float up[1] = {l}, dn[1] = {r}, au = dec, ad = dec;
-        wave_affine_up(au, up);
-        wave_affine_down(ad, dn);
-        if (lane == WAVE - 1) { agg[3 * wv] = up[0]; agg[3 * wv + 2] = au; }
+        float up[1] = {l}, dn[1] = {r};
+        wave_affine_up(dec, up);
+        wave_affine_down(dec, dn);
+        if (lane == WAVE - 1) { agg[3 * wv] = up[0]; agg[3 * wv + 2] = dec.before * dec.own; }
         if (lane == 0) agg[3 * wv + 1] = dn[0];
         float L = dpp<WAVE_SHR1>(0.f, up[0]), R = dpp<WAVE_SHL1>(0.f, dn[0]);
-        const float aL = dpp<WAVE_SHR1>(1.f, au), aR = dpp<WAVE_SHL1>(1.f, ad);
         __syncthreads();
         float lin = 0.f, rin = 0.f;
         for (int x = 0; x < wv; ++x) lin = fmaf(agg[3 * x + 2], lin, agg[3 * x]);
         for (int x = W - 1; x > wv; --x) rin = fmaf(agg[3 * x + 2], rin, agg[3 * x + 1]);
-        L = fmaf(aL, lin, L);
-        R = fmaf(aR, rin, R);
+        L = fmaf(dec.before, lin, L);
+        R = fmaf(dec.after, rin, R);
 #pragma unroll
         for (int e = E - 1; e >= 0; --e) {               // R at the element (later keys), then at the one before
             R += wt[e];
@@ -471,7 +518,7 @@ __device__ __forceinline__ void emit_stream(const ColMergeArgs& A, float* sm, in
     for (int x = tid; x < M; x += T) uo[x] = sm[x];
 }
 
-// dynamic LDS: N + M words (values, then word indices, then the v == 1 terms), then the scan's aggregates
+// dynamic LDS: N + M words (values, then word indices, then the v == 1 terms), then the scans' 3 words a wave
 template <int KIND, int T, int E>
 __global__ __launch_bounds__(T)
 void col_merge(const ColMergeArgs A)
@@ -731,7 +778,7 @@ void col_sort(const ColMergeArgs A)
 // col_sum: one workgroup per (p, feature share, CH channels)
 // ---------------------------------------------------------------------------------------------------------------
 struct ColSumArgs {
-    const float* val; const uint16_t* tag; const float* xe;
+    const float* val; const uint16_t* tag; const float* xe; const float* xe2;
     const float* w;                  // [P][CW][Nw][CH] weight columns (col_weights): of v, or of g_w with SWAP
     float* out;                      // [P][DS][C][Ma]
     int P, D, N, M, C, DS, K0, CW;
@@ -745,7 +792,7 @@ void col_sum(const ColSumArgs A)
 {
     constexpr int W = T / WAVE;
     extern __shared__ float sm[];
-    const int tid = threadIdx.x, lane = lane_id(), wv = wave_in_block();
+    const int tid = threadIdx.x, wv = wave_in_block();
     const int D = A.D, N = A.N, M = A.M, C = A.C, DS = A.DS;
     const int Nw = SWAP ? M : N, Ma = SWAP ? N : M, w0 = SWAP ? 0 : A.K0, a0 = SWAP ? A.K0 : 0;
     const int CG = (C + CH - 1) / CH;
@@ -779,11 +826,20 @@ void col_sum(const ColSumArgs A)
     };
 #pragma unroll
     for (int g = 0; g < E / 4; ++g) load(d0, g);
-    const float* xp = A.xe + (s0 + d0) * T + tid;
-    float xs = *xp;
+    const float* xp = A.xe + (s0 + d0) * T + tid;        // abs
+    float xs = 0.f;
+    if constexpr (KIND == COL_ABS) xs = *xp;
     const uint32_t split = (uint32_t)A.K0 * CH * 4;      // queries' words lie below, keys' above
     auto addr = [&](int e) { return tag_addr<CH * 4>(tg[e / 2], e & 1); };
     for (int d = d0; d < d1; ++d) {
+        f4_t ya = {0.f, 0.f, 0.f, 0.f};                  // Laplace: its Decays, read after the thread's own sums
+        f2_t yb = {0.f, 0.f};
+        if constexpr (KIND == COL_LAPLACE) {
+            ya = buf_load4(make_rsrc(A.xe + s0 * T * 4, (uint32_t)(D * T * 16)), tid * 16, d * (T * 16));
+            yb = __builtin_bit_cast(f2_t, __builtin_amdgcn_raw_buffer_load_b64(
+                     make_rsrc(A.xe2 + s0 * T * 2, (uint32_t)(D * T * 8)), tid * 8, d * (T * 8), 0));
+            asm volatile("" ::: "memory");               // issued here, not where they are used
+        }
         float a[E][CH];
         uint64_t acc[E];                                 // lanes whose element is an accumulator
         // One workgroup per CU (CH = 1): reads run AHEAD elements before their use, in that order, so that a wave's arithmetic
@@ -799,7 +855,7 @@ void col_sum(const ColSumArgs A)
         for (int e = 0; e < AHEAD && e < E; ++e) read(e);
         const int dn = min(d + 1, d1 - 1);
         const uint32_t ab = aggb + (uint32_t)(d & 1) * AGGS;
-        const int el = min(lane & 15, W - 1);            // the wave whose aggregate this lane scans
+        const int lane = lane_now(), el = min(lane & 15, W - 1);         // the wave whose aggregate this lane scans
         if constexpr (KIND == COL_ABS) {
             // Half of sum_n |k_n - x| w_n is sum_{k < x} (x - k) w less half of the sum over all keys of (x - k) w. With x
             // and k relative to the thread's anchor, a thread's own keys below give x W - K from its running sums
@@ -880,7 +936,8 @@ void col_sum(const ColSumArgs A)
         } else {
             // L = sum over the keys below of e^-(x - k) w, R the same above. A thread's own sums, then the states
             // entering it from both sides, then each query adds L + R.
-            float l[CH], r[CH], au = xs, ad = xs, pr = 1.f;
+            const Decays y{ya[0], ya[1], ya[2], ya[3], yb.x, yb.y};
+            float l[CH], r[CH], pr = 1.f;
 #pragma unroll
             for (int h = 0; h < CH; ++h) l[h] = r[h] = 0.f;
 #pragma unroll
@@ -898,12 +955,12 @@ void col_sum(const ColSumArgs A)
                     r[h] = fmaf(pr, x, r[h]);
                 }
             }
-            wave_affine_up(au, l);
-            wave_affine_down(ad, r);
+            wave_affine_up(y, l);
+            wave_affine_down(y, r);
             if (lane == WAVE - 1) {
 #pragma unroll
                 for (int h = 0; h < CH; ++h) *(LDS_AS float*)(ab + (wv * CH + h) * 4) = l[h];
-                *(LDS_AS float*)(ab + (2 * W * CH + wv) * 4) = au;
+                *(LDS_AS float*)(ab + (2 * W * CH + wv) * 4) = y.before * y.own;
             }
             if (lane == 0) {
 #pragma unroll
@@ -915,7 +972,6 @@ void col_sum(const ColSumArgs A)
                 L[h] = dpp<WAVE_SHR1>(0.f, l[h]);
                 R[h] = dpp<WAVE_SHL1>(0.f, r[h]);
             }
-            const float aL = dpp<WAVE_SHR1>(1.f, au), aR = dpp<WAVE_SHL1>(1.f, ad);
             __syncthreads();
             {
                 const float a0_ = *(LDS_AS const float*)(ab + (2 * W * CH + el) * 4);
@@ -932,14 +988,12 @@ void col_sum(const ColSumArgs A)
                 for (int h = 0; h < CH; ++h) {
                     const float lin = wv > 0 ? bcast(up[h], wv > 0 ? wv - 1 : 0) : 0.f;
                     const float rin = wv < W - 1 ? bcast(dw[h], wv < W - 1 ? wv + 1 : 0) : 0.f;
-                    L[h] = fmaf(aL, lin, L[h]);
-                    R[h] = fmaf(aR, rin, R[h]);
+                    L[h] = fmaf(y.before, lin, L[h]);
+                    R[h] = fmaf(y.after, rin, R[h]);
                 }
             }
 #pragma unroll
             for (int g = 0; g < E / 2; ++g) asm volatile("" : "+v"(tg[g]));
-            xp += T;
-            if (d + 1 < d1) xs = *xp;
             // R at each element beside its word where the registers hold both (one rounding of the word per feature, and
             // fewer instructions: 372 -> 338 us at 12 x 8192, two channels); else added to the word on the way (27 spilled
             // registers at 32 elements: 930 -> 1975 us)
@@ -1397,21 +1451,22 @@ bool col_bwd_applies(int D, int N, int M) {
 
 int col_key0(const ColPlan& pl, int M) { return pad_words(M, pl.CH); }
 
-size_t col_stream_bytes(const ColPlan& pl, int S) {
-    const size_t L = (size_t)pl.T * pl.E;
+size_t col_stream_bytes(int kind, const ColPlan& pl, int S) {
+    const size_t L = (size_t)pl.T * pl.E, x = (size_t)S * pl.T * 4;
     auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
-    return al((size_t)S * L * 4) + al((size_t)S * L * 2) + 2 * al((size_t)S * pl.T * 4);
+    return al((size_t)S * L * 4) + al((size_t)S * L * 2) + (kind == COL_ABS ? 2 * al(x) : al(4 * x) + al(2 * x));
 }
 
-ColStream col_stream(const ColPlan& pl, void* base, int S) {
-    const size_t L = (size_t)pl.T * pl.E;
+ColStream col_stream(int kind, const ColPlan& pl, void* base, int S) {
+    const size_t L = (size_t)pl.T * pl.E, x = (size_t)S * pl.T * 4;
     auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
     char* b = (char*)base;
-    ColStream r;
+    ColStream r{};
     r.val = (float*)b;     b += al((size_t)S * L * 4);
     r.tag = (uint16_t*)b;  b += al((size_t)S * L * 2);
-    r.xe = (float*)b;      b += al((size_t)S * pl.T * 4);
-    r.eq = (uint32_t*)b;
+    r.xe = (float*)b;      b += al(kind == COL_ABS ? x : 4 * x);
+    if (kind == COL_ABS) r.eq = (uint32_t*)b;
+    else r.xe2 = (float*)b;
     return r;
 }
 
@@ -1475,7 +1530,7 @@ bool col_sort_applies(const ColPlan& pl) { return pl.E <= 16; }
 
 int col_sort_launch(int kind, const ColPlan& pl, const float* q, const float* k, const uint8_t* keep, ColStream str,
                     float* u, float* bad, int S, int D, int N, int M, hipStream_t st) {
-    const ColMergeArgs a{q, nullptr, k, nullptr, keep, str.val, str.tag, str.xe, nullptr, u, bad, D, N, M, M, 1};
+    const ColMergeArgs a{q, nullptr, k, nullptr, keep, str.val, str.tag, str.xe, str.xe2, nullptr, u, bad, D, N, M, M, 1};
     StageTimer t("col_sort", st);
     return dispatch_shape(pl, [&](auto T, auto E, auto) {
         if constexpr (E() > 16) {
@@ -1498,7 +1553,7 @@ int col_sort_launch(int kind, const ColPlan& pl, const float* q, const float* k,
 int col_merge_launch(int kind, const ColPlan& pl, const float* qs, const uint32_t* qp, const float* ks,
                      const uint32_t* kp, const uint8_t* keep, ColStream str, float* u, float* bad, int S, int D, int N,
                      int M, bool bwd, int sets, hipStream_t st) {
-    const ColMergeArgs a{qs, qp, ks, kp, keep, str.val, str.tag, str.xe, bwd ? str.eq : nullptr, u, bad, D, N, M,
+    const ColMergeArgs a{qs, qp, ks, kp, keep, str.val, str.tag, str.xe, str.xe2, bwd ? str.eq : nullptr, u, bad, D, N, M,
                          bwd ? col_key0(pl, M) : M, sets};
     S *= sets;
     StageTimer t("col_merge", st);
@@ -1521,7 +1576,7 @@ int col_weights_launch(const ColPlan& pl, const float* w, const uint8_t* keep, b
 
 int col_sum_launch(int kind, const ColPlan& pl, ColStream str, const float* wt, float* cols, int P, int D, int N, int M,
                    int C, int sets, hipStream_t st) {
-    const ColSumArgs a{str.val, str.tag, str.xe, wt, cols, P, D * sets, N, M, C, pl.DS, M, (C + pl.CH - 1) / pl.CH, sets};
+    const ColSumArgs a{str.val, str.tag, str.xe, str.xe2, wt, cols, P, D * sets, N, M, C, pl.DS, M, (C + pl.CH - 1) / pl.CH, sets};
     StageTimer t(kind == COL_ABS ? "col_sum_abs" : "col_sum_laplace", st);
     return dispatch_shape(pl, [&](auto T, auto E, auto CH) {
         return kind == COL_ABS ? launch_sum<COL_ABS, T(), E(), CH(), false>(a, st)
@@ -1530,7 +1585,7 @@ int col_sum_launch(int kind, const ColPlan& pl, ColStream str, const float* wt, 
 
 int col_grad_v_launch(const ColPlan& pl, ColStream str, const float* gt, int CW, float* cols, int P, int D, int N, int M,
                       int C, hipStream_t st) {
-    const ColSumArgs a{str.val, str.tag, str.xe, gt, cols, P, D, N, M, C, pl.DS, col_key0(pl, M), CW, 1};
+    const ColSumArgs a{str.val, str.tag, str.xe, str.xe2, gt, cols, P, D, N, M, C, pl.DS, col_key0(pl, M), CW, 1};
     StageTimer t("col_grad_v", st);
     return dispatch_shape(pl, [&](auto T, auto E, auto CH) { return launch_sum<COL_ABS, T(), E(), CH(), true>(a, st); });
 }

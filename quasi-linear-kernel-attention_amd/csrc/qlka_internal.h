@@ -264,11 +264,11 @@ constexpr int COL_MAX2 = 20352;          // two channels per workgroup: 2 words 
 constexpr int COL_SHARES = 16;           // most shares of the features
 // threads, elements per thread, channels per workgroup, shares of the features, features one after another in all rounds
 struct ColPlan { int T, E, CH, DS; int64_t cost; };
-struct ColStream { float* val; uint16_t* tag; float* xe; uint32_t* eq; };
+struct ColStream { float* val; uint16_t* tag; float* xe; float* xe2; uint32_t* eq; };
 bool col_applies(int D, int N, int M);
 ColPlan col_plan(int kind, int P, int D, int N, int M, int C);      // kind 0 abs, 1 Laplace (as below)
-size_t col_stream_bytes(const ColPlan& pl, int S);
-ColStream col_stream(const ColPlan& pl, void* base, int S);
+size_t col_stream_bytes(int kind, const ColPlan& pl, int S);
+ColStream col_stream(int kind, const ColPlan& pl, void* base, int S);
 // the merged stream of S sorted segments, and the v == 1 terms u (S, M) in query order (null: none); masked keys are padding.
 // bwd: the stream of the abs backward (keys' words from col_key0, runs of equal values). sets = 3 (kind 0): three streams
 // and rows of u per segment, of q, q + 1 and q - 1, which the sums weight -1, 1/2, 1/2 (add_bump); else 1. bad (P, M), with

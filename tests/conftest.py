@@ -40,7 +40,6 @@ def dev():
 # The library's own routing by size ("auto"), or every short segment too through sort + walk or, where N + M allows it, sort +
 # column sums: dense cutoff (None: as it is), column mode.
 ROUTES = {"auto": (None, 0), "walk": (0, 1), "columns": (0, 2)}
-COLUMN_MAX = 32768                 # longest segment (N + M) that goes by columns
 
 
 @pytest.fixture
