@@ -14,7 +14,8 @@
 // C / CH workgroups of a p read it, neighbours on one XCD at about the same time, so from its L2.
 //   val[s][E/4][T][4]   abs: the value less the thread's anchor, the end of its elements that lies towards the segment's
 //                       median key; Laplace: e^-distance to the previous element
-//   tag[s][E/4][T][4]   16-bit word index: m for query m, K0 + n for key n, K0 + N for padding (K0 = M, or M rounded up)
+//   tag[s][E/4][T][4]   16-bit word index: query m at spread(m), key n at K0 + spread(n), padding at K0 + N (K0 = M, or M
+//                       rounded up)
 //   xe[s][T]            abs: each thread's anchor less the median key; Laplace: its Decays
 //   eq[s][T]            (abs backward) bit e: element e of the thread has the value of the element before it
 // With 4 elements per 16-byte (8-byte) load, a wave's loads are contiguous.
@@ -286,8 +287,8 @@ struct ColMergeArgs {
     const float* qs; const uint32_t* qp; const float* ks; const uint32_t* kp;   // sorted queries and keys
     const uint8_t* keep;             // (P, N) key mask or null: masked keys become padding
     float* val; uint16_t* tag; float* xe; float* xe2; uint32_t* eq;  // eq: null unless wanted; xe2: Laplace only
-    float* u;                        // (S, M) v == 1 terms in query order, or null
-    float* bad;                      // (P, M), bwd: (P, N): NaN at the rows whose own value makes them NaN, 0 else; or null
+    float* u;                        // (S, M) v == 1 terms in the order of the words, or null
+    float* bad;                      // (P, M), bwd: (P, N), in the order of the words: NaN at the rows whose own value makes them NaN, 0 else; or null
     int D, N, M, K0;
     int sets;                        // 1, or 3: streams of q, q + 1 and q - 1 per segment (add_bump), their v == 1 terms weighted
 };
@@ -314,6 +315,12 @@ __device__ __forceinline__ bool any_of(bool x, uint32_t* flags) {
     __syncthreads();
     return __ballot(flags[lane_id() % W] != 0) != 0;
 }
+
+// The word of row i among the L of a side (and the row of word i): within each whole block of 64, shuffled by the block's
+// number. Where values tie, the sorts leave rows in order, and threads of E consecutive elements each would read words E
+// apart, 16 and more of them from one bank (12 x 64 x 16384, half the keys 0 as by a
+// mask multiplied in: abs 1.93 -> 1.35 ms, Laplace 2.11 -> 1.44, training 5.88 -> 3.81; walks 1.72, 1.71, 4.75).
+__device__ __forceinline__ int spread(int i, int L) { return i < (L & ~63) ? i ^ ((i >> 6) & 63) : i; }
 
 // 16-bit word indices, two in a register
 template <int E>
@@ -509,7 +516,7 @@ __device__ __forceinline__ void emit_stream(const ColMergeArgs& A, float* sm, in
 #pragma unroll
         for (int e = 0; e < E; ++e) { L = fmaf(dist[e], L, wt[e]); out[e] += L; }
     }
-    // to query order through LDS (every thread has read its word indices before the scan's barrier)
+    // in the order of the words through LDS (every thread has read its word indices before the scan's barrier)
 #pragma unroll
     for (int e = 0; e < E; ++e)
         if ((int)src.get(e) < M) sm[src.get(e)] = out[e];
@@ -553,8 +560,9 @@ void col_merge(const ColMergeArgs A)
             sm[i] = no_nan(x);
             const bool weight = (i >= M) == (A.eq == nullptr);
             const int row = i < M ? (int)A.qp[(size_t)seg * M + i] : (int)A.kp[(size_t)seg * N + i - M];
+            const int rows = i < M ? M : N;
             if (weight) nan |= !keep || keep[row] != 0;
-            else if (A.bad) A.bad[(size_t)(seg / A.D) * (A.eq ? N : M) + row] = x;
+            else if (A.bad) A.bad[(size_t)(seg / A.D) * rows + spread(row, rows)] = x;
         }
         __syncthreads();
         poison = any_of<T / WAVE>(nan, (uint32_t*)sm + n);
@@ -601,9 +609,12 @@ void col_merge(const ColMergeArgs A)
         const uint32_t* qp = A.qp + (size_t)seg * M;
         const uint32_t* kp = A.kp + (size_t)seg * N;
 #pragma unroll 8
-        for (int x = tid; x < M; x += T) w[x] = qp[x];
+        for (int x = tid; x < M; x += T) w[x] = (uint32_t)spread((int)qp[x], M);
 #pragma unroll 8
-        for (int x = tid; x < N; x += T) w[M + x] = A.K0 + (!keep || keep[kp[x]] != 0 ? kp[x] : (uint32_t)N);
+        for (int x = tid; x < N; x += T) {
+            const int key = (int)kp[x];
+            w[M + x] = (uint32_t)(A.K0 + (!keep || keep[key] != 0 ? spread(key, N) : N));
+        }
         __syncthreads();
 #pragma unroll
         for (int e = 0; e < E; e += 2) {
@@ -675,7 +686,7 @@ void col_sort(const ColMergeArgs A)
             const bool on = i < n && (i < M || !keep || keep[i - M] != 0);
             odd |= on && !ordinary<KIND>(x);
             key[j] = on ? min(float_to_ordered(x), 0xfffffffeu) : 0xffffffffu;
-            idx.set(j, on ? (uint32_t)i : (uint32_t)n);
+            idx.set(j, on ? (uint32_t)(i < M ? spread(i, M) : M + spread(i - M, N)) : (uint32_t)n);
             live += (int)__popcll(__ballot(on));
         }
     }
@@ -1265,15 +1276,15 @@ void col_dot(const ColDotArgs A)
     }
     __syncthreads();
     float* gq = A.gq + (size_t)s * M;
-    for (int i = tid; i < M; i += T) gq[i] = sm[i];
+    for (int i = tid; i < M; i += T) gq[i] = sm[spread(i, M)];
     if (A.gk) {
         float* gk = A.gk + (size_t)s * N;
-        for (int i = tid; i < N; i += T) gk[i] = sm[K0 + i];
+        for (int i = tid; i < N; i += T) gk[i] = sm[K0 + spread(i, N)];
     }
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// col_weights: the weight rows (P, Nw, C) as columns [P][CW][Nw][CH], masked rows 0. With C1 = C + 1 there is one more
+// col_weights: the weight rows (P, Nw, C) as columns [P][CW][Nw][CH] in the order of their words, masked rows 0. With C1 = C + 1 there is one more
 // channel, `extra` (P, Nw) or all ones. Also clears `bad` (bads words; null: 0) for the merge that comes after it.
 // ---------------------------------------------------------------------------------------------------------------
 constexpr int CF_T = 256, CF_M = 64;        // threads, rows per workgroup (also of col_finish)
@@ -1303,7 +1314,7 @@ void col_weights(const float* __restrict__ w, const float* __restrict__ extra, c
         if (lane < rows) tile[cc][lane] = cc < C1 ? (extra ? extra[(size_t)p * Nw + n0 + lane] : 1.f) : 0.f;
     __syncthreads();
     if (lane >= rows) return;
-    float* dst = out + ((size_t)p * CW * Nw + n0 + lane) * CH;
+    float* dst = out + ((size_t)p * CW * Nw + spread(n0 + lane, Nw)) * CH;
     for (int g = threadIdx.x / CF_M; g < CW; g += CF_T / CF_M) {
         if constexpr (CH == 1) {
             dst[(size_t)g * Nw] = tile[g][lane];
@@ -1332,7 +1343,7 @@ void col_finish(const float* __restrict__ cols, const float* __restrict__ u, con
     const int mb = (M + CF_M - 1) / CF_M;
     const int p = blockIdx.x / mb, m0 = (blockIdx.x - p * mb) * CF_M;
     const int lane = threadIdx.x & (CF_M - 1), wv = threadIdx.x / CF_M;
-    const int m = min(m0 + lane, M - 1);
+    const int m = spread(min(m0 + lane, M - 1), M);         // its word
     const float* src = cols + (size_t)p * DS * C * M + m;
     const float spoilt = bad[(size_t)p * M + m];         // 0 or NaN
 #pragma unroll 4

@@ -269,7 +269,8 @@ bool col_applies(int D, int N, int M);
 ColPlan col_plan(int kind, int P, int D, int N, int M, int C);      // kind 0 abs, 1 Laplace (as below)
 size_t col_stream_bytes(int kind, const ColPlan& pl, int S);
 ColStream col_stream(int kind, const ColPlan& pl, void* base, int S);
-// the merged stream of S sorted segments, and the v == 1 terms u (S, M) in query order (null: none); masked keys are padding.
+// the merged stream of S sorted segments, and the v == 1 terms u (S, M) in the order of the words
+// (null: none); masked keys are padding.
 // bwd: the stream of the abs backward (keys' words from col_key0, runs of equal values). sets = 3 (kind 0): three streams
 // and rows of u per segment, of q, q + 1 and q - 1, which the sums weight -1, 1/2, 1/2 (add_bump); else 1. bad (P, M), with
 // bwd (P, N), cleared before (col_weights_launch): NaN where a row's own value makes it NaN (null: not wanted).

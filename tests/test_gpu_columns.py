@@ -324,3 +324,32 @@ def test_laplace_keys_whose_roundings_repeat(dev, no_dense, n, kind):
     ow, ou, _ = brute.laplace_sum(q, k, v, qidx=idx)
     assert np.linalg.norm(w[0][idx[0]] - ow[0]) <= 1e-6 * np.linalg.norm(ow[0])
     assert np.linalg.norm(u[0][idx[0]] - ou[0]) <= 1e-6 * np.linalg.norm(ou[0])
+
+
+@pytest.mark.parametrize("shape", [(1, 3, 63, 64, 2), (1, 3, 65, 127, 3), (2, 2, 4160, 4033, 5), (1, 2, 12352, 10000, 3)])
+def test_columns_of_equal_and_padded_values(dev, no_dense, shape):
+    # whole and broken blocks of 64 rows (their words are shuffled within whole ones), all values of a feature equal, and a
+    # tail of keys that a mask made 0
+    P, D, N, M, C = shape
+    from weighted_abs_sum import weighted_abs_sum_full
+    from weighted_laplace_sum import weighted_laplace_sum
+    print(f"equal and padded {shape}", flush=True)
+    q, k, v = _data(P, D, N, M, C, "normal", sum(shape))
+    q[:, 0], k[:, 0] = 0.5, 0.5
+    k[:, 1, N // 2:] = 0
+    v[:, N // 2:] = 0
+    g = np.random.default_rng(3).standard_normal((P, M, C), dtype=np.float32)
+    t = [torch.from_numpy(a).to(dev) for a in (q, k, v, g)]
+    idx, ik = inputs.query_subsample(P, M, per_p=24, seed=2), inputs.query_subsample(P, N, per_p=24, seed=3)
+    take = lambda a, i, ax=0: np.stack([np.take(a[p], i[p], axis=ax) for p in range(P)])  # noqa: E731
+    for op, oracle in ((lambda *a: weighted_abs_sum_full(*a, backend="cuda"), brute.abs_sum),
+                       (weighted_laplace_sum, brute.laplace_sum)):
+        w, u = (x.cpu().numpy() for x in op(*t[:3]))
+        ow, ou, nw = oracle(q, k, v, qidx=idx)
+        assert float(brute.rel_err(take(w, idx), ow, nw).max()) <= REL
+        assert float(brute.rel_err(take(u, idx), ou, ou).max()) <= REL
+    from weighted_abs_sum import _ext
+    got = [x.cpu().numpy() for x in _ext.weighted_abs_sum_backward(*t)]
+    (wq, wk, wv), (nq, nk, nv) = brute.abs_backward_sub(q, k, v, g, None, idx, ik)
+    for a, w, n in ((take(got[0], idx, 1), wq, nq), (take(got[1], ik, 1), wk, nk), (take(got[2], ik), wv, nv)):
+        assert float(brute.rel_err(a, w, n).max()) <= REL
