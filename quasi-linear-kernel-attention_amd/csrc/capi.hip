@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -463,39 +464,82 @@ int run_pipeline(int P, const Plan& pl, void* ws, size_t copy, hipStream_t st, P
 // The chunks run in order on the caller's stream: the sums keep every CU's LDS, so nothing would run beside them. Its
 // workspace is smaller than the walk's but for many more keys than queries, where the *_ws_bytes queries return the
 // larger of the two.
-// Its longer chain of launches, each too small to fill the chip, costs more than the walk's below about half a million
-// elements (a million with fewer than 128 segments, one workgroup each in its sort) forward, and backward, whose dot
-// products also take one workgroup per segment, below a million, 128 segments, or 192 where a workgroup fills a CU.
-// (P, D, M = N, C = 64:) Laplace 114 against 87 us at 1 x 64 x 2000, 99 against 139 at 12 x 64 x 520, abs 132 against 114 at
-// 1 x 64 x 4200; forward + backward 258 against 160 us at 1 x 64 x 1500, even at 12 x 64 x 640, 322 against 368 at
-// 12 x 64 x 1100, 796 against 774 at 2 x 64 x 16000. The sgn sum takes it with two channels per workgroup only
-// (12 x 64 x 3000: 253 against 277 us; 16384: 1525 against 1439). qlka_set_columns overrides all of this for tests.
-inline bool col_enough(int P, int D, int N, int M, int64_t elements, int64_t segments) {
+//
+// Which route a call takes is decided by estimates of both routes' times (us), linear in what each does and fitted (relative
+// least squares) to both routes' times of 840 calls on MI355X: P D (N + M) from 2^12 to 2^25, D from 1 to 300, N / M from 1/32
+// to 32, C from 1 to 128. They are within 8 to 18% of the times on average, and the columns are taken where theirs is below
+// the walk's by a margin. Over those calls, against the walk: Laplace 1.39 x, abs 1.45 x, add_bump 1.83 x, backward 1.37 x, sgn
+// 1.08 x on average, 2.2%, 2.4%, 2.3%, 3.2% and 8% off the faster route; 1 to 1.5% of them are more than 5% slower than
+// their walk, at most by 30%. Fixed limits on elements and segments instead took 2.2 x the walk's time with
+// few features per p (256 x 1 x 4000 x 4000 x 64 abs: 572 against 310 us; the columns are loaded for one feature) or many more
+// keys than queries (add_bump 12 x 64 x 20000 x 600 x 64: 2.73 against 1.54 ms; its three streams hold the keys three times),
+// and left small calls to the walk (2 x 64 x 1225 x 703 x 4 Laplace: 106 against 47 us). qlka_set_columns overrides it.
+enum ColOp : int { COL_OP_LAPLACE, COL_OP_ABS, COL_OP_BUMP, COL_OP_BWD, COL_OP_SGN };
+
+// The walk: its launches; per 1000 segment keys and queries (sorts, bounds, walk); per 10^6 words of gathered and written
+// rows, more of them with two channel slots a lane, unaligned rows and widths that are no power of two; keys past one LDS
+// sort; the length of its longest chain per segments beyond the chip's workgroups.
+struct WalkCost {
+    double launches, key, query, key_row, query_row, two, long_key, unaligned, unaligned_two, uneven, chain;
+};
+constexpr WalkCost WALK_COST[] = {
+    {55, 0.052, 0.043, 0.081, 0.79, 0.39, 0.010, 0.39, 0.15, 0.12, 2.2},
+    {55, 0.049, 0.042, 0.082, 0.80, 0.38, 0.010, 0.38, 0.14, 0.12, 2.2},
+    {99, 0.051, 0.130, 0, 2.2, 0.61, 0.009, 1.8, 0.30, 1.4, 2.8},
+    {71, 0.086, 0.067, 0.65, 0.20, 1.9, 0.036, 1.6, 0, 0.25, 3.2},
+    {35, 0.042, 0.029, 0.14, 0.42, 0.34, 0.016, 0.094, 0, 0.14, 3.3},
+};
+double walk_us(ColOp op, int P, int D, int N, int M, int C) {
+    const WalkCost& w = WALK_COST[op];
+    const double S = (double)P * D, row = S * std::max(C, 8) * 1e-6, rows = row * ((double)N + M);
+    return w.launches + S * 1e-3 * (w.key * N + w.query * M + (N > LDS_SORT_MAX ? w.long_key * N : 0.)) +
+           row * (w.key_row * N + w.query_row * M) + (C > 64 ? w.two * rows : 0.) + (C % 4 ? (C > 64 ? w.unaligned_two : w.unaligned) * rows : 0.) +
+           ((C & (C - 1)) ? w.uneven * rows : 0.) + w.chain * std::ceil(S / 512) * std::max(N, M) * 1e-3;
+}
+
+// The columns: their launches; the sorts and merges, one workgroup per segment, by the waves a SIMD runs and the elements of
+// each thread, and per 1000 elements; the transposes per 1000 words; the sums, by waves and elements as the sorts and by the
+// features a workgroup walks (load and store of its columns: another 2, or 6 with a CU to itself); the finish, one thread
+// adding the shares of C / 4 channels. Backward: the dots, by rounds over the chip and by waves, elements and channel
+// groups, and per 10^6 words that they read.
+struct ColCost { double launches, sort, element, word, sum, finish, dot_round, dot, dot_word, margin, slack; };
+constexpr ColCost COL_COST[] = {
+    {28, 0.48, 0.0068, 0.0023, 0.036, 0.073, 0, 0, 0, 0.95, 8},
+    {27, 0.50, 0.0056, 0.0024, 0.030, 0.072, 0, 0, 0, 0.95, 8},
+    {43, 0.34, 0.0093, 0.0030, 0.033, 0.073, 0, 0, 0, 0.95, 8},
+    {39, 0.58, 0.0120, 0.0049, 0, 0.091, 0.060, 0.027, 0.34, 1.0, 15},
+    {43, 0.31, 0.0130, 0.0028, 0, 0, 0.035, 0, 0.42, 0.75, 5},
+};
+double col_us(ColOp op, int P, int D, int N, int M, int C) {
+    const ColCost& w = COL_COST[op];
+    const int sets = op == COL_OP_BUMP ? 3 : 1;
+    const ColPlan pl = col_plan(op == COL_OP_LAPLACE ? 1 : 0, P, D * sets, N, M, C);
+    const int DS = std::min(pl.DS, std::min(D, COL_SHARES));
+    const double S = (double)P * D, n = (double)N + M, waves = pl.T / 256. * pl.E, groups = (C + pl.CH - 1) / pl.CH;
+    const double sums = std::ceil(P * groups * DS / CUS) * waves * ((D * sets + DS - 1) / DS + (pl.CH == 1 ? 6 : 2));
+    const double rows = op == COL_OP_BWD ? N : M, dots = (C + 2) / pl.CH;
+    return w.launches + w.sort * std::ceil(S / CUS) * waves + S * n * sets * 1e-3 * w.element + P * n * C * 1e-3 * w.word +
+           w.sum * sums + w.finish * std::ceil(P * std::ceil(rows / 64) / (4 * CUS)) * C * DS +
+           w.dot_round * std::ceil(S / (CUS * pl.per_cu)) * pl.E * dots + w.dot * std::ceil(S / CUS) * waves * dots +
+           w.dot_word * S * n * C * 1e-6;
+}
+bool col_faster(ColOp op, int P, int D, int N, int M, int C) {
     const int mode = columns_mode();
     if (mode != QLKA_COLUMNS_AUTO) return mode == QLKA_COLUMNS_ALWAYS;
-    return (int64_t)P * D * ((int64_t)N + M) >= elements && (int64_t)P * D >= segments;
+    return col_us(op, P, D, N, M, C) < COL_COST[op].margin * walk_us(op, P, D, N, M, C) - COL_COST[op].slack;
 }
-inline bool col_fwd(int P, int D, int sets, int N, int M) {
-    return col_applies(D * sets, N, M) &&
-           (col_enough(P, D, N, M, 1 << 19, 128) || col_enough(P, D, N, M, 1 << 20, 1));
+
+// forward sums: COL_OP_LAPLACE, COL_OP_ABS or COL_OP_BUMP
+bool col_fwd(ColOp op, int P, int D, int N, int M, int C) {
+    return col_applies(op == COL_OP_BUMP ? 3 * D : D, N, M) && col_faster(op, P, D, N, M, C);
 }
-// The Laplace sums with one channel per workgroup (N + M > COL_MAX2) run about as long as the walk, so there the rounds that
-// the chip needs decide, by estimates of both in us: 4.75 per feature and round of 32-element threads, the sorts and the
-// merge, against the walk at this width (P, D, M = N, C: 10 x 64 x 15000 x 64 1336 against 1306 us, 9 x 64 x 15000 x 64 1308
-// against 1197, but 8 x 64 x 16300 x 64 1035 against 1188 and 12 x 64 x 16384 x 64 1540 against 1690).
-inline bool col_laplace(int P, int D, int N, int M, int C) {
-    if (!col_fwd(P, D, 1, N, M)) return false;
-    if (N + M <= COL_MAX2 || columns_mode() == QLKA_COLUMNS_ALWAYS) return true;
-    const ColPlan pl = col_plan(1, P, D, N, M, C);
-    const double el = (double)P * D * (N + M);
-    const double col = 60 + pl.cost * 4.75 * pl.E / 32 + el * 1.87e-5;
-    const double walk = el * 0.67e-4 * (C <= 32 ? 0.67 : C <= 64 ? 1 : 2.4) * (std::max(N, M) > LDS_SORT_MAX ? 1.35 : 1);
-    return col < walk;
+bool col_bwd(int P, int D, int N, int M, int C) {
+    return col_bwd_applies(D, N, M) && col_faster(COL_OP_BWD, P, D, N, M, C);
 }
-inline bool col_bwd(int P, int D, int N, int M) {
-    return col_bwd_applies(D, N, M) && col_enough(P, D, N, M, 1 << 20, N + M <= COL_MAX2 ? 128 : 192);
+// with two channels per workgroup only
+bool col_sgn(int P, int D, int N, int M, int C) {
+    return N + M <= COL_MAX2 && col_bwd_applies(D, N, M) && col_faster(COL_OP_SGN, P, D, N, M, C);
 }
-inline bool col_sgn(int P, int D, int N, int M) { return col_bwd(P, D, N, M) && N + M <= COL_MAX2; }
 
 struct ColWs { SortedWs s; ColStream str; float* u; float* cols; float* wt; float* bad; char* extra; };
 
@@ -700,7 +744,7 @@ int qlka_laplace_fwd(const float* q, const float* k, const float* v, float* out_
     auto b1 = [&](int pc) { return laplace_ws(pc, D, N, M, C); };
     const Plan pl = plan_chunks(P, ws_bytes_given, pipelined(P, D, M), b1);
     if (int e = check_ws(ws, ws_bytes_given, plan_bytes(pl, b1))) return e;
-    if (col_laplace(P, D, N, M, C))
+    if (col_fwd(COL_OP_LAPLACE, P, D, N, M, C))
         return run_columns(1, 1, q, k, v, nullptr, true, P, D, N, M, C, ws, ws_bytes_given, st, no_extra,
             [&](int p0, int np, ColWs& w, hipStream_t s) {
                 const size_t p = (size_t)p0;
@@ -831,7 +875,7 @@ int abs_fwd_impl(const float* q, const float* k, const float* v, float* out_w, f
     if (int e = check_ws(ws, ws_bytes_given, plan_bytes(pl, b1))) return e;
     // By columns no range states are formed, so only the sorts are kept, where the backward is expected to need no states;
     // should it walk all the same (the routes can be pinned in between), it forms its own.
-    if (col_fwd(P, D, 1, N, M) && (!keep_states || col_bwd(P, D, N, M))) {
+    if (col_fwd(COL_OP_ABS, P, D, N, M, C) && (!keep_states || col_bwd(P, D, N, M, C))) {
         const int e = run_columns(0, 1, keep_sorts ? nullptr : q, k, v, nullptr, out_u != nullptr, P, D, N, M, C, ws, ws_bytes_given, st, no_extra,
             [&](int p0, int np, ColWs& w, hipStream_t s) {
                 const size_t p = (size_t)p0;
@@ -1118,7 +1162,7 @@ int abs_bwd_impl(const float* q, const float* k, const float* v, const float* g_
     hipStream_t st = (hipStream_t)stream;
     if (dense_sign(P, N, M))     // the walks' convention: a tie counts -1 in both gradients
         return dense_bwd(-1.f, q, k, v, g_w, g_u, grad_q, grad_k, grad_v, P, D, N, M, C, st);
-    if (col_bwd(P, D, N, M)) {
+    if (col_bwd(P, D, N, M, C)) {
         if (int e = check_ws(ws, ws_bytes_given, col_bwd_bytes(1, D, N, M, C))) return e;
         return run_bwd_columns(v, g_w, g_u, 2.f, grad_q, grad_k, grad_v, P, D, N, M, C, ws, ws_bytes_given, st,
             [&](int p0, int np, SortedWs& w, hipStream_t s) {
@@ -1231,7 +1275,7 @@ int qlka_sgn_fwd(const float* q, const float* k, const float* v, const float* g,
     hipStream_t st = (hipStream_t)stream;
     if (dense_sign(P, N, M))     // sgn(k - q) with a tie counted +1 == -(s(q - k) with a tie counted -1)
         return hip_status(direct_sign(true, q, k, g, v, nullptr, out, -1.f, -1.f, P, D, M, N, C, st), "dense sgn sum");
-    if (col_sgn(P, D, N, M))   // sgn(k - q) with a tie counted +1, as above: -grad_q
+    if (col_sgn(P, D, N, M, C))   // sgn(k - q) with a tie counted +1, as above: -grad_q
         return run_bwd_columns(v, g, nullptr, -2.f, out, nullptr, nullptr, P, D, N, M, C, ws, ws_bytes_given, st,
             [&](int p0, int np, SortedWs& w, hipStream_t s) {
                 const size_t p = (size_t)p0;
@@ -1489,7 +1533,8 @@ static int layer_fwd(int kind, const float* q, const float* k, const float* v, c
         npc = n_pad ? n_pad + p : nullptr; keepc = keep ? keep + p * N : nullptr; outc = out + p * M * C;
     };
     const bool bump = kind == LAYER_ADD_BUMP;
-    const bool columns = kind == LAYER_ADD_LAPLACE ? col_laplace(P, D, N, M, C) : col_fwd(P, D, bump ? 3 : 1, N, M);
+    const ColOp op = kind == LAYER_ADD_LAPLACE ? COL_OP_LAPLACE : bump ? COL_OP_BUMP : COL_OP_ABS;
+    const bool columns = col_fwd(op, P, D, N, M, C);
     if (columns && !(kind == LAYER_ADD_RIESZ && keep == nullptr && few_keys(N)))
         return layer_columns(kind, q, k, v, n_pad, keep, out, P, D, N, M, C, ws, ws_bytes_given, st);
     if (kind == LAYER_ADD_RIESZ && keep == nullptr && few_keys(N))   // the abs sums dense (few_keys), then the epilogue

@@ -1443,13 +1443,13 @@ ColPlan col_plan(int kind, int P, int D, int N, int M, int C) {
     // Shares of the features: the fewest rounds of workgroups over the chip, in features walked one after another, plus the
     // loading and storing of the columns per round: about six features' time where a workgroup has a CU to itself, two
     // where others run beside it.
-    const int64_t wgs = (int64_t)P * ((C + pl.CH - 1) / pl.CH), slots = 256 * (int64_t)wgs_per_cu(kind, pl.T, pl.CH, n);
+    pl.per_cu = wgs_per_cu(kind, pl.T, pl.CH, n);
+    const int64_t wgs = (int64_t)P * ((C + pl.CH - 1) / pl.CH), slots = (int64_t)CUS * pl.per_cu;
     int64_t best = -1;
     for (int s = 1; s <= std::min(D, COL_SHARES); ++s) {
         const int64_t cost = ((wgs * s + slots - 1) / slots) * ((D + s - 1) / s + (pl.CH == 1 ? 6 : 2));
         if (best < 0 || cost < best) { best = cost; pl.DS = s; }
     }
-    pl.cost = best;
     return pl;
 }
 

@@ -262,8 +262,9 @@ int reduce_slabs_bump(bool masked, const ReduceEpilogue& ep, const float* const 
 constexpr int COL_MAX = 32768;           // 32 elements for each of 1024 threads
 constexpr int COL_MAX2 = 20352;          // two channels per workgroup: 2 words of LDS per element
 constexpr int COL_SHARES = 16;           // most shares of the features
-// threads, elements per thread, channels per workgroup, shares of the features, features one after another in all rounds
-struct ColPlan { int T, E, CH, DS; int64_t cost; };
+constexpr int CUS = 256;                 // compute units of an MI355X
+// threads, elements per thread, channels per workgroup, shares of the features, workgroups of the sums that a CU holds
+struct ColPlan { int T, E, CH, DS, per_cu; };
 struct ColStream { float* val; uint16_t* tag; float* xe; float* xe2; uint32_t* eq; };
 bool col_applies(int D, int N, int M);
 ColPlan col_plan(int kind, int P, int D, int N, int M, int C);      // kind 0 abs, 1 Laplace (as below)

@@ -353,3 +353,37 @@ def test_columns_of_equal_and_padded_values(dev, no_dense, shape):
     (wq, wk, wv), (nq, nk, nv) = brute.abs_backward_sub(q, k, v, g, None, idx, ik)
     for a, w, n in ((take(got[0], idx, 1), wq, nq), (take(got[1], ik, 1), wk, nk), (take(got[2], ik), wv, nv)):
         assert float(brute.rel_err(a, w, n).max()) <= REL
+
+
+# calls whose two routes were measured 1.3 x and more apart: the slower one is not taken
+@pytest.mark.parametrize("op,shape,columns", [
+    ("abs", (256, 1, 4000, 4000, 64), False), ("laplace", (256, 1, 4000, 4000, 64), False),      # one feature per p
+    ("abs", (40, 4, 14000, 14000, 64), False), ("bwd", (256, 1, 4000, 4000, 64), False),
+    ("add_bump", (12, 64, 20000, 600, 64), False),                  # the keys in three streams
+    ("sgn", (2, 64, 5200, 5200, 64), False), ("sgn", (512, 4, 1100, 1100, 64), False),
+    ("abs", (12, 64, 8192, 8192, 64), True), ("laplace", (12, 64, 8192, 8192, 64), True),
+    ("bwd", (12, 64, 8192, 8192, 64), True), ("add_bump", (12, 64, 8192, 8192, 64), True),
+    ("laplace", (2, 64, 1225, 703, 4), True), ("abs", (12, 64, 600, 20000, 64), True),
+])
+def test_the_measured_faster_route_is_taken(dev, op, shape, columns):
+    from qlka import _lib, layers
+    from weighted_abs_sum import _ext, weighted_abs_sum_full, weighted_sgn_sum
+    from weighted_laplace_sum import weighted_laplace_sum
+    P, D, N, M, C = shape
+    print(f"route {op} {shape}", flush=True)
+    g = torch.Generator(dev).manual_seed(1)
+    q, k, v, gw = (torch.randn(s, generator=g, device=dev) for s in ((P, D, M), (P, D, N), (P, N, C), (P, M, C)))
+    call = {"abs": lambda: weighted_abs_sum_full(q, k, v, backend="cuda"), "laplace": lambda: weighted_laplace_sum(q, k, v),
+            "bwd": lambda: _ext.weighted_abs_sum_backward(q, k, v, gw),
+            "sgn": lambda: weighted_sgn_sum(q, k, v, gw, backend="cuda"),
+            "add_bump": lambda: layers.layer_forward("add_bump", q, k, v)}[op]
+    lib = _lib.load()
+    lib.qlka_timing_enable(1)
+    try:
+        before = [_lib.stage_time(s)[1] for s in ("col_sort", "col_merge")]
+        call()
+        torch.cuda.synchronize()
+        ran = [_lib.stage_time(s)[1] for s in ("col_sort", "col_merge")] != before
+    finally:
+        lib.qlka_timing_enable(0)
+    assert ran == columns
