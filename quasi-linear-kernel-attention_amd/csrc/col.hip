@@ -525,6 +525,19 @@ __device__ __forceinline__ void emit_stream(const ColMergeArgs& A, float* sm, in
     for (int x = tid; x < M; x += T) uo[x] = sm[x];
 }
 
+// f(i, x[i]) for the n elements of x, shared out over T threads; eight loads of each are in flight at a time
+template <int T, class X, class F>
+__device__ __forceinline__ void each_of(const X* __restrict__ x, int n, F f) {
+    for (int i = threadIdx.x; i < n; i += 8 * T) {
+        X r[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) r[j] = x[min(i + j * T, n - 1)];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (i + j * T < n) f(i + j * T, r[j]);
+    }
+}
+
 // dynamic LDS: N + M words (values, then word indices, then the v == 1 terms), then the scans' 3 words a wave
 template <int KIND, int T, int E>
 __global__ __launch_bounds__(T)
@@ -538,18 +551,15 @@ void col_merge(const ColMergeArgs A)
     const float shift = set_shift(s - seg * A.sets);
     const uint8_t* keep = A.keep ? A.keep + (size_t)(seg / A.D) * N : nullptr;       // without A.eq only
     bool odd = false;
-#pragma unroll 8
-    for (int i = tid; i < M; i += T) {
-        const float x = qs[i] + shift;
+    each_of<T>(qs, M, [&](int i, float x) {
+        x += shift;
         odd |= !ordinary<KIND>(x);
         sm[i] = x;
-    }
-#pragma unroll 8
-    for (int i = tid; i < N; i += T) {
-        const float x = ks[i];
+    });
+    each_of<T>(ks, N, [&](int i, float x) {
         odd |= !ordinary<KIND>(x);
         sm[M + i] = x;
-    }
+    });
     const bool rare = any_of<T / WAVE>(odd, (uint32_t*)sm + n);
     bool poison = false;
     if (rare) {          // the merge compares floats: NaNs become infinities, on the side that the sort put them
@@ -608,13 +618,9 @@ void col_merge(const ColMergeArgs A)
         uint32_t* w = (uint32_t*)sm;
         const uint32_t* qp = A.qp + (size_t)seg * M;
         const uint32_t* kp = A.kp + (size_t)seg * N;
-#pragma unroll 8
-        for (int x = tid; x < M; x += T) w[x] = (uint32_t)spread((int)qp[x], M);
-#pragma unroll 8
-        for (int x = tid; x < N; x += T) {
-            const int key = (int)kp[x];
-            w[M + x] = (uint32_t)(A.K0 + (!keep || keep[key] != 0 ? spread(key, N) : N));
-        }
+        each_of<T>(qp, M, [&](int i, uint32_t x) { w[i] = (uint32_t)spread((int)x, M); });
+        if (!keep) each_of<T>(kp, N, [&](int i, uint32_t x) { w[M + i] = (uint32_t)(A.K0 + spread((int)x, N)); });
+        else each_of<T>(kp, N, [&](int i, uint32_t x) { w[M + i] = (uint32_t)(A.K0 + (keep[x] ? spread((int)x, N) : N)); });
         __syncthreads();
 #pragma unroll
         for (int e = 0; e < E; e += 2) {
