@@ -95,36 +95,6 @@ def test_laplace_infinite_keys_and_queries(dev, no_dense):
     assert float(brute.rel_err(u[0], A.sum(1), A.sum(1)).max()) <= REL
 
 
-@pytest.mark.parametrize("kernel", ["add_laplace", "add_riesz", "add_bump"])
-@pytest.mark.parametrize("N,M,C", [(1030, 1020, 6), (3111, 3111, 64), (12000, 9000, 31)])
-def test_masked_layer_columns(dev, no_dense, kernel, N, M, C):
-    # masked rows weigh 0 whatever they hold (NaN in v, large k), against the float64 layer over the kept keys
-    from qlka import layers
-    P, D = 2, 4
-    q, k, v = _data(P, D, N, M, C, "normal", N)
-    keep = np.random.default_rng(N).random((P, N)) < 0.7
-    k[np.broadcast_to(~keep[:, None], k.shape)] = 50.0
-    v[~keep] = np.nan
-    got = layers.layer_forward(kernel, *(torch.from_numpy(a).to(dev) for a in (q, k, v)),
-                               keep=torch.from_numpy(keep).to(dev)).cpu().numpy()
-    rows = np.arange(0, M, max(1, M // 50))
-    for p in range(P):
-        kk, vv, qq = k[p][:, keep[p]].astype(np.float64), v[p][keep[p]].astype(np.float64), q[p][:, rows].astype(np.float64)
-        dist = np.abs(qq[:, :, None] - kk[:, None])
-        if kernel == "add_laplace":
-            A = np.exp(-dist).sum(0)
-        elif kernel == "add_bump":
-            A = np.maximum(0, 1 - dist).sum(0)
-        else:
-            A = np.abs(qq).sum(0)[:, None] + np.abs(kk).sum(0)[None] - dist.sum(0) + layers.EPS
-        den = A.sum(1)
-        if kernel == "add_riesz":
-            den = den + (np.abs(qq).sum(0) + layers.EPS) * (M - N)
-        num = A @ vv
-        scale = np.abs(A) @ np.abs(vv)
-        np.testing.assert_array_less(np.abs(got[p][rows] * den[:, None] - num), 2e-4 * (scale + np.abs(num)) + 1e-6)
-
-
 @pytest.mark.parametrize("kind", ["normal", "ties", "runs"])
 @pytest.mark.parametrize("shape", [(1, 3, 18, 19, 1), (2, 2, 400, 369, 3), (1, 3, 700, 800, 65), (1, 2, 2100, 1990, 5),
                                    (1, 2, 5000, 5239, 2), (1, 2, 9000, 7385, 9), (1, 2, 9900, 10453, 3),
@@ -157,7 +127,7 @@ def test_column_backward(dev, no_dense, shape, kind):
     assert float(brute.rel_err(pick(sgn, iq, 1), -wq, nq).max()) <= REL
 
 
-# ---- queries and keys that are not finite, or huge: their own row only
+# ---- layers; queries and keys that are not finite, or huge: their own row only
 
 BAD = {"inf": np.inf, "-inf": -np.inf, "nan": np.nan, "-nan": -np.nan, "huge": 3e38}
 
@@ -188,6 +158,23 @@ def _assert_layer(kernel, got, q, k, v, keep, M):
     assert np.isfinite(got).all(), kernel
     err = np.abs(got * den[:, None] - num)
     np.testing.assert_array_less(err, REL * (snum + np.abs(got) * sden[:, None]) + 1e-30, err_msg=kernel)
+
+
+@pytest.mark.parametrize("kernel", ["add_laplace", "add_riesz", "add_bump"])
+@pytest.mark.parametrize("N,M,C", [(1030, 1020, 6), (3111, 3111, 64), (12000, 9000, 31)])
+def test_masked_layer_columns(dev, no_dense, kernel, N, M, C):
+    # masked rows weigh 0 whatever they hold (NaN in v, large k), against the float64 layer over the kept keys
+    from qlka import layers
+    P, D = 2, 4
+    q, k, v = _data(P, D, N, M, C, "normal", N)
+    keep = np.random.default_rng(N).random((P, N)) < 0.7
+    k[np.broadcast_to(~keep[:, None], k.shape)] = 50.0
+    v[~keep] = np.nan
+    got = layers.layer_forward(kernel, *(torch.from_numpy(a).to(dev) for a in (q, k, v)),
+                               keep=torch.from_numpy(keep).to(dev)).cpu().numpy()
+    rows = np.arange(0, M, max(1, M // 50))
+    for p in range(P):
+        _assert_layer(kernel, got[p][rows], q[p][:, rows], k[p], v[p], keep[p], M)
 
 
 @pytest.mark.parametrize("bad", sorted(BAD))

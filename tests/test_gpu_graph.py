@@ -133,3 +133,41 @@ def test_first_call_of_a_thread_captured(dev, route, pin_route):
     th.join()
     assert "error" not in result, result.get("error")
     assert result["equal"] == [True, True]
+
+
+FIRST_CALL = """
+import sys
+sys.path[:0] = [{pkg!r}]
+import torch
+from qlka import _lib
+from weighted_abs_sum import weighted_abs_sum_full
+from weighted_laplace_sum import weighted_laplace_sum
+_lib.load().qlka_set_columns(2)
+dev = torch.device("cuda", 0)
+g = torch.Generator().manual_seed(1)
+q, k = (torch.randn(2, 3, 9000, generator=g).to(dev) for _ in range(2))
+v = torch.randn(2, 9000, 4, generator=g).to(dev)
+torch.cuda.synchronize()
+graph = torch.cuda.CUDAGraph()
+with torch.no_grad(), torch.cuda.graph(graph):
+    out = [*weighted_abs_sum_full(q, k, v, backend="cuda"), *weighted_laplace_sum(q, k, v)]
+for _ in range(3):
+    for t in out:
+        t.fill_(float("nan"))
+    graph.replay()
+    torch.cuda.synchronize()
+    want = [*weighted_abs_sum_full(q, k, v, backend="cuda"), *weighted_laplace_sum(q, k, v)]
+    assert all(torch.equal(a, b) for a, b in zip(out, want))
+print("captured first")
+"""
+
+
+def test_first_call_of_a_process_captured():
+    # a process whose very first library call is captured: the columns' kernels raise their LDS limit on the way, which a
+    # capture must allow (a child process: nothing of the library may have run before)
+    import os
+    import subprocess
+    import sys
+    pkg = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "quasi-linear-kernel-attention_amd")
+    run = subprocess.run([sys.executable, "-c", FIRST_CALL.format(pkg=pkg)], capture_output=True, text=True, timeout=100)
+    assert run.returncode == 0 and "captured first" in run.stdout, run.stderr[-2000:]
