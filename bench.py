@@ -290,8 +290,9 @@ def kernel_algorithmic_bytes(name):
     feature, and write one contribution row per (p, d, query) plus one v == 1 term; the reduce reads the D rows of
     each query and writes one output row + out_u; the sort reads keys and writes sorted keys + perm; the range
     sums gather v once per key and feature; the query grouping reads q and writes values + indices. The column route:
-    one sort launch of q and k; the merge reads both with their perms and writes 6 bytes per element and the v == 1 terms;
-    the column sums read that stream once per p and v's columns, and write the output's; the finish makes them rows."""
+    one sort launch of q and k; the merge reads both with their perms and writes 6 bytes per element, 24 (Laplace) or 4 per
+    thread of 32 elements and the v == 1 terms; the column sums read that stream once per p and v's columns, and write the
+    output's; the finish makes them rows."""
     S = P * D
     walk = 4.0 * S * (2 * N + 2 * M + N * C + M * C + M)
     table = {
@@ -299,8 +300,8 @@ def kernel_algorithmic_bytes(name):
         "slab_reduce": 4.0 * P * M * (D * C + D + C + 1),
         "lds_radix_sort": 12.0 * S * (N + M), "lds_count_sort": 12.0 * S * (N + M),
         "col_merge": S * (14.0 * (N + M) + 4 * M),
-        "col_sum_laplace": 6.0 * S * (N + M) + 4.0 * P * C * (N + M),
-        "col_sum_abs": 6.0 * S * (N + M) + 4.0 * P * C * (N + M),
+        "col_sum_laplace": 6.75 * S * (N + M) + 4.0 * P * C * (N + M),
+        "col_sum_abs": 6.125 * S * (N + M) + 4.0 * P * C * (N + M),
         "col_weights": 8.0 * P * N * C, "col_finish": 8.0 * P * M * C + 4.0 * M * (S + P),
         "lap_range_sums": 4.0 * S * (2 * N + N * C), "abs_range_sums": 4.0 * S * (2 * N + N * C),
         "group_queries": 12.0 * S * M,
@@ -514,11 +515,12 @@ def main():
 
     # Roofline of the step: B_scan of both op calls / step time. The op is the unit the north-star target is set on;
     # its measured HBM traffic (sum over its kernels of FETCH_SIZE + WRITE_SIZE, copy-calibrated) is `traffic`.
-    # `kernel` is the kernel with the most GPU time in the step, on its own algorithmic bytes per launch.
+    # `kernel` is the kernel with the most GPU time in the step, on its own algorithmic bytes per launch. By columns the
+    # step moves a quarter of B_scan, and the column sums are bound by the VALU and LDS, not by HBM (`limiter`).
     achieved = 2 * bscan / (ms_per_step / 1e3) / 1e9
     dom = max(stages, key=lambda s_: stages[s_]["ms_total"])
     # the ops run their kernels once per chunk of p: a launch does (op-call bytes) / (launches per op call)
-    calls = args.steps * (1 if dom.startswith(("lap_", "abs_")) else 2)
+    calls = args.steps * (1 if dom.startswith(("lap_", "abs_")) or dom.endswith(("_laplace", "_abs")) else 2)
     per_call = kernel_algorithmic_bytes(dom)
     kbytes = per_call * calls / stages[dom]["launches"] if per_call else None
     kach = kbytes / (stages[dom]["ms_per_launch"] / 1e3) / 1e9 if kbytes else None
@@ -526,6 +528,7 @@ def main():
             "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": _op_traffic(),
             "algorithmic_bytes_per_step": 2 * bscan, "op_frac": op_frac,
+            "limiter": "VALU and LDS of the column sums; `frac` is B_scan (a walk's bytes) over the time, not HBM in use",
             "kernel": {"name": dom, "ms_per_launch": round(stages[dom]["ms_per_launch"], 4),
                        "launches_per_op_call": stages[dom]["launches"] / calls,
                        "algorithmic_bytes_per_launch": kbytes,
