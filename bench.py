@@ -280,7 +280,8 @@ def _cpu_model():
 
 STAGES = ("lds_radix_sort", "lds_count_sort", "merge_runs", "group_queries", "query_bounds", "fill_zero", "lap_range_sums",
           "lap_range_scan", "lap_range_walk", "abs_range_sums", "abs_range_scan", "abs_range_walk", "u_to_query",
-          "u_sum", "slab_reduce", "col_sort", "col_merge", "col_weights", "col_sum_laplace", "col_sum_abs", "col_finish")
+          "u_sum", "slab_reduce", "col_sort", "col_merge", "col_weights", "col_sum_laplace", "col_sum_abs",
+          "col_finish")
 DENSE_STAGES = ("direct_fwd", "direct_sign")
 
 
@@ -290,9 +291,9 @@ def kernel_algorithmic_bytes(name):
     feature, and write one contribution row per (p, d, query) plus one v == 1 term; the reduce reads the D rows of
     each query and writes one output row + out_u; the sort reads keys and writes sorted keys + perm; the range
     sums gather v once per key and feature; the query grouping reads q and writes values + indices. The column route:
-    one sort launch of q and k; the merge reads both with their perms and writes 6 bytes per element, 24 (Laplace) or 4 per
-    thread of 32 elements and the v == 1 terms; the column sums read that stream once per p and v's columns, and write the
-    output's; the finish makes them rows."""
+    one sort launch of q and k; the merge reads both with their perms and writes 6 bytes per element, 24 (Laplace) or
+    4 per thread of 32 elements and the v == 1 terms; the column sums read that stream once per p and v's columns, and
+    write the output's; the finish makes them rows."""
     S = P * D
     walk = 4.0 * S * (2 * N + 2 * M + N * C + M * C + M)
     table = {
@@ -528,7 +529,7 @@ def main():
             "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": _op_traffic(),
             "algorithmic_bytes_per_step": 2 * bscan, "op_frac": op_frac,
-            "limiter": "VALU and LDS of the column sums; `frac` is B_scan (a walk's bytes) over the time, not HBM in use",
+            "limiter": "VALU and LDS of the column sums; `frac` is B_scan (a walk's bytes) over the time, not HBM use",
             "kernel": {"name": dom, "ms_per_launch": round(stages[dom]["ms_per_launch"], 4),
                        "launches_per_op_call": stages[dom]["launches"] / calls,
                        "algorithmic_bytes_per_launch": kbytes,

@@ -43,9 +43,9 @@ int qlka_version(void);
 int qlka_set_direct_max(int n);
 /*
  * Which sorted route a call takes, for tests and measurements: segments of N + M <= 32768 elements can run column by
- * column, all others walk. AUTO (the default) takes the columns where they were measured faster, NEVER walks everything,
- * ALWAYS takes the columns wherever they apply. Results agree to fp32 rounding. What the dense evaluation takes stays
- * there (qlka_set_direct_max). Process-wide; returns the previous mode (or -QLKA_EINVAL for another one).
+ * column, all others walk. AUTO (the default) takes the columns where they were measured faster, NEVER walks
+ * everything, ALWAYS takes the columns wherever they apply. Results agree to fp32 rounding. What the dense evaluation
+ * takes stays there (qlka_set_direct_max). Process-wide; returns the previous mode (or -QLKA_EINVAL for another one).
  */
 #define QLKA_COLUMNS_AUTO   0
 #define QLKA_COLUMNS_NEVER  1
@@ -129,8 +129,9 @@ int qlka_abs_bwd(const float* q, const float* k, const float* v, const float* g_
  * dense kernels, or, at C <= 64 with C % 4 == 0, walks once over the merged sorted keys and queries): the forward
  * also leaves there the range states and query bounds of its walk over the sorted keys, which the backward's grad_q
  * walk would compute again (the same range sums, scan and bounds); it sets *kept = 3 when it wrote them (its own walk
- * ran; a forward on the dense kernels or by columns keeps only the sorts). Passing them to qlka_abs_bwd_sorted after *kept = 3
- * skips one range-sum pass, one scan and one bound search per chunk of the backward, with bit-identical gradients.
+ * ran; a forward on the dense kernels or by columns keeps only the sorts). Passing them to qlka_abs_bwd_sorted after
+ * *kept = 3 skips one range-sum pass, one scan and one bound search per chunk of the backward, with bit-identical
+ * gradients.
  */
 int qlka_abs_bwd_walks(int P, int N, int M);
 size_t qlka_abs_keep_state_bytes(int P, int D, int N, int M, int C);

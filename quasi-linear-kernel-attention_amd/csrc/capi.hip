@@ -457,28 +457,28 @@ int run_pipeline(int P, const Plan& pl, void* ws, size_t copy, hipStream_t st, P
     return w == hipSuccess ? QLKA_OK : hip_status((int)w, "join");
 }
 
-// ---- the forward sums column by column (col.hip): sort k and q, merge them into the stream the columns walk, the column
-// sums, and the finish that turns columns into rows (with the v == 1 terms and, for a layer, its epilogue). Segments of
-// N + M <= COL_MAX elements take it whatever the dense cutoff leaves; longer ones walk ranges of keys into a slab of
-// contribution rows. Measured against that walk on MI355X: see col.hip.
-// The chunks run in order on the caller's stream: the sums keep every CU's LDS, so nothing would run beside them. Its
-// workspace is smaller than the walk's but for many more keys than queries, where the *_ws_bytes queries return the
-// larger of the two.
+// ---- the forward sums column by column (col.hip): sort k and q, merge them into the stream the columns walk, the
+// column sums, and the finish that turns columns into rows (with the v == 1 terms and, for a layer, its epilogue).
+// Segments of N + M <= COL_MAX elements can take it, whatever the dense cutoff leaves; longer ones walk ranges of keys
+// into a slab of contribution rows. The chunks run in order on the caller's stream: the sums keep every CU's LDS, so
+// nothing would run beside them. Its workspace is smaller than the walk's but for many more keys than queries, where
+// the *_ws_bytes queries return the larger of the two.
 //
-// Which route a call takes is decided by estimates of both routes' times (us), linear in what each does and fitted (relative
-// least squares) to both routes' times of 840 calls on MI355X: P D (N + M) from 2^12 to 2^25, D from 1 to 300, N / M from 1/32
-// to 32, C from 1 to 128. They are within 8 to 18% of the times on average, and the columns are taken where theirs is below
-// the walk's by a margin. Over those calls, against the walk: Laplace 1.39 x, abs 1.45 x, add_bump 1.83 x, backward 1.37 x, sgn
-// 1.08 x on average, 2.2%, 2.4%, 2.3%, 3.2% and 8% off the faster route; 1 to 1.5% of them are more than 5% slower than
-// their walk, at most by 30%. Fixed limits on elements and segments instead took 2.2 x the walk's time with
-// few features per p (256 x 1 x 4000 x 4000 x 64 abs: 572 against 310 us; the columns are loaded for one feature) or many more
-// keys than queries (add_bump 12 x 64 x 20000 x 600 x 64: 2.73 against 1.54 ms; its three streams hold the keys three times),
-// and left small calls to the walk (2 x 64 x 1225 x 703 x 4 Laplace: 106 against 47 us). qlka_set_columns overrides it.
+// Which route a call takes is decided by estimates of both routes' times (us), linear in what each does and fitted
+// (relative least squares) to both routes' times of 840 calls on MI355X: P D (N + M) from 2^12 to 2^25, D from 1 to
+// 300, N / M from 1/32 to 32, C from 1 to 128. They are within 8 to 18% of the times on average, and the columns are
+// taken where theirs is below the walk's by a margin. Over those calls, against the walk: Laplace 1.39 x, abs 1.45 x,
+// add_bump 1.83 x, backward 1.37 x, sgn 1.08 x on average, 2.2%, 2.4%, 2.3%, 3.2% and 8% off the faster route; 1 to
+// 1.5% of them are more than 5% slower than their walk, at most by 30%. Fixed limits on elements and segments instead
+// took 2.2 x the walk's time with few features per p (256 x 1 x 4000 x 4000 x 64 abs: 572 against 310 us; the columns
+// are loaded for one feature) or many more keys than queries (add_bump 12 x 64 x 20000 x 600 x 64: 2.73 against 1.54
+// ms; its three streams hold the keys three times), and left small calls to the walk (2 x 64 x 1225 x 703 x 4 Laplace:
+// 106 against 47 us). qlka_set_columns overrides it.
 enum ColOp : int { COL_OP_LAPLACE, COL_OP_ABS, COL_OP_BUMP, COL_OP_BWD, COL_OP_SGN };
 
-// The walk: its launches; per 1000 segment keys and queries (sorts, bounds, walk); per 10^6 words of gathered and written
-// rows, more of them with two channel slots a lane, unaligned rows and widths that are no power of two; keys past one LDS
-// sort; the length of its longest chain per segments beyond the chip's workgroups.
+// The walk: its launches; per 1000 segment keys and queries (sorts, bounds, walk); per 10^6 words of gathered and
+// written rows, more of them with two channel slots a lane, unaligned rows and widths that are no power of two; keys
+// past one LDS sort; the length of its longest chain per segments beyond the chip's workgroups.
 struct WalkCost {
     double launches, key, query, key_row, query_row, two, long_key, unaligned, unaligned_two, uneven, chain;
 };
@@ -493,15 +493,16 @@ double walk_us(ColOp op, int P, int D, int N, int M, int C) {
     const WalkCost& w = WALK_COST[op];
     const double S = (double)P * D, row = S * std::max(C, 8) * 1e-6, rows = row * ((double)N + M);
     return w.launches + S * 1e-3 * (w.key * N + w.query * M + (N > LDS_SORT_MAX ? w.long_key * N : 0.)) +
-           row * (w.key_row * N + w.query_row * M) + (C > 64 ? w.two * rows : 0.) + (C % 4 ? (C > 64 ? w.unaligned_two : w.unaligned) * rows : 0.) +
+           row * (w.key_row * N + w.query_row * M) + (C > 64 ? w.two * rows : 0.) +
+           (C % 4 ? (C > 64 ? w.unaligned_two : w.unaligned) * rows : 0.) +
            ((C & (C - 1)) ? w.uneven * rows : 0.) + w.chain * std::ceil(S / 512) * std::max(N, M) * 1e-3;
 }
 
-// The columns: their launches; the sorts and merges, one workgroup per segment, by the waves a SIMD runs and the elements of
-// each thread, and per 1000 elements; the transposes per 1000 words; the sums, by waves and elements as the sorts and by the
-// features a workgroup walks (load and store of its columns: another 2, or 6 with a CU to itself); the finish, one thread
-// adding the shares of C / 4 channels. Backward: the dots, by rounds over the chip and by waves, elements and channel
-// groups, and per 10^6 words that they read.
+// The columns: their launches; the sorts and merges, one workgroup per segment, by the waves a SIMD runs and the
+// elements of each thread, and per 1000 elements; the transposes per 1000 words; the sums, by waves and elements as the
+// sorts and by the features a workgroup walks (load and store of its columns: another 2, or 6 with a CU to itself); the
+// finish, one thread adding the shares of C / 4 channels. Backward: the dots, by rounds over the chip and by waves,
+// elements and channel groups, and per 10^6 words that they read.
 struct ColCost { double launches, sort, element, word, sum, finish, dot_round, dot, dot_word, margin, slack; };
 constexpr ColCost COL_COST[] = {
     {28, 0.48, 0.0068, 0.0023, 0.036, 0.073, 0, 0, 0, 0.95, 8},
@@ -518,8 +519,9 @@ double col_us(ColOp op, int P, int D, int N, int M, int C) {
     const double S = (double)P * D, n = (double)N + M, waves = pl.T / 256. * pl.E, groups = (C + pl.CH - 1) / pl.CH;
     const double sums = std::ceil(P * groups * DS / CUS) * waves * ((D * sets + DS - 1) / DS + (pl.CH == 1 ? 6 : 2));
     const double rows = op == COL_OP_BWD ? N : M, dots = (C + 2) / pl.CH;
-    return w.launches + w.sort * std::ceil(S / CUS) * waves + S * n * sets * 1e-3 * w.element + P * n * C * 1e-3 * w.word +
-           w.sum * sums + w.finish * std::ceil(P * std::ceil(rows / 64) / (4 * CUS)) * C * DS +
+    return w.launches + w.sort * std::ceil(S / CUS) * waves + S * n * sets * 1e-3 * w.element +
+           P * n * C * 1e-3 * w.word + w.sum * sums +
+           w.finish * std::ceil(P * std::ceil(rows / 64) / (4 * CUS)) * C * DS +
            w.dot_round * std::ceil(S / (CUS * pl.per_cu)) * pl.E * dots + w.dot * std::ceil(S / CUS) * waves * dots +
            w.dot_word * S * n * C * 1e-6;
 }
@@ -560,8 +562,8 @@ size_t col_part(int kind, const ColPlan& pl, int P, int D, int N, int M, int C, 
 
 constexpr int COL_PARTS = 10;
 
-// Workspace of a chunk of P p, the columns sized for the most feature shares: their number depends on the whole call's P,
-// and neither the sizes nor (the plan being the whole call's) the results may depend on the chunking.
+// Workspace of a chunk of P p, the columns sized for the most feature shares: their number depends on the whole call's
+// P, and neither the sizes nor (the plan being the whole call's) the results may depend on the chunking.
 size_t col_bytes(int kind, int P, int D, int N, int M, int C, int sets = 1) {
     if (!col_applies(D * sets, N, M)) return 0;
     ColPlan pl = col_plan(kind, 1, D, N, M, C);
@@ -589,11 +591,12 @@ ColWs col_carve(int kind, ColPlan pl, void* ws, int P, int D, int N, int M, int 
 }
 
 // q and k (null: always by sort) go to the stream in one kernel where col_sort_applies; else
-// sort(p0, np, w, stream) leaves the sorted k and q in w.s, which are merged. finish(p0, np, w, plan, stream) reads w.cols and w.u (null
-// without want_u). extra(np): bytes of the caller's own after the columns (w.extra).
+// sort(p0, np, w, stream) leaves the sorted k and q in w.s, which are merged. finish(p0, np, w, plan, stream) reads
+// w.cols and w.u (null without want_u). extra(np): bytes of the caller's own after the columns (w.extra).
 template <class Extra, class Sort, class Finish>
-int run_columns(int kind, int sets, const float* q, const float* k, const float* v, const uint8_t* keep, bool want_u, int P, int D, int N, int M, int C, void* ws,
-                size_t given, hipStream_t st, Extra extra, Sort sort, Finish finish) {
+int run_columns(int kind, int sets, const float* q, const float* k, const float* v, const uint8_t* keep, bool want_u,
+                int P, int D, int N, int M, int C, void* ws, size_t given, hipStream_t st, Extra extra, Sort sort,
+                Finish finish) {
     ColPlan pl = col_plan(kind, P, D * sets, N, M, C);
     pl.DS = std::min(pl.DS, std::min(D, COL_SHARES));        // as many as the workspace is sized for
     auto bytes = [&](int pc) { return col_bytes(kind, pc, D, N, M, C, sets) + extra(pc); };
@@ -607,7 +610,8 @@ int run_columns(int kind, int sets, const float* q, const float* k, const float*
         if (int e = col_weights_launch(pl, v + p * N * C, kc, false, nullptr, w.wt, w.bad, np * M, np, N, C, st))
             return hip_status(e, "weight columns");
         if (q && sets == 1 && col_sort_applies(pl)) {
-            if (int e = col_sort_launch(kind, pl, q + p * D * M, k + p * D * N, kc, w.str, w.u, w.bad, np * D, D, N, M, st))
+            if (int e = col_sort_launch(kind, pl, q + p * D * M, k + p * D * N, kc, w.str, w.u, w.bad, np * D, D, N, M,
+                                        st))
                 return hip_status(e, "sort of q and k");
         } else {
             if (int e = sort(p0, np, w, st)) return e;
@@ -624,10 +628,10 @@ int run_columns(int kind, int sets, const float* q, const float* k, const float*
 
 inline size_t no_extra(int) { return 0; }
 
-// The abs backward by columns (col.hip), and the sgn sum, its grad_q negated: the merge of the sorted k and q, the columns
-// of g_w and v (with g_u: one more channel, g_u against ones), grad_q and grad_k per segment, grad_v by the forward's
-// column sums with the roles of q and k exchanged. Workspace of a chunk of P p: as the forward's, the columns of N rows,
-// and those of g_w.
+// The abs backward by columns (col.hip), and the sgn sum, its grad_q negated: the merge of the sorted k and q, the
+// columns of g_w and v (with g_u: one more channel, g_u against ones), grad_q and grad_k per segment, grad_v by the
+// forward's column sums with the roles of q and k exchanged. Workspace of a chunk of P p: as the forward's, the columns
+// of N rows, and those of g_w.
 size_t col_bwd_part(const ColPlan& pl, int P, int D, int N, int M, int C, int i) {
     const size_t S = (size_t)P * D, C1 = (size_t)(C + 1 + pl.CH) / pl.CH * pl.CH;      // C + 1 channels in whole groups
     switch (i) {
@@ -673,24 +677,26 @@ int run_bwd_columns(const float* v, const float* g_w, const float* g_u, float sc
         float* bad = grad_v ? (float*)part[9] : nullptr;
         const size_t p = (size_t)p0;
         const int CW = (C + (g_u ? 1 : 0) + pl.CH - 1) / pl.CH;
-        if (int e = col_weights_launch(pl, v + p * N * C, nullptr, g_u != nullptr, nullptr, vt, bad, bad ? np * N : 0, np,
-                                       N, C, st))
+        if (int e = col_weights_launch(pl, v + p * N * C, nullptr, g_u != nullptr, nullptr, vt, bad, bad ? np * N : 0,
+                                       np, N, C, st))
             return hip_status(e, "value columns");
         if (int e = col_weights_launch(pl, g_w + p * M * C, nullptr, g_u != nullptr, g_u ? g_u + p * M : nullptr, gt,
                                        nullptr, 0, np, M, C, st))
             return hip_status(e, "gradient columns");
         if (int e = sorts(p0, np, w, st)) return e;
-        if (int e = col_merge_launch(0, pl, w.qs, w.qp, w.ks, w.kp, nullptr, str, nullptr, bad, np * D, D, N, M, true, 1,
-                                     st))
+        if (int e = col_merge_launch(0, pl, w.qs, w.qp, w.ks, w.kp, nullptr, str, nullptr, bad, np * D, D, N, M, true,
+                                     1, st))
             return hip_status(e, "merge of q and k");
         if (grad_v) {
-            if (int e = col_grad_v_launch(pl, str, gt, CW, cols, np, D, N, M, C, st)) return hip_status(e, "grad_v columns");
-            if (int e = col_finish_launch(0, -1, false, pl, cols, nullptr, bad, grad_v + p * N * C, nullptr, ReduceEpilogue{}, np, D,
-                                          N, C, st))
+            if (int e = col_grad_v_launch(pl, str, gt, CW, cols, np, D, N, M, C, st))
+                return hip_status(e, "grad_v columns");
+            if (int e = col_finish_launch(0, -1, false, pl, cols, nullptr, bad, grad_v + p * N * C, nullptr,
+                                          ReduceEpilogue{}, np, D, N, C, st))
                 return hip_status(e, "columns to rows");
         }
-        return hip_status(col_dot_launch(pl, str, gt, vt, CW, scale, grad_q + p * D * M,
-                                         grad_k ? grad_k + p * D * N : nullptr, np * D, D, N, M, st), "column dots"); });
+        float* gk = grad_k ? grad_k + p * D * N : nullptr;
+        return hip_status(col_dot_launch(pl, str, gt, vt, CW, scale, grad_q + p * D * M, gk, np * D, D, N, M, st),
+                          "column dots"); });
 }
 
 }  // namespace
@@ -751,8 +757,9 @@ int qlka_laplace_fwd(const float* q, const float* k, const float* v, float* out_
                 return sort_both(q + p * D * M, k + p * D * N, w.s, np * D, N, M, s); },
             [&](int p0, int np, ColWs& w, const ColPlan& cp, hipStream_t s) {
                 const size_t p = (size_t)p0;
-                return hip_status(col_finish_launch(1, -1, false, cp, w.cols, w.u, w.bad, out_w + p * M * C, out_u + p * M,
-                                                    ReduceEpilogue{}, np, D, M, C, s), "columns to rows"); });
+                return hip_status(col_finish_launch(1, -1, false, cp, w.cols, w.u, w.bad, out_w + p * M * C,
+                                                    out_u + p * M, ReduceEpilogue{}, np, D, M, C, s),
+                                  "columns to rows"); });
     // per chunk: sort k and group q; range passes and walk; reduce
     auto prep = [&](int p0, int np, void* buf, hipStream_t s) {
         SortedWs w = carve(buf, laplace_spec(np, D, N, M, C));
@@ -873,10 +880,11 @@ int abs_fwd_impl(const float* q, const float* k, const float* v, float* out_w, f
     auto b1 = [&](int pc) { return abs_fwd_ws(pc, D, N, M, C); };
     const Plan pl = plan_chunks(P, ws_bytes_given, pipelined(P, D, M), b1);
     if (int e = check_ws(ws, ws_bytes_given, plan_bytes(pl, b1))) return e;
-    // By columns no range states are formed, so only the sorts are kept, where the backward is expected to need no states;
-    // should it walk all the same (the routes can be pinned in between), it forms its own.
+    // By columns no range states are formed, so only the sorts are kept, where the backward is expected to need no
+    // states; should it walk all the same (the routes can be pinned in between), it forms its own.
     if (col_fwd(COL_OP_ABS, P, D, N, M, C) && (!keep_states || col_bwd(P, D, N, M, C))) {
-        const int e = run_columns(0, 1, keep_sorts ? nullptr : q, k, v, nullptr, out_u != nullptr, P, D, N, M, C, ws, ws_bytes_given, st, no_extra,
+        const int e = run_columns(0, 1, keep_sorts ? nullptr : q, k, v, nullptr, out_u != nullptr, P, D, N, M, C, ws,
+                                  ws_bytes_given, st, no_extra,
             [&](int p0, int np, ColWs& w, hipStream_t s) {
                 const size_t p = (size_t)p0;
                 if (keep_sorts) {
@@ -1097,10 +1105,10 @@ size_t qlka_abs_bwd_ws_bytes(int P, int D, int N, int M, int C) {
 }  // extern "C"
 
 namespace {
-// The merged backward (mbw.hip), per chunk: the sorts (unless the forward kept them) and the merge of the sorted q and k
-// with its range summaries (prep); the scans (early, before the wait for the previous chunk's reduce); the walk (main);
-// the grad_v reduce (back). Copy j % 2's slab region, which holds the summaries, is free at prep of chunk j: main of
-// chunk j - 1 waited for the reduce of chunk j - 2.
+// The merged backward (mbw.hip), per chunk: the sorts (unless the forward kept them) and the merge of the sorted q and
+// k with its range summaries (prep); the scans (early, before the wait for the previous chunk's reduce); the walk
+// (main); the grad_v reduce (back). Copy j % 2's slab region, which holds the summaries, is free at prep of chunk j:
+// main of chunk j - 1 waited for the reduce of chunk j - 2.
 int abs_bwd_mbw(const float* q, const float* k, const float* v, const float* g_w, const float* g_u, float* grad_q,
                 float* grad_k, float* grad_v, int P, int D, int N, int M, int C, const Presorted* pre, void* ws,
                 size_t ws_bytes_given, hipStream_t st) {
@@ -1504,16 +1512,16 @@ static int layer_columns(int kind, const float* q, const float* k, const float* 
             const size_t p = (size_t)p0;
             void* pre = w.extra + align256((size_t)np * M * 4);
             if (riesz)
-                if (int e = riesz_prefix(k + p * D * N, v + p * N * C, keep ? keep + p * N : nullptr, pre, np, D, N, C, s))
+                if (int e = riesz_prefix(k + p * D * N, v + p * N * C, keep ? keep + p * N : nullptr, pre, np, D, N, C,
+                                         s))
                     return hip_status(e, "riesz prefixes");
             ReduceEpilogue ep{};
             if (int e = layer_epilogue_params(kind, keep != nullptr, q + p * D * M, n_pad ? n_pad + p : nullptr, pre,
                                               (float*)w.extra, out + p * M * C, np, D, M, C, &ep, s))
                 return hip_status(e, "layer query terms");
-            return hip_status(col_finish_launch(laplace ? 1 : 0, kind, keep != nullptr, cp, w.cols, w.u, w.bad, nullptr, nullptr, ep,
-                                                np,
-                                                D * sets, M, C,
-                                                s), "columns to rows"); });
+            const int e = col_finish_launch(laplace ? 1 : 0, kind, keep != nullptr, cp, w.cols, w.u, w.bad, nullptr,
+                                            nullptr, ep, np, D * sets, M, C, s);
+            return hip_status(e, "columns to rows"); });
 }
 
 static int layer_fwd(int kind, const float* q, const float* k, const float* v, const float* n_pad,

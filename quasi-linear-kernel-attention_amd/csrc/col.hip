@@ -10,23 +10,23 @@
 // sum happens in LDS, so no per-feature contribution ever goes to memory, which is what a walk with one row per (p, d,
 // query) has to write and a reduce to read back (6.6 of 10.4 GB per call at P = 12, D = 64, N = M = 16384, C = 64).
 //
-// The merged sequence of a segment does not depend on the channel: col_merge writes it once (6 bytes per element) and the
-// C / CH workgroups of a p read it, neighbours on one XCD at about the same time, so from its L2.
-//   val[s][E/4][T][4]   abs: the value less the thread's anchor, the end of its elements that lies towards the segment's
-//                       median key; Laplace: e^-distance to the previous element
-//   tag[s][E/4][T][4]   16-bit word index: query m at spread(m), key n at K0 + spread(n), padding at K0 + N (K0 = M, or M
-//                       rounded up)
+// The merged sequence of a segment does not depend on the channel: col_merge writes it once (6 bytes per element) and
+// the C / CH workgroups of a p read it, neighbours on one XCD at about the same time, so from its L2.
+//   val[s][E/4][T][4]   abs: the value less the thread's anchor, its value nearest the segment's median key; Laplace:
+//                       e^-distance to the previous element
+//   tag[s][E/4][T][4]   16-bit word index: query m at spread(m), key n at K0 + spread(n), padding at K0 + N (K0 = M,
+//                       or M rounded up)
 //   xe[s][T]            abs: each thread's anchor less the median key; Laplace: its Decays
 //   eq[s][T]            (abs backward) bit e: element e of the thread has the value of the element before it
 // With 4 elements per 16-byte (8-byte) load, a wave's loads are contiguous.
 //
-// What bounds col_sum: per element and channel one LDS read and, for a query, one masked write at random addresses (about
-// 8 and 6 cycles a wave, bank conflicts of 64 random words), beside some 10 (abs) or 15 (Laplace) vector instructions; at
-// N = M = 16384, one channel per workgroup, that is 0.6 ms of LDS and 0.5 ms of VALU for the measured 0.81 ms (abs,
-// P = 12, D = C = 64; Laplace 0.91). LDS float atomics in place of the read and the write ran at 100 cycles a wave
-// (4.3 ms). Whole calls against the walk: abs 1.70 -> 1.36 ms, Laplace 1.69 -> 1.54 ms at that size, Laplace 0.81 ->
-// 0.52 ms at N = M = 8192, add_riesz 0.97 -> 0.55 ms at 24 x 3111, add_bump 8.9 -> 5.5 ms at 48 x 8192, abs forward +
-// backward 4.76 -> 3.65 ms at 12 x 16384.
+// What bounds col_sum: per element and channel one LDS read and, for a query, one masked write at random addresses
+// (about 8 and 6 cycles a wave, bank conflicts of 64 random words), beside some 10 (abs) or 15 (Laplace) vector
+// instructions. At N = M = 16384, one channel per workgroup, P = 12, D = C = 64, a kernel trace has 0.90 ms (abs; VALU
+// 59%, LDS 61% of it by the counters) and 1.01 ms (Laplace; 76%, 55%). LDS float atomics in place of the read and the
+// write ran at 100 cycles a wave (4.3 ms). Whole calls against the walk: abs 1.70 -> 1.35 ms, Laplace 1.69 -> 1.44 ms
+// at that size, Laplace 0.81 -> 0.54 ms at N = M = 8192, add_riesz 0.97 -> 0.55 ms at 24 x 3111, add_bump 8.9 -> 5.4 ms
+// at 48 x 8192, abs forward + backward 4.76 -> 3.61 ms at 12 x 16384.
 #include <algorithm>
 #include <cfloat>
 #include <utility>
@@ -53,9 +53,9 @@ __device__ __forceinline__ float dpp(float old, float x) {
 }
 constexpr int WAVE_SHR1 = 0x138, WAVE_SHL1 = 0x130;
 
-// Steps of the scans as one DPP instruction each (the compiler's form moves the other lane's value first): x += y of the
-// lane the pattern names, x = a y + x and a *= that lane's a; lanes without a source keep x. A DPP read needs two wait
-// states after the register's write (as a lane read does after the last step: settle), which the compiler does not
+// Steps of the scans as one DPP instruction each (the compiler's form moves the other lane's value first): x += y of
+// the lane the pattern names, x = a y + x and a *= that lane's a; lanes without a source keep x. A DPP read needs two
+// wait states after the register's write (as a lane read does after the last step: settle), which the compiler does not
 // know of around an asm statement.
 #define QLKA_DPP_STEP(NAME, PATTERN)                                                                                  \
     struct NAME {                                                                                                     \
@@ -117,15 +117,17 @@ __device__ __forceinline__ void affine_step(float& a, float (&b)[CH]) {
     for (int c = 0; c < CH; ++c) Step::fma(b[c], a);
     Step::mul(a);
 }
-// lane_id() counted again, for a loop whose registers cannot hold it (spilled, its reload waits for every load in flight)
+// lane_id() counted again, for a loop whose registers cannot hold it (spilled, its reload waits for every load in
+// flight)
 __device__ __forceinline__ int lane_now() {
     int r;
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(r));
     return r;
 }
 
-// The Laplace decays of a thread and around it in its wave, each formed from its own distance: a scan that multiplies the
-// threads' decays up doubles their errors at every step, to thousands of times a rounding that repeats (a grid of keys).
+// The Laplace decays of a thread and around it in its wave, each formed from its own distance: a scan that multiplies
+// the threads' decays up doubles their errors at every step, to thousands of times a rounding that repeats (a grid of
+// keys).
 struct Decays {
     float own;                       // over the thread
     float row, half;                 // from the start of its row of 16 lanes, and of lane 32, to the thread's end
@@ -201,9 +203,9 @@ __device__ __forceinline__ void lds_read(float (&x)[CH], uint32_t byte) {
         x[1] = v.y;
     }
 }
-// Store in the lanes of `mask` only, without a branch around it (the compiler's form of a masked store jumps over it when
-// no lane stores, which costs more than the store: half of a wave's elements are queries). Every lane of the wave is
-// active here. The compiler does not count this store: a wait for lgkmcnt(0) must come before the next barrier.
+// Store in the lanes of `mask` only, without a branch around it (the compiler's form of a masked store jumps over it
+// when no lane stores, which costs more than the store: half of a wave's elements are queries). Every lane of the wave
+// is active here. The compiler does not count this store: a wait for lgkmcnt(0) must come before the next barrier.
 template <int CH>
 __device__ __forceinline__ void lds_write_masked(const float (&x)[CH], uint32_t byte, uint64_t mask) {
     if constexpr (CH == 1) {
@@ -217,8 +219,8 @@ __device__ __forceinline__ void lds_write_masked(const float (&x)[CH], uint32_t 
                      : "memory");
     }
 }
-// Byte address of the low / high 16-bit word index of a tag pair, words of B bytes (one instruction each; the compiler takes
-// two for the low half).
+// Byte address of the low / high 16-bit word index of a tag pair, words of B bytes (one instruction each; the compiler
+// takes two for the low half).
 template <int B>
 __device__ __forceinline__ uint32_t tag_addr(uint32_t pair, bool high) {
     uint32_t r;
@@ -231,16 +233,16 @@ __device__ __forceinline__ uint32_t tag_addr(uint32_t pair, bool high) {
             : "=v"(r) : "v"(sh), "v"(pair));
     return r;
 }
-// b where the lane's bit of mask is set, else a; the empty asm keeps it one select (the compiler otherwise branches around
-// the arithmetic that follows)
+// b where the lane's bit of mask is set, else a; the empty asm keeps it one select (the compiler otherwise branches
+// around the arithmetic that follows)
 __device__ __forceinline__ float pick(float a, float b, uint64_t mask) {
     float r = __builtin_amdgcn_inverse_ballot_w64(mask) ? b : a;
     asm("" : "+v"(r));
     return r;
 }
 __device__ __forceinline__ float unless(float a, uint64_t mask) { return pick(a, 0.f, mask); }
-// All ones where bit e of x is set, else 0; and b where m is all ones, a where it is 0. As asm, or the compiler turns the
-// bits of a loop into one lane mask each, more than there are scalar registers.
+// All ones where bit e of x is set, else 0; and b where m is all ones, a where it is 0. As asm, or the compiler turns
+// the bits of a loop into one lane mask each, more than there are scalar registers.
 template <int e>
 __device__ __forceinline__ uint32_t bit_mask(uint32_t x) {
     uint32_t r;
@@ -254,19 +256,21 @@ __device__ __forceinline__ float bit_pick(float a, float b, uint32_t m) {
 }
 // f(integral_constant<int, 0>) ... f(integral_constant<int, E - 1>)
 template <class F, int... I>
-__device__ __forceinline__ void each_of(F f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+__device__ __forceinline__ void each_index(F f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
 template <int E, class F>
-__device__ __forceinline__ void each(F f) { each_of(f, std::make_integer_sequence<int, E>{}); }
+__device__ __forceinline__ void each(F f) { each_index(f, std::make_integer_sequence<int, E>{}); }
 
 // ---------------------------------------------------------------------------------------------------------------
 // col_merge: one workgroup per segment
 // ---------------------------------------------------------------------------------------------------------------
-// e^-x, x >= 0, for a chain of products. Below 1/2 as 1 - h with h = 1 - e^-x by its Taylor series (9 terms: to 2^-26 of h),
-// so that it rounds to nearest: near 1 the library's expf is off to one side by up to an ulp, which thousands of factors add
-// up. And `rest`, what rounding the factors before has left to be taken off, is taken off here and left anew: where the
-// distances repeat (a grid) or are all below half an ulp, factors rounded one by one err to one side as well.
-// With this and Decays, Laplace at N = M = 8192, relative 2-norm against 64 bits, a grid over +-3 and uniform keys in +-2e-5:
-// 5.1e-6 and 3.5e-6 -> 3.9e-7 and 1.5e-7 (walks: 5.7e-7 and 2.1e-7); N(0, 1) 1.4e-7 -> 7.6e-8 (2.9e-7).
+// e^-x, x >= 0, for a chain of products. Below 1/2 as 1 - h with h = 1 - e^-x by its Taylor series (9 terms: to 2^-26
+// of h), so that it rounds to nearest: near 1 the library's expf is off to one side by up to an ulp, which thousands of
+// factors add up. And `rest`, what rounding the factors before has left to be taken off, is taken off here and left
+// anew: where the distances repeat (a grid) or are all below half an ulp, factors rounded one by one err to one side as
+// well. With this and Decays, Laplace at N = M = 8192, relative 2-norm against 64 bits, a grid over +-3 and uniform
+// keys in +-2e-5: 5.1e-6 and 3.5e-6 -> 3.9e-7 and 1.5e-7 (walks: 5.7e-7 and 2.1e-7); N(0, 1) 1.4e-7 -> 7.6e-8 (2.9e-7).
 __device__ __forceinline__ float decay(float x, float& rest) {
     if (x >= 0.5f) return expf(-x);
     float h = fmaf(x, -1.f / 362880.f, 1.f / 40320.f);
@@ -288,26 +292,29 @@ struct ColMergeArgs {
     const uint8_t* keep;             // (P, N) key mask or null: masked keys become padding
     float* val; uint16_t* tag; float* xe; float* xe2; uint32_t* eq;  // eq: null unless wanted; xe2: Laplace only
     float* u;                        // (S, M) v == 1 terms in the order of the words, or null
-    float* bad;                      // (P, M), bwd: (P, N), in the order of the words: NaN at the rows whose own value makes them NaN, 0 else; or null
+    float* bad;                      // (P, M), bwd: (P, N), in the order of the words: NaN at the rows whose own value
+                                     // makes them NaN, 0 else; or null
     int D, N, M, K0;
-    int sets;                        // 1, or 3: streams of q, q + 1 and q - 1 per segment (add_bump), their v == 1 terms weighted
+    int sets;                        // 1, or 3: streams of q, q + 1 and q - 1 per segment (add_bump), their v == 1
+                                     // terms weighted
 };
 
-// add_bump: max(0, 1 - |x|) = (|x + 1| + |x - 1|) / 2 - |x|, one feature's three abs sums after one another. The same sorted
-// order serves all three: adding a constant in fp32 is monotone.
+// add_bump: max(0, 1 - |x|) = (|x + 1| + |x - 1|) / 2 - |x|, one feature's three abs sums after one another. The same
+// sorted order serves all three: adding a constant in fp32 is monotone.
 __device__ __forceinline__ float set_shift(int set) { return set == 0 ? 0.f : set == 1 ? 1.f : -1.f; }
 __device__ __forceinline__ float set_weight(int sets, int set) { return sets == 1 ? 1.f : set == 0 ? -1.f : 0.5f; }
 
-// A finite stand-in for an element that carries no weight: x, or the largest float on x's side. Its value enters the shared
-// sums as value x 0, which an infinity or a NaN would turn into NaN for every row of the p.
+// A finite stand-in for an element that carries no weight: x, or the largest float on x's side. Its value enters the
+// shared sums as value x 0, which an infinity or a NaN would turn into NaN for every row of the p.
 __device__ __forceinline__ float bounded(float x) { return fabsf(x) <= FLT_MAX ? x : copysignf(FLT_MAX, x); }
 // a NaN as the infinity on its side
 __device__ __forceinline__ float no_nan(float x) { return x == x ? x : copysignf(__int_as_float(0x7f800000), x); }
-// Values with which all below is finite without looking at each (abs: their differences are; Laplace: not a NaN); a segment
-// with another one is `rare`
+// Values with which all below is finite without looking at each (abs: their differences are; Laplace: not a NaN); a
+// segment with another one is `rare`
 template <int KIND>
 __device__ __forceinline__ bool ordinary(float x) { return KIND == COL_ABS ? fabsf(x) <= 1e37f : x == x; }
-// true in the whole workgroup if x is in any of its threads; flags: W words of LDS, read before they may be written again
+// true in the whole workgroup if x is in any of its threads; flags: W words of LDS, read before they may be written
+// again
 template <int W>
 __device__ __forceinline__ bool any_of(bool x, uint32_t* flags) {
     const uint64_t b = __ballot(x);
@@ -316,10 +323,10 @@ __device__ __forceinline__ bool any_of(bool x, uint32_t* flags) {
     return __ballot(flags[lane_id() % W] != 0) != 0;
 }
 
-// The word of row i among the L of a side (and the row of word i): within each whole block of 64, shuffled by the block's
-// number. Where values tie, the sorts leave rows in order, and threads of E consecutive elements each would read words E
-// apart, 16 and more of them from one bank (12 x 64 x 16384, half the keys 0 as by a
-// mask multiplied in: abs 1.93 -> 1.35 ms, Laplace 2.11 -> 1.44, training 5.88 -> 3.81; walks 1.72, 1.71, 4.75).
+// The word of row i among the L of a side (and the row of word i): within each whole block of 64, shuffled by the
+// block's number. Where values tie, the sorts leave rows in order, and threads of E consecutive elements each would
+// read words E apart, 16 and more of them from one bank (12 x 64 x 16384, half the keys 0 as by a mask multiplied in:
+// abs 1.93 -> 1.35 ms, Laplace 2.11 -> 1.44, training 5.88 -> 3.81; walks 1.72, 1.71, 4.75).
 __device__ __forceinline__ int spread(int i, int L) { return i < (L & ~63) ? i ^ ((i >> 6) & 63) : i; }
 
 // 16-bit word indices, two in a register
@@ -333,12 +340,15 @@ struct Halves {
     }
 };
 
-__device__ __forceinline__ bool is_key(int word, const ColMergeArgs& A) { return (uint32_t)(word - A.K0) < (uint32_t)A.N; }
+__device__ __forceinline__ bool is_key(int word, const ColMergeArgs& A) {
+    return (uint32_t)(word - A.K0) < (uint32_t)A.N;
+}
 
-// The median of a segment's keys that are not padding, from its merged order (as emit_stream's), 0 without any; scratch:
-// 1 + W words of LDS.
+// The median of a segment's keys that are not padding, from its merged order (as emit_stream's), 0 without any;
+// scratch: 1 + W words of LDS.
 template <int T, int E>
-__device__ __forceinline__ float median_key(const ColMergeArgs& A, const float (&val)[E], const Halves<E>& src, uint32_t* scratch)
+__device__ __forceinline__ float median_key(const ColMergeArgs& A, const float (&val)[E], const Halves<E>& src,
+                                            uint32_t* scratch)
 {
     constexpr int W = T / WAVE;
     const int lane = lane_id(), wv = wave_in_block();
@@ -369,17 +379,18 @@ __device__ __forceinline__ float median_key(const ColMergeArgs& A, const float (
     return __uint_as_float(scratch[0]);
 }
 
-// The stream and the v == 1 terms of one segment, from its merged order: thread t's elements as word indices src (padding,
-// masked keys among it: K0 + N) and as values val (padding: the value before); x0 the median key, xs the value before the thread's first element.
-// sm: N + M words and 3 words a wave, free to use.
+// The stream and the v == 1 terms of one segment, from its merged order: thread t's elements as word indices src
+// (padding, masked keys among it: K0 + N) and as values val (padding: the value before); x0 the median key, xs the
+// value before the thread's first element. sm: N + M words and 3 words a wave, free to use.
 //
-// A query (bwd: a key) only receives sums, so whatever it holds stays in its own row. In a rare segment abs sums take its
-// value bounded, Laplace sums a NaN as the infinity on its side, and the row is marked in A.bad, which the finish makes NaN:
-// for abs where the value is infinite or NaN (as the walks' rows are), for Laplace where it is NaN (an infinite one is far
-// from every finite key). poison: a NaN among the weights' values that val no longer shows; every row is NaN.
+// A query (bwd: a key) only receives sums, so whatever it holds stays in its own row. In a rare segment abs sums take
+// its value bounded, Laplace sums a NaN as the infinity on its side, and the row is marked in A.bad, which the finish
+// makes NaN: for abs where the value is infinite or NaN (as the walks' rows are), for Laplace where it is NaN (an
+// infinite one is far from every finite key). poison: a NaN among the weights' values that val no longer shows; every
+// row is NaN.
 template <int KIND, int T, int E>
-__device__ __forceinline__ void emit_stream(const ColMergeArgs& A, float* sm, int s, float x0, float xs, float (&val)[E],
-                                            const Halves<E>& src, bool rare, bool poison)
+__device__ __forceinline__ void emit_stream(const ColMergeArgs& A, float* sm, int s, float x0, float xs,
+                                            float (&val)[E], const Halves<E>& src, bool rare, bool poison)
 {
     constexpr int W = T / WAVE;
     const int N = A.N, M = A.M, n = N + M, tid = threadIdx.x, seg = s / A.sets, p = seg / A.D;
@@ -396,9 +407,9 @@ __device__ __forceinline__ void emit_stream(const ColMergeArgs& A, float* sm, in
         }
     }
     float dist[E];
-    // A thread's values are taken relative to its anchor, its value nearest the median, so that every value an element's sums
-    // are formed from is bounded by distances to keys: on either side of the median the end towards it, and the median
-    // itself in a thread on both sides
+    // A thread's values are taken relative to its anchor, its value nearest the median, so that every value an
+    // element's sums are formed from is bounded by distances to keys: on either side of the median the end towards it,
+    // and the median itself in a thread on both sides
     float anchor = 0.f;
     Decays dec;
     if constexpr (KIND == COL_ABS) {
@@ -430,7 +441,8 @@ __device__ __forceinline__ void emit_stream(const ColMergeArgs& A, float* sm, in
         dec.before = over(__shfl(xs, 0, WAVE), xs);
         dec.after = over(prev, __shfl(prev, WAVE - 1, WAVE));
         dec.rest = over(xs, __shfl(prev, lane | 15, WAVE));
-        if (rare && poison) dec.own = dec.row = dec.half = dec.before = dec.after = dec.rest = __int_as_float(0x7fc00000);
+        if (rare && poison)
+            dec.own = dec.row = dec.half = dec.before = dec.after = dec.rest = __int_as_float(0x7fc00000);
     }
     float* vo = A.val + (size_t)s * T * E;
     uint16_t* to = A.tag + (size_t)s * T * E;
@@ -486,7 +498,8 @@ __device__ __forceinline__ void emit_stream(const ColMergeArgs& A, float* sm, in
         const float S = we + fmaf(-0.5f, wtot, wp);
         const float F = fmaf(anchor, S, -(ke + fmaf(-0.5f, ktot, kp)));
 #pragma unroll
-        for (int e = 0; e < E; ++e) out[e] = 2.f * set_weight(A.sets, s - seg * A.sets) * (out[e] + fmaf(dist[e], S, F));
+        for (int e = 0; e < E; ++e)
+            out[e] = 2.f * set_weight(A.sets, s - seg * A.sets) * (out[e] + fmaf(dist[e], S, F));
     } else {
         float l = 0.f, r = 0.f, pr = 1.f;
 #pragma unroll
@@ -619,8 +632,9 @@ void col_merge(const ColMergeArgs A)
         const uint32_t* qp = A.qp + (size_t)seg * M;
         const uint32_t* kp = A.kp + (size_t)seg * N;
         each_of<T>(qp, M, [&](int i, uint32_t x) { w[i] = (uint32_t)spread((int)x, M); });
-        if (!keep) each_of<T>(kp, N, [&](int i, uint32_t x) { w[M + i] = (uint32_t)(A.K0 + spread((int)x, N)); });
-        else each_of<T>(kp, N, [&](int i, uint32_t x) { w[M + i] = (uint32_t)(A.K0 + (keep[x] ? spread((int)x, N) : N)); });
+        auto key = [&](int i, int word) { w[M + i] = (uint32_t)(A.K0 + word); };
+        if (!keep) each_of<T>(kp, N, [&](int i, uint32_t x) { key(i, spread((int)x, N)); });
+        else each_of<T>(kp, N, [&](int i, uint32_t x) { key(i, keep[x] ? spread((int)x, N) : N); });
         __syncthreads();
 #pragma unroll
         for (int e = 0; e < E; e += 2) {
@@ -639,13 +653,13 @@ void col_merge(const ColMergeArgs A)
 // ---------------------------------------------------------------------------------------------------------------
 // col_sort: one workgroup per segment, from the unsorted queries and keys (A.qs, A.ks) to the stream
 //
-// A stable radix sort of queries (first) and keys together, 4 passes of 8 bits. A wave owns 64 E consecutive positions and
-// takes them 64 at a time: the lanes with an equal digit find each other by 8 ballots, so that a position's rank in its
-// wave is a running count per digit (a wave's own 256 counters in LDS) plus the equal lanes below it; one scan over
+// A stable radix sort of queries (first) and keys together, 4 passes of 8 bits. A wave owns 64 E consecutive positions
+// and takes them 64 at a time: the lanes with an equal digit find each other by 8 ballots, so that a position's rank in
+// its wave is a running count per digit (a wave's own 256 counters in LDS) plus the equal lanes below it; one scan over
 // (digit, wave) makes the counts first positions, and values and word indices go to their places through LDS. Nothing
-// is read from or written to memory between the inputs and the stream. Masked keys sort last, as padding.
-// What bounds it: about 60 vector instructions per element and pass (the ballots), then some 38 cycles of LDS, one after the
-// other: 155 us for 768 segments of 16384 elements (the two sorts and the merge: 178).
+// is read from or written to memory between the inputs and the stream. Masked keys sort last, as padding. What bounds
+// it: about 60 vector instructions per element and pass (the ballots), then some 38 cycles of LDS, one after the other:
+// 155 us for 768 segments of 16384 elements (the two sorts and the merge: 178).
 // ---------------------------------------------------------------------------------------------------------------
 __host__ __device__ constexpr int sort_words(int T, int E) { return T * E + T * E / 32 + 1 + 256 * (T / WAVE) + 32; }
 
@@ -859,9 +873,10 @@ void col_sum(const ColSumArgs A)
         }
         float a[E][CH];
         uint64_t acc[E];                                 // lanes whose element is an accumulator
-        // One workgroup per CU (CH = 1): reads run AHEAD elements before their use, in that order, so that a wave's arithmetic
-        // overlaps the other waves' reads (abs at N = M = 16384: 957 -> 856 us with the reads first and in order). With
-        // several workgroups per CU the compiler's order is better (text size, 16384 elements: 302 against 336 us).
+        // One workgroup per CU (CH = 1): reads run AHEAD elements before their use, in that order, so that a wave's
+        // arithmetic overlaps the other waves' reads (abs at N = M = 16384: 957 -> 856 us with the reads first and in
+        // order). With several workgroups per CU the compiler's order is better (text size, 16384 elements: 302 against
+        // 336 us).
         auto read = [&](int e) {
             const uint32_t x = addr(e);
             lds_read<CH>(a[e], x);
@@ -874,11 +889,11 @@ void col_sum(const ColSumArgs A)
         const uint32_t ab = aggb + (uint32_t)(d & 1) * AGGS;
         const int lane = lane_now(), el = min(lane & 15, W - 1);         // the wave whose aggregate this lane scans
         if constexpr (KIND == COL_ABS) {
-            // Half of sum_n |k_n - x| w_n is sum_{k < x} (x - k) w less half of the sum over all keys of (x - k) w. With x
-            // and k relative to the thread's anchor, a thread's own keys below give x W - K from its running sums
-            // W = sum w, K = sum k w; the keys of the threads before, and the totals, then make one linear term S x + F
-            // per thread. Across threads K runs relative to the median
-            // key: |k - median| w sums to no more than the terms |k - q| w that the result is measured by.
+            // Half of sum_n |k_n - x| w_n is sum_{k < x} (x - k) w less half of the sum over all keys of (x - k) w.
+            // With x and k relative to the thread's anchor, a thread's own keys below give x W - K from its running
+            // sums W = sum w, K = sum k w; the keys of the threads before, and the totals, then make one linear term S
+            // x + F per thread. Across threads K runs relative to the median key: |k - median| w sums to no more than
+            // the terms |k - q| w that the result is measured by.
             float own[E][CH], sw[CH], sk[CH], we[CH], ke[CH];
 #pragma unroll
             for (int h = 0; h < CH; ++h) sw[h] = sk[h] = 0.f;
@@ -1011,9 +1026,9 @@ void col_sum(const ColSumArgs A)
             }
 #pragma unroll
             for (int g = 0; g < E / 2; ++g) asm volatile("" : "+v"(tg[g]));
-            // R at each element beside its word where the registers hold both (one rounding of the word per feature, and
-            // fewer instructions: 372 -> 338 us at 12 x 8192, two channels); else added to the word on the way (27 spilled
-            // registers at 32 elements: 930 -> 1975 us)
+            // R at each element beside its word where the registers hold both (one rounding of the word per feature,
+            // and fewer instructions: 372 -> 338 us at 12 x 8192, two channels); else added to the word on the way (27
+            // spilled registers at 32 elements: 930 -> 1975 us)
             constexpr bool BESIDE = CH == 2 ? E <= 16 : E <= 24;
             float above[BESIDE ? E : 1][CH];
 #pragma unroll
@@ -1064,22 +1079,22 @@ void col_sum(const ColSumArgs A)
 // ---------------------------------------------------------------------------------------------------------------
 // col_dot: one workgroup per segment (p, d), all channels: the gradients of the abs sums in q and k
 //
-//   grad_q[m] = sum_c g_mc (2 W_c - Wtot_c), W_c the sum of v_nc over the keys below q_m      (an equal key counts above)
-//   grad_k[n] = sum_c v_nc (2 G_c - Gtot_c), G_c the sum of g_mc over the queries below k_n   (an equal query counts above)
+//   grad_q[m] = sum_c g_mc (2 W_c - Wtot_c), W_c the sum of v_nc over the keys below q_m    (an equal key counts above)
+//   grad_k[n] = sum_c v_nc (2 G_c - Gtot_c), G_c the sum of g_mc over the queries below k_n (an equal query, too)
 //
 // The transposed loop of col_sum: a segment's merged order stays in registers (tags, and each element's running dot
 // product), and the columns of g_w and v of one channel group after another go through LDS (copied there without
 // registers while the previous group's arithmetic finishes). Per element and channel one random LDS read, two running
 // sums and two multiply-adds. With g_u there is one more channel, g_u against ones.
 // Queries come before equal keys in the merged order, so W is right as it runs; G is taken where the key's run of equal
-// values began: kept as the thread goes, and where a run crosses threads (else a workgroup skips it) through LDS from the
-// thread in which it began.
+// values began: kept as the thread goes, and where a run crosses threads (else a workgroup skips it) through LDS from
+// the thread in which it began.
 // ---------------------------------------------------------------------------------------------------------------
 struct ColDotArgs {
     const uint16_t* tag; const uint32_t* eq;
     const float* gt; const float* vt;        // [P][CW][M][CH], [P][CW][N][CH]
     float* gq; float* gk;                    // (P, D, M) and, or null, (P, D, N)
-    float* sums;                             // [S][E/4][T][4] scratch: the dot products, where they are not in registers
+    float* sums;                             // [S][E/4][T][4] scratch: the dot products where no registers are left
     float scale;                             // 2, or -2 for the sgn sum
     int D, N, M, K0, NP, CW;                 // NP: keys' words, N rounded up like K0
 };
@@ -1146,19 +1161,22 @@ void col_dot(const ColDotArgs A)
         from = max(ex, 0);
     }
 
-    // one channel group's columns into LDS: chunks of 64 x 16 bytes, shared out over the waves; lanes past a column read 0
+    // one channel group's columns into LDS: chunks of 64 x 16 bytes, shared out over the waves; lanes past a column
+    // read 0
     auto fetch = [&](int cg) {
         const rsrc_t rg = make_rsrc(A.gt + ((size_t)p * A.CW + cg) * M * CH, (uint32_t)(M * CH * 4));
         const rsrc_t rv = make_rsrc(A.vt + ((size_t)p * A.CW + cg) * N * CH, (uint32_t)(N * CH * 4));
         const int qc = K0 * CH / 256, kc = A.NP * CH / 256;
         for (int i = wv; i < qc; i += W)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rg, (LDS_AS void*)(uint32_t)(i * 1024), 16, lane * 16, i * 1024, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rg, (LDS_AS void*)(uint32_t)(i * 1024), 16, lane * 16, i * 1024, 0,
+                                                     0);
         for (int i = wv; i < kc; i += W)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (LDS_AS void*)(uint32_t)((qc + i) * 1024), 16, lane * 16, i * 1024,
-                                                     0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (LDS_AS void*)(uint32_t)((qc + i) * 1024), 16, lane * 16,
+                                                     i * 1024, 0, 0);
     };
-    // The dot products over 8 groups at a time, then over those: sequential sums over all channels lost half a digit. The
-    // latter in memory where registers do not hold both (spilled, their reloads would wait for the columns in flight).
+    // The dot products over 8 groups at a time, then over those: sequential sums over all channels lost half a digit.
+    // The latter in memory where registers do not hold both (spilled, their reloads would wait for the columns in
+    // flight).
     constexpr bool IN_MEMORY = CH == 1 && E > 24;
     float sum[IN_MEMORY ? 1 : E], part[E];
     f4_t* sums = (f4_t*)(A.sums + (size_t)s * T * E) + tid;
@@ -1177,7 +1195,7 @@ void col_dot(const ColDotArgs A)
 #pragma unroll
         for (int e = 0; e < AHEAD && e < E; ++e) lds_read<CH>(a[e], addr(e));
         uint32_t eqc = eq, contc = cont;
-        asm volatile("" : "+v"(eqc), "+v"(contc));           // their bits' masks are formed here, not kept from channel to channel
+        asm volatile("" : "+v"(eqc), "+v"(contc));           // their bits' masks are formed here, not kept all along
         float w[CH], g[CH], gr[CH];                          // running W and G, G where the element's run of equals began
 #pragma unroll
         for (int h = 0; h < CH; ++h) w[h] = g[h] = gr[h] = 0.f;
@@ -1290,15 +1308,17 @@ void col_dot(const ColDotArgs A)
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// col_weights: the weight rows (P, Nw, C) as columns [P][CW][Nw][CH] in the order of their words, masked rows 0. With C1 = C + 1 there is one more
-// channel, `extra` (P, Nw) or all ones. Also clears `bad` (bads words; null: 0) for the merge that comes after it.
+// col_weights: the weight rows (P, Nw, C) as columns [P][CW][Nw][CH] in the order of their words, masked rows 0. With
+// C1 = C + 1 there is one more channel, `extra` (P, Nw) or all ones. Also clears `bad` (bads words; null: 0) for the
+// merge that comes after it.
 // ---------------------------------------------------------------------------------------------------------------
 constexpr int CF_T = 256, CF_M = 64;        // threads, rows per workgroup (also of col_finish)
 
 template <int CH>
 __global__ __launch_bounds__(CF_T)
 void col_weights(const float* __restrict__ w, const float* __restrict__ extra, const uint8_t* __restrict__ keep,
-                 float* __restrict__ out, float* __restrict__ bad, const int bads, const int Nw, const int C, const int C1)
+                 float* __restrict__ out, float* __restrict__ bad, const int bads, const int Nw, const int C,
+                 const int C1)
 {
     __shared__ float tile[130][CF_M + 1];
     for (int i = blockIdx.x * CF_T + threadIdx.x; i < bads; i += gridDim.x * CF_T) bad[i] = 0.f;
@@ -1336,13 +1356,13 @@ void col_weights(const float* __restrict__ w, const float* __restrict__ extra, c
 // ---------------------------------------------------------------------------------------------------------------
 // col_finish: the feature shares' columns summed, turned into rows, with the v == 1 terms summed over the features
 // ---------------------------------------------------------------------------------------------------------------
-// scale: 2 for the abs sums, whose columns hold halves. bad (P, M): NaN at the rows that are NaN whatever the columns hold
-// (emit_stream), 0 else. kind < 0: out = w and out_u = u; else the layer's epilogue on
-// them, as layer_epilogue_kernel
+// scale: 2 for the abs sums, whose columns hold halves. bad (P, M): NaN at the rows that are NaN whatever the columns
+// hold (emit_stream), 0 else. kind < 0: out = w and out_u = u; else the layer's epilogue on them, as
+// layer_epilogue_kernel
 __global__ __launch_bounds__(CF_T)
 void col_finish(const float* __restrict__ cols, const float* __restrict__ u, const float* __restrict__ bad,
-                float* __restrict__ out, float* __restrict__ out_u, const float scale, const int kind, const int masked, const ReduceEpilogue ep,
-                const int D, const int M, const int C, const int DS)
+                float* __restrict__ out, float* __restrict__ out_u, const float scale, const int kind, const int masked,
+                const ReduceEpilogue ep, const int D, const int M, const int C, const int DS)
 {
     __shared__ float tile[128][CF_M + 1];
     __shared__ float us[CF_T / CF_M][CF_M];
@@ -1405,7 +1425,8 @@ namespace {
 constexpr size_t LDS_BYTES = 160 * 1024;
 
 size_t sum_lds(int kind, int T, int CH, int n) {
-    return (((size_t)(n + 1) * CH * 4 + 15) & ~size_t(15)) + 2 * (size_t)(kind == COL_ABS ? 2 : 3) * CH * (T / WAVE) * 4;
+    const size_t words = ((size_t)(n + 1) * CH * 4 + 15) & ~size_t(15);
+    return words + 2 * (size_t)(kind == COL_ABS ? 2 : 3) * CH * (T / WAVE) * 4;
 }
 
 // words of a region rounded up to the 1 KB chunks col_dot copies
@@ -1416,7 +1437,8 @@ size_t dot_lds(int T, int CH, int N, int M) {
     return words + (size_t)(T / WAVE) * 2 * CH * 4 + (size_t)T * CH * 4;
 }
 
-// Workgroups of one col_sum launch that a CU holds at once: by LDS, and by the wave slots of 4 waves per SIMD (128 VGPRs)
+// Workgroups of one col_sum launch that a CU holds at once: by LDS, and by the wave slots of 4 waves per SIMD (128
+// VGPRs)
 int wgs_per_cu(int kind, int T, int CH, int n) {
     return std::max(1, std::min((int)(LDS_BYTES / sum_lds(kind, T, CH, n)), 1024 / T));
 }
@@ -1433,8 +1455,8 @@ ColPlan col_plan(int kind, int P, int D, int N, int M, int C) {
     const int n = N + M;
     ColPlan pl{};
     // Two channels per workgroup where their words fit LDS (an 8-byte LDS read costs what a 4-byte one does, and the
-    // stream is read once for both; the second of one channel is 0); the smallest workgroup whose threads hold at most 16
-    // elements then, so that several run per CU and fill each other's waits. The shape depends on n alone: what a
+    // stream is read once for both; the second of one channel is 0); the smallest workgroup whose threads hold at most
+    // 16 elements then, so that several run per CU and fill each other's waits. The shape depends on n alone: what a
     // stream takes (col_applies) is the same for every C.
     if (n <= COL_MAX2) {
         pl.CH = 2;
@@ -1446,9 +1468,9 @@ ColPlan col_plan(int kind, int P, int D, int N, int M, int C) {
         pl.T = 1024;
         pl.E = n <= pl.T * 20 ? 20 : n <= pl.T * 24 ? 24 : n <= pl.T * 28 ? 28 : 32;
     }
-    // Shares of the features: the fewest rounds of workgroups over the chip, in features walked one after another, plus the
-    // loading and storing of the columns per round: about six features' time where a workgroup has a CU to itself, two
-    // where others run beside it.
+    // Shares of the features: the fewest rounds of workgroups over the chip, in features walked one after another, plus
+    // the loading and storing of the columns per round: about six features' time where a workgroup has a CU to itself,
+    // two where others run beside it.
     pl.per_cu = wgs_per_cu(kind, pl.T, pl.CH, n);
     const int64_t wgs = (int64_t)P * ((C + pl.CH - 1) / pl.CH), slots = (int64_t)CUS * pl.per_cu;
     int64_t best = -1;
@@ -1463,7 +1485,8 @@ ColPlan col_plan(int kind, int P, int D, int N, int M, int C) {
 bool col_bwd_applies(int D, int N, int M) {
     if (!col_applies(D, N, M)) return false;
     const ColPlan pl = col_plan(COL_ABS, 1, D, N, M, 1);
-    return dot_lds(pl.T, pl.CH, N, M) <= LDS_BYTES && sum_lds(COL_ABS, pl.T, pl.CH, pad_words(M, pl.CH) + N) <= LDS_BYTES;
+    return dot_lds(pl.T, pl.CH, N, M) <= LDS_BYTES &&
+           sum_lds(COL_ABS, pl.T, pl.CH, pad_words(M, pl.CH) + N) <= LDS_BYTES;
 }
 
 int col_key0(const ColPlan& pl, int M) { return pad_words(M, pl.CH); }
@@ -1494,7 +1517,8 @@ template <class F>
 int dispatch_shape(const ColPlan& pl, F f) {
 #define QLKA_COL(TT, EE, CC) \
     if (pl.T == TT && pl.E == EE && pl.CH == CC) \
-        return f(std::integral_constant<int, TT>{}, std::integral_constant<int, EE>{}, std::integral_constant<int, CC>{})
+        return f(std::integral_constant<int, TT>{}, std::integral_constant<int, EE>{},                                 \
+                 std::integral_constant<int, CC>{})
     QLKA_COL(64, 12, 2); QLKA_COL(64, 16, 2); QLKA_COL(128, 12, 2); QLKA_COL(128, 16, 2); QLKA_COL(256, 12, 2);
     QLKA_COL(256, 16, 2); QLKA_COL(512, 12, 2); QLKA_COL(512, 16, 2); QLKA_COL(1024, 12, 2); QLKA_COL(1024, 16, 2);
     QLKA_COL(512, 20, 2); QLKA_COL(1024, 20, 2);
@@ -1503,8 +1527,8 @@ int dispatch_shape(const ColPlan& pl, F f) {
     return (int)hipErrorInvalidValue;
 }
 
-// Lets the kernel use all of a CU's LDS on the stream's device. The attribute belongs to one device's copy of the kernel (and
-// is set for the current device's), so `once`, one per kernel, keeps account by device.
+// Lets the kernel use all of a CU's LDS on the stream's device. The attribute belongs to one device's copy of the
+// kernel (and is set for the current device's), so `once`, one per kernel, keeps account by device.
 template <class K>
 int allow_lds(K kernel, PerDevice& once, hipStream_t st) {
     int cur = 0;
@@ -1534,20 +1558,22 @@ int launch_sum(const ColSumArgs& a, hipStream_t st) {
     static PerDevice once;
     if (int e = allow_lds(col_sum<KIND, T, E, CH, SWAP, 4>, once, st)) return e;
     const unsigned blocks = (unsigned)(a.P * a.DS * ((a.C + CH - 1) / CH));
-    hipLaunchKernelGGL((col_sum<KIND, T, E, CH, SWAP, 4>), dim3(blocks), dim3(T), sum_lds(KIND, T, CH, a.K0 + a.N), st, a);
+    hipLaunchKernelGGL((col_sum<KIND, T, E, CH, SWAP, 4>), dim3(blocks), dim3(T), sum_lds(KIND, T, CH, a.K0 + a.N), st,
+                       a);
     return (int)hipGetLastError();
 }
 
 }  // namespace
 
-// Against the two sorts and the merge, whole prep of a call: 1536 elements 66 -> 47 us (2048 segments), 8192 210 -> 126 us
-// (1536; with a key mask also the 60 us of its fill), 16384 178 -> 156 us (768). Threads of more than 16 elements spill
-// here (32768: 629 against 412 us).
+// Against the two sorts and the merge, whole prep of a call: 1536 elements 66 -> 47 us (2048 segments), 8192 210 -> 126
+// us (1536; with a key mask also the 60 us of its fill), 16384 178 -> 156 us (768). Threads of more than 16 elements
+// spill here (32768: 629 against 412 us).
 bool col_sort_applies(const ColPlan& pl) { return pl.E <= 16; }
 
 int col_sort_launch(int kind, const ColPlan& pl, const float* q, const float* k, const uint8_t* keep, ColStream str,
                     float* u, float* bad, int S, int D, int N, int M, hipStream_t st) {
-    const ColMergeArgs a{q, nullptr, k, nullptr, keep, str.val, str.tag, str.xe, str.xe2, nullptr, u, bad, D, N, M, M, 1};
+    const ColMergeArgs a{q, nullptr, k, nullptr, keep, str.val, str.tag, str.xe, str.xe2, nullptr, u, bad, D, N, M, M,
+                         1};
     StageTimer t("col_sort", st);
     return dispatch_shape(pl, [&](auto T, auto E, auto) {
         if constexpr (E() > 16) {
@@ -1570,12 +1596,13 @@ int col_sort_launch(int kind, const ColPlan& pl, const float* q, const float* k,
 int col_merge_launch(int kind, const ColPlan& pl, const float* qs, const uint32_t* qp, const float* ks,
                      const uint32_t* kp, const uint8_t* keep, ColStream str, float* u, float* bad, int S, int D, int N,
                      int M, bool bwd, int sets, hipStream_t st) {
-    const ColMergeArgs a{qs, qp, ks, kp, keep, str.val, str.tag, str.xe, str.xe2, bwd ? str.eq : nullptr, u, bad, D, N, M,
-                         bwd ? col_key0(pl, M) : M, sets};
+    const ColMergeArgs a{qs, qp, ks, kp, keep, str.val, str.tag, str.xe, str.xe2, bwd ? str.eq : nullptr, u, bad, D, N,
+                         M, bwd ? col_key0(pl, M) : M, sets};
     S *= sets;
     StageTimer t("col_merge", st);
     return dispatch_shape(pl, [&](auto T, auto E, auto) {
-        return kind == COL_ABS ? launch_merge<COL_ABS, T(), E()>(a, S, st) : launch_merge<COL_LAPLACE, T(), E()>(a, S, st); });
+        return kind == COL_ABS ? launch_merge<COL_ABS, T(), E()>(a, S, st)
+                               : launch_merge<COL_LAPLACE, T(), E()>(a, S, st); });
 }
 
 int col_weights_launch(const ColPlan& pl, const float* w, const uint8_t* keep, bool more, const float* extra, float* wt,
@@ -1593,23 +1620,26 @@ int col_weights_launch(const ColPlan& pl, const float* w, const uint8_t* keep, b
 
 int col_sum_launch(int kind, const ColPlan& pl, ColStream str, const float* wt, float* cols, int P, int D, int N, int M,
                    int C, int sets, hipStream_t st) {
-    const ColSumArgs a{str.val, str.tag, str.xe, str.xe2, wt, cols, P, D * sets, N, M, C, pl.DS, M, (C + pl.CH - 1) / pl.CH, sets};
+    const int CW = (C + pl.CH - 1) / pl.CH;
+    const ColSumArgs a{str.val, str.tag, str.xe, str.xe2, wt, cols, P, D * sets, N, M, C, pl.DS, M, CW, sets};
     StageTimer t(kind == COL_ABS ? "col_sum_abs" : "col_sum_laplace", st);
     return dispatch_shape(pl, [&](auto T, auto E, auto CH) {
         return kind == COL_ABS ? launch_sum<COL_ABS, T(), E(), CH(), false>(a, st)
                                : launch_sum<COL_LAPLACE, T(), E(), CH(), false>(a, st); });
 }
 
-int col_grad_v_launch(const ColPlan& pl, ColStream str, const float* gt, int CW, float* cols, int P, int D, int N, int M,
-                      int C, hipStream_t st) {
+int col_grad_v_launch(const ColPlan& pl, ColStream str, const float* gt, int CW, float* cols, int P, int D, int N,
+                      int M, int C, hipStream_t st) {
     const ColSumArgs a{str.val, str.tag, str.xe, str.xe2, gt, cols, P, D, N, M, C, pl.DS, col_key0(pl, M), CW, 1};
     StageTimer t("col_grad_v", st);
-    return dispatch_shape(pl, [&](auto T, auto E, auto CH) { return launch_sum<COL_ABS, T(), E(), CH(), true>(a, st); });
+    return dispatch_shape(pl, [&](auto T, auto E, auto CH) {
+        return launch_sum<COL_ABS, T(), E(), CH(), true>(a, st); });
 }
 
 int col_dot_launch(const ColPlan& pl, ColStream str, const float* gt, const float* vt, int CW, float scale, float* gq,
                    float* gk, int S, int D, int N, int M, hipStream_t st) {
-    const ColDotArgs a{str.tag, str.eq, gt, vt, gq, gk, str.val, scale, D, N, M, col_key0(pl, M), pad_words(N, pl.CH), CW};
+    const ColDotArgs a{str.tag, str.eq, gt, vt, gq, gk, str.val, scale, D, N, M, col_key0(pl, M), pad_words(N, pl.CH),
+                       CW};
     StageTimer t("col_dot", st);
     return dispatch_shape(pl, [&](auto T, auto E, auto CH) {
         static PerDevice once;
@@ -1619,10 +1649,11 @@ int col_dot_launch(const ColPlan& pl, ColStream str, const float* gt, const floa
 }
 
 int col_finish_launch(int kind, int layer, bool masked, const ColPlan& pl, const float* cols, const float* u,
-                      const float* bad, float* out, float* out_u, const ReduceEpilogue& ep, int P, int D, int M, int C, hipStream_t st) {
+                      const float* bad, float* out, float* out_u, const ReduceEpilogue& ep, int P, int D, int M, int C,
+                      hipStream_t st) {
     StageTimer t("col_finish", st);
-    hipLaunchKernelGGL(col_finish, dim3((unsigned)(P * ((M + CF_M - 1) / CF_M))), dim3(CF_T), 0, st, cols, u, bad, out, out_u,
-                       kind == COL_ABS ? 2.f : 1.f, layer, masked ? 1 : 0, ep, D, M, C, pl.DS);
+    hipLaunchKernelGGL(col_finish, dim3((unsigned)(P * ((M + CF_M - 1) / CF_M))), dim3(CF_T), 0, st, cols, u, bad, out,
+                       out_u, kind == COL_ABS ? 2.f : 1.f, layer, masked ? 1 : 0, ep, D, M, C, pl.DS);
     return (int)hipGetLastError();
 }
 

@@ -6,8 +6,8 @@
 
 namespace qlka {
 
-// once(device, f) runs f() unless it has succeeded for that device before, and returns its status (0: success, and later
-// calls return 0 at once). A failure is not remembered. Threads that come together may each run f.
+// once(device, f) runs f() unless it has succeeded for that device before, and returns its status (0: success, and
+// later calls return 0 at once). A failure is not remembered. Threads that come together may each run f.
 class PerDevice {
 public:
     template <class F>

@@ -212,8 +212,8 @@ int mbw_walk_launch(const float* mv, const uint32_t* mt, const float* v, const f
 int direct_fwd(int kind, const float* q, const float* k, const float* v, float* out_w, float* out_u,
                int P, int D, int N, int M, int C, hipStream_t st);
 // The dense abs forward keeping its kernel matrix A[p][m][n] = sum_d |q[p,d,m] - k[p,d,n]| (P*M rows of pad4(N) floats)
-// in a_out, where the tiled kernel runs (direct_fwd_tiled); and out[p,n,:] = sum_m A[p,m,n] g[p,m,:] from such an A (the
-// dense grad_v, bit-identical to forming A again)
+// in a_out, where the tiled kernel runs (direct_fwd_tiled); and out[p,n,:] = sum_m A[p,m,n] g[p,m,:] from such an A
+// (the dense grad_v, bit-identical to forming A again)
 bool direct_fwd_tiled(int D, int N, int M, int C);
 int direct_fwd_keep_a(const float* q, const float* k, const float* v, float* out_w, float* out_u, float* a_out,
                       int P, int D, int N, int M, int C, hipStream_t st);
@@ -272,9 +272,10 @@ size_t col_stream_bytes(int kind, const ColPlan& pl, int S);
 ColStream col_stream(int kind, const ColPlan& pl, void* base, int S);
 // the merged stream of S sorted segments, and the v == 1 terms u (S, M) in the order of the words
 // (null: none); masked keys are padding.
-// bwd: the stream of the abs backward (keys' words from col_key0, runs of equal values). sets = 3 (kind 0): three streams
-// and rows of u per segment, of q, q + 1 and q - 1, which the sums weight -1, 1/2, 1/2 (add_bump); else 1. bad (P, M), with
-// bwd (P, N), cleared before (col_weights_launch): NaN where a row's own value makes it NaN (null: not wanted).
+// bwd: the stream of the abs backward (keys' words from col_key0, runs of equal values). sets = 3 (kind 0): three
+// streams and rows of u per segment, of q, q + 1 and q - 1, which the sums weight -1, 1/2, 1/2 (add_bump); else 1. bad
+// (P, M), with bwd (P, N), cleared before (col_weights_launch): NaN where a row's own value makes it NaN (null: not
+// wanted).
 int col_merge_launch(int kind, const ColPlan& pl, const float* qs, const uint32_t* qp, const float* ks,
                      const uint32_t* kp, const uint8_t* keep, ColStream str, float* u, float* bad, int S, int D, int N,
                      int M, bool bwd, int sets, hipStream_t st);
@@ -282,25 +283,26 @@ int col_merge_launch(int kind, const ColPlan& pl, const float* qs, const uint32_
 bool col_sort_applies(const ColPlan& pl);
 int col_sort_launch(int kind, const ColPlan& pl, const float* q, const float* k, const uint8_t* keep, ColStream str,
                     float* u, float* bad, int S, int D, int N, int M, hipStream_t st);
-// wt: the columns of rows w (P, Nw, C) in groups of pl.CH, rows masked by keep (null: none) 0; `more`: one more channel,
-// extra (P, Nw) or ones. Clears the `bads` words of bad.
+// wt: the columns of rows w (P, Nw, C) in groups of pl.CH, rows masked by keep (null: none) 0; `more`: one more
+// channel, extra (P, Nw) or ones. Clears the `bads` words of bad.
 int col_weights_launch(const ColPlan& pl, const float* w, const uint8_t* keep, bool more, const float* extra, float* wt,
                        float* bad, int bads, int P, int Nw, int C, hipStream_t st);
 // The abs backward over a bwd stream and the columns gt, vt (CW groups each) of g_w and v: cols[P][DS][C][N] = half of
 // grad_v; and gq = scale / 2 times grad_q, gk (or null) the same of grad_k (last: it overwrites str.val)
 bool col_bwd_applies(int D, int N, int M);
 int col_key0(const ColPlan& pl, int M);
-int col_grad_v_launch(const ColPlan& pl, ColStream str, const float* gt, int CW, float* cols, int P, int D, int N, int M,
-                      int C, hipStream_t st);
+int col_grad_v_launch(const ColPlan& pl, ColStream str, const float* gt, int CW, float* cols, int P, int D, int N,
+                      int M, int C, hipStream_t st);
 int col_dot_launch(const ColPlan& pl, ColStream str, const float* gt, const float* vt, int CW, float scale, float* gq,
                    float* gk, int S, int D, int N, int M, hipStream_t st);
 // cols[P][DS][C][M]: the sums of each feature share over the weights wt (P, C, N); half of them for kind 0
 int col_sum_launch(int kind, const ColPlan& pl, ColStream str, const float* wt, float* cols, int P, int D, int N, int M,
                    int C, int sets, hipStream_t st);
-// layer < 0: out (P, M, C) and, with u, out_u (P, M); else the epilogue of layer kind `layer` written to ep.out. Rows marked
-// in bad are NaN.
+// layer < 0: out (P, M, C) and, with u, out_u (P, M); else the epilogue of layer kind `layer` written to ep.out. Rows
+// marked in bad are NaN.
 int col_finish_launch(int kind, int layer, bool masked, const ColPlan& pl, const float* cols, const float* u,
-                      const float* bad, float* out, float* out_u, const ReduceEpilogue& ep, int P, int D, int M, int C, hipStream_t st);
+                      const float* bad, float* out, float* out_u, const ReduceEpilogue& ep, int P, int D, int M, int C,
+                      hipStream_t st);
 
 // ---- capi.hip helpers for noalloc.hip
 // check_dims of the C ABI (clears the thread's error first); the workspace of a Laplace forward over pc p at a time;

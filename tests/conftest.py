@@ -37,8 +37,8 @@ def dev():
     return torch.device("cuda", 0)
 
 
-# The library's own routing by size ("auto"), or every short segment too through sort + walk or, where N + M allows it, sort +
-# column sums: dense cutoff (None: as it is), column mode.
+# The library's own routing by size ("auto"), or every short segment too through sort + walk or, where N + M allows it,
+# sort + column sums: dense cutoff (None: as it is), column mode.
 ROUTES = {"auto": (None, 0), "walk": (0, 1), "columns": (0, 2)}
 
 

@@ -2,8 +2,8 @@
 counts N + M where the threads or elements per thread change, the switch from two channels per workgroup to one, odd
 channel counts, one-sided sizes and the last size before the ranges take over.
 
-Against the fp64 oracle on a subsample of the queries, at the bar of every forward sum: 1e-5 of sum |term|. The fp32 error
-of these sums is a few roundings of partial sums no larger than sum |term| (measured: below 1e-6), so 1e-5 has room.
+Against the fp64 oracle on a subsample of the queries, at the bar of every forward sum: 1e-5 of sum |term|. The fp32
+error of these sums is a few roundings of partial sums no larger than sum |term| (measured: below 1e-6), so 1e-5 has room.
 """
 
 import numpy as np
@@ -67,7 +67,8 @@ def test_column_capacity_edges(dev, no_dense, n, kind):
 
 
 @pytest.mark.parametrize("shape", [(1, 1, 17, 1, 1), (2, 1, 18, 40, 2), (1, 2, 32000, 700, 5), (1, 2, 700, 32000, 2),
-                                   (2, 5, 600, 610, 1), (1, 2, 9000, 8000, 1), (3, 33, 900, 1100, 7), (40, 2, 1200, 900, 128), (2, 64, 5003, 3001, 33)])
+                                   (2, 5, 600, 610, 1), (1, 2, 9000, 8000, 1), (3, 33, 900, 1100, 7),
+                                   (40, 2, 1200, 900, 128), (2, 64, 5003, 3001, 33)])
 @pytest.mark.parametrize("kind", ["normal", "far"])
 def test_column_shapes(dev, no_dense, shape, kind):
     _check(dev, *shape, kind, seed=sum(shape))
@@ -100,8 +101,9 @@ def test_laplace_infinite_keys_and_queries(dev, no_dense):
                                    (1, 2, 5000, 5239, 2), (1, 2, 9000, 7385, 9), (1, 2, 9900, 10453, 3),
                                    (1, 2, 16384, 16384, 18), (1, 2, 31000, 900, 2), (2, 1, 900, 30000, 1)])
 def test_column_backward(dev, no_dense, shape, kind):
-    # grad_q, grad_k, grad_v with and without g_u, and the sgn sum, at the workgroup shapes' edges; "ties": runs of equal
-    # queries and keys that cross threads and waves, "runs": one value for long stretches. Ties count -1 (sgn: +1).
+    # grad_q, grad_k, grad_v with and without g_u, and the sgn sum, at the workgroup shapes' edges; "ties": runs of
+    # equal queries and keys that cross threads and waves, "runs": one value for long stretches. Ties count -1 (sgn:
+    # +1).
     from weighted_abs_sum import _ext, weighted_sgn_sum
     P, D, N, M, C = shape
     print(f"column backward {shape} {kind}", flush=True)
@@ -133,8 +135,8 @@ BAD = {"inf": np.inf, "-inf": -np.inf, "nan": np.nan, "-nan": -np.nan, "huge": 3
 
 
 def _layer64(kernel, q, k, v, keep, M):
-    """float64 num (rows, C) and den (rows) of one p's layer at queries q (D, rows) over its kept keys k (D, N) with rows v,
-    and the sums of |term| that the abs or Laplace sums and the epilogue form them from: each is within REL of those."""
+    """float64 num (rows, C) and den (rows) of one p's layer at queries q (D, rows) over its kept keys k (D, N) with
+    rows v, and the sums of |term| that the abs or Laplace sums and the epilogue form them from: each is within REL of those."""
     from qlka import layers
     n_pad = int((~keep).sum())
     q, k, v = q.astype(np.float64), k[:, keep].astype(np.float64), v[keep].astype(np.float64)
@@ -180,8 +182,9 @@ def test_masked_layer_columns(dev, no_dense, kernel, N, M, C):
 @pytest.mark.parametrize("bad", sorted(BAD))
 @pytest.mark.parametrize("shape", [(2, 3, 700, 650, 5), (1, 2, 12000, 11000, 3), (1, 2, 16000, 16000, 2)])
 def test_a_bad_query_spoils_only_its_row(dev, no_dense, shape, bad):
-    # as by the walks: abs and layer rows of an infinite or NaN query are NaN, Laplace's are 0 for an infinite one; every
-    # other row is what the oracle says. A huge finite query (differences past the largest float) spoils no other row.
+    # as by the walks: abs and layer rows of an infinite or NaN query are NaN, Laplace's are 0 for an infinite one;
+    # every other row is what the oracle says. A huge finite query (differences past the largest float) spoils no other
+    # row.
     from qlka import layers
     from weighted_abs_sum import weighted_abs_sum, weighted_abs_sum_full
     from weighted_laplace_sum import weighted_laplace_sum
@@ -239,8 +242,8 @@ def test_a_bad_key_spoils_only_its_row_of_grad_v(dev, no_dense, shape, bad):
 
 
 def test_a_thread_on_both_sides_of_the_median(dev, no_dense):
-    # a far query, then the keys, all in the first thread's elements: the others' sums stay as precise as their distances to
-    # the keys are (1.5e-3 of sum |term| where such a thread's values were relative to the far query)
+    # a far query, then the keys, all in the first thread's elements: the others' sums stay as precise as their
+    # distances to the keys are (1.5e-3 of sum |term| where such a thread's values were relative to the far query)
     from weighted_abs_sum import weighted_abs_sum_full
     P, D, N, M, C = 2, 2, 17, 700, 3
     rng = np.random.default_rng(8)
@@ -257,10 +260,11 @@ def test_a_thread_on_both_sides_of_the_median(dev, no_dense):
 
 @pytest.mark.parametrize("kernel", ["add_laplace", "add_riesz", "add_bump"])
 @pytest.mark.parametrize("far", ["low", "both", "nan"])
-@pytest.mark.parametrize("N,M,kept", [(3000, 2000, 0.4), (3000, 2000, 0.01), (12000, 11000, 0.4), (12000, 11000, 0.001)])
+@pytest.mark.parametrize("N,M,kept", [(3000, 2000, 0.4), (3000, 2000, 0.01), (12000, 11000, 0.4),
+                                      (12000, 11000, 0.001)])
 def test_mostly_masked_keys_far_out(dev, no_dense, kernel, far, N, M, kept):
-    # masked keys weigh nothing wherever they lie: most of a segment's keys masked and far below the kept ones, on both sides
-    # of them, or NaN of either sign, with kept keys and queries of scale 1
+    # masked keys weigh nothing wherever they lie: most of a segment's keys masked and far below the kept ones, on both
+    # sides of them, or NaN of either sign, with kept keys and queries of scale 1
     from qlka import layers
     P, D, C = 2, 3, 4
     print(f"mostly masked {kernel} N={N} kept={kept} {far}", flush=True)
@@ -282,13 +286,14 @@ def test_mostly_masked_keys_far_out(dev, no_dense, kernel, far, N, M, kept):
         _assert_layer(kernel, got[p][idx[p]], q[p][:, idx[p]], k[p], v[p], keep[p], M)
 
 
-@pytest.mark.parametrize("kind", ["grid 1e-4", "grid 0.1", "grid 3", "uniform 2e-5", "normal 1e-5", "dyadic", "normal 1"])
+@pytest.mark.parametrize("kind", ["grid 1e-4", "grid 0.1", "grid 3", "uniform 2e-5", "normal 1e-5", "dyadic",
+                                  "normal 1"])
 @pytest.mark.parametrize("n", [1100, 3000, 8192, 16384])
 def test_laplace_keys_whose_roundings_repeat(dev, no_dense, n, kind):
-    # Decays between neighbours that are all alike (grids) or all below a rounding of 1 (narrow keys), where the errors of a
-    # chain of products add up. Relative 2-norm: at most 31 products in a thread and 15 across waves, half of them on
-    # average, each off by up to 2^-25 to the same side: 7e-7; by factors rounded one by one and multiplied up through the
-    # scans 1.2e-6 to 6.1e-6 (measured, the grids and narrow keys here), by the walks up to 1.4e-6.
+    # Decays between neighbours that are all alike (grids) or all below a rounding of 1 (narrow keys), where the errors
+    # of a chain of products add up. Relative 2-norm: at most 31 products in a thread and 15 across waves, half of them
+    # on average, each off by up to 2^-25 to the same side: 7e-7; by factors rounded one by one and multiplied up
+    # through the scans 1.2e-6 to 6.1e-6 (measured, the grids and narrow keys here), by the walks up to 1.4e-6.
     from weighted_laplace_sum import weighted_laplace_sum
     P, D, C = 1, 4, 5
     print(f"repeating roundings {kind} n={n}", flush=True)
@@ -313,10 +318,11 @@ def test_laplace_keys_whose_roundings_repeat(dev, no_dense, n, kind):
     assert np.linalg.norm(u[0][idx[0]] - ou[0]) <= 1e-6 * np.linalg.norm(ou[0])
 
 
-@pytest.mark.parametrize("shape", [(1, 3, 63, 64, 2), (1, 3, 65, 127, 3), (2, 2, 4160, 4033, 5), (1, 2, 12352, 10000, 3)])
+@pytest.mark.parametrize("shape", [(1, 3, 63, 64, 2), (1, 3, 65, 127, 3), (2, 2, 4160, 4033, 5),
+                                   (1, 2, 12352, 10000, 3)])
 def test_columns_of_equal_and_padded_values(dev, no_dense, shape):
-    # whole and broken blocks of 64 rows (their words are shuffled within whole ones), all values of a feature equal, and a
-    # tail of keys that a mask made 0
+    # whole and broken blocks of 64 rows (their words are shuffled within whole ones), all values of a feature equal,
+    # and a tail of keys that a mask made 0
     P, D, N, M, C = shape
     from weighted_abs_sum import weighted_abs_sum_full
     from weighted_laplace_sum import weighted_laplace_sum
@@ -360,7 +366,8 @@ def test_the_measured_faster_route_is_taken(dev, op, shape, columns):
     print(f"route {op} {shape}", flush=True)
     g = torch.Generator(dev).manual_seed(1)
     q, k, v, gw = (torch.randn(s, generator=g, device=dev) for s in ((P, D, M), (P, D, N), (P, N, C), (P, M, C)))
-    call = {"abs": lambda: weighted_abs_sum_full(q, k, v, backend="cuda"), "laplace": lambda: weighted_laplace_sum(q, k, v),
+    call = {"abs": lambda: weighted_abs_sum_full(q, k, v, backend="cuda"),
+            "laplace": lambda: weighted_laplace_sum(q, k, v),
             "bwd": lambda: _ext.weighted_abs_sum_backward(q, k, v, gw),
             "sgn": lambda: weighted_sgn_sum(q, k, v, gw, backend="cuda"),
             "add_bump": lambda: layers.layer_forward("add_bump", q, k, v)}[op]

@@ -163,11 +163,12 @@ print("captured first")
 
 
 def test_first_call_of_a_process_captured():
-    # a process whose very first library call is captured: the columns' kernels raise their LDS limit on the way, which a
-    # capture must allow (a child process: nothing of the library may have run before)
+    # a process whose very first library call is captured: the columns' kernels raise their LDS limit on the way, which
+    # a capture must allow (a child process: nothing of the library may have run before)
     import os
     import subprocess
     import sys
     pkg = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "quasi-linear-kernel-attention_amd")
-    run = subprocess.run([sys.executable, "-c", FIRST_CALL.format(pkg=pkg)], capture_output=True, text=True, timeout=100)
+    run = subprocess.run([sys.executable, "-c", FIRST_CALL.format(pkg=pkg)], capture_output=True, text=True,
+                         timeout=100)
     assert run.returncode == 0 and "captured first" in run.stdout, run.stderr[-2000:]

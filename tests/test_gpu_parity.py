@@ -70,8 +70,9 @@ SHAPES = [
 
 @pytest.fixture(params=["auto", "walk", "columns"])
 def route(request, pin_route):
-    """auto: the library's size routing (dense kernels for short segments, columns for large calls); walk, columns: sort +
-    walk or sort + column sums at every size, so both stay covered on the short segments the routing sends elsewhere."""
+    """auto: the library's size routing (dense kernels for short segments, columns where they are faster); walk,
+    columns: sort + walk or sort + column sums at every size, so both stay covered on the segments the routing sends
+    elsewhere."""
     return pin_route(request.param)
 
 
@@ -491,8 +492,8 @@ def test_backward_with_workspace_above_a_2gib_address_boundary(dev):
 
 def test_fwd_keep_leaves_unsized_states_untouched(dev, pin_route):
     # Through the C ABI: where qlka_abs_keep_state_bytes is 0 (the merged backward, C <= 64, C % 4 == 0) the forward
-    # keeps the sorts only (*kept = 1) even when handed a states pointer, and writes nothing through it; at a width whose
-    # backward walks twice it fills a buffer of the stated size (*kept = 3).
+    # keeps the sorts only (*kept = 1) even when handed a states pointer, and writes nothing through it; at a width
+    # whose backward walks twice it fills a buffer of the stated size (*kept = 3).
     from qlka import _lib
     lib = _lib.load()
     pin_route("walk")
@@ -921,9 +922,9 @@ def test_largest_inputs_dense(dev):
 
 @pytest.mark.parametrize("forward,backward", [("columns", "walk"), ("walk", "columns"), ("columns", "columns")])
 def test_kept_sorts_across_routes(dev, pin_route, forward, backward):
-    # The two directions choose their routes apart, and the pins are process-wide: whatever the forward kept, the backward's
-    # gradients are right. By columns no range states are formed, so none are handed on (at C = 18, whose walking backward
-    # reads them).
+    # The two directions choose their routes apart, and the pins are process-wide: whatever the forward kept, the
+    # backward's gradients are right. By columns no range states are formed, so none are handed on (at C = 18, whose
+    # walking backward reads them).
     from weighted_abs_sum import _ext
     P, D, N, M, C = 2, 3, 1500, 1300, 18
     print(f"kept sorts, forward {forward}, backward {backward}", flush=True)

@@ -44,7 +44,8 @@ def _ops(q, k, v, g_w, g_u):
     return [w, u, aw, au, gq, gk, gv]
 
 
-@pytest.mark.parametrize("shape,route", [("grouped", "walk"), ("grouped", "columns"), ("sorted_q", "walk"), ("dense", "auto")])
+@pytest.mark.parametrize("shape,route", [("grouped", "walk"), ("grouped", "columns"), ("sorted_q", "walk"),
+                                         ("dense", "auto")])
 def test_threads_on_own_streams_match_one_thread(dev, shape, route, pin_route):
     P, D, N, M, C = SHAPES[shape]
     pin_route(route)
