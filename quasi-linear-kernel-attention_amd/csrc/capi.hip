@@ -727,15 +727,17 @@ size_t qlka_set_workspace_budget(size_t bytes) { return g_ws_budget.exchange(byt
 // ------------------------------------------------------------------------------------------------ laplace forward
 static WsSpec laplace_spec(int P, int D, int N, int M, int C) { return WsSpec{P, D, N, M, C, N, M, true}; }
 
-// one chunk of P p, by columns or by ranges
-static size_t laplace_ws(int P, int D, int N, int M, int C) {
-    return std::max(ws_bytes(laplace_spec(P, D, N, M, C)), col_bytes(1, P, D, N, M, C));
+// One chunk of P p of a call that may go by columns, or that walks. (As for every operator below: a workspace sized for
+// fewer p than the call's may hold the walk alone, which then runs.)
+static size_t laplace_ws(bool columns, int P, int D, int N, int M, int C) {
+    return std::max(ws_bytes(laplace_spec(P, D, N, M, C)), columns ? col_bytes(1, P, D, N, M, C) : 0);
 }
 
 size_t qlka_laplace_fwd_ws_bytes(int P, int D, int N, int M, int C) {
     if (P <= 0 || D <= 0 || N <= 0 || M <= 0 || C <= 0) return 0;
     if (dense_laplace_fwd(N, M)) return 0;        // the dense route takes no workspace
-    auto b1 = [&](int pc) { return laplace_ws(pc, D, N, M, C); };
+    const bool columns = col_fwd(COL_OP_LAPLACE, P, D, N, M, C);
+    auto b1 = [&](int pc) { return laplace_ws(columns, pc, D, N, M, C); };
     return plan_bytes(plan_chunks(P, g_ws_budget.load(std::memory_order_relaxed), pipelined(P, D, M), b1), b1);
 }
 
@@ -747,10 +749,11 @@ int qlka_laplace_fwd(const float* q, const float* k, const float* v, float* out_
     hipStream_t st = (hipStream_t)stream;
     if (dense_laplace_fwd(N, M))
         return hip_status(direct_fwd(1, q, k, v, out_w, out_u, P, D, N, M, C, st), "laplace direct sum");
-    auto b1 = [&](int pc) { return laplace_ws(pc, D, N, M, C); };
+    const bool columns = col_fwd(COL_OP_LAPLACE, P, D, N, M, C) && ws_bytes_given >= col_bytes(1, 1, D, N, M, C);
+    auto b1 = [&](int pc) { return ws_bytes(laplace_spec(pc, D, N, M, C)); };
     const Plan pl = plan_chunks(P, ws_bytes_given, pipelined(P, D, M), b1);
     if (int e = check_ws(ws, ws_bytes_given, plan_bytes(pl, b1))) return e;
-    if (col_fwd(COL_OP_LAPLACE, P, D, N, M, C))
+    if (columns)
         return run_columns(1, 1, q, k, v, nullptr, true, P, D, N, M, C, ws, ws_bytes_given, st, no_extra,
             [&](int p0, int np, ColWs& w, hipStream_t s) {
                 const size_t p = (size_t)p0;
@@ -799,14 +802,15 @@ static size_t abs_dense_ws(int P, int pc, int D, int N, int M, int C) {
     return dense_sign(P, N, M) ? 0 : align256(sort_scratch_need(abs_fwd_spec(pc, D, N, M, C, true)));
 }
 
-static size_t abs_fwd_ws(int P, int D, int N, int M, int C) {
-    return std::max(ws_bytes(abs_fwd_spec(P, D, N, M, C, true)), col_bytes(0, P, D, N, M, C));
+static size_t abs_fwd_ws(bool columns, int P, int D, int N, int M, int C) {
+    return std::max(ws_bytes(abs_fwd_spec(P, D, N, M, C, true)), columns ? col_bytes(0, P, D, N, M, C) : 0);
 }
 
 size_t qlka_abs_fwd_ws_bytes(int P, int D, int N, int M, int C) {
     if (P <= 0 || D <= 0 || N <= 0 || M <= 0 || C <= 0) return 0;
     if (dense_abs_fwd(N, M)) return budget_bytes(P, [&](int pc) { return abs_dense_ws(P, pc, D, N, M, C); });
-    auto b1 = [&](int pc) { return abs_fwd_ws(pc, D, N, M, C); };
+    const bool columns = col_fwd(COL_OP_ABS, P, D, N, M, C);
+    auto b1 = [&](int pc) { return abs_fwd_ws(columns, pc, D, N, M, C); };
     return plan_bytes(plan_chunks(P, g_ws_budget.load(std::memory_order_relaxed), pipelined(P, D, M), b1), b1);
 }
 
@@ -877,12 +881,13 @@ int abs_fwd_impl(const float* q, const float* k, const float* v, float* out_w, f
         return hip_status(direct_fwd(0, q, k, v, out_w, out_u, P, D, N, M, C, st), "abs direct sum");
     }
     // the workspace is sized for the _full op (an upper bound of the plain one), so one size serves both
-    auto b1 = [&](int pc) { return abs_fwd_ws(pc, D, N, M, C); };
+    auto b1 = [&](int pc) { return abs_fwd_ws(false, pc, D, N, M, C); };
     const Plan pl = plan_chunks(P, ws_bytes_given, pipelined(P, D, M), b1);
     if (int e = check_ws(ws, ws_bytes_given, plan_bytes(pl, b1))) return e;
     // By columns no range states are formed, so only the sorts are kept, where the backward is expected to need no
     // states; should it walk all the same (the routes can be pinned in between), it forms its own.
-    if (col_fwd(COL_OP_ABS, P, D, N, M, C) && (!keep_states || col_bwd(P, D, N, M, C))) {
+    if (col_fwd(COL_OP_ABS, P, D, N, M, C) && (!keep_states || col_bwd(P, D, N, M, C)) &&
+        ws_bytes_given >= col_bytes(0, 1, D, N, M, C)) {
         const int e = run_columns(0, 1, keep_sorts ? nullptr : q, k, v, nullptr, out_u != nullptr, P, D, N, M, C, ws,
                                   ws_bytes_given, st, no_extra,
             [&](int p0, int np, ColWs& w, hipStream_t s) {
@@ -1094,11 +1099,13 @@ static MbwWs mbw_carve(void* ws, int P, int D, int N, int M, int C) {
 size_t qlka_abs_bwd_ws_bytes(int P, int D, int N, int M, int C) {
     if (P <= 0 || D <= 0 || N <= 0 || M <= 0 || C <= 0) return 0;
     if (dense_sign(P, N, M)) return 0;            // the dense route takes no workspace
+    const bool columns = col_bwd(P, D, N, M, C);
+    auto col = [&](int pc) { return columns ? col_bwd_bytes(pc, D, N, M, C) : 0; };
     if (mbw_applies(C)) {
-        auto bm = [&](int pc) { return std::max(mbw_ws_bytes(pc, D, N, M, C), col_bwd_bytes(pc, D, N, M, C)); };
+        auto bm = [&](int pc) { return std::max(mbw_ws_bytes(pc, D, N, M, C), col(pc)); };
         return plan_bytes(plan_chunks(P, g_ws_budget.load(std::memory_order_relaxed), pipelined(P, D, N), bm), bm);
     }
-    auto b1 = [&](int pc) { return std::max(ws_bytes(abs_bwd_spec(pc, D, N, M, C)), col_bwd_bytes(pc, D, N, M, C)); };
+    auto b1 = [&](int pc) { return std::max(ws_bytes(abs_bwd_spec(pc, D, N, M, C)), col(pc)); };
     return plan_bytes(plan_chunks(P, g_ws_budget.load(std::memory_order_relaxed), pipelined(P, D, N), b1), b1);
 }
 
@@ -1170,8 +1177,7 @@ int abs_bwd_impl(const float* q, const float* k, const float* v, const float* g_
     hipStream_t st = (hipStream_t)stream;
     if (dense_sign(P, N, M))     // the walks' convention: a tie counts -1 in both gradients
         return dense_bwd(-1.f, q, k, v, g_w, g_u, grad_q, grad_k, grad_v, P, D, N, M, C, st);
-    if (col_bwd(P, D, N, M, C)) {
-        if (int e = check_ws(ws, ws_bytes_given, col_bwd_bytes(1, D, N, M, C))) return e;
+    if (col_bwd(P, D, N, M, C) && ws_bytes_given >= col_bwd_bytes(1, D, N, M, C)) {
         return run_bwd_columns(v, g_w, g_u, 2.f, grad_q, grad_k, grad_v, P, D, N, M, C, ws, ws_bytes_given, st,
             [&](int p0, int np, SortedWs& w, hipStream_t s) {
                 const size_t p = (size_t)p0;
@@ -1271,8 +1277,9 @@ static WsSpec sgn_spec(int P, int D, int N, int M, int C) { return WsSpec{P, D, 
 size_t qlka_sgn_fwd_ws_bytes(int P, int D, int N, int M, int C) {
     if (P <= 0 || D <= 0 || N <= 0 || M <= 0 || C <= 0) return 0;
     if (dense_sign(P, N, M)) return 0;            // the dense route takes no workspace
+    const bool columns = col_sgn(P, D, N, M, C);
     return budget_bytes(P, [&](int pc) {
-        return std::max(ws_bytes(sgn_spec(pc, D, N, M, C)), col_bwd_bytes(pc, D, N, M, C)); });
+        return std::max(ws_bytes(sgn_spec(pc, D, N, M, C)), columns ? col_bwd_bytes(pc, D, N, M, C) : 0); });
 }
 
 int qlka_sgn_fwd(const float* q, const float* k, const float* v, const float* g, float* out,
@@ -1283,7 +1290,7 @@ int qlka_sgn_fwd(const float* q, const float* k, const float* v, const float* g,
     hipStream_t st = (hipStream_t)stream;
     if (dense_sign(P, N, M))     // sgn(k - q) with a tie counted +1 == -(s(q - k) with a tie counted -1)
         return hip_status(direct_sign(true, q, k, g, v, nullptr, out, -1.f, -1.f, P, D, M, N, C, st), "dense sgn sum");
-    if (col_sgn(P, D, N, M, C))   // sgn(k - q) with a tie counted +1, as above: -grad_q
+    if (col_sgn(P, D, N, M, C) && ws_bytes_given >= col_bwd_bytes(1, D, N, M, C))   // sgn(k - q) with a tie counted +1, as above: -grad_q
         return run_bwd_columns(v, g, nullptr, -2.f, out, nullptr, nullptr, P, D, N, M, C, ws, ws_bytes_given, st,
             [&](int p0, int np, SortedWs& w, hipStream_t s) {
                 const size_t p = (size_t)p0;
@@ -1416,19 +1423,25 @@ static size_t layer_col_extra(int kind, int P, int D, int N, int M, int C) {
                                           : kind == LAYER_ADD_LAPLACE ? align256((size_t)P * D * N * 4) : 0);
 }
 
-static bool col_layer(int kind, int D, int N, int M) { return col_applies(kind == LAYER_ADD_BUMP ? 3 * D : D, N, M); }
+static bool col_layer(int kind, int P, int D, int N, int M, int C) {
+    const ColOp op = kind == LAYER_ADD_LAPLACE ? COL_OP_LAPLACE : kind == LAYER_ADD_BUMP ? COL_OP_BUMP : COL_OP_ABS;
+    return col_fwd(op, P, D, N, M, C);
+}
 
-// one chunk of P p, by columns or by ranges
-static size_t layer_ws(int kind, int P, int D, int N, int M, int C) {
-    const size_t ranges = layer_ws_bytes(kind, WsSpec{P, D, N, M, C, N, M, true});
-    if (!col_layer(kind, D, N, M)) return ranges;
-    return std::max(ranges, col_bytes(kind == LAYER_ADD_LAPLACE, P, D, N, M, C, kind == LAYER_ADD_BUMP ? 3 : 1) +
-                            layer_col_extra(kind, P, D, N, M, C));
+static size_t layer_col_ws(int kind, int P, int D, int N, int M, int C) {
+    return col_bytes(kind == LAYER_ADD_LAPLACE, P, D, N, M, C, kind == LAYER_ADD_BUMP ? 3 : 1) +
+           layer_col_extra(kind, P, D, N, M, C);
+}
+
+static size_t layer_ws(bool columns, int kind, int P, int D, int N, int M, int C) {
+    return std::max(layer_ws_bytes(kind, WsSpec{P, D, N, M, C, N, M, true}),
+                    columns ? layer_col_ws(kind, P, D, N, M, C) : 0);
 }
 
 size_t qlka_layer_fwd_ws_bytes(int kind, int P, int D, int N, int M, int C) {
     if (P <= 0 || D <= 0 || N <= 0 || M <= 0 || C <= 0 || kind < 0 || kind > 2) return 0;
-    auto b1 = [&](int pc) { return layer_ws(kind, pc, D, N, M, C); };
+    const bool columns = col_layer(kind, P, D, N, M, C);
+    auto b1 = [&](int pc) { return layer_ws(columns, kind, pc, D, N, M, C); };
     const size_t cap = g_ws_budget.load(std::memory_order_relaxed);
     return plan_bytes(plan_chunks(P, cap, layer_pipelined(kind, P, D, M, C), b1), b1);
 }
@@ -1530,7 +1543,7 @@ static int layer_fwd(int kind, const float* q, const float* k, const float* v, c
     if (kind < 0 || kind > 2) return fail(QLKA_EINVAL, "kind must be 0 (add_laplace), 1 (add_riesz) or 2 (add_bump)");
     if (int e = check_dims(P, D, N, M, C)) return e;
     if (!q || !k || !v || !out) return fail(QLKA_EINVAL, "q, k, v and out must be non-null");
-    auto b1 = [&](int pc) { return layer_ws(kind, pc, D, N, M, C); };
+    auto b1 = [&](int pc) { return layer_ws(false, kind, pc, D, N, M, C); };
     const Plan pl = plan_chunks(P, ws_bytes_given, layer_pipelined(kind, P, D, M, C), b1);
     if (int e = check_ws(ws, ws_bytes_given, plan_bytes(pl, b1))) return e;
     hipStream_t st = (hipStream_t)stream;
@@ -1541,8 +1554,7 @@ static int layer_fwd(int kind, const float* q, const float* k, const float* v, c
         npc = n_pad ? n_pad + p : nullptr; keepc = keep ? keep + p * N : nullptr; outc = out + p * M * C;
     };
     const bool bump = kind == LAYER_ADD_BUMP;
-    const ColOp op = kind == LAYER_ADD_LAPLACE ? COL_OP_LAPLACE : bump ? COL_OP_BUMP : COL_OP_ABS;
-    const bool columns = col_fwd(op, P, D, N, M, C);
+    const bool columns = col_layer(kind, P, D, N, M, C) && ws_bytes_given >= layer_col_ws(kind, 1, D, N, M, C);
     if (columns && !(kind == LAYER_ADD_RIESZ && keep == nullptr && few_keys(N)))
         return layer_columns(kind, q, k, v, n_pad, keep, out, P, D, N, M, C, ws, ws_bytes_given, st);
     if (kind == LAYER_ADD_RIESZ && keep == nullptr && few_keys(N))   // the abs sums dense (few_keys), then the epilogue
@@ -1731,6 +1743,6 @@ int validate_dims(int P, int D, int N, int M, int C) {
     g_err.clear();
     return check_dims(P, D, N, M, C);
 }
-size_t laplace_fwd_chunk_ws(int pc, int D, int N, int M, int C) { return laplace_ws(pc, D, N, M, C); }
+size_t laplace_fwd_chunk_ws(int pc, int D, int N, int M, int C) { return laplace_ws(false, pc, D, N, M, C); }
 int report_error(int code, const char* msg) { return fail(code, "%s", msg); }
 }  // namespace qlka

@@ -181,9 +181,28 @@ def test_direct_cutoff_setter(lib):
 
 def test_workspace_of_one_channel_is_not_larger_than_of_two(lib):
     # the columns' shape depends on N + M alone (one channel once took 10240 elements for any short segment)
-    for N, M in ((600, 20), (20, 600), (700, 700), (9000, 9000)):
-        for fn in (lib.qlka_laplace_fwd_ws_bytes, lib.qlka_abs_fwd_ws_bytes, lib.qlka_abs_bwd_ws_bytes):
-            assert fn(4, 64, N, M, 1) <= fn(4, 64, N, M, 2)
+    prev = lib.qlka_set_columns(2)
+    try:
+        for N, M in ((600, 20), (20, 600), (700, 700), (9000, 9000)):
+            for fn in (lib.qlka_laplace_fwd_ws_bytes, lib.qlka_abs_fwd_ws_bytes, lib.qlka_abs_bwd_ws_bytes):
+                assert fn(4, 64, N, M, 1) <= fn(4, 64, N, M, 2)
+    finally:
+        lib.qlka_set_columns(prev)
+
+
+def test_a_walking_call_asks_for_its_walks_workspace(lib):
+    # calls whose walk was measured faster by far: the columns' workspace, up to 3 x the walk's here, is not counted
+    fns = {"laplace": lib.qlka_laplace_fwd_ws_bytes, "abs": lib.qlka_abs_fwd_ws_bytes, "bwd": lib.qlka_abs_bwd_ws_bytes,
+           "sgn": lib.qlka_sgn_fwd_ws_bytes, "add_riesz": lambda *s: lib.qlka_layer_fwd_ws_bytes(1, *s)}
+    for name, shape in (("laplace", (256, 1, 4000, 4000, 64)), ("abs", (256, 1, 4000, 4000, 64)),
+                        ("bwd", (256, 1, 4000, 4000, 64)), ("sgn", (12, 64, 16384, 16384, 64)),
+                        ("add_riesz", (256, 1, 4000, 4000, 64))):
+        auto = fns[name](*shape)
+        prev = lib.qlka_set_columns(1)
+        try:
+            assert auto == fns[name](*shape), name
+        finally:
+            lib.qlka_set_columns(prev)
 
 
 def test_column_mode_setter(lib):

@@ -70,6 +70,20 @@ def test_noalloc_equals_laplace_fwd(dev):
         del q, k, v, w, u, want_w, want_u
 
 
+def test_noalloc_takes_a_shape_whose_walk_alone_fits_its_scratch(dev):
+    """One p of 30000 keys and 600 queries in 580 features: the walk's workspace fits the static scratch, the columns' does
+    not (many more keys than queries); the call walks."""
+    P, D, N, M, C = 1, 580, 30000, 600, 4
+    print(f"noalloc P={P} D={D} N={N} M={M} C={C}", flush=True)
+    q, k, v = _inputs(P, D, N, M, C, 4, dev)
+    w, u = _call(_noalloc(), q, k, v)
+    qn, kn, vn = (t.cpu().numpy() for t in (q, k, v))
+    idx = np.array([[0, 7, 300, 599]])
+    ow, ou, nw = brute.laplace_sum(qn, kn, vn, qidx=idx)
+    assert float(brute.rel_err(w.cpu().numpy()[:, idx[0]], ow, nw).max()) <= 1e-5
+    assert float(brute.rel_err(u.cpu().numpy()[:, idx[0]], ou, ou).max()) <= 1e-5
+
+
 def test_noalloc_refuses_shapes_beyond_its_scratch(dev):
     """One p at N = M = 131072, D = C = 64 needs more than the static scratch: refused on the host with a message."""
     from qlka import _lib
