@@ -38,7 +38,7 @@ int hip_status(int e, const char* where) {
 inline size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 // Where the dense evaluation (direct.hip) beats sort + scans + walk + reduce, whose cost at short segments is launch
-// and per-segment overhead. With B = the base cutoff (qlka_set_direct_max, default 512; 0: always sort + walk) and
+// and per-segment overhead. With B = the base cutoff (qlka_set_direct_max, default 512; 0: none of them) and
 // L = max(N, M), measured on MI355X (P = 12, 32, 48, 512; D, C = 32, 64):
 //   abs forward      L <= 2B   (dense 0.28 vs walk 0.51 ms at L = 1024, P = 48)
 //   Laplace forward  L <= B    (its exp per term: about even at L = 700 for P = 12)
